@@ -275,11 +275,12 @@ def tolerance(case):
     """About four times the distance between the 32-bit (bf16) results and the same path in 64
     bits: the longest sums (weight gradients over a million pixels) are off by 1.4e-6 in 2-norm
     and 7e-6 at most, pooled and resampled sums of up to some tens of terms by 8e-8 and 6e-7,
-    bf16 results by 2.4e-3 and 1.3e-2 (their own rounding is 1.65e-3).  Whole numbers are
-    equal."""
+    bf16 results by 2.4e-3 and 1.3e-2 (their own rounding is 1.65e-3).  64-bit sums taken in
+    another order differ by 2e-15, but the bias gradient of a single output channel is one sum of
+    up to a million terms of both signs: 2e-14 of its value seen.  Whole numbers are equal."""
     if case["kind"] == "knn":
         return "exact"  # the order of a distance's three terms is fixed, ties go by index
     if case["kind"] in ("pool", "resample"):
         return {"rel": 4e-7, "max": 3e-6}
     return {"bf16": {"rel": 1e-2, "max": 0.05}, "fp32": {"rel": 5e-6, "max": 3e-5},
-            "fp64": {"rel": 4e-15, "max": 4e-14}}[case["dtype"]]
+            "fp64": {"rel": 2e-13, "max": 2e-13}}[case["dtype"]]
