@@ -284,3 +284,108 @@ def tolerance(case):
         return {"rel": 4e-7, "max": 3e-6}
     return {"bf16": {"rel": 1e-2, "max": 0.05}, "fp32": {"rel": 5e-6, "max": 3e-5},
             "fp64": {"rel": 2e-13, "max": 2e-13}}[case["dtype"]]
+
+
+# ------------------------------------------------------------------- the same in 64 bits
+def _corners(smap, weights, H, W, interp):
+    """[N, K, corners] element offsets and weights of a map's taps, in 64 bits."""
+    x, y = smap.double().unbind(-1)
+    if interp == "nearest":
+        half = [torch.trunc(v) + torch.where((v - torch.trunc(v)).abs() >= 0.5, v.sign(), 0 * v)
+                for v in (x, y)]
+        cols, rows, wts = [half[0]], [half[1]], [torch.ones_like(x)]
+    else:
+        x1, y1 = x.floor(), y.floor()
+        cols, rows = [x1, x1 + 1] * 2, [y1, y1, y1 + 1, y1 + 1]
+        A, B, C, D = y1 + 1 - y, x1 + 1 - x, x - x1, y - y1
+        wts = [A * B, A * C, D * B, D * C]
+        if interp == "bispherical":
+            cols = [c % W for c in cols]
+    off, wt = [], []
+    for c, r, a in zip(cols, rows, wts):
+        inside = (c >= 0) & (c < W) & (r >= 0) & (r < H)
+        off.append(torch.where(inside, r * W + c, 0 * c).long())
+        wt.append(torch.where(inside, a if weights is None else a * weights.double(), 0 * a))
+    off, wt = torch.stack(off, -1), torch.stack(wt, -1)
+    if weights is not None:  # [..., P, corners]: all of them belong to the same tap
+        off, wt = off.flatten(-2), wt.flatten(-2)
+    n = smap.shape[0] * smap.shape[1]
+    return off.reshape(n, -1, off.shape[-1]), wt.reshape(n, -1, off.shape[-1])
+
+
+def _gather(plane, off, wt):
+    """[C, N] samples of [C, HW] planes at [N, corners]."""
+    return sum(plane[:, off[:, i]] * wt[:, i] for i in range(off.shape[1]))
+
+
+def _scatter(plane, values, off, wt):
+    for i in range(off.shape[1]):
+        plane.index_add_(1, off[:, i], values * wt[:, i])
+
+
+def exact(case, seed):
+    if case["kind"] == "knn" or work(case)["flops"] > 2e12:
+        return None  # whole numbers beside distances of fixed order; over 20 seconds
+    s = prepare(case, seed)
+    kind, train, smap = case["kind"], s["train"], s["args"][0]
+    weights, (H, W) = None, s["x"].shape[2:]
+    x = s["x"].detach().double().flatten(2)
+    gy = s["gy"].double().flatten(2) if train else [None] * len(x)
+    if kind == "tconv":
+        H, W, smap = s["args"]
+    elif kind == "mesh":
+        weights = s["args"][1]
+    elif case.get("op") == "resample":
+        H, W = s["args"][1]
+    off, wt = _corners(smap, weights, H, W, case.get("interp", "nearest"))
+    taps = range(off.shape[1])
+    plane = lambda c: torch.zeros(c, H * W, dtype=torch.float64, device="cuda")
+    if kind in ("pool", "resample"):
+        y, gx = [], []
+        for xb, gb in zip(x, gy):
+            if case.get("op") == "resample":
+                y.append(plane(len(xb)))
+                _scatter(y[-1], xb, off[:, 0], wt[:, 0])
+                gx.append(_gather(gb, off[:, 0], wt[:, 0]))
+                continue
+            cols = (_gather(xb, off[:, k], wt[:, k]) for k in taps)
+            if case.get("op") == "max":
+                best = next(cols)
+                for c in cols:
+                    best = torch.maximum(best, c)
+                y.append(best)
+                continue
+            y.append(sum(cols) / len(taps))
+            gx.append(plane(len(xb)))
+            for k in taps:
+                _scatter(gx[-1], gb / len(taps), off[:, k], wt[:, k])
+        shape = s["gy"].shape
+        y = torch.stack(y).view(shape)
+        # which of two taps within rounding of each other wins is not a matter of precision
+        return (y, None, None) if case.get("op") == "max" else \
+            (y, torch.stack(gx).view(s["x"].shape))
+    w, bias = (p.detach().double() for p in s["params"])
+    y, gx, gw = [], [], torch.zeros_like(w)
+    for xb, gb in zip(x, gy):
+        if kind == "tconv":
+            y.append(plane(w.shape[1]) + bias[:, None])
+            gx.append(torch.zeros_like(xb))
+            for k in taps:
+                _scatter(y[-1], w[:, :, k].t() @ xb, off[:, k], wt[:, k])
+                if train:
+                    col = _gather(gb, off[:, k], wt[:, k])
+                    gx[-1] += w[:, :, k] @ col
+                    gw[:, :, k] += xb @ col.t()
+            continue
+        y.append(bias[:, None].repeat(1, len(off)))
+        gx.append(plane(len(xb)))
+        for k in taps:
+            col = _gather(xb, off[:, k], wt[:, k])
+            y[-1] += w[:, :, k] @ col
+            if train:
+                gw[:, :, k] += gb @ col.t()
+                _scatter(gx[-1], w[:, :, k].t() @ gb, off[:, k], wt[:, k])
+    y = torch.stack(y)
+    if not train:
+        return y.view(len(y), y.shape[1], *((H, W) if kind == "tconv" else smap.shape[:2]))
+    return (y.view(s["gy"].shape), torch.stack(gx).view(s["x"].shape), gw, gy.sum((0, 2)))
