@@ -23,6 +23,23 @@ template <typename T>
 int generic_weight_grad(const T *plain, const T *gath, const T *map, const T *iw, T *gw,
                         int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t N,
                         int64_t K, int64_t P, int interp, hipStream_t s);
+// ---- fp64 over channel-last records (mcx_conv_records.hip); ws: the *_bytes of the product ----
+bool records_supported(int64_t B, int64_t C1, int64_t C2, int64_t K);
+size_t records_gather_bytes(int64_t B, int64_t G, int64_t SN);
+int records_gather_product(const double *src, const double *map, const double *iw, const double *w,
+                           const double *bias, double *y, void *ws, int64_t B, int64_t G,
+                           int64_t O, int64_t SH, int64_t SW, int64_t N, int64_t K, int64_t P,
+                           int interp, hipStream_t s);
+size_t records_scatter_bytes(int64_t B, int64_t D, int64_t DN);
+int records_product_scatter(const double *src, const double *map, const double *iw,
+                            const double *w, const double *bias, double *dst, void *ws, int64_t B,
+                            int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,
+                            int64_t P, int interp, hipStream_t s);
+size_t records_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t GN, int64_t N, int64_t K);
+int records_weight_grad(const double *plain, const double *gath, const double *map,
+                        const double *iw, double *gw, void *ws, int64_t B, int64_t A, int64_t G,
+                        int64_t GH, int64_t GW, int64_t N, int64_t K, int64_t P, int interp,
+                        hipStream_t s);
 // scratch: channel_sum_scratch_bytes(...) bytes, or NULL for the single-kernel form.
 size_t channel_sum_scratch_bytes(int64_t B, int64_t C, int64_t N, size_t elem);
 template <typename T>

@@ -2,8 +2,8 @@
 // arguments, then routes each of the three products (gather-product,
 // product-scatter, weight gradient; see mcx_conv_generic.hip for the roles) to the
 // matrix-core kernels when they cover the case (fp32 and bf16 storage, at most 4
-// interpolation points per tap) and to the scalar kernels otherwise (fp64, or fp32
-// with more points).
+// interpolation points per tap), to the record kernels for fp64 with a workspace, and to
+// the scalar kernels otherwise.
 #include <algorithm>
 #include <initializer_list>
 #include <mutex>
@@ -99,18 +99,27 @@ int fill_zero<double>(double *p, int64_t n, hipStream_t s) { return fill_f64(p, 
 
 // ---- scratch sizes of the three operators -------------------------------------------
 // SH x SW: the image sampled; MH x MW: the map
+// (fp64 runs over channel-last records where the caller's scratch holds them, and on the scalar
+// kernels where it does not)
 size_t gather_product_ws(int dtype, int64_t G, int64_t O, int64_t K, int64_t P, int64_t B,
                          int64_t SH, int64_t SW, int64_t MH, int64_t MW) {
+  if (dtype == MCX_F64)
+    return records_supported(B, G, O, K) ? records_gather_bytes(B, G, SH * SW) : 0;
   return use_mfma(dtype, P)
              ? mfma_gather_product_bytes(O, G, K, B, SH, SW, (int)elem_size(dtype), MH, MW)
              : 0;
 }
 size_t weight_grad_ws(int dtype, int64_t B, int64_t A, int64_t G, int64_t MH, int64_t MW,
                       int64_t K, int64_t P, int64_t GH, int64_t GW) {
+  if (dtype == MCX_F64)
+    return records_supported(B, A, G, K)
+               ? records_weight_grad_bytes(B, A, G, GH * GW, MH * MW, K)
+               : 0;
   return use_mfma(dtype, P) ? mfma_weight_grad_bytes(B, A, G, MH, MW, K, GH, GW, elem_size(dtype)) : 0;
 }
 size_t product_scatter_ws(int dtype, int64_t B, int64_t S, int64_t D, int64_t K, int64_t P,
                           int64_t DH, int64_t DW, int64_t MH, int64_t MW) {
+  if (dtype == MCX_F64) return records_supported(B, S, D, K) ? records_scatter_bytes(B, D, DH * DW) : 0;
   return use_mfma(dtype, P)
              ? mfma_product_scatter_bytes(B, S, D, K, DH, DW, elem_size(dtype), MH, MW, P)
              : 0;
@@ -148,47 +157,64 @@ template <typename T>
 int bias_grad(const void *gy, void *gb, void *ws, size_t ws_bytes, int64_t B, int64_t C, int64_t N,
               hipStream_t s);
 
-#define MCX_SCALAR_OPS(T)                                                                          \
-  template <>                                                                                      \
-  int gather_product<T>(bool, const void *src, const void *map, const void *iw, const void *w,     \
-                        const void *bias, void *y, void *, size_t, int64_t B, int64_t G,           \
-                        int64_t O, int64_t SH, int64_t SW, int64_t MH, int64_t MW, int64_t K,      \
-                        int64_t P, int interp, hipStream_t s, const void *) {                      \
-    return generic_gather_product<T>((const T *)src, (const T *)map, (const T *)iw,                \
-                                     (const T *)w, (const T *)bias, (T *)y, B, G, O, SH, SW,       \
-                                     MH * MW, K, P, interp, s);                                    \
-  }                                                                                                \
-  template <>                                                                                      \
-  int product_scatter<T>(bool, const void *src, const void *map, const void *iw, const void *w,    \
-                         const void *bias, void *dst, void *, size_t, int64_t B, int64_t S,        \
-                         int64_t D, int64_t DH, int64_t DW, int64_t MH, int64_t MW, int64_t K,     \
-                         int64_t P, int interp, hipStream_t s, const void *) {                     \
-    int rc = bias ? fill_bias<T>((T *)dst, (const T *)bias, B, D, DH * DW, s)                      \
-                  : fill_zero<T>((T *)dst, B * D * DH * DW, s);                                    \
-    if (rc) return rc;                                                                             \
-    return generic_product_scatter<T>((const T *)src, (const T *)map, (const T *)iw,               \
-                                      (const T *)w, (T *)dst, B, S, D, DH, DW, MH * MW, K, P,      \
-                                      interp, s);                                                  \
-  }                                                                                                \
-  template <>                                                                                      \
-  int weight_grad<T>(bool, const void *plain, const void *gath, const void *map, const void *iw,   \
-                     void *gw, void *, size_t, int64_t B, int64_t A, int64_t G, int64_t GH,        \
-                     int64_t GW, int64_t MH, int64_t MW, int64_t K, int64_t P, int interp,         \
-                     hipStream_t s, void *, const void *) {                                        \
-    return generic_weight_grad<T>((const T *)plain, (const T *)gath, (const T *)map,               \
-                                  (const T *)iw, (T *)gw, B, A, G, GH, GW, MH * MW, K, P, interp,  \
-                                  s);                                                              \
-  }                                                                                                \
-  template <>                                                                                      \
-  int bias_grad<T>(const void *gy, void *gb, void *ws, size_t ws_bytes, int64_t B, int64_t C,      \
-                   int64_t N, hipStream_t s) {                                                     \
-    const size_t need = channel_sum_scratch_bytes(B, C, N, sizeof(T));                             \
-    T *scratch = (ws && need > 0 && ws_bytes >= need) ? (T *)ws : nullptr;                         \
-    return channel_sum<T>((const T *)gy, (T *)gb, scratch, B, C, N, s);                            \
-  }
+// double: records where there is scratch for them, scalar kernels otherwise
 
-// double: scalar kernels only
-MCX_SCALAR_OPS(double)
+template <>
+int gather_product<double>(bool, const void *src, const void *map, const void *iw, const void *w,
+                           const void *bias, void *y, void *ws, size_t ws_bytes, int64_t B,
+                           int64_t G, int64_t O, int64_t SH, int64_t SW, int64_t MH, int64_t MW,
+                           int64_t K, int64_t P, int interp, hipStream_t s, const void *) {
+  const size_t need = gather_product_ws(MCX_F64, G, O, K, P, B, SH, SW, MH, MW);
+  if (ws && need > 0 && ws_bytes >= need)
+    return records_gather_product((const double *)src, (const double *)map, (const double *)iw,
+                                  (const double *)w, (const double *)bias, (double *)y, ws, B, G,
+                                  O, SH, SW, MH * MW, K, P, interp, s);
+  return generic_gather_product<double>((const double *)src, (const double *)map,
+                                        (const double *)iw, (const double *)w,
+                                        (const double *)bias, (double *)y, B, G, O, SH, SW,
+                                        MH * MW, K, P, interp, s);
+}
+
+template <>
+int product_scatter<double>(bool, const void *src, const void *map, const void *iw, const void *w,
+                            const void *bias, void *dst, void *ws, size_t ws_bytes, int64_t B,
+                            int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t MH, int64_t MW,
+                            int64_t K, int64_t P, int interp, hipStream_t s, const void *) {
+  const size_t need = product_scatter_ws(MCX_F64, B, S, D, K, P, DH, DW, MH, MW);
+  if (ws && need > 0 && ws_bytes >= need)
+    return records_product_scatter((const double *)src, (const double *)map, (const double *)iw,
+                                   (const double *)w, (const double *)bias, (double *)dst, ws, B,
+                                   S, D, DH, DW, MH * MW, K, P, interp, s);
+  int rc = bias ? fill_bias<double>((double *)dst, (const double *)bias, B, D, DH * DW, s)
+                : fill_zero<double>((double *)dst, B * D * DH * DW, s);
+  if (rc) return rc;
+  return generic_product_scatter<double>((const double *)src, (const double *)map,
+                                         (const double *)iw, (const double *)w, (double *)dst, B,
+                                         S, D, DH, DW, MH * MW, K, P, interp, s);
+}
+
+template <>
+int weight_grad<double>(bool, const void *plain, const void *gath, const void *map, const void *iw,
+                        void *gw, void *ws, size_t ws_bytes, int64_t B, int64_t A, int64_t G,
+                        int64_t GH, int64_t GW, int64_t MH, int64_t MW, int64_t K, int64_t P,
+                        int interp, hipStream_t s, void *, const void *) {
+  const size_t need = weight_grad_ws(MCX_F64, B, A, G, MH, MW, K, P, GH, GW);
+  if (ws && need > 0 && ws_bytes >= need)
+    return records_weight_grad((const double *)plain, (const double *)gath, (const double *)map,
+                               (const double *)iw, (double *)gw, ws, B, A, G, GH, GW, MH * MW, K,
+                               P, interp, s);
+  return generic_weight_grad<double>((const double *)plain, (const double *)gath,
+                                     (const double *)map, (const double *)iw, (double *)gw, B, A,
+                                     G, GH, GW, MH * MW, K, P, interp, s);
+}
+
+template <>
+int bias_grad<double>(const void *gy, void *gb, void *ws, size_t ws_bytes, int64_t B, int64_t C,
+                      int64_t N, hipStream_t s) {
+  const size_t need = channel_sum_scratch_bytes(B, C, N, sizeof(double));
+  double *scratch = (ws && need > 0 && ws_bytes >= need) ? (double *)ws : nullptr;
+  return channel_sum<double>((const double *)gy, (double *)gb, scratch, B, C, N, s);
+}
 
 // float: matrix-core kernels when `mfma`, scalar kernels otherwise
 
@@ -399,7 +425,9 @@ extern "C" int mcx_conv_forward_static(const void *x, const void *map, const voi
   if (int rc = check_ptrs(x, map, iw, w, P)) return rc;
   if (!bias || !y) return MCX_E_NULL;
   if (dtype != MCX_F32 && dtype != MCX_F64 && dtype != MCX_BF16) return MCX_E_DTYPE;
-  const size_t need = gather_product_ws(dtype, Ci, Co, K, P, B, IH, IW, OH, OW);
+  // (fp64 can do without scratch)
+  const size_t need =
+      dtype == MCX_F64 ? 0 : gather_product_ws(dtype, Ci, Co, K, P, B, IH, IW, OH, OW);
   if (need > kStaticScratchBytes) return MCX_E_STATIC_LIMIT;
   int rc = 0;
   void *ws = static_scratch_of_current_device(&rc);

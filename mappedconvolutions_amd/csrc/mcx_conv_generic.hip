@@ -244,7 +244,9 @@ int generic_weight_grad(const T *plain, const T *gath, const T *map, const T *iw
 }
 
 int channel_sum_splits(int64_t B, int64_t C, int64_t N) {
-  if (B * C * N < (1 << 20) || B > 65535) return 0;  // small: one kernel, no scratch
+  // One kernel (no scratch) while a channel is a few thousand values: its single workgroup
+  // adds about one value a nanosecond (100 000 values of one channel: 95 us, in two stages 13).
+  if (B * N < (1 << 14) || B > 65535) return 0;
   int splits = 1;
   while (B * C * splits < 2048 && N / (splits * 2) >= 4096 && splits < 64) splits *= 2;
   return splits;

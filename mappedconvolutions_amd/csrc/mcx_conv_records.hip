@@ -1,0 +1,546 @@
+// fp64 form of the three products (gather-product, product-scatter, weight gradient; roles in
+// mcx_conv_generic.hip) over channel-last records.  In the planar layout every corner of every
+// tap of every channel is an 8-byte access in a cache line of its own; a record holds all
+// channels of a pixel side by side, so a corner is one run of lines that LPR neighbouring
+// lanes read (or add to) together.  The operand that the map reaches is copied into records
+// in the caller's workspace (the scattered destination: accumulated there and copied back);
+// without a workspace the scalar kernels run.  All arithmetic is fp64 on the vector units: the
+// fp64 matrix instructions have the same rate here.
+// Bound: random record reads and fp64 atomics.  Measured at one image of 200x500 pixels, 10 -> 1
+// channels, nine taps of a shuffled map (scalar kernels -> these): forward
+// 210 -> 36 us (7 of them the copy), input gradient 1585 -> 375 us (the atomics: 36 M of them
+// as 3.6 M records; 2 x 8 lanes per record of 10 channels 385), weight gradient 579 -> 70 us.
+#include <algorithm>
+
+#include "mcx_conv.h"
+#include "mcx_device.h"
+
+namespace mcx {
+namespace {
+
+constexpr int kThreads = 256;
+
+// Lanes per record.  A reading lane handles two channels, so a pass covers 2 * LPR; a lane that
+// adds handles one.
+template <int LPR>
+struct RecShape {
+  static constexpr int kLocs = kThreads / LPR;  // map locations per workgroup
+  static constexpr int kCh = 2 * LPR;           // channels per pass
+  // taps resolved per pass (their cache is what limits the workgroups per CU)
+  static constexpr int kTaps = LPR == 2 ? 5 : 9;
+};
+
+// Record stride in doubles: 16-byte pairs for reading.
+inline int64_t read_stride(int64_t channels) { return (channels + 1) & ~(int64_t)1; }
+// Records that atomics add to: up to 16 channels a power of two, so that a run of eight
+// channels, one request of 64 bytes, never straddles a boundary.
+inline int64_t add_stride(int64_t channels) {
+  for (int64_t s = 2; s <= 16; s *= 2)
+    if (channels <= s) return s;
+  return (channels + 7) & ~(int64_t)7;
+}
+inline int lanes_per_record(int64_t channels) { return channels <= 4 ? 2 : channels <= 8 ? 4 : 8; }
+
+// [B][C][N] -> records [B][N + 1][stride]; the last record of an image is all zeros (what a
+// corner outside the image reads), as are the channels beyond C.
+__global__ __launch_bounds__(kThreads) void to_records_kernel(const double *__restrict__ x,
+                                                              double *__restrict__ rec, int C,
+                                                              int stride, int64_t N) {
+  const int64_t n = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int b = blockIdx.z;
+  if (n > N) return;
+  const double *src = x + (int64_t)b * C * N + (n < N ? n : 0);
+  double2 *dst = reinterpret_cast<double2 *>(rec + ((int64_t)b * (N + 1) + n) * stride);
+  const int c_end = min(stride, (int)(blockIdx.y + 1) * 16);
+  for (int c = blockIdx.y * 16; c < c_end; c += 2) {
+    double2 v = make_double2(0.0, 0.0);
+    if (n < N) {
+      if (c < C) v.x = src[(int64_t)c * N];
+      if (c + 1 < C) v.y = src[(int64_t)(c + 1) * N];
+    }
+    dst[c >> 1] = v;
+  }
+}
+
+// records [B][N][stride] -> [B][C][N], plus bias
+__global__ __launch_bounds__(kThreads) void from_records_kernel(const double *__restrict__ rec,
+                                                                const double *__restrict__ bias,
+                                                                double *__restrict__ y, int C,
+                                                                int stride, int64_t N) {
+  const int64_t n = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int b = blockIdx.z;
+  if (n >= N) return;
+  const double2 *src = reinterpret_cast<const double2 *>(rec + ((int64_t)b * N + n) * stride);
+  double *dst = y + (int64_t)b * C * N + n;
+  const int c_end = min(C, (int)(blockIdx.y + 1) * 16);
+  for (int c = blockIdx.y * 16; c < c_end; c += 2) {
+    const double2 v = src[c >> 1];
+    dst[(int64_t)c * N] = v.x + (bias ? bias[c] : 0.0);
+    if (c + 1 < C) dst[(int64_t)(c + 1) * N] = v.y + (bias ? bias[c + 1] : 0.0);
+  }
+}
+
+// Tap (n, k) of interpolation point p as NC (record index, weight) pairs; a corner outside the
+// image, or of weight zero, gets the index `none`.
+template <int NC>
+__device__ inline void resolve_records(const double *__restrict__ map,
+                                       const double *__restrict__ iw, int64_t e, int h, int w,
+                                       bool wrap, int none, int *off, double *wt, int step) {
+  const double x = map[e * 2], y = map[e * 2 + 1];
+  const double scale = iw ? iw[e] : 1.0;
+  if constexpr (NC == 1) {
+    Tap<double, kInterpNearest> t;
+    t.set(x, y, h, w);
+    off[0] = t.off < 0 ? none : t.off;
+    wt[0] = scale;
+  } else {
+    auto put = [&](const auto &t) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        off[i * step] = t.off[i] < 0 ? none : t.off[i];
+        wt[i * step] = t.wt[i] * scale;
+      }
+    };
+    if (wrap) {
+      Tap<double, kInterpBispherical> t;
+      t.set(x, y, h, w);
+      put(t);
+    } else {
+      Tap<double, kInterpBilinear> t;
+      t.set(x, y, h, w);
+      put(t);
+    }
+  }
+}
+
+// The taps [k0, k0 + taps) of a workgroup's locations into its cache, [corner][tap][location].
+template <int NC, int LPR>
+__device__ inline void fill_tap_cache(const double *__restrict__ map,
+                                      const double *__restrict__ iw, int n0, int N, int K, int pm,
+                                      int p, int k0, int taps, int h, int w, bool wrap, int none,
+                                      int *s_off, double *s_wt) {
+  using S = RecShape<LPR>;
+  constexpr int kStep = S::kTaps * S::kLocs;
+  for (int e = threadIdx.x; e < taps * S::kLocs; e += kThreads) {
+    const int l = e / taps, t = e - l * taps;
+    const int slot = t * S::kLocs + l;
+    if (n0 + l < N) {
+      resolve_records<NC>(map, iw, ((int64_t)(n0 + l) * K + k0 + t) * pm + p, h, w, wrap, none,
+                          s_off + slot, s_wt + slot, kStep);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NC; i++) {
+        s_off[i * kStep + slot] = none;
+        s_wt[i * kStep + slot] = 0.0;
+      }
+    }
+  }
+}
+
+// y[b,o,n] = bias[o] + sum_{g,k} W[o,g,k] * sample(src[b,g], map[n,k]).  A location belongs to
+// LPR lanes; every lane sums its two channels into OT outputs, the lanes' sums are added at
+// the end.  Taps and the weights of a pass sit in LDS.
+template <int NC, int LPR, int OT>
+__global__ __launch_bounds__(kThreads) void gather_records_kernel(
+    const double *__restrict__ rec, const double *__restrict__ map, const double *__restrict__ iw,
+    const double *__restrict__ w, const double *__restrict__ bias, double *__restrict__ y, int G,
+    int stride, int O, int SH, int SW, int N, int K, int P, int wrap) {
+  using S = RecShape<LPR>;
+  constexpr int kStep = S::kTaps * S::kLocs;
+  __shared__ int s_off[NC * kStep];
+  __shared__ double s_wt[NC * kStep];
+  __shared__ double2 s_w[S::kTaps * OT * LPR];
+  const int loc = threadIdx.x / LPR, j = threadIdx.x % LPR;
+  const int n0 = blockIdx.x * S::kLocs, o0 = blockIdx.y * OT, b = blockIdx.z;
+  const int64_t SN = (int64_t)SH * SW;
+  const double *recb = rec + (int64_t)b * (SN + 1) * stride;
+  const int pm = P == 0 ? 1 : P;
+  double acc[OT];
+#pragma unroll
+  for (int o = 0; o < OT; o++) acc[o] = 0.0;
+  for (int k0 = 0; k0 < K; k0 += S::kTaps) {
+    const int taps = min(S::kTaps, K - k0);
+    for (int g0 = 0; g0 < stride; g0 += S::kCh) {
+      __syncthreads();
+      for (int i = threadIdx.x; i < taps * OT * LPR; i += kThreads) {
+        const int jj = i % LPR, o = i / LPR % OT, t = i / (LPR * OT);
+        const int g = g0 + 2 * jj;
+        double2 v = make_double2(0.0, 0.0);
+        if (o0 + o < O) {
+          const double *row = w + ((int64_t)(o0 + o) * G + g) * K + k0 + t;
+          if (g < G) v.x = row[0];
+          if (g + 1 < G) v.y = row[K];
+        }
+        s_w[i] = v;
+      }
+      for (int p = 0; p < pm; p++) {
+        if (p) __syncthreads();
+        fill_tap_cache<NC, LPR>(map, iw, n0, N, K, pm, p, k0, taps, SH, SW, wrap != 0, (int)SN,
+                                s_off, s_wt);
+        __syncthreads();
+        if (g0 + 2 * j < stride) {
+          const double *src = recb + g0 + 2 * j;
+#pragma unroll 3
+          for (int t = 0; t < taps; t++) {
+            double2 d[NC];
+#pragma unroll
+            for (int i = 0; i < NC; i++)
+              d[i] = *reinterpret_cast<const double2 *>(
+                  src + (int64_t)s_off[i * kStep + t * S::kLocs + loc] * stride);
+            double vx = 0.0, vy = 0.0;
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+              const double a = s_wt[i * kStep + t * S::kLocs + loc];
+              vx = mcx_fma(a, d[i].x, vx);
+              vy = mcx_fma(a, d[i].y, vy);
+            }
+#pragma unroll
+            for (int o = 0; o < OT; o++) {
+              const double2 ww = s_w[(t * OT + o) * LPR + j];
+              acc[o] = mcx_fma(ww.y, vy, mcx_fma(ww.x, vx, acc[o]));
+            }
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < OT; o++) {
+#pragma unroll
+    for (int m = LPR / 2; m > 0; m >>= 1) acc[o] += __shfl_xor(acc[o], m);
+    if (o % LPR == j && o0 + o < O && n0 + loc < N)
+      y[((int64_t)b * O + o0 + o) * N + n0 + loc] = acc[o] + (bias ? bias[o0 + o] : 0.0);
+  }
+}
+
+// rec[b, corner] += weight * sum_s W[s,d,k] * src[b,s,n]: the products of a pass of taps stay
+// in registers, one channel a lane, then go out corner by corner: an atomic instruction adds to
+// whole records of up to sixteen channels (128 bytes).
+template <int NC, int LPR>
+__global__ __launch_bounds__(kThreads) void scatter_records_kernel(
+    const double *__restrict__ src, const double *__restrict__ map, const double *__restrict__ iw,
+    const double *__restrict__ w, double *__restrict__ rec, int S_, int D, int stride, int DH,
+    int DW, int N, int K, int P, int wrap) {
+  using S = RecShape<LPR>;
+  constexpr int kStep = S::kTaps * S::kLocs;
+  constexpr int kSrc = 16;  // source channels per pass
+  constexpr int kCh = LPR;
+  __shared__ int s_off[NC * kStep];
+  __shared__ double s_wt[NC * kStep];
+  __shared__ double s_w[S::kTaps * kSrc * kCh];
+  __shared__ double s_src[kSrc * S::kLocs];
+  const int loc = threadIdx.x / LPR, j = threadIdx.x % LPR;
+  const int n0 = blockIdx.x * S::kLocs, d0 = blockIdx.y * kCh, b = blockIdx.z;
+  const int64_t DN = (int64_t)DH * DW;
+  double *recb = rec + (int64_t)b * DN * stride + d0 + j;
+  const bool live = d0 + j < D;
+  const int pm = P == 0 ? 1 : P;
+  for (int k0 = 0; k0 < K; k0 += S::kTaps) {
+    const int taps = min(S::kTaps, K - k0);
+    double acc[S::kTaps];
+#pragma unroll
+    for (int t = 0; t < S::kTaps; t++) acc[t] = 0.0;
+    for (int s0 = 0; s0 < S_; s0 += kSrc) {
+      const int ns = min(kSrc, S_ - s0);
+      __syncthreads();
+      for (int i = threadIdx.x; i < ns * S::kTaps * kCh; i += kThreads) {
+        const int t = i % S::kTaps, c = i / S::kTaps % kCh, ss = i / (S::kTaps * kCh);
+        s_w[(ss * S::kTaps + t) * kCh + c] =
+            (t < taps && d0 + c < D) ? w[((int64_t)(s0 + ss) * D + d0 + c) * K + k0 + t] : 0.0;
+      }
+      for (int i = threadIdx.x; i < ns * S::kLocs; i += kThreads) {
+        const int l = i % S::kLocs, ss = i / S::kLocs;
+        s_src[i] = n0 + l < N ? src[((int64_t)b * S_ + s0 + ss) * N + n0 + l] : 0.0;
+      }
+      __syncthreads();
+      for (int ss = 0; ss < ns; ss++) {
+        const double v = s_src[ss * S::kLocs + loc];
+#pragma unroll
+        for (int t = 0; t < S::kTaps; t++) {
+          acc[t] = mcx_fma(s_w[(ss * S::kTaps + t) * kCh + j], v, acc[t]);
+        }
+      }
+    }
+    for (int p = 0; p < pm; p++) {
+      __syncthreads();
+      fill_tap_cache<NC, LPR>(map, iw, n0, N, K, pm, p, k0, taps, DH, DW, wrap != 0, -1, s_off,
+                              s_wt);
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < S::kTaps; t++) {
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+          const int slot = i * kStep + t * S::kLocs + loc;
+          const int off = t < taps ? s_off[slot] : -1;
+          if (live && off >= 0) atomic_add(recb + (int64_t)off * stride, s_wt[slot] * acc[t]);
+        }
+      }
+    }
+  }
+}
+
+// part[range][k][a][g] = sum over a range of (b, n) of plain[b,a,n] * sample(gath[b,g], map[n,k]).
+// A workgroup takes one tap, AT plain channels and 2 * LPR gathered ones; a tile is kSub runs of
+// kLocs locations, whose record reads are in flight together.
+template <int NC, int LPR, int AT>
+__global__ __launch_bounds__(kThreads) void weight_grad_records_kernel(
+    const double *__restrict__ plain, const double *__restrict__ rec,
+    const double *__restrict__ map, const double *__restrict__ iw, double *__restrict__ part,
+    int A, int G, int stride, int GH, int GW, int N, int K, int P, int wrap, int tiles_per_img,
+    int64_t total_tiles, int ranges) {
+  using S = RecShape<LPR>;
+  constexpr int kSub = LPR == 2 ? 2 : 4;  // (tiles of 128 or 256 locations)
+  constexpr int kTile = kSub * S::kLocs;
+  __shared__ int s_off[NC * kTile];
+  __shared__ double s_wt[NC * kTile];
+  __shared__ double s_plain[AT * kTile];
+  const int loc = threadIdx.x / LPR, j = threadIdx.x % LPR;
+  const int k = blockIdx.x % K, range = blockIdx.x / K;
+  const int a0 = blockIdx.y * AT, g0 = blockIdx.z * S::kCh;
+  const int64_t GN = (int64_t)GH * GW;
+  const int pm = P == 0 ? 1 : P;
+  const bool live = g0 + 2 * j < stride;
+  double2 acc[AT];
+#pragma unroll
+  for (int a = 0; a < AT; a++) acc[a] = make_double2(0.0, 0.0);
+  const int64_t t0 = total_tiles * range / ranges, t1 = total_tiles * (range + 1) / ranges;
+  for (int64_t tile = t0; tile < t1; tile++) {
+    const int b = (int)(tile / tiles_per_img);
+    const int n0 = (int)(tile - (int64_t)b * tiles_per_img) * kTile;
+    const double *src = rec + (int64_t)b * (GN + 1) * stride + g0 + 2 * j;
+    for (int p = 0; p < pm; p++) {
+      __syncthreads();
+      if (p == 0)
+        for (int i = threadIdx.x; i < AT * kTile; i += kThreads) {
+          const int l = i % kTile, a = a0 + i / kTile;
+          s_plain[i] = (a < A && n0 + l < N) ? plain[((int64_t)b * A + a) * N + n0 + l] : 0.0;
+        }
+      for (int l = threadIdx.x; l < kTile; l += kThreads) {
+        if (n0 + l < N) {
+          resolve_records<NC>(map, iw, ((int64_t)(n0 + l) * K + k) * pm + p, GH, GW, wrap != 0,
+                              (int)GN, s_off + l, s_wt + l, kTile);
+        } else {
+#pragma unroll
+          for (int i = 0; i < NC; i++) {
+            s_off[i * kTile + l] = (int)GN;
+            s_wt[i * kTile + l] = 0.0;
+          }
+        }
+      }
+      __syncthreads();
+      if (live) {
+        double2 d[kSub][NC];
+#pragma unroll
+        for (int u = 0; u < kSub; u++)
+#pragma unroll
+          for (int i = 0; i < NC; i++)
+            d[u][i] = *reinterpret_cast<const double2 *>(
+                src + (int64_t)s_off[i * kTile + u * S::kLocs + loc] * stride);
+#pragma unroll
+        for (int u = 0; u < kSub; u++) {
+          double vx = 0.0, vy = 0.0;
+#pragma unroll
+          for (int i = 0; i < NC; i++) {
+            const double f = s_wt[i * kTile + u * S::kLocs + loc];
+            vx = mcx_fma(f, d[u][i].x, vx);
+            vy = mcx_fma(f, d[u][i].y, vy);
+          }
+#pragma unroll
+          for (int a = 0; a < AT; a++) {
+            const double q = s_plain[a * kTile + u * S::kLocs + loc];
+            acc[a].x = mcx_fma(q, vx, acc[a].x);
+            acc[a].y = mcx_fma(q, vy, acc[a].y);
+          }
+        }
+      }
+    }
+  }
+  // sum over the locations' lanes of each wave, then over the four waves through LDS
+  __shared__ double2 s_red[kThreads / 64][AT][LPR];
+#pragma unroll
+  for (int a = 0; a < AT; a++) {
+#pragma unroll
+    for (int m = 32; m >= LPR; m >>= 1) {
+      acc[a].x += __shfl_xor(acc[a].x, m);
+      acc[a].y += __shfl_xor(acc[a].y, m);
+    }
+    if ((int)(threadIdx.x & 63) < LPR) s_red[threadIdx.x >> 6][a][j] = acc[a];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < AT * LPR; i += kThreads) {
+    const int a = i / LPR, jj = i % LPR, g = g0 + 2 * jj;
+    double2 v = s_red[0][a][jj];
+    for (int q = 1; q < kThreads / 64; q++) {
+      v.x += s_red[q][a][jj].x;
+      v.y += s_red[q][a][jj].y;
+    }
+    if (a0 + a < A) {
+      double *out = part + (((int64_t)range * K + k) * A + a0 + a) * G + g;
+      if (g < G) out[0] = v.x;
+      if (g + 1 < G) out[1] = v.y;
+    }
+  }
+}
+
+// gw[a][g][k] = sum over the ranges of part[range][k][a][g]: a wave per element
+__global__ __launch_bounds__(kThreads) void reduce_records_kernel(const double *__restrict__ part,
+                                                                  double *__restrict__ gw, int AG,
+                                                                  int K, int ranges) {
+  const int64_t e = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (e >= (int64_t)AG * K) return;
+  double v = 0.0;
+  for (int r = lane; r < ranges; r += 64) v += part[(int64_t)r * AG * K + e];
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
+  if (lane == 0) {
+    const int64_t k = e / AG, ag = e - k * AG;
+    gw[ag * K + k] = v;
+  }
+}
+
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Tiles, ranges and channel blocks of the weight gradient: about 2048 workgroups, eight per CU.
+struct GradShape {
+  int lpr, at;
+  int64_t tiles_per_img, total, ranges, ablocks, gblocks;
+};
+GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
+  GradShape q;
+  q.lpr = lanes_per_record(G);
+  q.at = A == 1 ? 1 : A <= 4 ? 4 : 16;
+  q.ablocks = (A + q.at - 1) / q.at;
+  q.gblocks = (read_stride(G) + 2 * q.lpr - 1) / (2 * q.lpr);
+  const int64_t tile = (q.lpr == 2 ? 2 : 4) * (kThreads / q.lpr);
+  q.tiles_per_img = (N + tile - 1) / tile;
+  q.total = B * q.tiles_per_img;
+  const int64_t per_range = K * q.ablocks * q.gblocks;
+  q.ranges = std::max<int64_t>(1, std::min(q.total, 2048 / per_range));
+  return q;
+}
+
+bool wraps(int interp) { return canonical_interp(interp) == kInterpBispherical; }
+
+int make_records(const double *x, double *rec, int64_t B, int64_t C, int64_t N, hipStream_t s) {
+  const int64_t stride = read_stride(C);
+  const dim3 grid(div_up(N + 1, kThreads), div_up(stride, 16), (unsigned)B);
+  hipLaunchKernelGGL(to_records_kernel, grid, dim3(kThreads), 0, s, x, rec, (int)C, (int)stride, N);
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // namespace
+
+// A grid has at most 65535 workgroups in its second and third direction.
+bool records_supported(int64_t B, int64_t C1, int64_t C2, int64_t K) {
+  return B <= 65535 && C1 <= 65535 && C2 <= 65535 && K <= 2048;
+}
+
+#define MCX_LPR(C, CALL)              \
+  switch (lanes_per_record(C)) {      \
+    case 2: { CALL(2) } break;        \
+    case 4: { CALL(4) } break;        \
+    default: { CALL(8) } break;       \
+  }
+
+size_t records_gather_bytes(int64_t B, int64_t G, int64_t SN) {
+  return align256((size_t)(B * (SN + 1) * read_stride(G)) * sizeof(double));
+}
+
+int records_gather_product(const double *src, const double *map, const double *iw, const double *w,
+                           const double *bias, double *y, void *ws, int64_t B, int64_t G,
+                           int64_t O, int64_t SH, int64_t SW, int64_t N, int64_t K, int64_t P,
+                           int interp, hipStream_t s) {
+  double *rec = (double *)ws;
+  if (int rc = make_records(src, rec, B, G, SH * SW, s)) return rc;
+  const int stride = (int)read_stride(G);
+  const bool one = canonical_interp(interp) == kInterpNearest;
+#define MCX_RUN(NC, LPR, OT)                                                                     \
+  hipLaunchKernelGGL((gather_records_kernel<NC, LPR, OT>),                                       \
+                     dim3(div_up(N, kThreads / LPR), div_up(O, OT), (unsigned)B), dim3(kThreads), \
+                     0, s, rec, map, iw, w, bias, y, (int)G, stride, (int)O, (int)SH, (int)SW,   \
+                     (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0);
+#define MCX_OT(NC, LPR)                             \
+  if (O == 1) { MCX_RUN(NC, LPR, 1) }               \
+  else if (O <= 4) { MCX_RUN(NC, LPR, 4) }          \
+  else { MCX_RUN(NC, LPR, 16) }
+#define MCX_NC(LPR) if (one) { MCX_OT(1, LPR) } else { MCX_OT(4, LPR) }
+  MCX_LPR(G, MCX_NC)
+#undef MCX_NC
+#undef MCX_OT
+#undef MCX_RUN
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+
+size_t records_scatter_bytes(int64_t B, int64_t D, int64_t DN) {
+  return align256((size_t)(B * DN * add_stride(D)) * sizeof(double));
+}
+
+int records_product_scatter(const double *src, const double *map, const double *iw,
+                            const double *w, const double *bias, double *dst, void *ws, int64_t B,
+                            int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,
+                            int64_t P, int interp, hipStream_t s) {
+  double *rec = (double *)ws;
+  const int64_t DN = DH * DW, stride = add_stride(D);
+  if (int rc = fill_f64(rec, B * DN * stride, 0.0, s)) return rc;
+  const bool one = canonical_interp(interp) == kInterpNearest;
+#define MCX_RUN(NC, LPR)                                                                          \
+  hipLaunchKernelGGL((scatter_records_kernel<NC, LPR>),                                           \
+                     dim3(div_up(N, kThreads / LPR), div_up(D, LPR), (unsigned)B),                \
+                     dim3(kThreads), 0, s, src, map, iw, w, rec, (int)S, (int)D, (int)stride,     \
+                     (int)DH, (int)DW, (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0);
+#define MCX_NC(LPR) if (one) { MCX_RUN(1, LPR) } else { MCX_RUN(4, LPR) }
+  if (D <= 2) { MCX_NC(2) }
+  else if (D <= 4) { MCX_NC(4) }
+  else if (D <= 8) { MCX_NC(8) }
+  else { MCX_NC(16) }
+#undef MCX_NC
+#undef MCX_RUN
+  MCX_HIP_CHECK_LAUNCH();
+  hipLaunchKernelGGL(from_records_kernel, dim3(div_up(DN, kThreads), div_up(D, 16), (unsigned)B),
+                     dim3(kThreads), 0, s, rec, bias, dst, (int)D, (int)stride, DN);
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+
+size_t records_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t GN, int64_t N,
+                                 int64_t K) {
+  const GradShape q = grad_shape(B, A, G, N, K);
+  return records_gather_bytes(B, G, GN) + align256((size_t)(q.ranges * K * A * G) * sizeof(double));
+}
+
+int records_weight_grad(const double *plain, const double *gath, const double *map,
+                        const double *iw, double *gw, void *ws, int64_t B, int64_t A, int64_t G,
+                        int64_t GH, int64_t GW, int64_t N, int64_t K, int64_t P, int interp,
+                        hipStream_t s) {
+  double *rec = (double *)ws;
+  double *part = (double *)((char *)ws + records_gather_bytes(B, G, GH * GW));
+  if (int rc = make_records(gath, rec, B, G, GH * GW, s)) return rc;
+  const GradShape q = grad_shape(B, A, G, N, K);
+  const bool one = canonical_interp(interp) == kInterpNearest;
+#define MCX_RUN(NC, LPR, AT)                                                                     \
+  hipLaunchKernelGGL((weight_grad_records_kernel<NC, LPR, AT>),                                  \
+                     dim3((unsigned)(q.ranges * K), (unsigned)q.ablocks, (unsigned)q.gblocks),   \
+                     dim3(kThreads), 0, s, plain, rec, map, iw, part, (int)A, (int)G,            \
+                     (int)read_stride(G), (int)GH, (int)GW, (int)N, (int)K, (int)P,              \
+                     wraps(interp) ? 1 : 0, (int)q.tiles_per_img, q.total, (int)q.ranges);
+#define MCX_AT(NC, LPR)                             \
+  if (q.at == 1) { MCX_RUN(NC, LPR, 1) }            \
+  else if (q.at == 4) { MCX_RUN(NC, LPR, 4) }       \
+  else { MCX_RUN(NC, LPR, 16) }
+#define MCX_NC(LPR) if (one) { MCX_AT(1, LPR) } else { MCX_AT(4, LPR) }
+  MCX_LPR(G, MCX_NC)
+#undef MCX_NC
+#undef MCX_AT
+#undef MCX_RUN
+  MCX_HIP_CHECK_LAUNCH();
+  hipLaunchKernelGGL(reduce_records_kernel, dim3(div_up(A * G * K, kThreads / 64)), dim3(kThreads),
+                     0, s, part, gw, (int)(A * G), (int)K, (int)q.ranges);
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+#undef MCX_LPR
+
+}  // namespace mcx

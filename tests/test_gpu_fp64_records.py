@@ -1,0 +1,83 @@
+"""fp64 convolutions over channel-last records against the CPU oracle, at the edges of their
+tiles: channel counts around the widths a pass of lanes covers (2, 4 and 8 lanes of two
+channels; 1, 4 and 16 outputs), more channels and taps than one pass takes, locations around a
+workgroup's share, weighted taps, and the call without a workspace (the scalar kernels)."""
+import ctypes
+
+import pytest
+import torch
+
+import helpers
+from helpers import rel_err
+from oracle import ops as O
+
+from mappedconvolutions_amd import _C, _lib
+
+pytestmark = pytest.mark.gpu
+
+# (Ci, Co, K, map height, map width, P): sums of up to a few hundred terms in 64 bits differ by
+# some 1e-15 of the result with their order; 1e-12 is what the fp64 tests beside this one allow
+SHAPES = [(1, 1, 1, 1, 1, 0), (2, 1, 9, 5, 7, 0), (3, 4, 6, 4, 32, 0), (4, 5, 9, 8, 17, 0),
+          (5, 16, 10, 3, 43, 0), (8, 17, 9, 9, 15, 0), (9, 2, 5, 16, 16, 3), (16, 3, 9, 4, 33, 0),
+          (17, 9, 4, 6, 11, 6), (33, 20, 11, 5, 13, 0)]
+
+
+@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES)
+@pytest.mark.parametrize("interp", [0, 1, 2])
+def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
+    g = torch.Generator().manual_seed(ci * 100 + co)
+    B, ih, iw_ = 2, 6, 9
+    smap, wts = helpers.random_map(g, mh, mw, k, p, ih, iw_, torch.float64,
+                                   integer=interp == 1 and k == 9)
+    rnd = lambda *s: torch.randn(s, generator=g, dtype=torch.float64)
+    cuda = lambda t: None if t is None else t.cuda()
+    pre = "weighted_" if p else ""
+    maps = [smap] + ([wts] if p else [])
+    x, w, b, gy = rnd(B, ci, ih, iw_), rnd(co, ci, k), rnd(co), rnd(B, co, mh, mw)
+    for name, args in ((pre + "mapped_conv_forward", [x, *maps, w, b, k, interp]),
+                       (pre + "mapped_conv_backward", [gy, *maps, x, w, b, k, interp])):
+        want = getattr(O, name)(*args)
+        got = getattr(_C, name)(*[cuda(a) if torch.is_tensor(a) else a for a in args])
+        for i, (a, c) in enumerate(zip(*[v if isinstance(v, (list, tuple)) else [v]
+                                         for v in (got, want)])):
+            assert rel_err(a, c) < 1e-12, (name, i)
+    # the transposed convolution: the map's locations are the input's pixels
+    xt, wt, bt, gt = rnd(B, ci, mh, mw), rnd(ci, co, k), rnd(co), rnd(B, co, ih, iw_)
+    for name, args in (
+            (pre + "mapped_transposed_conv_forward", [xt, *maps, wt, bt, ih, iw_, k, interp]),
+            (pre + "mapped_transposed_conv_backward", [gt, *maps, xt, wt, bt, k, interp])):
+        want = getattr(O, name)(*args)
+        got = getattr(_C, name)(*[cuda(a) if torch.is_tensor(a) else a for a in args])
+        for i, (a, c) in enumerate(zip(*[v if isinstance(v, (list, tuple)) else [v]
+                                         for v in (got, want)])):
+            assert rel_err(a, c) < 1e-12, (name, i)
+
+
+def test_fp64_without_a_workspace(device):
+    g = torch.Generator().manual_seed(5)
+    B, ci, co, k, h, w_ = 2, 5, 3, 9, 7, 8
+    smap, _ = helpers.random_map(g, h, w_, k, 0, h, w_, torch.float64)
+    x, w, b = (torch.randn(s, generator=g, dtype=torch.float64)
+               for s in ((B, ci, h, w_), (co, ci, k), (co,)))
+    want = O.mapped_conv_forward(x, smap, w, b, k, 1)
+    dx, dm, dw, db = (t.cuda() for t in (x, smap, w, b))
+    out = torch.empty(B, co, h, w_, dtype=torch.float64, device=device)
+    lib = _lib.load()
+    rc = lib.mcx_conv_forward(dx.data_ptr(), dm.data_ptr(), None, dw.data_ptr(), db.data_ptr(),
+                              out.data_ptr(), None, 0, B, ci, co, h, w_, h, w_, k, 0, 1,
+                              _lib.MCX_F64, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert rel_err(out, want) < 1e-12
+
+
+@pytest.mark.parametrize("n", [1 << 13, (1 << 13) + 1, 100003])
+def test_bias_gradient_of_one_channel(n, device):
+    """The sum's two stages set in at 2^14 values of a channel."""
+    g = torch.Generator().manual_seed(n)
+    gy = torch.randn(2, 1, 1, n, generator=g, dtype=torch.float64)
+    smap = torch.zeros(1, n, 1, 2, dtype=torch.float64)
+    x, w, b = torch.zeros(2, 1, 2, 2).double(), torch.zeros(1, 1, 1).double(), torch.zeros(1).double()
+    gb = _C.mapped_conv_backward(gy.cuda(), smap.cuda(), x.cuda(), w.cuda(), b.cuda(), 1, 1)[2]
+    want = gy.sum().item()
+    # n terms of magnitude one in 64 bits: at most n * 2^-53 * sum|gy| apart, far less in practice
+    assert abs(gb.item() - want) <= 1e-12 * gy.abs().sum().item()
