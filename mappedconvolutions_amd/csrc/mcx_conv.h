@@ -53,9 +53,12 @@ struct bf16_t;
 bool mfma_supported(int64_t P);
 size_t mfma_gather_product_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
                                  int64_t SW, int elem, int64_t MH, int64_t MW);
+// (enough for every result; with all of mfma_gather_product_bytes fp32 storage is faster)
+size_t mfma_gather_product_min_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
+                                     int64_t SW, int elem, int64_t MH, int64_t MW);
 template <typename TD>
 int mfma_gather_product(const TD *src, const float *map, const float *iw, const TD *w,
-                        const TD *bias, TD *y, void *scratch, int64_t B, int64_t G, int64_t O,
+                        const TD *bias, TD *y, void *scratch, size_t scratch_bytes, int64_t B, int64_t G, int64_t O,
                         int64_t SH, int64_t SW, int64_t OH, int64_t OW, int64_t K, int64_t P,
                         int interp, hipStream_t s, const void *plan = nullptr);
 size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64_t MW, int64_t K,

@@ -228,10 +228,10 @@ int gather_product<float>(bool mfma, const void *src, const void *map, const voi
     return generic_gather_product<float>((const float *)src, (const float *)map,
                                          (const float *)iw, (const float *)w, (const float *)bias,
                                          (float *)y, B, G, O, SH, SW, MH * MW, K, P, interp, s);
-  if (!ws || ws_bytes < mfma_gather_product_bytes(O, G, K, B, SH, SW, 4, MH, MW))
+  if (!ws || ws_bytes < mfma_gather_product_min_bytes(O, G, K, B, SH, SW, 4, MH, MW))
     return MCX_E_WORKSPACE;
   return mfma_gather_product<float>((const float *)src, (const float *)map, (const float *)iw,
-                                    (const float *)w, (const float *)bias, (float *)y, ws, B, G, O,
+                                    (const float *)w, (const float *)bias, (float *)y, ws, ws_bytes, B, G, O,
                                     SH, SW, MH, MW, K, P, interp, s, plan);
 }
 
@@ -291,7 +291,7 @@ int gather_product<bf16_t>(bool mfma, const void *src, const void *map, const vo
   if (!ws || ws_bytes < mfma_gather_product_bytes(O, G, K, B, SH, SW, 2, MH, MW))
     return MCX_E_WORKSPACE;
   return mfma_gather_product<bf16_t>((const bf16_t *)src, (const float *)map, (const float *)iw,
-                                     (const bf16_t *)w, (const bf16_t *)bias, (bf16_t *)y, ws, B,
+                                     (const bf16_t *)w, (const bf16_t *)bias, (bf16_t *)y, ws, ws_bytes, B,
                                      G, O, SH, SW, MH, MW, K, P, interp, s, plan);
 }
 
@@ -425,9 +425,12 @@ extern "C" int mcx_conv_forward_static(const void *x, const void *map, const voi
   if (int rc = check_ptrs(x, map, iw, w, P)) return rc;
   if (!bias || !y) return MCX_E_NULL;
   if (dtype != MCX_F32 && dtype != MCX_F64 && dtype != MCX_BF16) return MCX_E_DTYPE;
-  // (fp64 can do without scratch)
+  // (what the product cannot do without: nothing for fp64, the packed weights for fp32)
   const size_t need =
-      dtype == MCX_F64 ? 0 : gather_product_ws(dtype, Ci, Co, K, P, B, IH, IW, OH, OW);
+      dtype == MCX_F64 ? 0
+      : dtype == MCX_F32 && mfma_supported(P)
+          ? mfma_gather_product_min_bytes(Co, Ci, K, B, IH, IW, 4, OH, OW)
+          : gather_product_ws(dtype, Ci, Co, K, P, B, IH, IW, OH, OW);
   if (need > kStaticScratchBytes) return MCX_E_STATIC_LIMIT;
   int rc = 0;
   void *ws = static_scratch_of_current_device(&rc);

@@ -73,6 +73,16 @@ struct PairMaskJob {
   int64_t total;   // (location, tap) entries
 };
 
+//   * SplitJob: the weights in three bf16 parts as well, and the flag word that the kernels
+//     which read them set cleared (mcx_conv_split.h).
+struct SplitJob {
+  uint16_t *w;     // nullptr: no job
+  int *nonfinite;
+  int planar;      // the source they meet is planar (else channel-last)
+};
+
+__host__ __device__ inline int split_channel(int c, int kg, int j, int G, int planar);
+
 // Bits of the (point, corner) pairs with a nonzero weight anywhere among the entries this
 // block walks (block `block` of `blocks`); valid in every thread on return.
 template <int NCORN>
@@ -134,8 +144,12 @@ __device__ inline float dot_bf16_first(unsigned word, unsigned w) {
 template <typename TD>
 __global__ __launch_bounds__(256) void pack_weights_kernel(
     const TD *__restrict__ w, void *__restrict__ packed_out, int O, int G, int K, int Opad,
-    int Gpad, int transposed, int *__restrict__ clear, ZeroJob zero, PairMaskJob pm) {
-  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // a flag word of the caller
+    int Gpad, int transposed, int *__restrict__ clear, ZeroJob zero, PairMaskJob pm,
+    SplitJob split) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // flag words of the caller
+    if (clear) *clear = 0;
+    if (split.nonfinite) *split.nonfinite = 0;
+  }
   int blocks = gridDim.x;
   if (pm.mask) {
     blocks -= pm.blocks;
@@ -174,6 +188,25 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
       const int k = (int)(e / ((int64_t)Opad * Gpad));
       const int64_t wi = transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k;
       wp[e] = (o < O && g < G) ? to_f32(w[wi]) : 0.f;
+    }
+    // the same in three bf16 parts, [k][chunk][part][kg][o][8 channels] (mcx_conv_split.h)
+    if (split.w) {
+      const int chunks = Gpad / kGC;
+      for (int64_t e = first; e < total; e += stride) {
+        const int o = (int)((e >> 3) % Opad);
+        const int64_t u = (e >> 3) / Opad;  // (tap, chunk, half)
+        const int kg = (int)(u & 1), c = (int)((u >> 1) % chunks), k = (int)((u >> 1) / chunks);
+        const int g = split_channel(c, kg, (int)(e & 7), G, split.planar);
+        float x = 0.f;
+        if (o < O && g >= 0)
+          x = to_f32(w[transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k]);
+#pragma unroll
+        for (int part = 0; part < 3; part++) {
+          const uint16_t q = from_f32<bf16_t>(x).v;
+          split.w[((((u >> 1) * 3 + part) * 2 + kg) * Opad + o) * 8 + (e & 7)] = q;
+          x -= __builtin_bit_cast(float, (uint32_t)q << 16);
+        }
+      }
     }
   }
   for (int64_t i = first; i < zero.count; i += stride) zero.ptr[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -319,7 +352,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
     int tiles_x, int tiles_per_img, int tw_shift, const int *__restrict__ gate, int run_if_zero,
     const float *__restrict__ addend, const int *__restrict__ pair_mask, int run_if_leading,
     int packed_map, int accumulate, int cl_blocked, const int *__restrict__ row_mask,
-    int mask_words) {
+    int mask_words, const int *__restrict__ only_if) {
   constexpr int NE = NP * NCORN;         // (offset, weight) pairs per pixel and tap
   static_assert(NA >= 1 && NA <= NE, "NA counts leading pairs");
   constexpr bool kMasked = NA == NE;
@@ -336,6 +369,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
   // (bilinear corners of integral coordinates, unused slots) are neither loaded nor
   // accumulated.
   __shared__ unsigned TapMask[TG][2][2];
+  if (only_if && *only_if == 0) return;  // nothing to recompute (see mcx_conv_split.h)
   if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
   if (pair_mask && !row_mask &&
       (!later_pairs_in_use(pair_mask, mask_words) != (run_if_leading != 0)))
@@ -1030,6 +1064,8 @@ __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel
       }
   }
 }
+
+#include "mcx_conv_split.h"
 
 // ---------------------------------------------------------------------------------
 // weight_grad: gW[a,g,k] = sum_{b,n} plain[b,a,n] * sample(gath[b,g], map[n,k])
@@ -2332,6 +2368,65 @@ int launch_channel_blocks(const TD *src, TD *stage, int64_t B, int64_t G, int64_
 
 // `stage`: room for the channel-last copy (B * SH * SW * Gpad elements) when
 // use_channel_last(SH, interp), unused otherwise.
+// ---- fp32 on the bf16 matrix instructions (mcx_conv_split.h) ----
+// Room for the split weights and the flag word, at the end of a product's scratch.
+size_t split_bytes(int64_t O, int64_t G, int64_t K, int elem) {
+  if (elem != 4) return 0;
+  return 256 + align256((size_t)(K * round_up(G, kGC) * round_up(O, kOT)) * 6);
+}
+SplitJob split_job(char *region, bool planar) {
+  return SplitJob{reinterpret_cast<uint16_t *>(region + 256), reinterpret_cast<int *>(region),
+                  planar ? 1 : 0};
+}
+// A tap of the source is one, or for planar images four, (offset, weight) entries; operands
+// are addressed as buffers of less than 4 GiB.
+bool split_applies(int64_t G, int64_t O, int64_t SH, int64_t SW, int64_t K, const ModeArgs &m,
+                   bool packed, bool cl) {
+  const int64_t Gpad = round_up(G, kGC), Opad = round_up(O, kOT);
+  if (K * (Gpad / kGC) * 6 * Opad * 16 >= (int64_t)kOobOffset) return false;
+  if (SH * SW * (cl ? Gpad : G) * 4 >= (int64_t)kOobOffset) return false;
+  if (cl) return m.mode == kInterpNearest && m.np <= 4;
+  return packed ? m.np == 4 : m.np == 1;
+}
+
+int launch_gather_split(SplitArgs a, const PixelTiling &t, bool cl, hipStream_t s) {
+  a.tiles_x = t.tiles_x;
+  a.tiles_per_img = t.tiles_per_img;
+  a.tw_shift = t.tw_shift;
+  const bool wide = a.Opad % (2 * kOT) == 0;
+  const dim3 grid((unsigned)t.total, (unsigned)(a.Opad / (wide ? 2 * kOT : kOT)));
+#define MCX_SPLIT(KERNEL, ...) \
+  hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(kThreads), 0, s, a)
+#define MCX_SPLIT_OG(KERNEL, ...)        \
+  if (wide) {                            \
+    MCX_SPLIT(KERNEL, __VA_ARGS__, 2);   \
+  } else {                               \
+    MCX_SPLIT(KERNEL, __VA_ARGS__, 1);   \
+  }
+  if (cl) {
+    if (a.map2) {
+      MCX_SPLIT_OG(gather_product_split_cl_kernel, 4, true)
+    } else {
+      switch (a.packed ? 4 : a.np) {
+        case 1: MCX_SPLIT_OG(gather_product_split_cl_kernel, 1, false) break;
+        case 2: MCX_SPLIT_OG(gather_product_split_cl_kernel, 2, false) break;
+        case 3: MCX_SPLIT_OG(gather_product_split_cl_kernel, 3, false) break;
+        default: MCX_SPLIT_OG(gather_product_split_cl_kernel, 4, false) break;
+      }
+    }
+  } else if (!a.packed && a.ncorn == 1) {
+    MCX_SPLIT_OG(gather_product_split_kernel, 1)
+  } else {
+    MCX_SPLIT_OG(gather_product_split_kernel, 4)
+  }
+#undef MCX_SPLIT_OG
+#undef MCX_SPLIT
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+
+// `split` (fp32 storage; w NULL: not available): where the packing launch put the split weights.
+// `map2`: second-level entries of a packed map, read by the split kernels only.
 template <typename TD>
 int launch_gather_product(const TD *src, const float *map, const float *iw, const float *wp,
                           const TD *bias, TD *y, TD *stage, int64_t B, int64_t G, int64_t O,
@@ -2340,7 +2435,8 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
                           const float *addend = nullptr, bool staged = false,
                           const int *pair_mask = nullptr, bool packed_map = false,
                           bool accumulate = false, const int *row_mask = nullptr,
-                          int mask_words = 1) {
+                          int mask_words = 1, SplitJob split = SplitJob{},
+                          const float2 *map2 = nullptr, const int *only_if = nullptr) {
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const bool blocked = stage != nullptr && use_channel_blocks(SH, interp, sizeof(TD)) &&
                        SH * SW * 8 * (int64_t)sizeof(TD) <= 0xffffffffLL;
@@ -2418,6 +2514,26 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
   }
   dim3 grid((unsigned)t.total, (unsigned)(Opad / (wide ? 2 * kOT : kOT)));
   const ModeArgs m = mode_args(interp, P);
+  if constexpr (sizeof(TD) == 4) {
+    if (split.w) {
+      SplitArgs a{};
+      a.src = src; a.map = map; a.iw = iw; a.map2 = map2; a.w = split.w; a.bias = bias; a.y = y;
+      a.addend = addend; a.gate = gate; a.pair_mask = pair_mask; a.row_mask = row_mask;
+      a.nonfinite = split.nonfinite;
+      a.G = (int)G; a.O = (int)O; a.Opad = Opad; a.Gpad = Gpad; a.SH = (int)SH; a.SW = (int)SW;
+      a.OH = (int)OH; a.OW = (int)OW; a.K = (int)K; a.np = m.np;
+      a.ncorn = m.mode == kInterpNearest ? 1 : 4;
+      a.weighted = m.weighted; a.wrap = m.wrap; a.packed = packed_map ? 1 : 0;
+      a.run_if_zero = run_if_zero; a.mask_words = mask_words;
+      profile_begin(s);
+      const int rc = launch_gather_split(a, t, cl, s);
+      profile_end(s);
+      if (rc) return rc;
+      // the fp32 form below recomputes everything where a result was not finite
+      only_if = split.nonfinite;
+    }
+    if (only_if) pair_mask = row_mask = nullptr;  // (its general form alone)
+  }
   // `pair_mask` (four-pair taps only): launch the two-pair form as well; the mask picks one
 #define MCX_LAUNCH_NA(NCORN, NP, OG, CL, NA, MASK, LEAD)                                         \
   hipLaunchKernelGGL((gather_product_mfma_kernel<TD, NCORN, NP, OG, CL, NA>), grid,              \
@@ -2425,7 +2541,7 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
                      Gpad, (int)SH, (int)SW, (int)OH, (int)OW, (int)K, m.weighted, m.wrap,       \
                      t.tiles_x, t.tiles_per_img, t.tw_shift, gate, run_if_zero, addend, MASK,    \
                      LEAD, packed_map ? 1 : 0, accumulate ? 1 : 0, blocked ? 1 : 0, row_mask,     \
-                     mask_words)
+                     mask_words, only_if)
 #define MCX_LAUNCH_CL(NCORN, NP, OG, CL)                                      \
   if constexpr (NCORN * NP == 4) {                                            \
     if (pair_mask) {                                                          \
@@ -2477,7 +2593,7 @@ constexpr int64_t kTinyMapEntries = 4096;
 template <typename TD>
 int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K, int transposed,
                         hipStream_t s, int *clear = nullptr, ZeroJob zero = ZeroJob{nullptr, 0},
-                        PairMaskJob pm = PairMaskJob{}) {
+                        PairMaskJob pm = PairMaskJob{}, SplitJob split = SplitJob{}) {
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const int64_t packed = (int64_t)K * Gpad * Opad;
   // (bf16 storage: the bf16 MFMA operand layout in the same scratch, half the bytes)
@@ -2485,7 +2601,7 @@ int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K,
   const dim3 grid((unsigned)std::min<int64_t>((work + 255) / 256, 4096) +
                   (pm.mask ? (unsigned)pm.blocks : 0u));
   hipLaunchKernelGGL(pack_weights_kernel<TD>, grid, dim3(256), 0, s, w, (void *)wp, (int)O, (int)G,
-                     (int)K, Opad, Gpad, transposed, clear, zero, pm);
+                     (int)K, Opad, Gpad, transposed, clear, zero, pm, split);
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }
@@ -2543,8 +2659,9 @@ size_t mfma_gather_plan_offset(int64_t DH, int64_t DW, int64_t MH, int64_t MW, i
 // ---- gather-product --------------------------------------------------------------
 // Packed weights, then (single-row sources) the channel-last copy of the source, sized
 // for 4-byte elements.
-size_t mfma_gather_product_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
-                                 int64_t SW, int elem, int64_t MH, int64_t MW) {
+// (without the room for split weights, see mfma_gather_product_bytes)
+size_t mfma_gather_product_min_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
+                                     int64_t SW, int elem, int64_t MH, int64_t MW) {
   size_t n = align256((size_t)(K * round_up(G, kGC) * round_up(O, kOT)) * sizeof(float));
   n += 256;  // the map's pair mask
   if (SH == 1 || elem == 2)
@@ -2554,14 +2671,26 @@ size_t mfma_gather_product_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int
     n += align256((size_t)(MH * MW * K) * kPlanSlots * sizeof(float2));
   return n;
 }
+size_t mfma_gather_product_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
+                                 int64_t SW, int elem, int64_t MH, int64_t MW) {
+  return mfma_gather_product_min_bytes(O, G, K, B, SH, SW, elem, MH, MW) +
+         split_bytes(O, G, K, elem);
+}
 
-// scratch: mfma_gather_product_bytes(...) bytes.
+// scratch: mfma_gather_product_bytes(...) bytes; with mfma_gather_product_min_bytes(...) the fp32
+// matrix instructions serve fp32 storage.
 template <typename TD>
 int mfma_gather_product(const TD *src, const float *map, const float *iw, const TD *w,
-                        const TD *bias, TD *y, void *scratch, int64_t B, int64_t G, int64_t O,
-                        int64_t SH, int64_t SW, int64_t OH, int64_t OW, int64_t K, int64_t P,
+                        const TD *bias, TD *y, void *scratch, size_t scratch_bytes, int64_t B,
+                        int64_t G, int64_t O, int64_t SH, int64_t SW, int64_t OH, int64_t OW, int64_t K, int64_t P,
                         int interp, hipStream_t s, const void *plan) {
   float *wp = (float *)scratch;
+  const size_t min_bytes =
+      mfma_gather_product_min_bytes(O, G, K, B, SH, SW, (int)sizeof(TD), OH, OW);
+  const bool room = sizeof(TD) == 4 && scratch_bytes >= min_bytes + split_bytes(O, G, K, 4);
+  const bool cl = use_channel_last(SH, interp) &&
+                  SH * SW * round_up(G, kGC) * (int64_t)sizeof(TD) <= 0xffffffffLL;
+  const SplitJob with_split = split_job((char *)scratch + min_bytes, !cl);
   // (fp32 images with four-corner taps: resolving the taps in the kernel and reading them
   // resolved measured the same within 1 %, so there only the plan's pair mask is used and the
   // 32 bytes per tap of the resolved form are not read; single-row sources and bf16 storage
@@ -2580,12 +2709,20 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
                                              align256((size_t)(K * round_up(G, kGC) *
                                                                round_up(O, kOT)) * 4))
                     : nullptr;
-    if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s)) return rc;
     const ModeArgs pm = mode_args(interp, P);
     const bool four_pairs = pm.np * (pm.mode == kInterpNearest ? 1 : 4) == 4;
+    // (a plan's cells hold four entries, the unused ones of weight zero)
+    const SplitJob split =
+        room && split_applies(G, O, SH, SW, K, mode_args(kInterpNearest, kPlanSlots), true, cl)
+            ? with_split
+            : SplitJob{};
+    if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s, nullptr, ZeroJob{nullptr, 0},
+                                         PairMaskJob{}, split))
+      return rc;
     return launch_gather_product<TD>(src, gmap, nullptr, wp, bias, y, stage, B, G, O, SH, SW, OH,
                                      OW, K, kPlanSlots, kInterpNearest, nullptr, 0, s, nullptr,
-                                     false, four_pairs ? flags + 4 : nullptr, true);
+                                     false, four_pairs ? flags + 4 : nullptr, true, false,
+                                     nullptr, 1, split);
   }
   int *pair_mask = reinterpret_cast<int *>(
       (char *)scratch + align256((size_t)(K * round_up(G, kGC) * round_up(O, kOT)) * 4));
@@ -2612,10 +2749,13 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   const int *mask = pair_mask;
   // the pair mask of a small map is made by the last block of the packing launch
   const bool mask_on_pack = four_pairs && !plan && OH * OW * K <= kSmallMapEntries;
+  const SplitJob split =
+      room && split_applies(G, O, SH, SW, K, m, false, cl) ? with_split : SplitJob{};
   if (int rc = launch_pack_weights<TD>(
           w, wp, O, G, K, 0, s, mask_on_pack ? nullptr : pair_mask, ZeroJob{nullptr, 0},
           mask_on_pack ? pair_mask_job(map, iw, pair_mask, m, SH, SW, OH * OW * K)
-                       : PairMaskJob{}))
+                       : PairMaskJob{},
+          split))
     return rc;
   if (four_pairs) {
     if (plan)  // flag word 4 of a plan built for this map
@@ -2629,7 +2769,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   return launch_gather_product<TD>(src, map, iw, wp, bias, y, stage, B, G, O, SH, SW, OH, OW, K,
                                    P, interp, nullptr, 0, s, nullptr, false,
                                    four_pairs ? mask : nullptr, false, false, nullptr,
-                                   mask_on_pack ? job.blocks : 1);
+                                   mask_on_pack ? job.blocks : 1, split);
 }
 
 // ---- weight gradient ---------------------------------------------------------------
@@ -3066,7 +3206,7 @@ bool gather_plan_applies(int interp, int64_t P) {
 }
 
 struct ScatterScratch {
-  size_t wq, wpt, cnt, tmap, tmap2, acc32, ovf, stage, total;  // byte offsets
+  size_t wq, wpt, cnt, tmap, tmap2, acc32, ovf, stage, split, total;  // byte offsets
   bool two_level;  // a second four-slot level, applied by a second gather pass
   int64_t ovf_cap;  // entries of the overflow list (0: none)
   bool transposed_path;
@@ -3118,6 +3258,8 @@ ScatterScratch scatter_scratch(int64_t B, int64_t S, int64_t D, int64_t K, int64
   sc.stage = off;
   if (sc.transposed_path && (MH == 1 || elem == 2))
     off += align256((size_t)(B * MH * MW * round_up(S, kGC)) * 4);
+  sc.split = off;
+  if (sc.transposed_path) off += split_bytes(D, S, K, (int)elem);
   sc.total = off;
   return sc;
 }
@@ -3238,11 +3380,20 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     gate = flag;
     OverflowEntry *ovf = (OverflowEntry *)(pbase + sc.ovf);
     TD *stage = (MH == 1 || sizeof(TD) == 2) ? (TD *)(base + sc.stage) : nullptr;
+    const int64_t Spad16 = round_up(S, kGC);
+    const bool cl = stage != nullptr && use_channel_last(MH, kInterpNearest) &&
+                    MH * MW * Spad16 * (int64_t)sizeof(TD) <= 0xffffffffLL;
+    const SplitJob split =
+        sizeof(TD) == 4 && (cl || !sc.two_level) &&
+                split_applies(S, D, MH, MW, K, mode_args(kInterpNearest, kTransSlots), true, cl)
+            ? split_job(base + sc.split, !cl)
+            : SplitJob{};
     // (the packing launch also clears the transposed map's counters, flags and slots)
     if (int rc = launch_pack_weights<TD>(
             w, wpt, D, S, K, 1, s, nullptr,
             plan ? ZeroJob{nullptr, 0}
-                 : ZeroJob{reinterpret_cast<uint4 *>(cnt), (int64_t)((sc.ovf - sc.cnt) / 16)}))
+                 : ZeroJob{reinterpret_cast<uint4 *>(cnt), (int64_t)((sc.ovf - sc.cnt) / 16)},
+            PairMaskJob{}, split))
       return rc;
     if (!plan)
       if (int rc = build_transposed_map(sc, map, iw, cnt, m, DH, DW, MH, MW, K, s, true))
@@ -3250,9 +3401,6 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     // What did not fit the four slots of its cell is accumulated with float atomics into a
     // channel-last fp32 image (cleared only when there is anything to add), which the
     // gather's epilogue adds.
-    const int64_t Spad16 = round_up(S, kGC);
-    const bool cl = stage != nullptr && use_channel_last(MH, kInterpNearest) &&
-                    MH * MW * Spad16 * (int64_t)sizeof(TD) <= 0xffffffffLL;
     float *img = (float *)(base + sc.acc32);
     const int64_t total_img = B * DH * DW * round_up(D, kOT);
     // flag[2]: at least 4 iff some cell holds more than two entries (a plan has it already)
@@ -3276,13 +3424,15 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     if (int rc = launch_gather_product<TD>(src, (const float *)tmap, nullptr, wpt, bias, dst,
                                            stage, B, S, D, MH, MW, DH, DW, K, kTransSlots,
                                            kInterpNearest, gate, 1, s, img, cl, flag + 2, true,
-                                           false, flag + 8))
+                                           false, flag + 8, 1, split, tmap2))
       return rc;
-    if (sc.two_level)  // entries five to eight of every cell, added onto dst
+    // entries five to eight of every cell, added onto dst (the split form took them along)
+    if (sc.two_level)
       if (int rc = launch_gather_product<TD>(src, (const float *)tmap2, nullptr, wpt,
                                              (const TD *)nullptr, dst, stage, B, S, D, MH, MW, DH,
                                              DW, K, kTransSlots, kInterpNearest, gate, 1, s,
-                                             nullptr, cl, flag + 3, true, true))
+                                             nullptr, cl, flag + 3, true, true, nullptr, 1,
+                                         SplitJob{}, nullptr, split.nonfinite))
         return rc;
   }
 
@@ -3371,9 +3521,9 @@ int mfma_bias_grad(const TD *g, TD *gb, void *scratch, int64_t B, int64_t C, int
 
 #define MCX_INSTANTIATE_TD(TD)                                                                     \
   template int mfma_gather_product<TD>(const TD *, const float *, const float *, const TD *,      \
-                                       const TD *, TD *, void *, int64_t, int64_t, int64_t,       \
-                                       int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, \
-                                       hipStream_t, const void *);                                \
+                                       const TD *, TD *, void *, size_t, int64_t, int64_t,        \
+                                       int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,      \
+                                       int64_t, int, hipStream_t, const void *);                  \
   template int mfma_weight_grad<TD>(const TD *, const TD *, const float *, const float *, TD *,   \
                                     void *, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, \
                                     int64_t, int64_t, int64_t, int, hipStream_t, TD *,            \

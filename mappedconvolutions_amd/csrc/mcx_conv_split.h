@@ -1,0 +1,528 @@
+// fp32 gather-product on the bf16 matrix instructions, without giving up fp32: every operand is
+// split exactly into three bf16 parts (8 + 8 + 8 significant bits, round to nearest each, the
+// remainders exact), and a product is the six of the nine partial products that are larger
+// than 2^-26 of it, summed in fp32 by the matrix unit.  The rounding of single products is then
+// finer than fp32's own, and a matrix instruction adds 16 products per rounding of its sum
+// where the fp32 one adds 2.  v_mfma_f32_32x32x16_bf16 does sixteen times the work of
+// v_mfma_f32_32x32x2_f32 per clock, so six of them cost 384 clocks a unit (one tap x 16 channels
+// x 32 pixels x 64 outputs) where the fp32 form costs 1024.
+//   * What the split cannot represent - an infinity or NaN among the operands, whose
+//     remainders are NaN, or a sum that overflows - always ends as a value that is not finite.  A wave
+//     that sees one sets a flag, and the launch of the fp32 kernel that follows every launch of
+//     these runs only then and recomputes the whole product.
+//   * Parts below 2^-133 are lost: operands smaller than 2^-110 keep fewer than 24 bits.
+//   * A lane gathers, interpolates and splits exactly the elements its matrix B operand holds
+//     (lane (l31, lhi): channels lhi * 8 .. + 7 of pixel l31 of the wave), so samples never pass
+//     through LDS; only the weights do, pre-split by the packing launch.
+// Bound: the matrix instructions (384 clocks a unit) and the vector instructions around them
+// (some 60 x 4), which all but take turns, and what three waves per SIMD leave exposed of the
+// loads' latency.  Measured, fp32 instructions -> these: 8 x 64 channels of 256 x 512 -> 64, nine
+// taps: forward 798 -> 597 us, input gradient 768 -> 597 us; 4 x 64 -> 32 channels onto 256 x 512
+// (transposed) 379 -> 269 us; mesh of 40 962 vertices, 4 x 64 -> 128 channels, four points a tap:
+// forward 411 -> 292 us, input gradient (both levels in one pass) 952 -> 509 us.  Distance from
+// the 64-bit result, in 2-norm: 4.3e-7 -> 3.6e-7 (576 terms).
+// Included by mcx_conv_mfma.hip, inside its anonymous namespace.
+
+struct SplitArgs {
+  const float *src, *map, *iw;
+  const float2 *map2;     // second-level entries of a transposed map, or NULL (channel-last only)
+  const uint16_t *w;      // split weights, see pack_split_weight
+  const float *bias;
+  float *y;
+  const float *addend;    // see gather_product_mfma_kernel, like the gates and masks below
+  const int *gate, *pair_mask, *row_mask;
+  int *nonfinite;
+  int G, O, Opad, Gpad, SH, SW, OH, OW, K, np, ncorn, weighted, wrap, packed;
+  int tiles_x, tiles_per_img, tw_shift, run_if_zero, mask_words;
+};
+
+// x = p[0] + p[1] + p[2] for 8 values: words of two bf16 each
+__device__ inline void split8(const float *x, bf16x8 *p) {
+  unsigned h[4], m[4], l[4];
+  // {-1, 0} and {0, -1} from registers: as immediates the compiler renders both as the inline
+  // constant -1.0, which the instruction takes for one and the same word.
+  unsigned neg_lo = 0x0000bf80u, neg_hi = 0xbf800000u;
+  asm("" : "+s"(neg_lo), "+s"(neg_hi));
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    // (a remainder is the dot product of the pair word with {-1, 0} or {0, -1} plus the value)
+    h[j] = __builtin_bit_cast(unsigned,
+                              __builtin_convertvector(floatx2{x[2 * j], x[2 * j + 1]}, bf16x2));
+    const float r0 = dot_bf16(h[j], neg_lo, x[2 * j]);
+    const float r1 = dot_bf16(h[j], neg_hi, x[2 * j + 1]);
+    m[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r0, r1}, bf16x2));
+    const float q0 = dot_bf16(m[j], neg_lo, r0);
+    const float q1 = dot_bf16(m[j], neg_hi, r1);
+    l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{q0, q1}, bf16x2));
+  }
+  p[0] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+  p[1] = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
+  p[2] = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// Channel (of G) that element j of half kg of chunk c stands for, or -1 (a weight of zero).
+// Planar sources read the second half of a partial last chunk `rem - 8` channels after the
+// first, so that no lane reads past the last channel (see split_upper_half).
+__host__ __device__ inline int split_channel(int c, int kg, int j, int G, int planar) {
+  const int g0 = c * 16, rem = G - g0;
+  if (!planar || rem >= 16) return g0 + kg * 8 + j < G ? g0 + kg * 8 + j : -1;
+  if (kg == 0) return j < rem ? g0 + j : -1;
+  if (rem <= 8) return -1;
+  return g0 + rem - 8 + j >= g0 + 8 ? g0 + rem - 8 + j : -1;
+}
+// Channels between the two halves of chunk c of a planar source.
+__device__ inline int split_upper_half(int c, int G) {
+  const int rem = G - c * 16;
+  return rem >= 16 ? 8 : rem > 8 ? rem - 8 : 0;
+}
+
+// The weights of a unit through LDS: [part][kg][output][8 channels], double buffered.
+template <int OG>
+struct SplitWeights {
+  static constexpr int kPieces = 3 * 2 * kOT * OG;                        // of 16 bytes
+  static constexpr int kPer = (kPieces + kThreads - 1) / kThreads;        // per thread
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  unsigned off[kPer];
+  int tid;
+  bool last_round;  // (wave-uniform) this wave stores a piece in the last, partial round
+  __device__ inline void init(int t, int Opad, int o0) {
+    tid = t;
+    last_round = __builtin_amdgcn_readfirstlane(t >> 6) * 64 + (kPer - 1) * kThreads < kPieces;
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+      const int i = min(t + j * kThreads, kPieces - 1);  // (a last, partial round is not stored)
+      off[j] = (unsigned)((i / (kOT * OG)) * Opad + o0 + i % (kOT * OG)) * 16u;
+    }
+  }
+  __device__ inline void load(plane_buf_t r, unsigned unit_off, u32x4 *v) const {
+#pragma unroll
+    for (int j = 0; j < kPer; j++)
+      v[j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], (int)unit_off, 0));
+  }
+  __device__ inline void store(uint4 *lds, const u32x4 *v) const {
+#pragma unroll
+    for (int j = 0; j < kPer; j++)
+      if ((j + 1) * kThreads <= kPieces || last_round)
+        *reinterpret_cast<u32x4 *>(lds + tid + j * kThreads) = v[j];
+  }
+};
+
+template <int OG>
+__device__ inline void split_products(const uint4 *lds, const bf16x8 *b, int l31, int lhi,
+                                      floatx16 *acc) {
+  bf16x8 a[2 * OG][3];
+#pragma unroll
+  for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+    for (int part = 0; part < 3; part++)
+      a[m][part] =
+          __builtin_bit_cast(bf16x8, lds[(part * 2 + lhi) * (kOT * OG) + 32 * m + l31]);
+  // (smallest first; the chains of the output blocks are independent)
+  constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+  for (int t = 0; t < 6; t++)
+#pragma unroll
+    for (int m = 0; m < 2 * OG; m++)
+      acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m][pa[t]], b[pb[t]], acc[m], 0, 0, 0);
+}
+
+// Bias, addend and stores of a lane's pixel; flags results that are not finite.
+template <int OG>
+__device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, int b, int o0,
+                                      int ei, int ej, int lhi) {
+  const int64_t N = (int64_t)s.OH * s.OW;
+  bool bad = false;
+  if (ei < s.OH && ej < s.OW) {
+    const int64_t n = (int64_t)ei * s.OW + ej;
+    float *yb = s.y + (int64_t)b * s.O * N + n;
+    const float *ab = (s.addend && s.gate && s.gate[1] > 0)
+                          ? s.addend + ((int64_t)b * N + n) * s.Opad
+                          : nullptr;
+#pragma unroll
+    for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int o = o0 + 32 * m + (i >> 2) * 8 + lhi * 4 + (i & 3);
+        bad |= !(__builtin_fabsf(acc[m][i]) <= 3.402823466e+38f);
+        if (o < s.O)
+          yb[(int64_t)o * N] = acc[m][i] + (s.bias ? s.bias[o] : 0.f) + (ab ? ab[o] : 0.f);
+      }
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) != 0 && (threadIdx.x & 63) == 0)
+    *s.nonfinite = 1;  // (every writer stores the same value)
+}
+
+// Planar images.  NE: (offset, weight) entries per tap, 1 or 4; with 4, tiles none of whose taps
+// uses a later entry run with the leading two.  Two entries of a tap that are neighbours in
+// memory for every pixel of the tile (the corners of a row, two contributions of a
+// transposed map) are fetched with one 8-byte load: the texture path takes 16 clocks for a
+// wave's load whatever its width, and 16 single loads a unit would cost it as much as the fp32
+// matrix instructions did.
+template <int NE, int OG>
+__global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gather_product_split_kernel(
+    const SplitArgs s) {
+  constexpr int kCache = NE == 1 ? 6 : kTapCache;  // cached entries per pixel
+  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<OG>::kPieces];
+  __shared__ __attribute__((aligned(16))) unsigned TapOff[kCache * kTilePx];
+  __shared__ __attribute__((aligned(16))) float TapWt[kCache * kTilePx];
+  __shared__ int unpaired;
+  if (s.gate && ((*s.gate == 0) != (s.run_if_zero != 0))) return;
+  const int tid = threadIdx.x;
+  const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const int b = tile / s.tiles_per_img;
+  const int t_in = tile - b * s.tiles_per_img;
+  const int tile_y = t_in / s.tiles_x, tile_x = t_in - tile_y * s.tiles_x;
+  const int tw_mask = (1 << s.tw_shift) - 1, th = kTilePx >> s.tw_shift;
+  bool leading = false;
+  if (NE == 4 && s.pair_mask) {
+    leading = !later_pairs_in_use(s.pair_mask, s.mask_words);
+    if (!leading && s.row_mask) {
+      int any = 0;
+      for (int r = tile_y * th; r < min(tile_y * th + th, s.OH); r++) any |= s.row_mask[r];
+      leading = any == 0;
+    }
+  }
+  const int o0 = blockIdx.y * (kOT * OG);
+  const int N = s.OH * s.OW;
+  const unsigned plane_bytes = (unsigned)s.SH * (unsigned)s.SW * 4u;
+  const int chunks = s.Gpad / kGC;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, lhi = lane >> 5;
+  const int pe = wave * 32 + l31;
+  const auto img = plane_buf(s.src + (int64_t)b * s.G * s.SH * s.SW, (unsigned)s.G * plane_bytes);
+  const auto wbuf = plane_buf(s.w, (unsigned)s.K * chunks * 6u * s.Opad * 16u);
+  const unsigned w_unit = 6u * s.Opad * 16u;
+
+  // resolving role: pixel p of the tile, every other tap
+  const int p = tid & (kTilePx - 1), half = tid >> 7;
+  const int gi = tile_y * th + (p >> s.tw_shift), gj = (tile_x << s.tw_shift) + (p & tw_mask);
+  const bool live = gi < s.OH && gj < s.OW;
+  const int64_t n_g = live ? (int64_t)gi * s.OW + gj : 0;
+
+  floatx16 acc[2 * OG];
+#pragma unroll
+  for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[m][i] = 0.f;
+  SplitWeights<OG> wts;
+  wts.init(tid, s.Opad, o0);
+  int buf = 0;
+
+  // units of a tap group: chunk-major, the tap fastest (a chunk's source rows stay in cache)
+  auto units_of = [&](int k0, int kn, auto na_tag, auto paired_tag) __attribute__((always_inline)) {
+    constexpr int NA = decltype(na_tag)::value;
+    constexpr bool PAIRED = decltype(paired_tag)::value;
+    constexpr int NL = PAIRED ? NA / 2 : NA;  // loads per channel
+    // Units whose loads are in flight.  With one, every unit waits out what its 12 matrix
+    // instructions do not cover of a load's latency: 657 us a product at 8 x 64 channels of
+    // 256 x 512 -> 64, 9 taps.  (Two of four single loads a channel do not fit the registers.)
+    constexpr int kDepth = NL * (PAIRED ? 2 : 1) <= 2 ? 2 : 1;
+    const int units = chunks * kn;
+    float v[kDepth][8][NA];
+    float wgt[kDepth][NA];
+    typename SplitWeights<OG>::u32x4 wv[kDepth][SplitWeights<OG>::kPer];
+    int kl = 0, c = 0;  // the unit whose loads are issued next
+    // (issued unconditionally, past the last unit too, where it reads the last chunk again: a
+    // load behind a branch would make every wait a full one)
+    auto issue = [&](int d) __attribute__((always_inline)) {
+      const int cc = min(c, chunks - 1);
+      unsigned off[NL];
+      const unsigned upper =
+          (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)split_upper_half(cc, s.G) *
+                                                         plane_bytes));
+#pragma unroll
+      for (int i = 0; i < NL; i++)
+        off[i] = TapOff[(kl * kTilePx + pe) * NA + (PAIRED ? 2 * i : i)] + (lhi ? upper : 0u);
+#pragma unroll
+      for (int i = 0; i < NA; i++) wgt[d][i] = TapWt[(kl * kTilePx + pe) * NA + i];
+      wts.load(wbuf, __builtin_amdgcn_readfirstlane((unsigned)((k0 + kl) * chunks + cc) * w_unit),
+               wv[d]);
+      const int last = s.G - 1 - cc * kGC;  // (channels past the last one: weights of zero)
+#pragma unroll
+      for (int ch = 0; ch < 8; ch++) {
+        const unsigned so = __builtin_amdgcn_readfirstlane((unsigned)(cc * kGC + min(ch, last)) *
+                                                           plane_bytes);
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+          if constexpr (PAIRED) {
+            const float_pair q = __builtin_bit_cast(
+                float_pair, __builtin_amdgcn_raw_buffer_load_b64(img, (int)off[i], (int)so, 0));
+            v[d][ch][2 * i] = q.x;
+            v[d][ch][2 * i + 1] = q.y;
+          } else {
+            v[d][ch][i] = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(img, (int)off[i], (int)so, 0));
+          }
+        }
+      }
+      if (++kl == kn) {
+        kl = 0;
+        ++c;
+      }
+    };
+    bf16x8 bq[3];
+    auto stage = [&](int d) __attribute__((always_inline)) {
+      float sv[8];
+#pragma unroll
+      for (int ch = 0; ch < 8; ch++) {
+        sv[ch] = wgt[d][0] * v[d][ch][0];
+#pragma unroll
+        for (int i = 1; i < NA; i++) sv[ch] = __builtin_fmaf(wgt[d][i], v[d][ch][i], sv[ch]);
+      }
+      split8(sv, bq);
+      wts.store(Wt[buf], wv[d]);
+    };
+#pragma unroll
+    for (int d = 0; d < kDepth; d++) issue(d);
+    int u = 0;
+    for (; u + kDepth <= units; u += kDepth) {
+#pragma unroll
+      for (int d = 0; d < kDepth; d++) {
+        stage(d);
+        __syncthreads();
+        issue(d);
+        split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+        buf ^= 1;
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < kDepth - 1; d++) {
+      if (u + d < units) {
+        stage(d);
+        __syncthreads();
+        split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+        buf ^= 1;
+      }
+    }
+  };
+
+  auto run = [&](auto na_tag) __attribute__((always_inline)) {
+    constexpr int NA = decltype(na_tag)::value;
+    constexpr int TG = kCache / NA;
+    for (int k0 = 0; k0 < s.K; k0 += TG) {
+      const int kn = min(TG, s.K - k0);
+      __syncthreads();  // the previous group's units are done with the cache
+      if (tid == 0) unpaired = NA == 1 ? 1 : 0;
+      __syncthreads();
+      for (int kl = half; kl < kn; kl += 2) {
+        unsigned off[4];
+        float wt[4];
+        if (s.packed) {
+          // pre-resolved entries [tap][slot][pixel]: (pixel index as bits, weight)
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            const float2 q =
+                reinterpret_cast<const float2 *>(s.map)[((int64_t)(k0 + kl) * 4 + i) * N + n_g];
+            off[i] = __builtin_bit_cast(unsigned, q.x) * 4u;
+            wt[i] = live ? q.y : 0.f;
+          }
+        } else {
+          const int64_t e = n_g * s.K + k0 + kl;
+          const float scale = live ? (s.weighted ? s.iw[e] : 1.f) : 0.f;
+          PairTap<NE> t;
+          resolve_pairs<NE, 4>(s.map[e * 2], s.map[e * 2 + 1], s.SH, s.SW, s.wrap != 0, scale, t);
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            off[i] = t.off[i];
+            wt[i] = t.wt[i];
+          }
+        }
+        if constexpr (NA > 1) {
+          bool fits = plane_bytes >= 8u;
+#pragma unroll
+          for (int i = 0; i < NA; i += 2) {
+            // entries i and i + 1 as two neighbours, where they are (an entry of weight zero
+            // may move anywhere)
+            const bool u0 = wt[i] != 0.f, u1 = wt[i + 1] != 0.f;
+            if (u0 && u1) {
+              if (off[i] == off[i + 1] + 4u) {
+                const unsigned o = off[i];
+                const float w = wt[i];
+                off[i] = off[i + 1];
+                wt[i] = wt[i + 1];
+                off[i + 1] = o;
+                wt[i + 1] = w;
+              }
+              fits = fits && off[i] + 4u == off[i + 1];
+            } else if (plane_bytes >= 8u) {
+              const unsigned o = u0 ? off[i] : u1 ? off[i + 1] : 0u;
+              const float w = u0 ? wt[i] : u1 ? wt[i + 1] : 0.f;
+              const bool end = o + 4u >= plane_bytes;  // the plane's last pixel: its left neighbour
+              off[i] = end ? o - 4u : o;
+              off[i + 1] = off[i] + 4u;
+              wt[i] = end ? 0.f : w;
+              wt[i + 1] = end ? w : 0.f;
+            }
+          }
+          if (!fits) unpaired = 1;  // (every writer stores the same value)
+        }
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+          TapOff[(kl * kTilePx + p) * NA + i] = off[i];
+          TapWt[(kl * kTilePx + p) * NA + i] = wt[i];
+        }
+      }
+      __syncthreads();
+      if constexpr (NA > 1) {
+        if (!__builtin_amdgcn_readfirstlane(unpaired)) {
+          units_of(k0, kn, na_tag, std::true_type());
+          continue;
+        }
+      }
+      units_of(k0, kn, na_tag, std::false_type());
+    }
+  };
+  if (NE == 4 && leading)
+    run(std::integral_constant<int, NE == 4 ? 2 : 1>());
+  else
+    run(std::integral_constant<int, NE>());
+  split_epilogue<OG>(s, acc, b, o0, tile_y * th + (pe >> s.tw_shift),
+                     (tile_x << s.tw_shift) + (pe & tw_mask), lhi);
+}
+
+// Channel-last sources (mesh signals): a lane's 8 channels of an entry are 32 contiguous bytes
+// of a record.  Tap-major, a tap's entries in registers; NE entries a tap, and with TWO (a
+// transposed map with a second level) four more where any lane of the wave uses one: both levels
+// go through one product.
+template <int NE, bool TWO, int OG>
+__global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_product_split_cl_kernel(const SplitArgs s) {
+  constexpr int NT = TWO ? NE + 4 : NE;
+  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<OG>::kPieces];
+  if (s.gate && ((*s.gate == 0) != (s.run_if_zero != 0))) return;
+  const int tid = threadIdx.x;
+  const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const int b = tile / s.tiles_per_img;
+  const int t_in = tile - b * s.tiles_per_img;
+  const int tile_y = t_in / s.tiles_x, tile_x = t_in - tile_y * s.tiles_x;
+  const int tw_mask = (1 << s.tw_shift) - 1, th = kTilePx >> s.tw_shift;
+  const int o0 = blockIdx.y * (kOT * OG);
+  const int N = s.OH * s.OW;
+  const int chunks = s.Gpad / kGC;
+  const unsigned record = (unsigned)s.Gpad * 4u;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, lhi = lane >> 5;
+  const int pe = wave * 32 + l31;
+  const int ei = tile_y * th + (pe >> s.tw_shift), ej = (tile_x << s.tw_shift) + (pe & tw_mask);
+  const bool live = ei < s.OH && ej < s.OW;
+  const int64_t n = live ? (int64_t)ei * s.OW + ej : 0;
+  const int64_t pixels = (int64_t)s.SH * s.SW;
+  const auto img = plane_buf(s.src + (int64_t)b * pixels * s.Gpad, (unsigned)pixels * record);
+  const auto wbuf = plane_buf(s.w, (unsigned)s.K * chunks * 6u * s.Opad * 16u);
+  const unsigned w_unit = 6u * s.Opad * 16u;
+
+  floatx16 acc[2 * OG];
+#pragma unroll
+  for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[m][i] = 0.f;
+  SplitWeights<OG> wts;
+  wts.init(tid, s.Opad, o0);
+
+  // entries of a tap as they come from memory, fetched a tap ahead
+  float2 raw[NT];
+  float raw_w[NE];
+  auto fetch = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      if (s.packed) {
+        raw[i] = reinterpret_cast<const float2 *>(s.map)[((int64_t)k * 4 + i) * N + n];
+        raw_w[i] = 0.f;
+      } else {
+        const int64_t e = (n * s.K + k) * NE + i;
+        raw[i] = reinterpret_cast<const float2 *>(s.map)[e];
+        raw_w[i] = s.weighted ? s.iw[e] : 1.f;
+      }
+    }
+    if constexpr (TWO) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) raw[NE + i] = s.map2[((int64_t)k * 4 + i) * N + n];
+    }
+  };
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  unsigned off[NT];
+  float wgt[NT];
+  f32x4 v[NT][2];
+  typename SplitWeights<OG>::u32x4 wv[SplitWeights<OG>::kPer];
+  bool more = false;  // (wave-uniform) an entry beyond the first NE is in use
+  auto resolve = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+      if (s.packed || i >= NE) {
+        off[i] = __builtin_bit_cast(unsigned, raw[i].x) * record;
+        wgt[i] = live ? raw[i].y : 0.f;
+      } else {
+        PairTap<1> t;
+        resolve_pairs<1, 1>(raw[i].x, raw[i].y, s.SH, s.SW, false, live ? raw_w[i < NE ? i : 0] : 0.f, t);
+        off[i] = t.off[0] * record;
+        wgt[i] = t.wt[0];
+      }
+      off[i] += lhi ? 32u : 0u;
+    }
+    if constexpr (TWO) {
+      bool any = false;
+#pragma unroll
+      for (int i = NE; i < NT; i++) any |= wgt[i] != 0.f;
+      more = __builtin_amdgcn_ballot_w64(any) != 0;
+    }
+  };
+  auto issue = [&](int k, int c) __attribute__((always_inline)) {
+    const int so = __builtin_amdgcn_readfirstlane(c * (kGC * 4));
+    auto load = [&](int i) __attribute__((always_inline)) {
+      v[i][0] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(img, (int)off[i], so, 0));
+      v[i][1] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(img, (int)(off[i] + 16u), so, 0));
+    };
+    wts.load(wbuf, __builtin_amdgcn_readfirstlane((unsigned)(k * chunks + c) * w_unit), wv);
+#pragma unroll
+    for (int i = 0; i < NE; i++) load(i);
+    if constexpr (TWO) {
+      if (more) {
+#pragma unroll
+        for (int i = NE; i < NT; i++) load(i);
+      }
+    }
+  };
+
+  fetch(0);
+  resolve();
+  fetch(min(1, s.K - 1));
+  issue(0, 0);
+  const int units = s.K * chunks;
+  int k = 0, c = 0, buf = 0;
+  for (int u = 0; u < units; u++) {
+    float sv[8];
+#pragma unroll
+    for (int ch = 0; ch < 8; ch++) {
+      sv[ch] = wgt[0] * v[0][ch >> 2][ch & 3];
+#pragma unroll
+      for (int i = 1; i < NE; i++) sv[ch] = __builtin_fmaf(wgt[i], v[i][ch >> 2][ch & 3], sv[ch]);
+    }
+    if constexpr (TWO) {
+      if (more) {
+#pragma unroll
+        for (int i = NE; i < NT; i++)
+#pragma unroll
+          for (int ch = 0; ch < 8; ch++)
+            sv[ch] = __builtin_fmaf(wgt[i], v[i][ch >> 2][ch & 3], sv[ch]);
+      }
+    }
+    bf16x8 bq[3];
+    split8(sv, bq);
+    wts.store(Wt[buf], wv);
+    __syncthreads();
+    if (u + 1 < units) {
+      if (++c == chunks) {
+        c = 0;
+        ++k;
+        resolve();
+        fetch(min(k + 1, s.K - 1));
+      }
+      issue(k, c);
+    }
+    split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+    buf ^= 1;
+  }
+  split_epilogue<OG>(s, acc, b, o0, ei, ej, lhi);
+}

@@ -18,6 +18,8 @@ class MappedMaxPoolFunction(torch.autograd.Function):
         else:
             pooled, idx_mask = _C.mapped_max_pool(input, sample_map, kernel_size, interp)
         ctx.mark_non_differentiable(idx_mask)
+        # (else autograd fills an int64 tensor of zeros, as large as idx_mask, on every backward)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(idx_mask, sample_map, interp_weights)
         ctx.input_hw = (int(input.shape[2]), int(input.shape[3]))
         ctx.kernel_size, ctx.interp = int(kernel_size), int(interp)
@@ -25,6 +27,8 @@ class MappedMaxPoolFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, idx_mask_grad=None):
+        if grad_output is None:
+            return None, None, None, None, None
         idx_mask, sample_map, interp_weights = ctx.saved_tensors
         ih, iw = ctx.input_hw
         grad_output = grad_output.contiguous()

@@ -1,0 +1,114 @@
+"""fp32 products on the bf16 matrix instructions (operands split into three bf16 parts): partial
+chunks of channels, taps whose entries are neighbours in memory or not, columns at the seam and
+at the last pixel of a plane, second levels of a mesh's transposed map, and operands the split
+cannot represent."""
+import pytest
+import torch
+
+import helpers
+from helpers import rel_err
+from oracle import ops as O
+
+from mappedconvolutions_amd import _C
+from mappedconvolutions_amd.util import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(h, w, k, dx, dy):
+    y, x = torch.meshgrid(torch.arange(h).float(), torch.arange(w).float(), indexing="ij")
+    taps = [torch.stack((x + i % 3 - 1 + dx, y + i // 3 - 1 + dy), -1) for i in range(k)]
+    return torch.stack(taps, 2).contiguous()
+
+
+# channels around 8 and 16 (the halves of a chunk), outputs around 64 and 128, widths whose rows
+# end inside a tile; 32-bit sums of up to 9 * 40 terms: a few 1e-7 of the result's magnitude,
+# 1e-5 allowed like everywhere in these tests
+@pytest.mark.parametrize("ci,co", [(1, 1), (7, 5), (8, 64), (9, 65), (15, 128), (16, 130), (17, 3),
+                                   (24, 40), (31, 64), (40, 129)])
+@pytest.mark.parametrize("interp,dx,dy", [(0, 0.0, 0.0), (1, 0.25, 0.0), (1, 0.4, 0.3),
+                                          (2, 0.25, 0.0), (2, -0.3, 0.6)])
+def test_split_products_over_images(ci, co, interp, dx, dy, device):
+    g = torch.Generator().manual_seed(ci * 1000 + co)
+    B, h, w_, k = 2, 5, 37, 9
+    smap = _grid(h, w_, k, dx, dy)
+    rnd = lambda *s: torch.randn(s, generator=g)
+    x, w, b, gy = rnd(B, ci, h, w_), rnd(co, ci, k), rnd(co), rnd(B, co, h, w_)
+    y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
+    assert rel_err(y, O.mapped_conv_forward(x, smap, w, b, k, interp)) < 1e-5
+    gx = _C.mapped_conv_backward(gy.cuda(), smap.cuda(), x.cuda(), w.cuda(), b.cuda(), k, interp,
+                                 needs=(True, False, False))[0]
+    assert rel_err(gx, O.mapped_conv_backward(gy, smap, x, w, b, k, interp)[0]) < 1e-5
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 2), (2, 1), (3, 2)])
+def test_split_products_over_the_smallest_planes(shape, device):
+    """A plane of one pixel has no neighbour to fetch along; the last pixel has none to its right."""
+    g = torch.Generator().manual_seed(3)
+    h, w_ = shape
+    k, ci, co = 9, 5, 6
+    smap = _grid(h, w_, k, 0.25, 0.5)
+    x, w, b = (torch.randn(s, generator=g) for s in ((2, ci, h, w_), (co, ci, k), (co,)))
+    for interp in (0, 1, 2):
+        y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
+        assert rel_err(y, O.mapped_conv_forward(x, smap, w, b, k, interp)) < 1e-5
+
+
+@pytest.mark.parametrize("per_cell", [1, 3, 4, 5, 8, 11])
+@pytest.mark.parametrize("ci,co", [(16, 64), (20, 128)])
+def test_split_products_over_meshes(per_cell, ci, co, device):
+    """`per_cell` contributions to every cell of the transposed map: within its first four slots,
+    in the second level, beyond it (the overflow list)."""
+    g = torch.Generator().manual_seed(per_cell)
+    V, k = 300, 3
+    idx = (torch.arange(V) // per_cell).view(1, V, 1, 1).expand(1, V, k, 1).float()
+    smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    iw = torch.rand(1, V, k, 1, generator=g)
+    x, w, b, gy = (torch.randn(s, generator=g)
+                   for s in ((2, ci, 1, V), (co, ci, k), (co,), (2, co, 1, V)))
+    y = _C.weighted_mapped_conv_forward(*[t.cuda() for t in (x, smap, iw, w, b)], k, 0)
+    assert rel_err(y, O.weighted_mapped_conv_forward(x, smap, iw, w, b, k, 0)) < 1e-5
+    gx = _C.weighted_mapped_conv_backward(*[t.cuda() for t in (gy, smap, iw, x, w, b)], k, 0,
+                                          needs=(True, False, False))[0]
+    assert rel_err(gx, O.weighted_mapped_conv_backward(gy, smap, iw, x, w, b, k, 0)[0]) < 1e-5
+
+
+@pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_inf", "overflow", "large"])
+def test_operands_without_a_split(what, device):
+    """An infinity or NaN among the operands and sums beyond fp32 come out as the fp32
+    instructions have them: infinite or NaN exactly where the sum over the taps is, finite values
+    unchanged.  (Values of 3e38 round up to an infinite bf16.)"""
+    g = torch.Generator().manual_seed(1)
+    B, ci, co, h, w_, k = 1, 16, 64, 6, 40, 9
+    smap = _grid(h, w_, k, 0.25, 0.25)
+    x, w, b = (torch.randn(s, generator=g) for s in ((B, ci, h, w_), (co, ci, k), (co,)))
+    if what == "x_inf":
+        x[0, 3, 2, 7] = float("inf")
+    elif what == "x_nan":
+        x[0, 0, 5, 39] = float("nan")
+    elif what == "w_inf":
+        w[5, 3, 4], x = float("-inf"), x.abs()
+    elif what == "overflow":
+        x[0, :, 3, 20], w = 3e38, w.abs()
+    else:
+        x[0, 2, 3, 20], w = 3.4e38, w * 1e-3
+    y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, 1).cpu()
+    want = O.mapped_conv_forward(x, smap, w, b, k, 1)
+    ok = torch.isfinite(want)
+    if what != "w_inf":  # (there a zero-weighted corner outside the image meets the infinity)
+        assert torch.equal(torch.isfinite(y), ok)
+    both = ok & torch.isfinite(y)
+    assert both.any()
+    assert ((y - want).abs()[both] <= 1e-5 * want.abs()[both].max()).all()
+
+
+def test_accuracy_is_not_below_fp32(device):
+    """Against 64 bits the split products are at least as close as fp32 sums of the same length:
+    2-norm 1e-6 of the result at 576 terms (fp32 instructions 4.3e-7, split 3.6e-7 measured)."""
+    g = torch.Generator().manual_seed(9)
+    h, w_, c, k = 32, 64, 64, 9
+    smap = synthetic.latitude_map(h, w_, 1)
+    x, w, b = (torch.randn(s, generator=g) for s in ((1, c, h, w_), (c, c, k), (c,)))
+    y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, 1).double().cpu()
+    want = O.mapped_conv_forward(x.double(), smap.double(), w.double(), b.double(), k, 1)
+    assert ((y - want).norm() / want.norm()).item() < 1e-6
