@@ -26,10 +26,14 @@ constexpr int kThreads = 256;
 __host__ __device__ constexpr size_t align_up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Grid search (second half of this file): per batch element, at the start of its workspace slice
+// Workgroups (per batch element) that share the bounding box and the clearing of the counters;
+// the counting launch puts the boxes together, a lane each.
+constexpr int kBoxParts = 64;
 template <typename T>
 struct GridHead {
   T lo[3], inv_h[3], h[3];
   int skewed;  // nonzero: a quarter of the points share one cell; the plain walk runs instead
+  T part_lo[3][kBoxParts], part_hi[3][kBoxParts];  // bounding boxes of runs of the points
 };
 template <typename T>
 struct alignas(sizeof(T) * 4) GridPoint {
@@ -229,14 +233,14 @@ __device__ inline int cell_of(const GridHead<T> &h, const int *g, const T *c, in
   return cell;
 }
 
-// One workgroup per batch element: bounding box of the finite reference points, cell size,
-// counters cleared.
+// Bounding box of a run of the finite reference points, and a run of the counters cleared.
+// (One workgroup for all of them took 24 us at 40 962 points and 85 184 cells.)
 template <typename T, int D>
-__global__ __launch_bounds__(kGridThreads) void knn_grid_box_kernel(
-    const T *__restrict__ ref, char *__restrict__ ws, size_t slice, int R, int g0, int g1, int g2,
-    int cells) {
-  __shared__ T smin[D][kGridThreads / 64], smax[D][kGridThreads / 64];
-  const int b = blockIdx.x;
+__global__ __launch_bounds__(256) void knn_grid_box_kernel(const T *__restrict__ ref,
+                                                           char *__restrict__ ws, size_t slice,
+                                                           int R, int cells) {
+  __shared__ T smin[D][4], smax[D][4];
+  const int b = blockIdx.y, part = blockIdx.x;
   const T *rb = ref + (int64_t)b * D * R;
   char *base = ws + (size_t)b * slice;
   GridHead<T> *head = reinterpret_cast<GridHead<T> *>(base);
@@ -249,7 +253,7 @@ __global__ __launch_bounds__(kGridThreads) void knn_grid_box_kernel(
     mn[d] = inf_t<T>();
     mx[d] = -inf_t<T>();
   }
-  for (int r = threadIdx.x; r < R; r += kGridThreads) {
+  for (int r = part * 256 + threadIdx.x; r < R; r += kBoxParts * 256) {
     T c[D];
     bool ok = true;
 #pragma unroll
@@ -278,31 +282,41 @@ __global__ __launch_bounds__(kGridThreads) void knn_grid_box_kernel(
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int g[3] = {g0, g1, g2};
-    for (int d = 0; d < 3; d++) {
-      T lo = T(0), hi = T(0);
-      if (d < D) {
-        lo = smin[d][0];
-        hi = smax[d][0];
-        for (int w = 1; w < kGridThreads / 64; w++) {
-          lo = smin[d][w] < lo ? smin[d][w] : lo;
-          hi = smax[d][w] > hi ? smax[d][w] : hi;
-        }
-      }
-      const T width = hi - lo;  // not finite: no finite point, or the box overflows
-      const bool usable = d < D && width > T(0) && finite_t(width);
-      head->lo[d] = usable ? lo : T(0);
-      head->h[d] = usable ? width / (T)g[d] : T(0);
-      head->inv_h[d] = usable ? (T)g[d] / width : T(0);  // unusable: everything in cell 0
+  if (threadIdx.x < D) {
+    const int d = threadIdx.x;
+    T lo = smin[d][0], hi = smax[d][0];
+    for (int w = 1; w < 4; w++) {
+      lo = smin[d][w] < lo ? smin[d][w] : lo;
+      hi = smax[d][w] > hi ? smax[d][w] : hi;
     }
-    head->skewed = 0;
+    head->part_lo[d][part] = lo;
+    head->part_hi[d][part] = hi;
   }
-  for (int c = threadIdx.x; c < cells; c += kGridThreads) {
-    start[c] = 0;
-    cursor[c] = 0;
+  for (int c = part * 256 + threadIdx.x; c < cells; c += kBoxParts * 256) cursor[c] = 0;
+}
+
+// The grid from the parts of the bounding box, by one wave: valid in its every lane.
+template <typename T, int D>
+__device__ inline void grid_of_box(const GridHead<T> &parts, const int *g, int lane, T *glo, T *gh,
+                                   T *ginv) {
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    T lo = T(0), hi = T(0);
+    if (d < D) {
+      lo = parts.part_lo[d][lane];
+      hi = parts.part_hi[d][lane];
+      for (int o = 32; o > 0; o >>= 1) {
+        const T a = __shfl_xor(lo, o), c = __shfl_xor(hi, o);
+        lo = a < lo ? a : lo;
+        hi = c > hi ? c : hi;
+      }
+    }
+    const T width = hi - lo;  // not finite: no finite point, or the box overflows
+    const bool usable = d < D && width > T(0) && finite_t(width);
+    glo[d] = usable ? lo : T(0);
+    gh[d] = usable ? width / (T)g[d] : T(0);
+    ginv[d] = usable ? (T)g[d] / width : T(0);  // unusable: everything in cell 0
   }
-  if (threadIdx.x == 0) start[cells] = 0;
 }
 
 template <typename T, int D>
@@ -310,18 +324,31 @@ __global__ __launch_bounds__(256) void knn_grid_count_kernel(const T *__restrict
                                                             char *__restrict__ ws, size_t slice,
                                                             int R, int g0, int g1, int g2,
                                                             int cells, int fill) {
+  static_assert(kBoxParts == 64, "a lane takes a part");
   const int b = blockIdx.y;
   const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= R) return;
   const T *rb = ref + (int64_t)b * D * R;
   char *base = ws + (size_t)b * slice;
-  const GridHead<T> &head = *reinterpret_cast<const GridHead<T> *>(base);
+  GridHead<T> *head = reinterpret_cast<GridHead<T> *>(base);
   int *start = reinterpret_cast<int *>(base + align_up256(sizeof(GridHead<T>)));
   int *cursor = reinterpret_cast<int *>(reinterpret_cast<char *>(start) +
                                         align_up256((size_t)(cells + 1) * 4));
   GridPoint<T> *pts = reinterpret_cast<GridPoint<T> *>(reinterpret_cast<char *>(cursor) +
                                                        align_up256((size_t)cells * 4));
   const int g[3] = {g0, g1, g2};
+  // (every wave puts the box together for itself; the counting launch leaves the grid in the
+  // head for the launches that follow it)
+  GridHead<T> h;
+  grid_of_box<T, D>(*head, g, threadIdx.x & 63, h.lo, h.h, h.inv_h);
+  if (!fill && blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int d = 0; d < 3; d++) {
+      head->lo[d] = h.lo[d];
+      head->h[d] = h.h[d];
+      head->inv_h[d] = h.inv_h[d];
+    }
+    head->skewed = 0;
+  }
+  if (r >= R) return;
   T c[3] = {T(0), T(0), T(0)};
   bool ok = true;
 #pragma unroll
@@ -331,90 +358,79 @@ __global__ __launch_bounds__(256) void knn_grid_count_kernel(const T *__restrict
   }
   if (!ok) return;
   int cd[3];
-  const int cell = cell_of<T, D>(head, g, c, cd);
+  const int cell = cell_of<T, D>(h, g, c, cd);
   if (!fill) {
-    atomicAdd(&start[cell], 1);  // counts now, offsets after the scan
+    atomicAdd(&cursor[cell], 1);
   } else {
     GridPoint<T> p;
     p.c[0] = c[0]; p.c[1] = c[1]; p.c[2] = c[2];
     p.idx = r + 1;
-    pts[start[cell] + atomicAdd(&cursor[cell], 1)] = p;
+    pts[start[cell] + atomicAdd(&cursor[cell], -1) - 1] = p;
   }
 }
 
-// counts -> offsets (exclusive prefix sum, start[cells] = number of binned points), one
-// workgroup per batch element, 1024 cells per step; also decides whether the grid is worth
-// walking.
+// counts (in cursor) -> offsets (exclusive prefix sum; start[cells] = number of binned points);
+// also decides whether the grid is worth walking.  A workgroup takes kScanCells cells and adds up
+// every count before them by itself: 85 184 cells are at most 340 KB to read from L2, where one
+// workgroup walking all of them paid a round trip to memory and two barriers per 4096 cells (25 us
+// against 6).
+constexpr int kScanCells = kGridThreads * 4;
 template <typename T>
 __global__ __launch_bounds__(kGridThreads) void knn_grid_scan_kernel(char *__restrict__ ws,
                                                                     size_t slice, int cells,
                                                                     int R) {
-  __shared__ int wave_sum[kGridThreads / 64];
-  __shared__ int biggest[kGridThreads / 64];
-  char *base = ws + (size_t)blockIdx.x * slice;
+  constexpr int kWaves = kGridThreads / 64;
+  __shared__ int before_sum[kWaves], wave_sum[kWaves], biggest[kWaves];
+  char *base = ws + (size_t)blockIdx.y * slice;
   GridHead<T> *head = reinterpret_cast<GridHead<T> *>(base);
   int *start = reinterpret_cast<int *>(base + align_up256(sizeof(GridHead<T>)));
+  const int *cursor = reinterpret_cast<int *>(reinterpret_cast<char *>(start) +
+                                              align_up256((size_t)(cells + 1) * 4));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int carry = 0, big = 0;
-  // four consecutive cells per thread and step (the slice is 256-byte aligned and padded, so
-  // 16-byte accesses past `cells` stay inside it); the next step's counts are fetched before
-  // this step's barriers
-  constexpr int kStep = kGridThreads * 4;
-  int4 *cell4 = reinterpret_cast<int4 *>(start);
-  auto fetch = [&](int c0) {
-    const int c = c0 + threadIdx.x * 4;
-    int4 v = c < cells ? cell4[c >> 2] : make_int4(0, 0, 0, 0);
-    if (c + 1 >= cells) v.y = 0;
-    if (c + 2 >= cells) v.z = 0;
-    if (c + 3 >= cells) v.w = 0;
-    return v;
-  };
-  int4 next = fetch(0);
-  for (int c0 = 0; c0 < cells; c0 += kStep) {
-    const int c = c0 + threadIdx.x * 4;
-    const int4 v = next;
-    if (c0 + kStep < cells) next = fetch(c0 + kStep);
-    big = max(max(big, max(v.x, v.y)), max(v.z, v.w));
-    const int mine = v.x + v.y + v.z + v.w;
-    int incl = mine;  // inclusive scan within the wave
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(incl, o);
-      if (lane >= o) incl += t;
-    }
-    __syncthreads();  // the previous step's wave sums have been read
-    if (lane == 63) wave_sum[wave] = incl;
-    __syncthreads();
-    int before = carry, total = 0;
-    for (int w = 0; w < kGridThreads / 64; w++) {
-      const int t = wave_sum[w];
-      if (w < wave) before += t;
-      total += t;
-    }
-    if (c < cells) {  // (entries past `cells` inside the last 16 bytes are padding or start[cells])
-      int4 o;
-      o.x = before + incl - mine;
-      o.y = o.x + v.x;
-      o.z = o.y + v.y;
-      o.w = o.z + v.z;
-      if (c + 3 < cells) {
-        cell4[c >> 2] = o;
-      } else {
-        start[c] = o.x;
-        if (c + 1 < cells) start[c + 1] = o.y;
-        if (c + 2 < cells) start[c + 2] = o.z;
-      }
-    }
-    carry += total;
+  const int c0 = blockIdx.x * kScanCells;
+  const int4 *count4 = reinterpret_cast<const int4 *>(cursor);  // (256-byte aligned)
+  int sum = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < c0 / 4; i += kGridThreads) {
+    const int4 v = count4[i];
+    sum += v.x + v.y + v.z + v.w;
   }
-  for (int o = 32; o > 0; o >>= 1) big = max(big, __shfl_xor(big, o));
+  const int c = c0 + threadIdx.x * 4;
+  int v[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) v[j] = c + j < cells ? cursor[c + j] : 0;
+  int big = max(max(v[0], v[1]), max(v[2], v[3]));
+  const int mine = v[0] + v[1] + v[2] + v[3];
+  int incl = mine;  // inclusive scan within the wave
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o);
+    big = max(big, __shfl_xor(big, o));
+  }
+  if (lane == 63) {
+    wave_sum[wave] = incl;
+    before_sum[wave] = sum;
+    biggest[wave] = big;
+  }
   __syncthreads();
-  if (lane == 0) biggest[wave] = big;
-  __syncthreads();
+  int run = incl - mine;
+  for (int w = 0; w < kWaves; w++) {
+    run += before_sum[w];
+    if (w < wave) run += wave_sum[w];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (c + j < cells) start[c + j] = run;
+    run += v[j];
+    if (c + j == cells - 1) start[cells] = run;
+  }
   if (threadIdx.x == 0) {
-    start[cells] = carry;
     int m = 0;
-    for (int w = 0; w < kGridThreads / 64; w++) m = max(m, biggest[w]);
-    head->skewed = m > max(256, R / 4) ? 1 : 0;
+    for (int w = 0; w < kWaves; w++) m = max(m, biggest[w]);
+    if (m > max(256, R / 4)) head->skewed = 1;  // (every writer stores the same value)
   }
 }
 
@@ -580,15 +596,15 @@ int launch_knn_grid(const T *ref, const T *query, int64_t *idx, T *dist, void *w
   const size_t slice = grid_slice_bytes<T>(D, R);
   char *ws = (char *)workspace;
   const int cells = (int)gs.cells;
-  hipLaunchKernelGGL((knn_grid_box_kernel<T, D>), dim3((unsigned)B), dim3(kGridThreads), 0, s, ref,
-                     ws, slice, (int)R, gs.g[0], gs.g[1], gs.g[2], cells);
+  hipLaunchKernelGGL((knn_grid_box_kernel<T, D>), dim3(kBoxParts, (unsigned)B), dim3(256), 0, s,
+                     ref, ws, slice, (int)R, cells);
   MCX_HIP_CHECK_LAUNCH();
   const dim3 rgrid(div_up(R, 256), (unsigned)B);
   hipLaunchKernelGGL((knn_grid_count_kernel<T, D>), rgrid, dim3(256), 0, s, ref, ws, slice, (int)R,
                      gs.g[0], gs.g[1], gs.g[2], cells, 0);
   MCX_HIP_CHECK_LAUNCH();
-  hipLaunchKernelGGL(knn_grid_scan_kernel<T>, dim3((unsigned)B), dim3(kGridThreads), 0, s, ws,
-                     slice, cells, (int)R);
+  hipLaunchKernelGGL(knn_grid_scan_kernel<T>, dim3(div_up(cells, kScanCells), (unsigned)B),
+                     dim3(kGridThreads), 0, s, ws, slice, cells, (int)R);
   MCX_HIP_CHECK_LAUNCH();
   hipLaunchKernelGGL((knn_grid_count_kernel<T, D>), rgrid, dim3(256), 0, s, ref, ws, slice, (int)R,
                      gs.g[0], gs.g[1], gs.g[2], cells, 1);
