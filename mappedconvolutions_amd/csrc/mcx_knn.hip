@@ -589,6 +589,268 @@ __global__ __launch_bounds__(kThreads) void knn_grid_kernel(
   }
 }
 
+// The k best so far of a lane in fp32, ordered by (distance, index); an empty slot (infinite
+// distance, index 0) yields to any finite distance only.
+// The pair is one 64-bit key, distance above index, read as a double: the bits of
+// numbers that are not negative are ordered like the numbers, and no key is an infinity or NaN (a
+// finite or infinite fp32 distance in the upper word is a finite double; a distance of zero makes
+// a subnormal one, which the 64-bit unit keeps).  Entry j after an insertion of x is then
+// max(entry j - 1, min(entry j, x)): two instructions an entry, where the comparisons and moves
+// of a pair are about eight.
+template <int KMAX>
+struct TopK {
+  double key[KMAX];
+  __device__ static inline double key_of(float d, int i) {
+    return __builtin_bit_cast(double, ((uint64_t)__builtin_bit_cast(unsigned, d) << 32) |
+                                          (unsigned)i);
+  }
+  // (written out: the compiler would quiet every operand first, for fear of a signalling NaN)
+  __device__ static inline double min2(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
+  __device__ static inline double max2(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
+  __device__ inline void init() {
+#pragma unroll
+    for (int j = 0; j < KMAX; j++) key[j] = key_of(inf_t<float>(), 0);
+  }
+  __device__ inline void insert(float ssd, int pi) {
+    const double x = key_of(ssd, pi);
+    if (!(x < key[KMAX - 1])) return;
+#pragma unroll
+    for (int j = KMAX - 1; j > 0; j--) key[j] = max2(key[j - 1], min2(key[j], x));
+    key[0] = min2(key[0], x);
+  }
+  __device__ inline float dist(int j) const {
+    return __builtin_bit_cast(float, (unsigned)(__builtin_bit_cast(uint64_t, key[j]) >> 32));
+  }
+  __device__ inline int index(int j) const { return (int)__builtin_bit_cast(uint64_t, key[j]); }
+};
+
+// Bound: vector instructions under divergence (a lane whose cells hold fewer points waits for the
+// wave's fullest).  So the runs of points of a lane's cells go into a list in LDS first and each
+// lane walks its own list through: the wave pays for the largest sum over its lanes, not for the
+// sum of each row's largest, and the loads of the row bounds are in flight together.
+// Rings beyond the first hold few points a lane still needs; rows that its k-th distance rules
+// out are not listed.
+// Measured, the kernel above -> this one (whole calls, us; Q queries among R points, k):
+// sphere, 524 288 among 40 962, 8: 318 -> 151; 1 000 among 642, 1: 76 -> 30; cube, 262 144
+// among 40 962, 8: 251 -> 136; plane 150 -> 84; line 122 -> 76; sphere, 50 000 among 10 000, 33:
+// 2388 -> 189; 40 tight clusters, 100 000 among 40 962, 8: 1126 -> 381.  (All but the first pair
+// hold the binning's own gain too, some 35 us among 40 962 points.)  In fp64 the key does not fit an instruction's operand and the same walk, with
+// pairs, needs more registers than there are: 2.7 -> 9.8 ms at k = 33, 410 -> 496 us for the cube
+// at k = 16 (and 265 -> 195 for the sphere at 8); fp64 keeps the kernel above.
+constexpr int kCrowded = 256;  // points in a query's 27 cells
+constexpr int kRuns = 12;  // runs listed per lane (24 KB of LDS: six workgroups a CU)
+template <int KMAX, int D>
+__global__ __launch_bounds__(kThreads) void knn_grid_lists_kernel(
+    const float *__restrict__ query, int64_t *__restrict__ idx, float *__restrict__ dist,
+    const char *__restrict__ ws, size_t slice, int Q, int k, int g0, int g1, int g2, int cells) {
+  using T = float;
+  const int b = blockIdx.y;
+  const char *base = ws + (size_t)b * slice;
+  const GridHead<T> head = *reinterpret_cast<const GridHead<T> *>(base);
+  if (head.skewed) return;
+  const int *start = reinterpret_cast<const int *>(base + align_up256(sizeof(GridHead<T>)));
+  const GridPoint<T> *pts = reinterpret_cast<const GridPoint<T> *>(
+      reinterpret_cast<const char *>(start) + align_up256((size_t)(cells + 1) * 4) +
+      align_up256((size_t)cells * 4));
+  const int q = blockIdx.x * kThreads + threadIdx.x;
+  if (q >= Q) return;
+  const T *qb = query + (int64_t)b * D * Q;
+  const int g[3] = {g0, g1, g2};
+
+  T qv[3] = {T(0), T(0), T(0)};
+  bool finite = true;
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    qv[d] = qb[(int64_t)d * Q + q];
+    finite = finite && finite_t(qv[d]);
+  }
+  TopK<KMAX> best;
+  best.init();
+  __shared__ int2 runs[kRuns][kThreads];  // (a lane reads only what it wrote: no barrier)
+  int listed = 0;
+  // The points of the listed runs, four at a time so that their loads are in flight together
+  // (a load past the run re-reads its last point and is not used).
+  constexpr int kUnroll = 4;
+  auto walk = [&]() __attribute__((always_inline)) {
+    int next = 0, r = 0, e = 0;
+    for (;;) {
+      if (r >= e) {
+        if (next == listed) break;
+        const int2 run = runs[next++][threadIdx.x];
+        r = run.x;
+        e = run.y;
+      }
+      GridPoint<T> p[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; u++) p[u] = pts[min(r + u, e - 1)];
+      T ssd[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; u++) {
+        ssd[u] = T(0);
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          const T t = p[u].c[d] - qv[d];
+          ssd[u] = fma_t(t, t, ssd[u]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; u++)
+        if (r + u < e) best.insert(ssd[u], p[u].idx);
+      r += kUnroll;
+    }
+    listed = 0;
+  };
+  auto list = [&](int r, int e) __attribute__((always_inline)) {
+    if (r < e) runs[listed++][threadIdx.x] = make_int2(r, e);
+  };
+  auto kth_dist = [&]() __attribute__((always_inline)) {
+    // (the largest of the first k.  They are in order; but written as the choice of entry k - 1,
+    // it is compiled to an access at a variable index, and the list then lives in scratch memory)
+    T kth = best.dist(0);
+#pragma unroll
+    for (int j = 1; j < KMAX; j++) {
+      const T d = best.dist(j);
+      kth = j < k && d > kth ? d : kth;
+    }
+    return kth;
+  };
+
+  if (finite && start[cells] > 0) {  // a query with a non-finite coordinate is near nothing
+    int c[3] = {0, 0, 0};
+    const int cell = cell_of<T, D>(head, g, qv, c);
+    // a dimension the points do not spread over (cell size 0) has them all in its cell 0
+    int ge[3] = {1, 1, 1};
+    T hmin = inf_t<T>();
+    // largest coordinate magnitude of a cell face: the face lo + n * h is rounded to one unit in
+    // the last place of that magnitude, and the cell index floor((c - lo) / h) of a point next to
+    // face n is off by a few units in the last place of n, i.e. of (n * h) in coordinates
+    T reach = T(0);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      if (head.h[d] > T(0)) {
+        ge[d] = g[d];
+        hmin = head.h[d] < hmin ? head.h[d] : hmin;
+        const T lo = head.lo[d] < T(0) ? -head.lo[d] : head.lo[d];
+        const T span = (T)g[d] * head.h[d];
+        reach = lo + span > reach ? lo + span : reach;
+      }
+    }
+    const int gmax = max(ge[0], max(ge[1], ge[2]));
+    constexpr T kUlp = 1.1920929e-7f;
+    // a thousandth of a cell, plus the rounding above (which outgrows it on long one-dimensional
+    // grids: 65536 cells in fp32 put a face off by hundredths of a cell)
+    const T slack = hmin * T(1e-3) + T(16) * kUlp * reach;
+    // a lower bound on the distance to the points of cells n along dimension d, squared
+    auto gap2 = [&](int d, int n) {
+      T f = T(0);
+      if (n > c[d]) f = head.lo[d] + (T)n * head.h[d] - qv[d];
+      if (n < c[d]) f = qv[d] - (head.lo[d] + (T)(n + 1) * head.h[d]);
+      f -= slack;
+      return f > T(0) ? f * f : T(0);
+    };
+    // the query's cell and its neighbours at once: a wave whose 64 lanes all find their k in the
+    // one cell is rare, and each row of cells is one run of points.  Where the points crowd (some
+    // 60 on a sphere, 14 in a cube filled evenly) the one cell comes first, so that its k-th
+    // distance rules the neighbours out.
+    bool crowded;
+    {
+      const int x0 = max(c[0] - 1, 0), x1 = min(c[0] + 1, ge[0] - 1) + 1;
+      int ra[9], re[9];
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        const int z = c[2] + i / 3 - 1, y = c[1] + i % 3 - 1;
+        ra[i] = re[i] = 0;
+        if (z >= 0 && z < ge[2] && y >= 0 && y < ge[1]) {
+          const int row = (z * g1 + y) * g0;
+          ra[i] = start[row + x0];
+          re[i] = start[row + x1];
+        }
+      }
+      int held = 0;
+#pragma unroll
+      for (int i = 0; i < 9; i++) held += re[i] - ra[i];
+      crowded = held > kCrowded;
+      if (crowded) {
+        list(start[cell], start[cell + 1]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 9; i++) list(ra[i], re[i]);
+      }
+    }
+    bool first = true;
+    for (int rho = crowded ? 0 : 1; rho < max(gmax, 2); rho++) {
+      const int z0 = max(c[2] - rho, 0), z1 = min(c[2] + rho, ge[2] - 1);
+      const int y0 = max(c[1] - rho, 0), y1 = min(c[1] + rho, ge[1] - 1);
+      const int xa = c[0] - rho, xb = c[0] + rho;
+      int z = first ? z1 + 1 : z0, y = y0;  // the next row of the ring
+      first = false;
+      do {
+        // ring rho: rows of cells along the first dimension; rows on the ring's outer faces
+        // are contiguous runs of cells (one run of points), the others contribute their ends.
+        // A row that lies beyond the k-th distance holds none of the k (the margin is that of
+        // the test below).
+        const T kth = kth_dist();
+        while (z <= z1 && listed <= kRuns - 2) {
+          const T gyz = (D > 2 ? gap2(2, z) : T(0)) + (D > 1 ? gap2(1, y) : T(0));
+          if (!(kth < gyz * T(1.0 - 1e-5))) {
+            const int row = (z * g1 + y) * g0;
+            const bool face = (D > 2 && (z == c[2] - rho || z == c[2] + rho)) ||
+                              (D > 1 && (y == c[1] - rho || y == c[1] + rho));
+            if (face) {
+              list(start[row + max(xa, 0)], start[row + min(xb, ge[0] - 1) + 1]);
+            } else {
+              if (xa >= 0 && !(kth < (gyz + gap2(0, xa)) * T(1.0 - 1e-5)))
+                list(start[row + xa], start[row + xa + 1]);
+              if (xb < ge[0] && !(kth < (gyz + gap2(0, xb)) * T(1.0 - 1e-5)))
+                list(start[row + xb], start[row + xb + 1]);
+            }
+          }
+          if (++y > y1) {
+            y = y0;
+            z++;
+          }
+        }
+        walk();
+      } while (z <= z1);
+      // every point not seen lies beyond a face of the cube of cells seen that is not on the
+      // grid's boundary; m: distance from the query to the nearest such face
+      T m = inf_t<T>();
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        if (c[d] - rho > 0) {
+          const T f = head.lo[d] + (T)(c[d] - rho) * head.h[d];
+          m = qv[d] - f < m ? qv[d] - f : m;
+        }
+        if (c[d] + rho < ge[d] - 1) {
+          const T f = head.lo[d] + (T)(c[d] + rho + 1) * head.h[d];
+          m = f - qv[d] < m ? f - qv[d] : m;
+        }
+      }
+      if (!(m < inf_t<T>())) break;  // the whole grid has been seen
+      const T kth = kth_dist();
+      // (the margins cover the rounding of cell assignment, faces and distances)
+      const T safe = m - slack;
+      if (safe > T(0) && kth < safe * safe * T(1.0 - 1e-5)) break;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < KMAX; j++) {
+    if (j < k) {
+      const int64_t o = ((int64_t)b * k + j) * Q + q;
+      idx[o] = best.index(j);
+      dist[o] = best.index(j) > 0 ? sqrt_t(best.dist(j)) : T(0);
+    }
+  }
+}
+
 template <typename T, int KMAX, int D>
 int launch_knn_grid(const T *ref, const T *query, int64_t *idx, T *dist, void *workspace,
                     int64_t B, int64_t R, int64_t Q, int64_t k, hipStream_t s) {
@@ -610,8 +872,12 @@ int launch_knn_grid(const T *ref, const T *query, int64_t *idx, T *dist, void *w
                      gs.g[0], gs.g[1], gs.g[2], cells, 1);
   MCX_HIP_CHECK_LAUNCH();
   const dim3 qgrid(div_up(Q, kThreads), (unsigned)B);
-  hipLaunchKernelGGL((knn_grid_kernel<T, KMAX, D>), qgrid, dim3(kThreads), 0, s, query, idx, dist,
-                     ws, slice, (int)Q, (int)k, gs.g[0], gs.g[1], gs.g[2], cells);
+  if constexpr (sizeof(T) == 4)
+    hipLaunchKernelGGL((knn_grid_lists_kernel<KMAX, D>), qgrid, dim3(kThreads), 0, s, query, idx,
+                       dist, ws, slice, (int)Q, (int)k, gs.g[0], gs.g[1], gs.g[2], cells);
+  else
+    hipLaunchKernelGGL((knn_grid_kernel<T, KMAX, D>), qgrid, dim3(kThreads), 0, s, query, idx,
+                       dist, ws, slice, (int)Q, (int)k, gs.g[0], gs.g[1], gs.g[2], cells);
   MCX_HIP_CHECK_LAUNCH();
   // the plain walk, for batch elements whose grid came out skewed (it returns at once otherwise)
   hipLaunchKernelGGL((knn_kernel<T, KMAX, D>), qgrid, dim3(kThreads), 0, s, ref, query, idx, dist,

@@ -172,3 +172,24 @@ def test_grid_knn_long_one_dimensional_grid(offset, device):
     assert torch.equal(gi, wi) and torch.equal(gd, wd)
     io, do = O.knn_forward(ref, qry[:, :, :256].contiguous(), 8)
     assert torch.equal(gi[:, :, :256].cpu(), io) and torch.equal(gd[:, :, :256].cpu(), do)
+
+
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 16, 17, 32, 33, 64])
+def test_grid_knn_lists_of_every_length(k, device):
+    """Lists at the edges of the compiled lengths, over points that make long ones of the runs a
+    query lists (rings of single points, more runs a ring than the list holds), distances of
+    zero, and distances that overflow fp32 (nearer to nothing): equal to the oracle bit for bit."""
+    g = torch.Generator().manual_seed(100 + k)
+    ref = torch.rand(1, 3, 700, generator=g)           # about half a point a cell
+    ref[0, :, 350:390] = ref[0, :, :40]                # the same place twice
+    qry = torch.rand(1, 3, 400, generator=g) * 1.5 - 0.25
+    qry[0, :, :80] = ref[0, :, :80]
+    _check(ref, qry, k)
+    huge = ref.clone()
+    huge[0, 0] = (huge[0, 0] - 0.5) * 1e20             # squares up to 1e40, fp32 ends at 3.4e38
+    big_q = qry.clone()
+    big_q[0, 0] = (big_q[0, 0] - 0.5) * 1e20
+    gi, gd = _raw_knn(huge.cuda(), big_q.cuda(), k, True)
+    wi, wd = _raw_knn(huge.cuda(), big_q.cuda(), k, False)
+    assert torch.equal(gi, wi) and torch.equal(gd, wd)
+    _check(ref.double(), qry.double(), k)
