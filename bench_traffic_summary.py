@@ -57,14 +57,16 @@ def per_kernel(folder, counter):
 
 
 def label_of(kernel):
-    """The timed C-ABI call whose work this kernel does (None: a helper kernel)."""
+    """The timed C-ABI calls whose work this kernel does (none: a helper kernel)."""
     if kernel.startswith("weight_grad_mfma_kernel<"):
-        return "conv_backward_weight"
+        return ["conv_backward_weight"]
+    if kernel.startswith("gather_product_split_kernel<"):
+        return ["conv_forward", "conv_backward_input"]  # (one kernel: the average of both calls)
     m = re.match(r"gather_product_mfma_kernel<\w+,(\d+),(\d+),", kernel)
     if m:  # the forward resolves the four bilinear corners itself; the input gradient reads a
         # packed transposed map of one pair per slot
-        return "conv_forward" if m.group(1) == "4" else "conv_backward_input"
-    return None
+        return ["conv_forward" if m.group(1) == "4" else "conv_backward_input"]
+    return []
 
 
 def main(argv):
@@ -95,9 +97,9 @@ def main(argv):
     print("@source sha256=%s file=%s" % (source_hash(), KERNEL_SOURCE))
     best = {}
     for k, n, f, w, rb, wb in rows:
-        lab = label_of(k)
-        if lab and (lab not in best or rb + wb > best[lab][1] + best[lab][2]):
-            best[lab] = (k, rb, wb)  # of two launched variants, the one that did the work
+        for lab in label_of(k):
+            if lab not in best or rb + wb > best[lab][1] + best[lab][2]:
+                best[lab] = (k, rb, wb)  # of two launched variants, the one that did the work
     for lab, (k, rb, wb) in sorted(best.items()):
         print('@traffic label=%s kernel="%s" read_bytes=%d written_bytes=%d' % (lab, k, rb, wb))
 
