@@ -103,8 +103,12 @@ int fill_zero<double>(double *p, int64_t n, hipStream_t s) { return fill_f64(p, 
 // kernels where it does not)
 size_t gather_product_ws(int dtype, int64_t G, int64_t O, int64_t K, int64_t P, int64_t B,
                          int64_t SH, int64_t SW, int64_t MH, int64_t MW) {
+  // (not for an image and a map of one wavefront each: there is nothing to spread, and the source
+  // is cached whole as it lies)
   if (dtype == MCX_F64)
-    return records_supported(B, G, O, K) ? records_gather_bytes(B, G, SH * SW) : 0;
+    return (SH * SW > 64 || MH * MW > 64) && records_supported(B, G, O, K)
+               ? records_gather_bytes(B, G, SH * SW)
+               : 0;
   return use_mfma(dtype, P)
              ? mfma_gather_product_bytes(O, G, K, B, SH, SW, (int)elem_size(dtype), MH, MW)
              : 0;
