@@ -2351,6 +2351,15 @@ inline ModeArgs mode_args(int interp, int64_t P) {
 inline bool use_channel_last(int64_t SH, int interp) {
   return SH == 1 && canonical_interp(interp) == kInterpNearest;
 }
+// Whether launch_gather_product samples a channel-last copy of the source, for the interpolation
+// that it is CALLED with (a plan's or a transposed map's entries are nearest taps, whatever the
+// map's interpolation was) and given room for the copy.  The split weights are laid out for the
+// source they meet (see split_channel), so whoever packs them asks here too.
+inline bool gathers_channel_last(bool room, int64_t SH, int64_t SW, int64_t G, int interp,
+                                 size_t elem) {
+  return room && use_channel_last(SH, interp) &&
+         SH * SW * ((G + kGC - 1) / kGC * kGC) * (int64_t)elem <= 0xffffffffLL;
+}
 // Blocked staging ([B][Gpad/8][pixels][8]) of an image-like source: bf16 storage only.
 inline bool use_channel_blocks(int64_t SH, int interp, size_t elem) {
   return elem == 2 && !use_channel_last(SH, interp) && SH > 1;
@@ -2440,8 +2449,7 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const bool blocked = stage != nullptr && use_channel_blocks(SH, interp, sizeof(TD)) &&
                        SH * SW * 8 * (int64_t)sizeof(TD) <= 0xffffffffLL;
-  const bool cl = blocked || (stage != nullptr && use_channel_last(SH, interp) &&
-                              SH * SW * Gpad * (int64_t)sizeof(TD) <= 0xffffffffLL);
+  const bool cl = blocked || gathers_channel_last(stage != nullptr, SH, SW, G, interp, sizeof(TD));
   if (cl && staged) {
     src = stage;  // the caller has made the copy already
   } else if (blocked) {
@@ -2688,9 +2696,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   const size_t min_bytes =
       mfma_gather_product_min_bytes(O, G, K, B, SH, SW, (int)sizeof(TD), OH, OW);
   const bool room = sizeof(TD) == 4 && scratch_bytes >= min_bytes + split_bytes(O, G, K, 4);
-  const bool cl = use_channel_last(SH, interp) &&
-                  SH * SW * round_up(G, kGC) * (int64_t)sizeof(TD) <= 0xffffffffLL;
-  const SplitJob with_split = split_job((char *)scratch + min_bytes, !cl);
+  char *const split_region = (char *)scratch + min_bytes;
   // (fp32 images with four-corner taps: resolving the taps in the kernel and reading them
   // resolved measured the same within 1 %, so there only the plan's pair mask is used and the
   // 32 bytes per tap of the resolved form are not read; single-row sources and bf16 storage
@@ -2712,9 +2718,11 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
     const ModeArgs pm = mode_args(interp, P);
     const bool four_pairs = pm.np * (pm.mode == kInterpNearest ? 1 : 4) == 4;
     // (a plan's cells hold four entries, the unused ones of weight zero)
+    const bool cl =
+        gathers_channel_last(stage != nullptr, SH, SW, G, kInterpNearest, sizeof(TD));
     const SplitJob split =
         room && split_applies(G, O, SH, SW, K, mode_args(kInterpNearest, kPlanSlots), true, cl)
-            ? with_split
+            ? split_job(split_region, !cl)
             : SplitJob{};
     if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s, nullptr, ZeroJob{nullptr, 0},
                                          PairMaskJob{}, split))
@@ -2749,8 +2757,10 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   const int *mask = pair_mask;
   // the pair mask of a small map is made by the last block of the packing launch
   const bool mask_on_pack = four_pairs && !plan && OH * OW * K <= kSmallMapEntries;
-  const SplitJob split =
-      room && split_applies(G, O, SH, SW, K, m, false, cl) ? with_split : SplitJob{};
+  const bool cl = gathers_channel_last(stage != nullptr, SH, SW, G, interp, sizeof(TD));
+  const SplitJob split = room && split_applies(G, O, SH, SW, K, m, false, cl)
+                             ? split_job(split_region, !cl)
+                             : SplitJob{};
   if (int rc = launch_pack_weights<TD>(
           w, wp, O, G, K, 0, s, mask_on_pack ? nullptr : pair_mask, ZeroJob{nullptr, 0},
           mask_on_pack ? pair_mask_job(map, iw, pair_mask, m, SH, SW, OH * OW * K)
@@ -3381,8 +3391,8 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     OverflowEntry *ovf = (OverflowEntry *)(pbase + sc.ovf);
     TD *stage = (MH == 1 || sizeof(TD) == 2) ? (TD *)(base + sc.stage) : nullptr;
     const int64_t Spad16 = round_up(S, kGC);
-    const bool cl = stage != nullptr && use_channel_last(MH, kInterpNearest) &&
-                    MH * MW * Spad16 * (int64_t)sizeof(TD) <= 0xffffffffLL;
+    const bool cl =
+        gathers_channel_last(stage != nullptr, MH, MW, S, kInterpNearest, sizeof(TD));
     const SplitJob split =
         sizeof(TD) == 4 && (cl || !sc.two_level) &&
                 split_applies(S, D, MH, MW, K, mode_args(kInterpNearest, kTransSlots), true, cl)

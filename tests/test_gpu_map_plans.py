@@ -87,6 +87,35 @@ def test_transposed_conv_with_one_plan(interp, p, dtype, device):
         assert rel_err(a.float(), r) < tol, nm
 
 
+@pytest.mark.parametrize("channels", [8, 9, 12, 15, 16, 28])
+@pytest.mark.parametrize("interp,p", [(0, 0), (0, 4), (1, 0), (2, 0), (1, 2)])
+def test_plans_over_one_row_signals(channels, interp, p, device):
+    """A plan's taps over a signal of one row are read from a channel-last copy whatever the map's
+    interpolation was; unplanned bilinear taps read the planes.  The weights have to be laid out
+    for the one that runs: the halves of a partial last chunk of 16 channels differ (9 to 15
+    channels in it).  Forward of a convolution and input gradient of a transposed one."""
+    g = torch.Generator().manual_seed(2300 + channels)
+    B, Co, V, N, K = 2, 10, 45, 37, 3
+    smap, iw = helpers.random_map(g, 1, N, K, p, 1, V, torch.float32)
+    smap[..., 1] *= 0.2  # (rows around the only one)
+    rnd = lambda *s: torch.randn(s, generator=g)
+    x, w, b = rnd(B, channels, 1, V), rnd(Co, channels, K), rnd(Co)
+    wt, xt = rnd(Co, channels, K), rnd(B, Co, 1, N)
+    sd, iwd = dev(smap, iw)
+    plan = _C.conv_map_plan(sd, iwd, 1, V, interp)
+    maps, dmaps, pre = ((smap, iw), (sd, iwd), "weighted_") if p else ((smap,), (sd,), "")
+    y = getattr(_C, pre + "mapped_conv_forward")(x.cuda(), *dmaps, w.cuda(), b.cuda(), K, interp,
+                                                 plan=plan)
+    assert rel_err(y, getattr(O, pre + "mapped_conv_forward")(x, *maps, w, b, K, interp)) < 1e-5
+    # (the transposed convolution's output is the one-row signal; x serves as its gradient)
+    gx = getattr(_C, pre + "mapped_transposed_conv_backward")(
+        x.cuda(), *dmaps, xt.cuda(), wt.cuda(), torch.zeros(channels).cuda(), K, interp, plan=plan,
+        needs=(True, False, False))[0]
+    want = getattr(O, pre + "mapped_transposed_conv_backward")(x, *maps, xt, wt,
+                                                               torch.zeros(channels), K, interp)[0]
+    assert rel_err(gx, want) < 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("interp", [0, 1, 2])
 @pytest.mark.parametrize("p", [0, 3])
