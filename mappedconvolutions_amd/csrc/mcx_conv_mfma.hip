@@ -81,6 +81,8 @@ struct SplitJob {
   int planar;      // the source they meet is planar (else channel-last)
 };
 
+// Factor of the weights and of the samples before they are split.
+constexpr float kSplitScale = 16777216.f;  // 2^24
 __host__ __device__ inline int split_channel(int c, int kg, int j, int G, int planar);
 
 // Bits of the (point, corner) pairs with a nonzero weight anywhere among the entries this
@@ -199,7 +201,8 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
         const int g = split_channel(c, kg, (int)(e & 7), G, split.planar);
         float x = 0.f;
         if (o < O && g >= 0)
-          x = to_f32(w[transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k]);
+          x = to_f32(w[transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k]) *
+              kSplitScale;
 #pragma unroll
         for (int part = 0; part < 3; part++) {
           const uint16_t q = from_f32<bf16_t>(x).v;

@@ -6,11 +6,14 @@
 // where the fp32 one adds 2.  v_mfma_f32_32x32x16_bf16 does sixteen times the work of
 // v_mfma_f32_32x32x2_f32 per clock, so six of them cost 384 clocks a unit (one tap x 16 channels
 // x 32 pixels x 64 outputs) where the fp32 form costs 1024.
+//   * Interpolation weights and product weights are scaled by 2^24 before they are split, the sums by
+//     2^-48 at the end: exact, and the lowest bit of the smallest fp32 number (2^-149) is then a
+//     normal bf16.  (Without it parts below 2^-133 are lost, and with them bits of operands smaller
+//     than 2^-110: 216 products of 2^-124 and 2^30 came out 4e-4 off in 2-norm, now 2.4e-7.)
 //   * What the split cannot represent - an infinity or NaN among the operands, whose
-//     remainders are NaN, or a sum that overflows - always ends as a value that is not finite.  A wave
-//     that sees one sets a flag, and the launch of the fp32 kernel that follows every launch of
-//     these runs only then and recomputes the whole product.
-//   * Parts below 2^-133 are lost: operands smaller than 2^-110 keep fewer than 24 bits.
+//     remainders are NaN, samples or weights from 2^104 up, or sums from 2^80 up - always ends as a
+//     value that is not finite.  A wave that sees one sets a flag, and the launch of the fp32
+//     kernel that follows every launch of these runs only then and recomputes the whole product.
 //   * A lane gathers, interpolates and splits exactly the elements its matrix B operand holds
 //     (lane (l31, lhi): channels lhi * 8 .. + 7 of pixel l31 of the wave), so samples never pass
 //     through LDS; only the weights do, pre-split by the packing launch.
@@ -22,6 +25,8 @@
 // forward 411 -> 292 us, input gradient (both levels in one pass) 952 -> 509 us.  Distance from
 // the 64-bit result, in 2-norm: 4.3e-7 -> 3.6e-7 (576 terms).
 // Included by mcx_conv_mfma.hip, inside its anonymous namespace.
+
+constexpr float kSplitUnscale = 1.f / (kSplitScale * kSplitScale);
 
 struct SplitArgs {
   const float *src, *map, *iw;
@@ -146,7 +151,9 @@ __device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, i
         const int o = o0 + 32 * m + (i >> 2) * 8 + lhi * 4 + (i & 3);
         bad |= !(__builtin_fabsf(acc[m][i]) <= 3.402823466e+38f);
         if (o < s.O)
-          yb[(int64_t)o * N] = acc[m][i] + (s.bias ? s.bias[o] : 0.f) + (ab ? ab[o] : 0.f);
+          yb[(int64_t)o * N] =
+              __builtin_fmaf(acc[m][i], kSplitUnscale, s.bias ? s.bias[o] : 0.f) +
+              (ab ? ab[o] : 0.f);
       }
   }
   if (__builtin_amdgcn_ballot_w64(bad) != 0 && (threadIdx.x & 63) == 0)
@@ -315,11 +322,11 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
             const float2 q =
                 reinterpret_cast<const float2 *>(s.map)[((int64_t)(k0 + kl) * 4 + i) * N + n_g];
             off[i] = __builtin_bit_cast(unsigned, q.x) * 4u;
-            wt[i] = live ? q.y : 0.f;
+            wt[i] = live ? q.y * kSplitScale : 0.f;
           }
         } else {
           const int64_t e = n_g * s.K + k0 + kl;
-          const float scale = live ? (s.weighted ? s.iw[e] : 1.f) : 0.f;
+          const float scale = live ? (s.weighted ? s.iw[e] * kSplitScale : kSplitScale) : 0.f;
           PairTap<NE> t;
           resolve_pairs<NE, 4>(s.map[e * 2], s.map[e * 2 + 1], s.SH, s.SW, s.wrap != 0, scale, t);
 #pragma unroll
@@ -450,10 +457,11 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
     for (int i = 0; i < NT; i++) {
       if (s.packed || i >= NE) {
         off[i] = __builtin_bit_cast(unsigned, raw[i].x) * record;
-        wgt[i] = live ? raw[i].y : 0.f;
+        wgt[i] = live ? raw[i].y * kSplitScale : 0.f;
       } else {
         PairTap<1> t;
-        resolve_pairs<1, 1>(raw[i].x, raw[i].y, s.SH, s.SW, false, live ? raw_w[i < NE ? i : 0] : 0.f, t);
+        resolve_pairs<1, 1>(raw[i].x, raw[i].y, s.SH, s.SW, false,
+                            live ? raw_w[i < NE ? i : 0] * kSplitScale : 0.f, t);
         off[i] = t.off[0] * record;
         wgt[i] = t.wt[0];
       }

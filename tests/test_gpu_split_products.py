@@ -102,6 +102,43 @@ def test_operands_without_a_split(what, device):
     assert ((y - want).abs()[both] <= 1e-5 * want.abs()[both].max()).all()
 
 
+# (x = 2^p * u, w = 2^q * v with u, v of ordinary size: the result is 2^(p + q) times the one
+# for u and v, to the last bit, wherever fp32 holds the operands in full: |x| >= 2^-126.  The
+# split's own range ends at operands of 2^104 and results of 2^80, where the fp32 form takes
+# over: another order of summation, a few 2^-24 of the result's size.)
+@pytest.mark.parametrize("p,q,bits", [(0, 0, True), (-108, 60, True), (-112, 100, True),
+                                      (-118, 100, True), (-124, 30, True), (60, -112, True),
+                                      (100, -124, True), (30, -124, True), (-60, -60, True),
+                                      (110, -110, False), (-110, 110, False), (45, 45, False)])
+@pytest.mark.parametrize("mesh", [False, True])
+def test_operands_of_every_magnitude_count_in_full(p, q, bits, mesh, device):
+    g = torch.Generator().manual_seed(13)
+    B, ci, co, h, w_, k = 1, 24, 40, 9, 40, 9
+    if mesh:
+        h, w_ = 1, 360
+        idx = torch.randint(w_, (1, w_, k), generator=g).float()
+        smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    else:
+        smap = _grid(h, w_, k, 0.0, 0.0)
+    interp = 0 if mesh else 1  # (whole rows and columns: interpolation weights of one)
+    unit = lambda *s: (1 + torch.rand(s, generator=g)) * (1 - 2 * torch.randint(2, s, generator=g))
+    u, v, gu = unit(B, ci, h, w_), unit(co, ci, k), unit(B, co, h, w_)
+    b = torch.zeros(co)
+    run = lambda x, w: _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
+    y = run(u * 2.0 ** p, v * 2.0 ** q).double().cpu() * 2.0 ** -(p + q)
+    if bits:
+        assert torch.equal(y, run(u, v).double().cpu())
+    want = O.mapped_conv_forward(u.double(), smap.double(), v.double(), b.double(), k, interp)
+    assert ((y - want).norm() / want.norm()).item() < 1e-6
+    # the input gradient (slots of the transposed map are filled in any order: not the same bits)
+    gx = _C.mapped_conv_backward((gu * 2.0 ** p).cuda(), smap.cuda(), u.cuda(),
+                                 (v * 2.0 ** q).cuda(), b.cuda(), k, interp,
+                                 needs=(True, False, False))[0].double().cpu() * 2.0 ** -(p + q)
+    want = O.mapped_conv_backward(gu.double(), smap.double(), u.double(), v.double(), b.double(),
+                                  k, interp)[0]
+    assert ((gx - want).norm() / want.norm()).item() < 1e-6
+
+
 def test_accuracy_is_not_below_fp32(device):
     """Against 64 bits the split products are at least as close as fp32 sums of the same length:
     2-norm 1e-6 of the result at 576 terms (fp32 instructions 4.3e-7, split 3.6e-7 measured)."""
