@@ -1,11 +1,14 @@
 // fp32 gather-product on the bf16 matrix instructions, without giving up fp32: every operand is
 // split exactly into three bf16 parts (8 + 8 + 8 significant bits, round to nearest each, the
-// remainders exact), and a product is the six of the nine partial products that are larger
-// than 2^-26 of it, summed in fp32 by the matrix unit.  The rounding of single products is then
-// finer than fp32's own, and a matrix instruction adds 16 products per rounding of its sum
-// where the fp32 one adds 2.  v_mfma_f32_32x32x16_bf16 does sixteen times the work of
-// v_mfma_f32_32x32x2_f32 per clock, so six of them cost 384 clocks a unit (one tap x 16 channels
-// x 32 pixels x 64 outputs) where the fp32 form costs 1024.
+// remainders exact; the decomposition into leading part and remainders is Dekker's, Numerische
+// Mathematik 18, 1971), and of the nine partial products six are summed in fp32 by the matrix unit.
+// Each of the other three is at most 2^-25 of the product, all of them 2^-24 (half a unit in the
+// last place of fp32; their root mean square over random operands is about 2^-26.5), and a matrix
+// instruction adds 16 products per rounding of its sum where the fp32 one adds 2: measured against
+// 64 bits the sum is no further off (see split_applies for where that holds).
+// v_mfma_f32_32x32x16_bf16 does sixteen times the work of v_mfma_f32_32x32x2_f32 per clock, so six
+// of them cost 384 clocks a unit (one tap x 16 channels x 32 pixels x 64 outputs) where the fp32
+// form costs 1024.
 //   * Interpolation weights and product weights are scaled by 2^24 before they are split, the sums by
 //     2^-48 at the end: exact, and the lowest bit of the smallest fp32 number (2^-149) is then a
 //     normal bf16.  (Without it parts below 2^-133 are lost, and with them bits of operands smaller

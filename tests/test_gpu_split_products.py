@@ -9,7 +9,7 @@ import helpers
 from helpers import rel_err
 from oracle import ops as O
 
-from mappedconvolutions_amd import _C
+from mappedconvolutions_amd import _C, _lib
 from mappedconvolutions_amd.util import synthetic
 
 pytestmark = pytest.mark.gpu
@@ -24,8 +24,8 @@ def _grid(h, w, k, dx, dy):
 # channels around 8 and 16 (the halves of a chunk), outputs around 64 and 128, widths whose rows
 # end inside a tile; 32-bit sums of up to 9 * 40 terms: a few 1e-7 of the result's magnitude,
 # 1e-5 allowed like everywhere in these tests
-@pytest.mark.parametrize("ci,co", [(1, 1), (7, 5), (8, 64), (9, 65), (15, 128), (16, 130), (17, 3),
-                                   (24, 40), (31, 64), (40, 129)])
+@pytest.mark.parametrize("ci,co", [(1, 1), (7, 5), (8, 64), (9, 65), (11, 6), (13, 27), (15, 128),
+                                   (16, 130), (17, 3), (24, 40), (31, 64), (40, 129)])
 @pytest.mark.parametrize("interp,dx,dy", [(0, 0.0, 0.0), (1, 0.25, 0.0), (1, 0.4, 0.3),
                                           (2, 0.25, 0.0), (2, -0.3, 0.6)])
 def test_split_products_over_images(ci, co, interp, dx, dy, device):
@@ -42,11 +42,12 @@ def test_split_products_over_images(ci, co, interp, dx, dy, device):
 
 
 @pytest.mark.parametrize("shape", [(1, 1), (1, 2), (2, 1), (3, 2)])
-def test_split_products_over_the_smallest_planes(shape, device):
+@pytest.mark.parametrize("ci", [5, 7, 12])
+def test_split_products_over_the_smallest_planes(ci, shape, device):
     """A plane of one pixel has no neighbour to fetch along; the last pixel has none to its right."""
     g = torch.Generator().manual_seed(3)
     h, w_ = shape
-    k, ci, co = 9, 5, 6
+    k, co = 9, 6
     smap = _grid(h, w_, k, 0.25, 0.5)
     x, w, b = (torch.randn(s, generator=g) for s in ((2, ci, h, w_), (co, ci, k), (co,)))
     for interp in (0, 1, 2):
@@ -139,13 +140,39 @@ def test_operands_of_every_magnitude_count_in_full(p, q, bits, mesh, device):
     assert ((gx - want).norm() / want.norm()).item() < 1e-6
 
 
-def test_accuracy_is_not_below_fp32(device):
-    """Against 64 bits the split products are at least as close as fp32 sums of the same length:
-    2-norm 1e-6 of the result at 576 terms (fp32 instructions 4.3e-7, split 3.6e-7 measured)."""
+def _forward_both(x, smap, w, b, k, interp):
+    """Through the split products, and (a byte of workspace short of their room) through the fp32
+    matrix instructions."""
+    lib = _lib.load()
+    B, ci, h, w_ = x.shape
+    co, (oh, ow) = w.shape[0], smap.shape[:2]
+    sizes = (B, ci, co, h, w_, oh, ow, k, 0)
+    need = lib.mcx_conv_forward_workspace(*sizes, _lib.MCX_F32)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    out = []
+    for given in (need, need - 1):
+        y = torch.empty(B, co, oh, ow, device=x.device)
+        rc = lib.mcx_conv_forward(x.data_ptr(), smap.data_ptr(), None, w.data_ptr(), b.data_ptr(),
+                                  y.data_ptr(), ws.data_ptr(), given, *sizes, interp,
+                                  _lib.MCX_F32, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        out.append(y.double().cpu())
+    return out
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 5, 6, 8, 9, 10, 11, 16, 17, 24, 33, 64, 128])
+@pytest.mark.parametrize("interp,shift", [(0, 0.0), (1, 0.0), (1, 0.3)])
+def test_accuracy_is_not_below_fp32(c, interp, shift, device):
+    """Distance from the 64-bit result in 2-norm: the forward's is no larger than that of the fp32
+    matrix instructions on the same operands, which serve it themselves where the split products'
+    would be (few channels).  (Some 130 000 results: their root mean square is known to better
+    than the 2 % allowed for.)"""
     g = torch.Generator().manual_seed(9)
-    h, w_, c, k = 32, 64, 64, 9
-    smap = synthetic.latitude_map(h, w_, 1)
-    x, w, b = (torch.randn(s, generator=g) for s in ((1, c, h, w_), (c, c, k), (c,)))
-    y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, 1).double().cpu()
-    want = O.mapped_conv_forward(x.double(), smap.double(), w.double(), b.double(), k, 1)
-    assert ((y - want).norm() / want.norm()).item() < 1e-6
+    h, w_, k, co = 32, 64, 9, 64
+    smap = synthetic.latitude_map(h, w_, 1) + shift
+    x, w, b = (torch.randn(s, generator=g) for s in ((1, c, h, w_), (co, c, k), (co,)))
+    split, fp32 = _forward_both(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
+    want = O.mapped_conv_forward(x.double(), smap.double(), w.double(), b.double(), k, interp)
+    far = lambda y: ((y - want).norm() / want.norm()).item()
+    assert torch.equal(split, fp32) == (c in (1, 2, 3, 4, 5, 9, 10))
+    assert far(split) <= 1.02 * far(fp32), (far(split), far(fp32))
