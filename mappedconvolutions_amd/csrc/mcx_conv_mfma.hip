@@ -73,11 +73,12 @@ struct PairMaskJob {
   int64_t total;   // (location, tap) entries
 };
 
-//   * SplitJob: the weights in three bf16 parts as well, and the flag word that the kernels
-//     which read them set cleared (mcx_conv_split.h).
+//   * SplitJob: the weights in three bf16 parts as well, and the flags that the kernels which
+//     read them set, a word per pixel tile, cleared (mcx_conv_split.h).
 struct SplitJob {
   uint16_t *w;     // nullptr: no job
   int *nonfinite;
+  int64_t tiles;
   int planar;      // the source they meet is planar (else channel-last)
 };
 
@@ -148,10 +149,7 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
     const TD *__restrict__ w, void *__restrict__ packed_out, int O, int G, int K, int Opad,
     int Gpad, int transposed, int *__restrict__ clear, ZeroJob zero, PairMaskJob pm,
     SplitJob split) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {  // flag words of the caller
-    if (clear) *clear = 0;
-    if (split.nonfinite) *split.nonfinite = 0;
-  }
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // a flag word of the caller
   int blocks = gridDim.x;
   if (pm.mask) {
     blocks -= pm.blocks;
@@ -213,6 +211,7 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
     }
   }
   for (int64_t i = first; i < zero.count; i += stride) zero.ptr[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (int64_t i = first; i < split.tiles; i += stride) split.nonfinite[i] = 0;
 }
 
 // x[b][g][n] -> xt[b][n][Gpad] (channels past G zero): 64 pixels x 64 channels per
@@ -372,7 +371,8 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
   // (bilinear corners of integral coordinates, unused slots) are neither loaded nor
   // accumulated.
   __shared__ unsigned TapMask[TG][2][2];
-  if (only_if && *only_if == 0) return;  // nothing to recompute (see mcx_conv_split.h)
+  // nothing of this tile to recompute (see mcx_conv_split.h)
+  if (only_if && only_if[xcd_contiguous_tile(blockIdx.x, gridDim.x)] == 0) return;
   if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
   if (pair_mask && !row_mask &&
       (!later_pairs_in_use(pair_mask, mask_words) != (run_if_leading != 0)))
@@ -2381,14 +2381,19 @@ int launch_channel_blocks(const TD *src, TD *stage, int64_t B, int64_t G, int64_
 // `stage`: room for the channel-last copy (B * SH * SW * Gpad elements) when
 // use_channel_last(SH, interp), unused otherwise.
 // ---- fp32 on the bf16 matrix instructions (mcx_conv_split.h) ----
-// Room for the split weights and the flag word, at the end of a product's scratch.
-size_t split_bytes(int64_t O, int64_t G, int64_t K, int elem) {
-  if (elem != 4) return 0;
-  return 256 + align256((size_t)(K * round_up(G, kGC) * round_up(O, kOT)) * 6);
+// Room for the flags (a word per tile of the B x OH x OW outputs) and the split weights, at the end
+// of a product's scratch.
+int64_t split_tiles(int64_t B, int64_t OH, int64_t OW) {
+  return make_tiling(B, OH, OW, (int)sizeof(float)).total;
 }
-SplitJob split_job(char *region, bool planar) {
-  return SplitJob{reinterpret_cast<uint16_t *>(region + 256), reinterpret_cast<int *>(region),
-                  planar ? 1 : 0};
+size_t split_bytes(int64_t O, int64_t G, int64_t K, int elem, int64_t tiles) {
+  if (elem != 4) return 0;
+  return align256((size_t)tiles * sizeof(int)) +
+         align256((size_t)(K * round_up(G, kGC) * round_up(O, kOT)) * 6);
+}
+SplitJob split_job(char *region, bool planar, int64_t tiles) {
+  return SplitJob{reinterpret_cast<uint16_t *>(region + align256((size_t)tiles * sizeof(int))),
+                  reinterpret_cast<int *>(region), tiles, planar ? 1 : 0};
 }
 // A tap of the source is one, or for planar images four, (offset, weight) entries; operands
 // are addressed as buffers of less than 4 GiB.
@@ -2546,7 +2551,7 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
       const int rc = launch_gather_split(a, t, cl, s);
       profile_end(s);
       if (rc) return rc;
-      // the fp32 form below recomputes everything where a result was not finite
+      // the fp32 form below recomputes the tiles that have a result that is not finite
       only_if = split.nonfinite;
     }
     if (only_if) pair_mask = row_mask = nullptr;  // (its general form alone)
@@ -2614,7 +2619,7 @@ int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K,
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const int64_t packed = (int64_t)K * Gpad * Opad;
   // (bf16 storage: the bf16 MFMA operand layout in the same scratch, half the bytes)
-  const int64_t work = std::max(packed, zero.count * 4);
+  const int64_t work = std::max({packed, zero.count * 4, split.tiles});
   const dim3 grid((unsigned)std::min<int64_t>((work + 255) / 256, 4096) +
                   (pm.mask ? (unsigned)pm.blocks : 0u));
   hipLaunchKernelGGL(pack_weights_kernel<TD>, grid, dim3(256), 0, s, w, (void *)wp, (int)O, (int)G,
@@ -2691,7 +2696,7 @@ size_t mfma_gather_product_min_bytes(int64_t O, int64_t G, int64_t K, int64_t B,
 size_t mfma_gather_product_bytes(int64_t O, int64_t G, int64_t K, int64_t B, int64_t SH,
                                  int64_t SW, int elem, int64_t MH, int64_t MW) {
   return mfma_gather_product_min_bytes(O, G, K, B, SH, SW, elem, MH, MW) +
-         split_bytes(O, G, K, elem);
+         split_bytes(O, G, K, elem, split_tiles(B, MH, MW));
 }
 
 // scratch: mfma_gather_product_bytes(...) bytes; with mfma_gather_product_min_bytes(...) the fp32
@@ -2704,7 +2709,8 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   float *wp = (float *)scratch;
   const size_t min_bytes =
       mfma_gather_product_min_bytes(O, G, K, B, SH, SW, (int)sizeof(TD), OH, OW);
-  const bool room = sizeof(TD) == 4 && scratch_bytes >= min_bytes + split_bytes(O, G, K, 4);
+  const int64_t tiles = split_tiles(B, OH, OW);
+  const bool room = sizeof(TD) == 4 && scratch_bytes >= min_bytes + split_bytes(O, G, K, 4, tiles);
   char *const split_region = (char *)scratch + min_bytes;
   // (fp32 images with four-corner taps: resolving the taps in the kernel and reading them
   // resolved measured the same within 1 %, so there only the plan's pair mask is used and the
@@ -2731,7 +2737,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
         gathers_channel_last(stage != nullptr, SH, SW, G, kInterpNearest, sizeof(TD));
     const SplitJob split =
         room && split_applies(G, O, SH, SW, K, mode_args(kInterpNearest, kPlanSlots), true, cl)
-            ? split_job(split_region, !cl)
+            ? split_job(split_region, !cl, tiles)
             : SplitJob{};
     if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s, nullptr, ZeroJob{nullptr, 0},
                                          PairMaskJob{}, split))
@@ -2768,7 +2774,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   const bool mask_on_pack = four_pairs && !plan && OH * OW * K <= kSmallMapEntries;
   const bool cl = gathers_channel_last(stage != nullptr, SH, SW, G, interp, sizeof(TD));
   const SplitJob split = room && split_applies(G, O, SH, SW, K, m, false, cl)
-                             ? split_job(split_region, !cl)
+                             ? split_job(split_region, !cl, tiles)
                              : SplitJob{};
   if (int rc = launch_pack_weights<TD>(
           w, wp, O, G, K, 0, s, mask_on_pack ? nullptr : pair_mask, ZeroJob{nullptr, 0},
@@ -3278,7 +3284,7 @@ ScatterScratch scatter_scratch(int64_t B, int64_t S, int64_t D, int64_t K, int64
   if (sc.transposed_path && (MH == 1 || elem == 2))
     off += align256((size_t)(B * MH * MW * round_up(S, kGC)) * 4);
   sc.split = off;
-  if (sc.transposed_path) off += split_bytes(D, S, K, (int)elem);
+  if (sc.transposed_path) off += split_bytes(D, S, K, (int)elem, split_tiles(B, DH, DW));
   sc.total = off;
   return sc;
 }
@@ -3405,7 +3411,7 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     const SplitJob split =
         sizeof(TD) == 4 && (cl || !sc.two_level) &&
                 split_applies(S, D, MH, MW, K, mode_args(kInterpNearest, kTransSlots), true, cl)
-            ? split_job(base + sc.split, !cl)
+            ? split_job(base + sc.split, !cl, split_tiles(B, DH, DW))
             : SplitJob{};
     // (the packing launch also clears the transposed map's counters, flags and slots)
     if (int rc = launch_pack_weights<TD>(

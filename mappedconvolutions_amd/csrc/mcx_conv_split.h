@@ -15,8 +15,13 @@
 //     than 2^-110: 216 products of 2^-124 and 2^30 came out 4e-4 off in 2-norm, now 2.4e-7.)
 //   * What the split cannot represent - an infinity or NaN among the operands, whose
 //     remainders are NaN, samples or weights from 2^104 up, or sums from 2^80 up - always ends as a
-//     value that is not finite.  A wave that sees one sets a flag, and the launch of the fp32
-//     kernel that follows every launch of these runs only then and recomputes the whole product.
+//     value that is not finite.  A wave that sees one sets its tile's flag, and the fp32 kernel,
+//     whose launch follows every launch of these with the same tiles, recomputes the tiles that
+//     have it (in its general form: a flagged tile costs both kernels).  8 x 64 channels of
+//     256 x 512 -> 64 forward: no NaN 599 us, one element 607, a quarter of the rows 766, all
+//     1285 (the fp32 kernel alone, in its two-pair form: 715 to 730; one flag for the whole
+//     product: 1300 in every case with a NaN).  2 x 24 -> 40 of 125 x 250, where the fp32 kernel's
+//     workgroups all run at once: 35, 59, 72, 72 (47).
 //   * A lane gathers, interpolates and splits exactly the elements its matrix B operand holds
 //     (lane (l31, lhi): channels lhi * 8 .. + 7 of pixel l31 of the wave), so samples never pass
 //     through LDS; only the weights do, pre-split by the packing launch.
@@ -39,7 +44,7 @@ struct SplitArgs {
   float *y;
   const float *addend;    // see gather_product_mfma_kernel, like the gates and masks below
   const int *gate, *pair_mask, *row_mask;
-  int *nonfinite;
+  int *nonfinite;         // a word per pixel tile
   int G, O, Opad, Gpad, SH, SW, OH, OW, K, np, ncorn, weighted, wrap, packed;
   int tiles_x, tiles_per_img, tw_shift, run_if_zero, mask_words;
 };
@@ -135,10 +140,10 @@ __device__ inline void split_products(const uint4 *lds, const bf16x8 *b, int l31
       acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m][pa[t]], b[pb[t]], acc[m], 0, 0, 0);
 }
 
-// Bias, addend and stores of a lane's pixel; flags results that are not finite.
+// Bias, addend and stores of a lane's pixel; flags a tile with a result that is not finite.
 template <int OG>
-__device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, int b, int o0,
-                                      int ei, int ej, int lhi) {
+__device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, int tile, int b,
+                                      int o0, int ei, int ej, int lhi) {
   const int64_t N = (int64_t)s.OH * s.OW;
   bool bad = false;
   if (ei < s.OH && ej < s.OW) {
@@ -160,7 +165,7 @@ __device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, i
       }
   }
   if (__builtin_amdgcn_ballot_w64(bad) != 0 && (threadIdx.x & 63) == 0)
-    *s.nonfinite = 1;  // (every writer stores the same value)
+    s.nonfinite[tile] = 1;  // (every writer stores the same value)
 }
 
 // Planar images.  NE: (offset, weight) entries per tap, 1 or 4; with 4, tiles none of whose taps
@@ -387,7 +392,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
     run(std::integral_constant<int, NE == 4 ? 2 : 1>());
   else
     run(std::integral_constant<int, NE>());
-  split_epilogue<OG>(s, acc, b, o0, tile_y * th + (pe >> s.tw_shift),
+  split_epilogue<OG>(s, acc, tile, b, o0, tile_y * th + (pe >> s.tw_shift),
                      (tile_x << s.tw_shift) + (pe & tw_mask), lhi);
 }
 
@@ -535,5 +540,5 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
     split_products<OG>(Wt[buf], bq, l31, lhi, acc);
     buf ^= 1;
   }
-  split_epilogue<OG>(s, acc, b, o0, ei, ej, lhi);
+  split_epilogue<OG>(s, acc, tile, b, o0, ei, ej, lhi);
 }

@@ -95,12 +95,91 @@ def test_operands_without_a_split(what, device):
         x[0, 2, 3, 20], w = 3.4e38, w * 1e-3
     y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, 1).cpu()
     want = O.mapped_conv_forward(x, smap, w, b, k, 1)
+    if what == "w_inf":
+        # one output channel has the infinity, or NaN where it meets a corner of weight zero; the
+        # others are what they are without it
+        assert not torch.isfinite(y[:, 5]).any()
+        y, want = (torch.cat((t[:, :5], t[:, 6:]), 1) for t in (y, want))
     ok = torch.isfinite(want)
-    if what != "w_inf":  # (there a zero-weighted corner outside the image meets the infinity)
-        assert torch.equal(torch.isfinite(y), ok)
-    both = ok & torch.isfinite(y)
-    assert both.any()
-    assert ((y - want).abs()[both] <= 1e-5 * want.abs()[both].max()).all()
+    assert ok.any() and torch.equal(torch.isfinite(y), ok)
+    assert ((y - want).abs()[ok] <= 1e-5 * want.abs()[ok].max()).all()
+
+
+def _like(got, want, tol=1e-5):
+    """Finite, infinite and NaN in the same places, finite values within `tol` of the largest."""
+    got, ok = got.cpu(), torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), ok) and ok.any() and not ok.all()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert ((got - want).abs()[ok] <= tol * want.abs()[ok].max()).all()
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("interp,planned", [(0, False), (0, True), (1, False), (1, True)])
+def test_not_finite_operands_over_images(value, interp, planned, device):
+    """The fp32 form takes over in the forward and in the input gradient of both convolutions.
+    (No tap leaves the image beside the element that is not finite, so no weight of zero meets
+    it.)"""
+    g = torch.Generator().manual_seed(11)
+    B, ci, co, h, w_, k = 2, 20, 40, 12, 70, 9
+    smap = _grid(h, w_, k, 0.25, 0.25)
+    x, w, b, gy = (torch.randn(s, generator=g)
+                   for s in ((B, ci, h, w_), (co, ci, k), (co,), (B, co, h, w_)))
+    x[1, 3, 5, 44] = value
+    gy[0, 7, 6, 12] = value
+    xd, sd, wd, bd, gd = (t.cuda() for t in (x, smap, w, b, gy))
+    plan = _C.conv_map_plan(sd, None, h, w_, interp) if planned else None
+    _like(_C.mapped_conv_forward(xd, sd, wd, bd, k, interp, plan=plan),
+          O.mapped_conv_forward(x, smap, w, b, k, interp))
+    gx = _C.mapped_conv_backward(gd, sd, xd, wd, bd, k, interp, plan=plan,
+                                 needs=(True, False, False))[0]
+    _like(gx, O.mapped_conv_backward(gy, smap, x, w, b, k, interp)[0])
+    # transposed: gy goes forward (co channels in), x comes back as the output's gradient
+    bt = torch.randn(ci, generator=g)
+    y = _C.mapped_transposed_conv_forward(gd, sd, wd, bt.cuda(), h, w_, k, interp, plan=plan)
+    _like(y, O.mapped_transposed_conv_forward(gy, smap, w, bt, h, w_, k, interp))
+    gt = _C.mapped_transposed_conv_backward(xd, sd, gd, wd, bt.cuda(), k, interp, plan=plan,
+                                            needs=(True, False, False))[0]
+    _like(gt, O.mapped_transposed_conv_backward(x, smap, gy, w, bt, k, interp)[0])
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("per_cell", [3, 5, 11])
+def test_not_finite_operands_over_meshes(value, planned, per_cell, device):
+    """Likewise over vertices: the fp32 form overwrites the destination and its second level is
+    added onto that; the overflow list's share comes once."""
+    g = torch.Generator().manual_seed(per_cell)
+    V, k, ci, co = 700, 3, 20, 130
+    idx = (torch.arange(V) // per_cell).view(1, V, 1, 1).expand(1, V, k, 1).float()
+    smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    iw = torch.rand(1, V, k, 1, generator=g) + 0.5
+    x, w, b, gy = (torch.randn(s, generator=g)
+                   for s in ((2, ci, 1, V), (co, ci, k), (co,), (2, co, 1, V)))
+    x[1, 3, 0, 17] = value
+    gy[0, 7, 0, 333] = value
+    d = [t.cuda() for t in (x, smap, iw, w, b, gy)]
+    plan = _C.conv_map_plan(d[1], d[2], 1, V, 0) if planned else None
+    _like(_C.weighted_mapped_conv_forward(*d[:5], k, 0, plan=plan),
+          O.weighted_mapped_conv_forward(x, smap, iw, w, b, k, 0))
+    gx = _C.weighted_mapped_conv_backward(d[5], *d[1:3], d[0], *d[3:5], k, 0, plan=plan,
+                                          needs=(True, False, False))[0]
+    _like(gx, O.weighted_mapped_conv_backward(gy, smap, iw, x, w, b, k, 0)[0])
+
+
+def test_only_the_tiles_with_a_value_that_is_not_finite_are_computed_again(device):
+    """Pixels far from a NaN keep the bits they have without it."""
+    g = torch.Generator().manual_seed(12)
+    B, ci, co, h, w_, k = 2, 16, 64, 32, 128, 9
+    smap = _grid(h, w_, k, 0.25, 0.25).cuda()
+    x, w, b = (torch.randn(s, generator=g).cuda() for s in ((B, ci, h, w_), (co, ci, k), (co,)))
+    clean = _C.mapped_conv_forward(x, smap, w, b, k, 1)
+    x[0, 3, 9, 40] = float("nan")
+    y = _C.mapped_conv_forward(x, smap, w, b, k, 1)
+    assert torch.isnan(y[0]).any()
+    # (tiles are 4 x 32 pixels, taps reach two pixels)
+    far = torch.ones(h, w_, dtype=torch.bool)
+    far[4:16, 32 - 32:64 + 32] = False
+    assert torch.equal(y[1], clean[1]) and torch.equal(y[0][:, far], clean[0][:, far])
 
 
 # (x = 2^p * u, w = 2^q * v with u, v of ordinary size: the result is 2^(p + q) times the one
