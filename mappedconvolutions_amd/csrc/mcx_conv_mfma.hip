@@ -2714,10 +2714,13 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   char *const split_region = (char *)scratch + min_bytes;
   // (fp32 images with four-corner taps: resolving the taps in the kernel and reading them
   // resolved measured the same within 1 %, so there only the plan's pair mask is used and the
-  // 32 bytes per tap of the resolved form are not read; single-row sources and bf16 storage
-  // gain from the resolved form)
+  // 32 bytes per tap of the resolved form are not read.  A single nearest point is one entry when
+  // resolved in the kernel and four when read: 8 x 64 channels of 256 x 512 -> 64, nine taps, 537
+  // against 800 us; 16 -> 32 of 64 x 128 20 against 25; a mesh of 40 962 vertices 160 against 202.
+  // Single-row sources otherwise and bf16 storage gain from the resolved form.)
+  const ModeArgs pt = mode_args(interp, P);
   const bool resolved_pays =
-      !(SH > 1 && canonical_interp(interp) != kInterpNearest && sizeof(TD) == 4);
+      !(sizeof(TD) == 4 && (pt.mode == kInterpNearest ? pt.np == 1 : SH > 1));
   if (plan && resolved_pays && gather_plan_applies(interp, P) &&
       OH * OW * K * kPlanSlots * 2 <= 0x7fffffffLL) {
     // the map's taps were resolved when the plan was built: read them as four pre-resolved

@@ -116,6 +116,23 @@ def test_plans_over_one_row_signals(channels, interp, p, device):
     assert rel_err(gx, want) < 1e-5
 
 
+@pytest.mark.parametrize("p", [0, 1])
+@pytest.mark.parametrize("rows", [1, 7])
+def test_plans_of_single_nearest_points(rows, p, device):
+    """fp32 forwards whose taps are one nearest point each decode the map, plan or not: the same
+    kernel on the same operands, the same bits."""
+    g = torch.Generator().manual_seed(2400 + p)
+    B, Ci, Co, IW, N, K = 2, 24, 36, 40, 33, 5
+    smap, iw = helpers.random_map(g, rows, N, K, p, rows, IW, torch.float32)
+    x, w, b = (torch.randn(s, generator=g) for s in ((B, Ci, rows, IW), (Co, Ci, K), (Co,)))
+    d = dev(x, smap, iw, w, b)
+    plan = _C.conv_map_plan(d[1], d[2], rows, IW, 0)
+    maps, op = (d[1:3], _C.weighted_mapped_conv_forward) if p else (d[1:2], _C.mapped_conv_forward)
+    y = op(d[0], *maps, *d[3:], K, 0, plan=plan)
+    assert torch.equal(y, op(d[0], *maps, *d[3:], K, 0))
+    assert rel_err(y, O.weighted_mapped_conv_forward(x, smap, iw, w, b, K, 0)) < 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("interp", [0, 1, 2])
 @pytest.mark.parametrize("p", [0, 3])
