@@ -94,11 +94,16 @@ __device__ inline void resolve_records(const double *__restrict__ map,
     off[0] = t.off < 0 ? none : t.off;
     wt[0] = scale;
   } else {
+    // (beside a corner that counts, one that does not weighs zero whatever the tap's scale: an
+    // infinite one times the zero it reads would make the whole sample NaN)
     auto put = [&](const auto &t) {
+      bool any = false;
+#pragma unroll
+      for (int i = 0; i < 4; i++) any |= t.off[i] >= 0;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         off[i * step] = t.off[i] < 0 ? none : t.off[i];
-        wt[i * step] = t.wt[i] * scale;
+        wt[i * step] = t.wt[i] * (any && t.off[i] < 0 ? 0.0 : scale);
       }
     };
     if (wrap) {
@@ -194,6 +199,7 @@ __global__ __launch_bounds__(kThreads) void gather_records_kernel(
               vx = mcx_fma(a, d[i].x, vx);
               vy = mcx_fma(a, d[i].y, vy);
             }
+            if (g0 + 2 * j + 1 >= G) vy = 0.0;  // (an odd last channel's pad, should `a` be infinite)
 #pragma unroll
             for (int o = 0; o < OT; o++) {
               const double2 ww = s_w[(t * OT + o) * LPR + j];

@@ -53,6 +53,36 @@ def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
             assert rel_err(a, c) < 1e-12, (name, i)
 
 
+@pytest.mark.parametrize("interp", [0, 1, 2])
+def test_infinite_interpolation_weights_at_the_border(interp, device):
+    """A tap that lies partly outside the image, or on whole rows and columns, has corners that do
+    not count; an infinite weight of such a tap makes its sample infinite, not NaN.  (Positive
+    operands: no two infinities of different signs meet.)"""
+    g = torch.Generator().manual_seed(21)
+    B, ci, co, k, p, h, w_ = 2, 5, 3, 9, 2, 12, 14
+    smap, wts = helpers.random_map(g, h, w_, k, p, h, w_, torch.float64)
+    smap.clamp_(-0.4, 13.25)                          # (no tap lies outside altogether)
+    smap[..., 1].clamp_(max=11.25)
+    smap[1] = smap[1].round().clamp_(0, 11)
+    for n in range(0, h * w_, 5):
+        wts.view(h * w_, k, p)[n, n % k, n % p] = float("inf")
+    x, w, b, gy = (torch.rand(s, generator=g, dtype=torch.float64) + 0.1
+                   for s in ((B, ci, h, w_), (co, ci, k), (co,), (B, co, h, w_)))
+    dev = [t.cuda() for t in (x, smap, wts, w, b, gy)]
+    got = [_C.weighted_mapped_conv_forward(*dev[:5], k, interp)]
+    got += _C.weighted_mapped_conv_backward(dev[5], *dev[1:3], dev[0], *dev[3:5], k, interp)
+    want = [O.weighted_mapped_conv_forward(x, smap, wts, w, b, k, interp)]
+    want += O.weighted_mapped_conv_backward(gy, smap, wts, x, w, b, k, interp)
+    assert torch.isinf(want[0]).any() and not torch.isinf(want[0]).all()
+    assert not torch.isnan(want[0]).any()
+    for i, (a, c) in enumerate(zip(got, want)):
+        # (the oracle's input gradient adds corners of weight zero too: NaN)
+        a, c = a.cpu()[~torch.isnan(c)], c[~torch.isnan(c)]
+        ok = torch.isfinite(c)
+        assert torch.equal(torch.isinf(a), torch.isinf(c)) and not torch.isnan(a).any(), i
+        assert not ok.any() or ((a - c).abs()[ok] <= 1e-12 * c.abs()[ok].max()).all(), i
+
+
 def test_fp64_without_a_workspace(device):
     g = torch.Generator().manual_seed(5)
     B, ci, co, k, h, w_ = 2, 5, 3, 9, 7, 8
