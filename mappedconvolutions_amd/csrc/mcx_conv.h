@@ -24,7 +24,9 @@ int generic_weight_grad(const T *plain, const T *gath, const T *map, const T *iw
                         int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t N,
                         int64_t K, int64_t P, int interp, hipStream_t s);
 // ---- fp64 over channel-last records (mcx_conv_records.hip); ws: the *_bytes of the product ----
-bool records_supported(int64_t B, int64_t C1, int64_t C2, int64_t K);
+bool records_gather_applies(int64_t B, int64_t G, int64_t O, int64_t N, int64_t K);
+bool records_scatter_applies(int64_t B, int64_t S, int64_t D, int64_t K);
+bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K);
 size_t records_gather_bytes(int64_t B, int64_t G, int64_t SN);
 int records_gather_product(const double *src, const double *map, const double *iw, const double *w,
                            const double *bias, double *y, void *ws, int64_t B, int64_t G,

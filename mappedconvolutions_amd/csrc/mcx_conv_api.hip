@@ -99,16 +99,12 @@ int fill_zero<double>(double *p, int64_t n, hipStream_t s) { return fill_f64(p, 
 
 // ---- scratch sizes of the three operators -------------------------------------------
 // SH x SW: the image sampled; MH x MW: the map
-// (fp64 runs over channel-last records where the caller's scratch holds them, and on the scalar
-// kernels where it does not)
+// (fp64 runs over channel-last records where they pay and the caller's scratch holds them, and on
+// the scalar kernels, without scratch, elsewhere)
 size_t gather_product_ws(int dtype, int64_t G, int64_t O, int64_t K, int64_t P, int64_t B,
                          int64_t SH, int64_t SW, int64_t MH, int64_t MW) {
-  // (not for an image and a map of one wavefront each: there is nothing to spread, and the source
-  // is cached whole as it lies)
   if (dtype == MCX_F64)
-    return (SH * SW > 64 || MH * MW > 64) && records_supported(B, G, O, K)
-               ? records_gather_bytes(B, G, SH * SW)
-               : 0;
+    return records_gather_applies(B, G, O, MH * MW, K) ? records_gather_bytes(B, G, SH * SW) : 0;
   return use_mfma(dtype, P)
              ? mfma_gather_product_bytes(O, G, K, B, SH, SW, (int)elem_size(dtype), MH, MW)
              : 0;
@@ -116,14 +112,15 @@ size_t gather_product_ws(int dtype, int64_t G, int64_t O, int64_t K, int64_t P, 
 size_t weight_grad_ws(int dtype, int64_t B, int64_t A, int64_t G, int64_t MH, int64_t MW,
                       int64_t K, int64_t P, int64_t GH, int64_t GW) {
   if (dtype == MCX_F64)
-    return records_supported(B, A, G, K)
+    return records_weight_grad_applies(B, A, G, MH * MW, K)
                ? records_weight_grad_bytes(B, A, G, GH * GW, MH * MW, K)
                : 0;
   return use_mfma(dtype, P) ? mfma_weight_grad_bytes(B, A, G, MH, MW, K, GH, GW, elem_size(dtype)) : 0;
 }
 size_t product_scatter_ws(int dtype, int64_t B, int64_t S, int64_t D, int64_t K, int64_t P,
                           int64_t DH, int64_t DW, int64_t MH, int64_t MW) {
-  if (dtype == MCX_F64) return records_supported(B, S, D, K) ? records_scatter_bytes(B, D, DH * DW) : 0;
+  if (dtype == MCX_F64)
+    return records_scatter_applies(B, S, D, K) ? records_scatter_bytes(B, D, DH * DW) : 0;
   return use_mfma(dtype, P)
              ? mfma_product_scatter_bytes(B, S, D, K, DH, DW, elem_size(dtype), MH, MW, P)
              : 0;

@@ -439,8 +439,38 @@ int make_records(const double *x, double *rec, int64_t B, int64_t C, int64_t N, 
 }  // namespace
 
 // A grid has at most 65535 workgroups in its second and third direction.
-bool records_supported(int64_t B, int64_t C1, int64_t C2, int64_t K) {
+static bool records_fit(int64_t B, int64_t C1, int64_t C2, int64_t K) {
   return B <= 65535 && C1 <= 65535 && C2 <= 65535 && K <= 2048;
+}
+
+// Where records pay (us, scalar kernel against records; 8x8 to 500x1000 pixels, one image unless
+// said otherwise, coherent and shuffled maps).
+// The scalar gather is one launch less and walks G * K samples per thread one after the other.
+// Few of them are sooner done, unless there are locations enough to fill the card many times
+// over: 8x8, two channels of 4 taps to one 5.5 / 7.7, to eight 8.4 / 7.9, 64 of 9 taps 653 / 40;
+// 500x1000, 2 -> 32 of 4 taps 105 / 77, shuffled 500 / 104.  One channel has no neighbours to
+// share a line with: 128x256 9 taps 8 / 10, 256x512 10 / 15; 362x724 33 / 28, shuffled 56 / 45, to
+// 32 channels 117 / 75.
+bool records_gather_applies(int64_t B, int64_t G, int64_t O, int64_t N, int64_t K) {
+  if (!records_fit(B, G, O, K)) return false;
+  const bool large = B * N >= 196608;
+  if (G == 1) return large && K >= 9;
+  return G * K >= (O >= 4 ? 8 : 16) || (large && G * K >= 3);
+}
+
+// The scalar scatter loses from two destination channels on (16x16 20 / 11 at ten; 256x512
+// shuffled 2008 / 450); with one on either side it writes what it must: 8.6 / 10.8, 203 / 214.
+bool records_scatter_applies(int64_t B, int64_t S, int64_t D, int64_t K) {
+  return records_fit(B, S, D, K) && (S > 1 || D > 1);
+}
+
+// The scalar weight gradient has one workgroup per (gathered channel, tap, eight plain channels)
+// walk all locations: short walks beat three launches as long as the workgroups are few.  10 -> 1
+// channels, 9 taps: 32x32 6.0 / 10.5, 45x45 9 / 10, 64x64 13 / 10, 91x91 28 / 12; 64 -> 64
+// 16x16 20 / 22 (9.4 M products), 45x45 98 / 57; 128 -> 128 8x8 51 / 42 (9.4 M).
+bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
+  if (!records_fit(B, A, G, K)) return false;
+  return B * N >= 2048 || A * G * K * B * N >= ((int64_t)1 << 23);
 }
 
 #define MCX_LPR(C, CALL)              \

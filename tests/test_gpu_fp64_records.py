@@ -22,7 +22,14 @@ SHAPES = [(1, 1, 1, 1, 1, 0), (2, 1, 9, 5, 7, 0), (3, 4, 6, 4, 32, 0), (4, 5, 9,
           (17, 9, 4, 6, 11, 6), (33, 20, 11, 5, 13, 0)]
 
 
-@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES)
+# Enough locations (of two images) for the weight gradient's records, too: tiles that end ragged,
+# more than one tile a workgroup; one channel, whose forward takes records from 196 608 on
+LARGER = [(1, 1, 1, 32, 32, 0), (2, 1, 9, 31, 67, 0), (3, 4, 6, 32, 33, 0), (5, 16, 10, 30, 43, 0),
+          (8, 17, 9, 29, 45, 0), (9, 2, 5, 48, 48, 3), (16, 3, 9, 34, 33, 0), (17, 9, 4, 36, 31, 6),
+          (33, 20, 3, 45, 53, 0), (1, 3, 9, 320, 308, 0)]
+
+
+@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES + LARGER)
 @pytest.mark.parametrize("interp", [0, 1, 2])
 def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
     g = torch.Generator().manual_seed(ci * 100 + co)
@@ -59,12 +66,12 @@ def test_infinite_interpolation_weights_at_the_border(interp, device):
     not count; an infinite weight of such a tap makes its sample infinite, not NaN.  (Positive
     operands: no two infinities of different signs meet.)"""
     g = torch.Generator().manual_seed(21)
-    B, ci, co, k, p, h, w_ = 2, 5, 3, 9, 2, 12, 14
+    B, ci, co, k, p, h, w_ = 2, 5, 3, 9, 2, 32, 34
     smap, wts = helpers.random_map(g, h, w_, k, p, h, w_, torch.float64)
-    smap.clamp_(-0.4, 13.25)                          # (no tap lies outside altogether)
-    smap[..., 1].clamp_(max=11.25)
-    smap[1] = smap[1].round().clamp_(0, 11)
-    for n in range(0, h * w_, 5):
+    smap.clamp_(-0.4, 33.25)                          # (no tap lies outside altogether)
+    smap[..., 1].clamp_(max=31.25)
+    smap[1] = smap[1].round().clamp_(0, 31)
+    for n in range(0, h * w_, 23):
         wts.view(h * w_, k, p)[n, n % k, n % p] = float("inf")
     x, w, b, gy = (torch.rand(s, generator=g, dtype=torch.float64) + 0.1
                    for s in ((B, ci, h, w_), (co, ci, k), (co,), (B, co, h, w_)))
@@ -83,21 +90,62 @@ def test_infinite_interpolation_weights_at_the_border(interp, device):
         assert not ok.any() or ((a - c).abs()[ok] <= 1e-12 * c.abs()[ok].max()).all(), i
 
 
-def test_fp64_without_a_workspace(device):
+def _every_call(lib, workspace):
+    """The six products of both convolutions through the C ABI, fp64; `workspace(bytes)` gives the
+    (pointer, size) that each call is handed.  [(what, bytes asked for, result, oracle's)]."""
     g = torch.Generator().manual_seed(5)
-    B, ci, co, k, h, w_ = 2, 5, 3, 9, 7, 8
+    B, ci, co, k, h, w_ = 2, 5, 3, 9, 33, 40
     smap, _ = helpers.random_map(g, h, w_, k, 0, h, w_, torch.float64)
-    x, w, b = (torch.randn(s, generator=g, dtype=torch.float64)
-               for s in ((B, ci, h, w_), (co, ci, k), (co,)))
-    want = O.mapped_conv_forward(x, smap, w, b, k, 1)
-    dx, dm, dw, db = (t.cuda() for t in (x, smap, w, b))
-    out = torch.empty(B, co, h, w_, dtype=torch.float64, device=device)
-    lib = _lib.load()
-    rc = lib.mcx_conv_forward(dx.data_ptr(), dm.data_ptr(), None, dw.data_ptr(), db.data_ptr(),
-                              out.data_ptr(), None, 0, B, ci, co, h, w_, h, w_, k, 0, 1,
-                              _lib.MCX_F64, torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    assert rel_err(out, want) < 1e-12
+    x, w, b, gy = (torch.randn(s, generator=g, dtype=torch.float64)
+                   for s in ((B, ci, h, w_), (co, ci, k), (co,), (B, co, h, w_)))
+    wt, bt = w.transpose(0, 1).contiguous(), b            # [ci, co, k] of the transposed one
+    dx, dm, dw, db, dg, dwt = (t.cuda() for t in (x, smap, w, b, gy, wt))
+    ptr = lambda t: None if t is None else t.data_ptr()
+    size, tail = (B, ci, co, h, w_, h, w_, k, 0), (1, _lib.MCX_F64,
+                                                    torch.cuda.current_stream().cuda_stream)
+    new = lambda t: torch.full(t.shape, float("nan"), dtype=torch.float64, device="cuda")
+    out = []
+
+    def forward(name, weight, weight_d, want):
+        need = getattr(lib, "mcx_%s_forward_workspace" % name)(*size, _lib.MCX_F64)
+        y = new(want)
+        rc = getattr(lib, "mcx_%s_forward" % name)(ptr(dx), ptr(dm), None, ptr(weight_d), ptr(db),
+                                                   ptr(y), *workspace(need), *size, *tail)
+        assert rc == 0
+        out.append((name, need, y, want))
+
+    def backward(name, weight_d, want):
+        need = getattr(lib, "mcx_%s_backward_workspace" % name)(*size, _lib.MCX_F64)
+        for i in range(3):                                # one gradient a call
+            grads = [new(t) if i == j else None for j, t in enumerate(want)]
+            rc = getattr(lib, "mcx_%s_backward" % name)(ptr(dg), ptr(dm), None, ptr(dx),
+                                                        ptr(weight_d), *map(ptr, grads),
+                                                        *workspace(need), *size, *tail)
+            assert rc == 0
+            out.append((name, need, grads[i], want[i]))
+
+    forward("conv", w, dw, O.mapped_conv_forward(x, smap, w, b, k, 1))
+    backward("conv", dw, O.mapped_conv_backward(gy, smap, x, w, b, k, 1))
+    forward("tconv", wt, dwt, O.mapped_transposed_conv_forward(x, smap, wt, bt, h, w_, k, 1))
+    backward("tconv", dwt, O.mapped_transposed_conv_backward(gy, smap, x, wt, bt, k, 1))
+    return out
+
+
+@pytest.mark.parametrize("given", ["all", "one byte less", "none"])
+def test_fp64_without_a_workspace(given, device):
+    """Every product asks for a workspace at this size and does without one, or with less: the
+    scalar kernels."""
+    lib, kept = _lib.load(), []
+
+    def workspace(need):
+        if given == "none":
+            return None, 0
+        kept.append(torch.empty(need, dtype=torch.uint8, device=device))
+        return kept[-1].data_ptr(), need - (given != "all")
+
+    for name, need, got, want in _every_call(lib, workspace):
+        assert need > 0, name
+        assert rel_err(got, want) < 1e-12, name
 
 
 @pytest.mark.parametrize("n", [1 << 13, (1 << 13) + 1, 100003])

@@ -41,7 +41,11 @@ def test_rejected_arguments_return_codes_without_a_gpu():
     assert lib.mcx_conv_forward(1, 1, None, 1, 1, 1, None, 0, 1, 1, 1, 4, 4, 4, 4, 1, 0, 1, 0,
                                 None) == -4
     assert lib.mcx_conv_forward_workspace(1, 64, 64, 8, 8, 8, 8, 9, 0, 0) > 0
-    assert lib.mcx_conv_forward_workspace(1, 64, 64, 8, 8, 8, 8, 9, 0, 1) == 0  # fp64: scalar kernels
+    # fp64: a copy of the sampled operand in records where the product runs over them, and nothing
+    # where the scalar kernels are as fast (one channel; few samples a location)
+    assert lib.mcx_conv_forward_workspace(1, 64, 64, 8, 8, 8, 8, 9, 0, 1) >= 64 * 64 * 8
+    assert lib.mcx_conv_forward_workspace(1, 1, 64, 8, 8, 8, 8, 9, 0, 1) == 0
+    assert lib.mcx_conv_forward_workspace(1, 3, 1, 8, 8, 8, 8, 4, 0, 1) == 0
     assert lib.mcx_resample_from_map(1, 1, None, 1, 0, 1, 4, 4, 4, 4, 0, 1, 0, None) == -2
     assert lib.mcx_resample_from_map(1, 1, None, 1, 1, 1, 4, 4, 4, 4, 0, 1, 7, None) == -1
     assert lib.mcx_knn(1, 1, 1, 1, None, 0, 1, 3, 10, 10, 65, 0, None) == -2
