@@ -11,14 +11,17 @@ namespace mcx {
 int fill_f32(float *p, int64_t n, float v, hipStream_t s);
 int fill_f64(double *p, int64_t n, double v, hipStream_t s);
 
+// only_if: a word on the device, the kernel returns at once where it is zero (NULL: always runs)
 template <typename T>
 int generic_gather_product(const T *src, const T *map, const T *iw, const T *w, const T *bias,
                            T *y, int64_t B, int64_t G, int64_t O, int64_t SH, int64_t SW,
-                           int64_t N, int64_t K, int64_t P, int interp, hipStream_t s);
+                           int64_t N, int64_t K, int64_t P, int interp, hipStream_t s,
+                           const int *only_if = nullptr);
 template <typename T>
 int generic_product_scatter(const T *src, const T *map, const T *iw, const T *w, T *dst,
                             int64_t B, int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N,
-                            int64_t K, int64_t P, int interp, hipStream_t s);
+                            int64_t K, int64_t P, int interp, hipStream_t s,
+                            const int *only_if = nullptr);
 template <typename T>
 int generic_weight_grad(const T *plain, const T *gath, const T *map, const T *iw, T *gw,
                         int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t N,
@@ -27,12 +30,12 @@ int generic_weight_grad(const T *plain, const T *gath, const T *map, const T *iw
 bool records_gather_applies(int64_t B, int64_t G, int64_t O, int64_t N, int64_t K);
 bool records_scatter_applies(int64_t B, int64_t S, int64_t D, int64_t K);
 bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K);
-size_t records_gather_bytes(int64_t B, int64_t G, int64_t SN);
+size_t records_gather_bytes(int64_t B, int64_t G, int64_t O, int64_t SN, int64_t N, int64_t K);
 int records_gather_product(const double *src, const double *map, const double *iw, const double *w,
                            const double *bias, double *y, void *ws, int64_t B, int64_t G,
                            int64_t O, int64_t SH, int64_t SW, int64_t N, int64_t K, int64_t P,
                            int interp, hipStream_t s);
-size_t records_scatter_bytes(int64_t B, int64_t D, int64_t DN);
+size_t records_scatter_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K);
 int records_product_scatter(const double *src, const double *map, const double *iw,
                             const double *w, const double *bias, double *dst, void *ws, int64_t B,
                             int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,

@@ -104,7 +104,8 @@ int fill_zero<double>(double *p, int64_t n, hipStream_t s) { return fill_f64(p, 
 size_t gather_product_ws(int dtype, int64_t G, int64_t O, int64_t K, int64_t P, int64_t B,
                          int64_t SH, int64_t SW, int64_t MH, int64_t MW) {
   if (dtype == MCX_F64)
-    return records_gather_applies(B, G, O, MH * MW, K) ? records_gather_bytes(B, G, SH * SW) : 0;
+    return records_gather_applies(B, G, O, MH * MW, K) ? records_gather_bytes(B, G, O, SH * SW, MH * MW, K)
+                                                      : 0;
   return use_mfma(dtype, P)
              ? mfma_gather_product_bytes(O, G, K, B, SH, SW, (int)elem_size(dtype), MH, MW)
              : 0;
@@ -120,7 +121,7 @@ size_t weight_grad_ws(int dtype, int64_t B, int64_t A, int64_t G, int64_t MH, in
 size_t product_scatter_ws(int dtype, int64_t B, int64_t S, int64_t D, int64_t K, int64_t P,
                           int64_t DH, int64_t DW, int64_t MH, int64_t MW) {
   if (dtype == MCX_F64)
-    return records_scatter_applies(B, S, D, K) ? records_scatter_bytes(B, D, DH * DW) : 0;
+    return records_scatter_applies(B, S, D, K) ? records_scatter_bytes(B, S, D, DH * DW, MH * MW, K) : 0;
   return use_mfma(dtype, P)
              ? mfma_product_scatter_bytes(B, S, D, K, DH, DW, elem_size(dtype), MH, MW, P)
              : 0;

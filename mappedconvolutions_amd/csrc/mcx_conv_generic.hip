@@ -43,7 +43,8 @@ template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads) void gather_product_kernel(
     const T *__restrict__ src, const T *__restrict__ map, const T *__restrict__ iw,
     const T *__restrict__ w, const T *__restrict__ bias, T *__restrict__ y, int G, int O, int SH,
-    int SW, int N, int K, int P) {
+    int SW, int N, int K, int P, const int *__restrict__ only_if) {
+  if (only_if && *only_if == 0) return;
   const int n = blockIdx.x * kThreads + threadIdx.x;
   if (n >= N) return;
   const int o0 = blockIdx.y * kOT;
@@ -72,7 +73,8 @@ template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads) void product_scatter_kernel(
     const T *__restrict__ src, const T *__restrict__ map, const T *__restrict__ iw,
     const T *__restrict__ w, T *__restrict__ dst, int S, int D, int DH, int DW, int N, int K,
-    int P) {
+    int P, const int *__restrict__ only_if) {
+  if (only_if && *only_if == 0) return;
   const int n = blockIdx.x * kThreads + threadIdx.x;
   if (n >= N) return;
   const int d0 = blockIdx.y * kOT;
@@ -208,12 +210,13 @@ __global__ void fill_bias_kernel(T *__restrict__ y, const T *__restrict__ bias, 
 template <typename T>
 int generic_gather_product(const T *src, const T *map, const T *iw, const T *w, const T *bias,
                            T *y, int64_t B, int64_t G, int64_t O, int64_t SH, int64_t SW,
-                           int64_t N, int64_t K, int64_t P, int interp, hipStream_t s) {
+                           int64_t N, int64_t K, int64_t P, int interp, hipStream_t s,
+                           const int *only_if) {
   dim3 grid(div_up(N, kThreads), div_up(O, kOT), (unsigned)B);
   MCX_DISPATCH_MODE(interp, hipLaunchKernelGGL((gather_product_kernel<T, MODE>), grid,
                                                dim3(kThreads), 0, s, src, map, iw, w, bias, y,
                                                (int)G, (int)O, (int)SH, (int)SW, (int)N, (int)K,
-                                               (int)P));
+                                               (int)P, only_if));
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }
@@ -221,11 +224,12 @@ int generic_gather_product(const T *src, const T *map, const T *iw, const T *w, 
 template <typename T>
 int generic_product_scatter(const T *src, const T *map, const T *iw, const T *w, T *dst,
                             int64_t B, int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N,
-                            int64_t K, int64_t P, int interp, hipStream_t s) {
+                            int64_t K, int64_t P, int interp, hipStream_t s, const int *only_if) {
   dim3 grid(div_up(N, kThreads), div_up(D, kOT), (unsigned)B);
   MCX_DISPATCH_MODE(interp, hipLaunchKernelGGL((product_scatter_kernel<T, MODE>), grid,
                                                dim3(kThreads), 0, s, src, map, iw, w, dst, (int)S,
-                                               (int)D, (int)DH, (int)DW, (int)N, (int)K, (int)P));
+                                               (int)D, (int)DH, (int)DW, (int)N, (int)K, (int)P,
+                                               only_if));
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }
@@ -287,10 +291,11 @@ int fill_bias(T *y, const T *bias, int64_t B, int64_t C, int64_t N, hipStream_t 
 #define MCX_INSTANTIATE(T)                                                                         \
   template int generic_gather_product<T>(const T *, const T *, const T *, const T *, const T *,   \
                                          T *, int64_t, int64_t, int64_t, int64_t, int64_t,        \
-                                         int64_t, int64_t, int64_t, int, hipStream_t);            \
+                                         int64_t, int64_t, int64_t, int, hipStream_t,             \
+                                         const int *);                                            \
   template int generic_product_scatter<T>(const T *, const T *, const T *, const T *, T *,        \
                                           int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,   \
-                                          int64_t, int64_t, int, hipStream_t);                    \
+                                          int64_t, int64_t, int, hipStream_t, const int *);       \
   template int generic_weight_grad<T>(const T *, const T *, const T *, const T *, T *, int64_t,   \
                                       int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,       \
                                       int64_t, int, hipStream_t);                                 \

@@ -32,20 +32,62 @@ struct RecShape {
 
 // Record stride in doubles: 16-byte pairs for reading.
 inline int64_t read_stride(int64_t channels) { return (channels + 1) & ~(int64_t)1; }
-// Records that atomics add to: up to 16 channels a power of two, so that a run of eight
-// channels, one request of 64 bytes, never straddles a boundary.
+// Records that atomics add to.  Requests are of 64 bytes: up to eight channels a power of two and
+// from 17 on a multiple of eight, so that no run of eight straddles a boundary (five channels
+// without a pad, shuffled map of 256x512: 224 -> 330 us).  Nine to sixteen lie side by side:
+// neighbouring records then share requests, and where they do not it costs nothing (ten channels
+// padded to sixteen, coherent 502 -> 341 us, shuffled 450 -> 445).
 inline int64_t add_stride(int64_t channels) {
-  for (int64_t s = 2; s <= 16; s *= 2)
+  for (int64_t s = 2; s <= 8; s *= 2)
     if (channels <= s) return s;
-  return (channels + 7) & ~(int64_t)7;
+  return channels <= 16 ? (channels + 1) & ~(int64_t)1 : (channels + 7) & ~(int64_t)7;
 }
 inline int lanes_per_record(int64_t channels) { return channels <= 4 ? 2 : channels <= 8 ? 4 : 8; }
+
+// *coherent = 1 if in three of four samples of the map (up to 1024 taps) the next location's tap
+// points at the pixel beside, else 0: what decides between planes and records where neither form
+// is better for every map.  Block 0; the others clear `count` pairs of doubles, it helps.
+__global__ __launch_bounds__(kThreads) void begin_records_kernel(const double *__restrict__ map,
+                                                                 int64_t N, int K, int pm,
+                                                                 int nearest,
+                                                                 int *__restrict__ coherent,
+                                                                 double2 *__restrict__ clear,
+                                                                 int64_t count) {
+  if (coherent && blockIdx.x == 0) {
+    constexpr int kSamples = 4 * kThreads;
+    int beside = 0;
+    for (int i = threadIdx.x; i < kSamples; i += kThreads) {
+      // (spread by the golden ratio, not by a stride that could meet a row's end every time;
+      // N > 1 where the map is asked, n <= N - 2)
+      const uint64_t u = (uint32_t)i * 2654435769u;
+      const int64_t n = (int64_t)((u * (uint64_t)(N - 1)) >> 32);
+      const int64_t e = (n * K + i % K) * pm, e2 = e + (int64_t)K * pm;
+      double x = map[e * 2], y = map[e * 2 + 1], x2 = map[e2 * 2], y2 = map[e2 * 2 + 1];
+      if (nearest) {
+        x = round_half_away(x), y = round_half_away(y);
+        x2 = round_half_away(x2), y2 = round_half_away(y2);
+      } else {
+        x = mcx_floor(x), y = mcx_floor(y), x2 = mcx_floor(x2), y2 = mcx_floor(y2);
+      }
+      const double d = x2 - x;
+      beside += __syncthreads_count(y == y2 && (d == 1.0 || d == -1.0));
+    }
+    if (threadIdx.x == 0) *coherent = beside * 4 >= kSamples * 3 ? 1 : 0;
+  }
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < count; i += stride)
+    clear[i] = make_double2(0.0, 0.0);
+}
+
+// `unless` below: a word that ends the kernel at once where it is not zero (NULL: always runs).
 
 // [B][C][N] -> records [B][N + 1][stride]; the last record of an image is all zeros (what a
 // corner outside the image reads), as are the channels beyond C.
 __global__ __launch_bounds__(kThreads) void to_records_kernel(const double *__restrict__ x,
                                                               double *__restrict__ rec, int C,
-                                                              int stride, int64_t N) {
+                                                              int stride, int64_t N,
+                                                              const int *__restrict__ unless) {
+  if (unless && *unless != 0) return;
   const int64_t n = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   const int b = blockIdx.z;
   if (n > N) return;
@@ -62,19 +104,21 @@ __global__ __launch_bounds__(kThreads) void to_records_kernel(const double *__re
   }
 }
 
-// records [B][N][stride] -> [B][C][N], plus bias
+// records [B][N][stride] -> [B][C][N], plus bias; the bias alone where `bias_only` says so
 __global__ __launch_bounds__(kThreads) void from_records_kernel(const double *__restrict__ rec,
                                                                 const double *__restrict__ bias,
                                                                 double *__restrict__ y, int C,
-                                                                int stride, int64_t N) {
+                                                                int stride, int64_t N,
+                                                                const int *__restrict__ bias_only) {
   const int64_t n = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   const int b = blockIdx.z;
   if (n >= N) return;
   const double2 *src = reinterpret_cast<const double2 *>(rec + ((int64_t)b * N + n) * stride);
   double *dst = y + (int64_t)b * C * N + n;
+  const bool skip = bias_only && *bias_only != 0;
   const int c_end = min(C, (int)(blockIdx.y + 1) * 16);
   for (int c = blockIdx.y * 16; c < c_end; c += 2) {
-    const double2 v = src[c >> 1];
+    const double2 v = skip ? make_double2(0.0, 0.0) : src[c >> 1];
     dst[(int64_t)c * N] = v.x + (bias ? bias[c] : 0.0);
     if (c + 1 < C) dst[(int64_t)(c + 1) * N] = v.y + (bias ? bias[c + 1] : 0.0);
   }
@@ -149,7 +193,9 @@ template <int NC, int LPR, int OT>
 __global__ __launch_bounds__(kThreads) void gather_records_kernel(
     const double *__restrict__ rec, const double *__restrict__ map, const double *__restrict__ iw,
     const double *__restrict__ w, const double *__restrict__ bias, double *__restrict__ y, int G,
-    int stride, int O, int SH, int SW, int N, int K, int P, int wrap) {
+    int stride, int O, int SH, int SW, int N, int K, int P, int wrap,
+    const int *__restrict__ unless) {
+  if (unless && *unless != 0) return;
   using S = RecShape<LPR>;
   constexpr int kStep = S::kTaps * S::kLocs;
   __shared__ int s_off[NC * kStep];
@@ -226,7 +272,8 @@ template <int NC, int LPR>
 __global__ __launch_bounds__(kThreads) void scatter_records_kernel(
     const double *__restrict__ src, const double *__restrict__ map, const double *__restrict__ iw,
     const double *__restrict__ w, double *__restrict__ rec, int S_, int D, int stride, int DH,
-    int DW, int N, int K, int P, int wrap) {
+    int DW, int N, int K, int P, int wrap, const int *__restrict__ unless) {
+  if (unless && *unless != 0) return;
   using S = RecShape<LPR>;
   constexpr int kStep = S::kTaps * S::kLocs;
   constexpr int kSrc = 16;  // source channels per pass
@@ -428,12 +475,56 @@ GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
 
 bool wraps(int interp) { return canonical_interp(interp) == kInterpBispherical; }
 
-int make_records(const double *x, double *rec, int64_t B, int64_t C, int64_t N, hipStream_t s) {
+int make_records(const double *x, double *rec, int64_t B, int64_t C, int64_t N, hipStream_t s,
+                 const int *unless = nullptr) {
   const int64_t stride = read_stride(C);
   const dim3 grid(div_up(N + 1, kThreads), div_up(stride, 16), (unsigned)B);
-  hipLaunchKernelGGL(to_records_kernel, grid, dim3(kThreads), 0, s, x, rec, (int)C, (int)stride, N);
+  hipLaunchKernelGGL(to_records_kernel, grid, dim3(kThreads), 0, s, x, rec, (int)C, (int)stride, N,
+                     unless);
   MCX_HIP_CHECK_LAUNCH();
   return 0;
+}
+
+// Whether the map is examined (coherent) and `count` doubles cleared.
+int begin_records(const double *map, int64_t N, int64_t K, int64_t P, int interp, int *coherent,
+                  double *clear, int64_t count, hipStream_t s) {
+  const unsigned blocks =
+      (unsigned)std::max<int64_t>(1, std::min<int64_t>((count / 2 + 1023) / 1024, 8192));
+  hipLaunchKernelGGL(begin_records_kernel, dim3(blocks), dim3(kThreads), 0, s, map, N, (int)K,
+                     (int)(P == 0 ? 1 : P), canonical_interp(interp) == kInterpNearest ? 1 : 0,
+                     coherent, (double2 *)clear, count / 2);
+  MCX_HIP_CHECK_LAUNCH();
+  return 0;
+}
+
+size_t gather_record_bytes(int64_t B, int64_t G, int64_t SN) {
+  return align256((size_t)(B * (SN + 1) * read_stride(G)) * sizeof(double));
+}
+size_t scatter_record_bytes(int64_t B, int64_t D, int64_t DN) {
+  return align256((size_t)(B * DN * add_stride(D)) * sizeof(double));
+}
+
+// ---- where the map decides ----
+// Neither form is better for every map, and which kind the map is only the device knows: it is
+// examined, both forms are launched, one returns at once.  That costs 5 to 9 us a call, which the
+// rules' lines leave below the difference.  (us, scalar / records / with the map examined)
+// One or two taps: those of a coherent map are reads of neighbouring pixels, which planes serve as
+// well, without the copy.  362x724, 64 -> 8 channels, one tap: 102 / 330 / 111, shuffled
+// 503 / 338 / 346; 16 -> 8, two taps 54 / 88 / 64, shuffled 243 / 90 / 98, but 16 -> 32 157 / 148,
+// and at 256x512 64 -> 8 of two taps 175 / 127, 64 -> 32 of one 174 / 163.
+bool gather_asks_map(int64_t B, int64_t G, int64_t O, int64_t N, int64_t K) {
+  return N > 1 && G > 1 && (K == 1 || (K == 2 && O <= 16)) && B * N >= 196608 &&
+         B * N * G >= ((int64_t)3 << 20);
+}
+// Scattering: neighbouring lanes of the scalar kernel add to neighbouring pixels of a plane, eight
+// a request, where records take a request or two each.  256x512, nine taps, latitude map: 1 -> 10
+// channels 124 / 142 / 134, 4 -> 5 66 / 106 / 78, 1 -> 17 203 / 292 / 224; fractional rows and
+// columns 1 -> 10 278 / 341 / 288; shuffled 2008 / 445 / 450.  (64x128 1 -> 10: 19 / 18 / 26.)  From
+// nine source channels on the products cost the scalar kernel what it saves (16 -> 5 98 / 113, 16 ->
+// 24 360 / 325), except where the last of three or more runs of eight holds a channel or two
+// (16 -> 17 239 / 315).
+bool scatter_asks_map(int64_t B, int64_t S, int64_t N, int64_t K) {
+  return N > 1 && S <= 8 && B * N * K >= ((int64_t)1 << 20);
 }
 
 }  // namespace
@@ -480,8 +571,9 @@ bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int
     default: { CALL(8) } break;       \
   }
 
-size_t records_gather_bytes(int64_t B, int64_t G, int64_t SN) {
-  return align256((size_t)(B * (SN + 1) * read_stride(G)) * sizeof(double));
+// (the word about the map last)
+size_t records_gather_bytes(int64_t B, int64_t G, int64_t O, int64_t SN, int64_t N, int64_t K) {
+  return gather_record_bytes(B, G, SN) + (gather_asks_map(B, G, O, N, K) ? 256 : 0);
 }
 
 int records_gather_product(const double *src, const double *map, const double *iw, const double *w,
@@ -489,14 +581,19 @@ int records_gather_product(const double *src, const double *map, const double *i
                            int64_t O, int64_t SH, int64_t SW, int64_t N, int64_t K, int64_t P,
                            int interp, hipStream_t s) {
   double *rec = (double *)ws;
-  if (int rc = make_records(src, rec, B, G, SH * SW, s)) return rc;
+  int *coherent = nullptr;
+  if (gather_asks_map(B, G, O, N, K)) {
+    coherent = (int *)((char *)ws + gather_record_bytes(B, G, SH * SW));
+    if (int rc = begin_records(map, N, K, P, interp, coherent, nullptr, 0, s)) return rc;
+  }
+  if (int rc = make_records(src, rec, B, G, SH * SW, s, coherent)) return rc;
   const int stride = (int)read_stride(G);
   const bool one = canonical_interp(interp) == kInterpNearest;
 #define MCX_RUN(NC, LPR, OT)                                                                     \
   hipLaunchKernelGGL((gather_records_kernel<NC, LPR, OT>),                                       \
                      dim3(div_up(N, kThreads / LPR), div_up(O, OT), (unsigned)B), dim3(kThreads), \
                      0, s, rec, map, iw, w, bias, y, (int)G, stride, (int)O, (int)SH, (int)SW,   \
-                     (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0);
+                     (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0, coherent);
 #define MCX_OT(NC, LPR)                             \
   if (O == 1) { MCX_RUN(NC, LPR, 1) }               \
   else if (O <= 4) { MCX_RUN(NC, LPR, 4) }          \
@@ -507,11 +604,13 @@ int records_gather_product(const double *src, const double *map, const double *i
 #undef MCX_OT
 #undef MCX_RUN
   MCX_HIP_CHECK_LAUNCH();
-  return 0;
+  if (!coherent) return 0;
+  return generic_gather_product<double>(src, map, iw, w, bias, y, B, G, O, SH, SW, N, K, P, interp,
+                                        s, coherent);
 }
 
-size_t records_scatter_bytes(int64_t B, int64_t D, int64_t DN) {
-  return align256((size_t)(B * DN * add_stride(D)) * sizeof(double));
+size_t records_scatter_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
+  return scatter_record_bytes(B, D, DN) + (scatter_asks_map(B, S, N, K) ? 256 : 0);
 }
 
 int records_product_scatter(const double *src, const double *map, const double *iw,
@@ -520,13 +619,16 @@ int records_product_scatter(const double *src, const double *map, const double *
                             int64_t P, int interp, hipStream_t s) {
   double *rec = (double *)ws;
   const int64_t DN = DH * DW, stride = add_stride(D);
-  if (int rc = fill_f64(rec, B * DN * stride, 0.0, s)) return rc;
+  int *coherent = scatter_asks_map(B, S, N, K)
+                      ? (int *)((char *)ws + scatter_record_bytes(B, D, DN))
+                      : nullptr;
+  if (int rc = begin_records(map, N, K, P, interp, coherent, rec, B * DN * stride, s)) return rc;
   const bool one = canonical_interp(interp) == kInterpNearest;
 #define MCX_RUN(NC, LPR)                                                                          \
   hipLaunchKernelGGL((scatter_records_kernel<NC, LPR>),                                           \
                      dim3(div_up(N, kThreads / LPR), div_up(D, LPR), (unsigned)B),                \
                      dim3(kThreads), 0, s, src, map, iw, w, rec, (int)S, (int)D, (int)stride,     \
-                     (int)DH, (int)DW, (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0);
+                     (int)DH, (int)DW, (int)N, (int)K, (int)P, wraps(interp) ? 1 : 0, coherent);
 #define MCX_NC(LPR) if (one) { MCX_RUN(1, LPR) } else { MCX_RUN(4, LPR) }
   if (D <= 2) { MCX_NC(2) }
   else if (D <= 4) { MCX_NC(4) }
@@ -536,15 +638,17 @@ int records_product_scatter(const double *src, const double *map, const double *
 #undef MCX_RUN
   MCX_HIP_CHECK_LAUNCH();
   hipLaunchKernelGGL(from_records_kernel, dim3(div_up(DN, kThreads), div_up(D, 16), (unsigned)B),
-                     dim3(kThreads), 0, s, rec, bias, dst, (int)D, (int)stride, DN);
+                     dim3(kThreads), 0, s, rec, bias, dst, (int)D, (int)stride, DN, coherent);
   MCX_HIP_CHECK_LAUNCH();
-  return 0;
+  if (!coherent) return 0;
+  return generic_product_scatter<double>(src, map, iw, w, dst, B, S, D, DH, DW, N, K, P, interp, s,
+                                         coherent);
 }
 
 size_t records_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t GN, int64_t N,
                                  int64_t K) {
   const GradShape q = grad_shape(B, A, G, N, K);
-  return records_gather_bytes(B, G, GN) + align256((size_t)(q.ranges * K * A * G) * sizeof(double));
+  return gather_record_bytes(B, G, GN) + align256((size_t)(q.ranges * K * A * G) * sizeof(double));
 }
 
 int records_weight_grad(const double *plain, const double *gath, const double *map,
@@ -552,7 +656,7 @@ int records_weight_grad(const double *plain, const double *gath, const double *m
                         int64_t GH, int64_t GW, int64_t N, int64_t K, int64_t P, int interp,
                         hipStream_t s) {
   double *rec = (double *)ws;
-  double *part = (double *)((char *)ws + records_gather_bytes(B, G, GH * GW));
+  double *part = (double *)((char *)ws + gather_record_bytes(B, G, GH * GW));
   if (int rc = make_records(gath, rec, B, G, GH * GW, s)) return rc;
   const GradShape q = grad_shape(B, A, G, N, K);
   const bool one = canonical_interp(interp) == kInterpNearest;

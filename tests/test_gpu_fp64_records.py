@@ -90,6 +90,45 @@ def test_infinite_interpolation_weights_at_the_border(interp, device):
         assert not ok.any() or ((a - c).abs()[ok] <= 1e-12 * c.abs()[ok].max()).all(), i
 
 
+# (S, D, K, map rows, columns, P): both sides of the rules that let the map decide (for the scatter
+# 2^20 taps of up to eight source channels; for the gather, from D channels into S, 196 608
+# locations of 3 * 2^20 samples at one tap, or at two for up to sixteen outputs), under maps that
+# are coherent, that are not, and half of whose neighbours are
+@pytest.mark.parametrize("s,d,k,mh,mw,p", [(1, 10, 9, 241, 242, 0), (2, 3, 9, 241, 241, 0),
+                                           (1, 17, 9, 241, 242, 2), (8, 9, 9, 241, 242, 0),
+                                           (9, 9, 9, 241, 242, 0), (3, 16, 1, 314, 314, 0),
+                                           (3, 15, 1, 314, 314, 0), (16, 16, 2, 314, 314, 2),
+                                           (17, 16, 2, 314, 314, 0)])
+@pytest.mark.parametrize("kind", ["coherent", "shuffled", "half"])
+def test_fp64_products_where_the_map_decides(s, d, k, mh, mw, p, kind, device):
+    g = torch.Generator().manual_seed(mh + s)
+    B, interp, np = 2, 1, max(p, 1)
+    at = torch.arange(mh * mw)
+    if kind == "shuffled":
+        at = torch.randperm(mh * mw, generator=g)
+    elif kind == "half":
+        at = torch.where(at // 2 % 2 == 0, at, at.flip(0))
+    base = torch.stack((at % mw, at // mw), -1).double().view(mh, mw, 1, 1, 2)
+    step = torch.randint(-2, 3, (1, 1, k, np, 2), generator=g)
+    smap = (base + step + 0.3).contiguous()
+    smap = smap if p else smap[:, :, :, 0].contiguous()
+    wts = torch.rand(mh, mw, k, p, generator=g, dtype=torch.float64) if p else None
+    rnd = lambda *size: torch.randn(size, generator=g, dtype=torch.float64)
+    # a transposed convolution: s channels scattered into d, and d gathered into s
+    x, w, b, gy = rnd(B, s, mh, mw), rnd(s, d, k), rnd(d), rnd(B, d, mh, mw)
+    pre, maps = ("weighted_", (smap, wts)) if p else ("", (smap,))
+    dm = [t.cuda() for t in maps]
+    y = getattr(_C, pre + "mapped_transposed_conv_forward")(x.cuda(), *dm, w.cuda(), b.cuda(), mh,
+                                                            mw, k, interp)
+    want = getattr(O, pre + "mapped_transposed_conv_forward")(x, *maps, w, b, mh, mw, k, interp)
+    assert rel_err(y, want) < 1e-12
+    gx = getattr(_C, pre + "mapped_transposed_conv_backward")(gy.cuda(), *dm, x.cuda(), w.cuda(),
+                                                              b.cuda(), k, interp,
+                                                              needs=(True, False, False))[0]
+    want = getattr(O, pre + "mapped_transposed_conv_backward")(gy, *maps, x, w, b, k, interp)[0]
+    assert rel_err(gx, want) < 1e-12
+
+
 def _every_call(lib, workspace):
     """The six products of both convolutions through the C ABI, fp64; `workspace(bytes)` gives the
     (pointer, size) that each call is handed.  [(what, bytes asked for, result, oracle's)]."""
