@@ -2399,12 +2399,12 @@ SplitJob split_job(char *region, bool planar, int64_t tiles) {
 // are addressed as buffers of less than 4 GiB.
 bool split_applies(int64_t G, int64_t O, int64_t SH, int64_t SW, int64_t K, const ModeArgs &m,
                    bool packed, bool cl) {
-  // Few channels: a tap's six instructions round their sums six times, the fp32 ones once per two
-  // channels.  Error of the split over that of the fp32 instructions, in 2-norm against 64 bits, at
-  // nine whole-pixel taps: 2.03, 1.55, 1.29, 1.13, 1.02 for one to five channels, 0.94 to 0.82 for
-  // six to eight, 1.01 and 0.99 (1.03 and 1.01 at 25 taps) for nine and ten, 0.81 to 0.98 from
-  // eleven up (0.84 at 64).
-  if (G <= 5 || G == 9 || G == 10) return false;
+  // Few channels: a tap's six instructions round their sums six times per eight channels, the fp32
+  // ones once a channel.  Error of the split over that of the fp32 instructions, in 2-norm against
+  // 64 bits, at nine whole-pixel taps: 2.03, 1.55, 1.29, 1.13, 1.02 for one to five channels, 0.94
+  // to 0.82 for six to eight, 1.01 and 0.99 for nine and ten (0.93 at three taps, 1.03 and 1.01 at
+  // 25: the same), 0.81 to 0.98 from eleven up (0.84 at 64).
+  if (G <= 5) return false;
   const int64_t Gpad = round_up(G, kGC), Opad = round_up(O, kOT);
   if (K * (Gpad / kGC) * 6 * Opad * 16 >= (int64_t)kOobOffset) return false;
   if (SH * SW * (cl ? Gpad : G) * 4 >= (int64_t)kOobOffset) return false;

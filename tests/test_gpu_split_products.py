@@ -244,8 +244,7 @@ def _forward_both(x, smap, w, b, k, interp):
 def test_accuracy_is_not_below_fp32(c, interp, shift, device):
     """Distance from the 64-bit result in 2-norm: the forward's is no larger than that of the fp32
     matrix instructions on the same operands, which serve it themselves where the split products'
-    would be (few channels).  (Some 130 000 results: their root mean square is known to better
-    than the 2 % allowed for.)"""
+    would be (few channels).  (2 % are allowed for: at nine and ten channels the two are equal.)"""
     g = torch.Generator().manual_seed(9)
     h, w_, k, co = 32, 64, 9, 64
     smap = synthetic.latitude_map(h, w_, 1) + shift
@@ -253,5 +252,5 @@ def test_accuracy_is_not_below_fp32(c, interp, shift, device):
     split, fp32 = _forward_both(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
     want = O.mapped_conv_forward(x.double(), smap.double(), w.double(), b.double(), k, interp)
     far = lambda y: ((y - want).norm() / want.norm()).item()
-    assert torch.equal(split, fp32) == (c in (1, 2, 3, 4, 5, 9, 10))
+    assert torch.equal(split, fp32) == (c <= 5)
     assert far(split) <= 1.02 * far(fp32), (far(split), far(fp32))
