@@ -99,6 +99,17 @@ def _workspace(nbytes, device):
     return torch.empty((max(int(nbytes), 1),), dtype=torch.uint8, device=device)
 
 
+def _conv_workspace(nbytes, dt, device):
+    """Scratch of a convolution call and its size.  float64 data needs none (the library then runs
+    its scalar kernels), so a call that leaves no memory for it goes through without."""
+    try:
+        return _workspace(nbytes, device), nbytes
+    except torch.OutOfMemoryError:
+        if dt != MCX_F64:
+            raise
+        return None, 0
+
+
 def _weighted_dims(sample_map, interp_weights, kernel):
     """Number of interpolation points P (0 = unweighted) after a shape check."""
     want = (4 if kernel else 3) + (0 if interp_weights is None else 1)
@@ -132,8 +143,8 @@ def _conv_forward(input, sample_map, interp_weights, weight, bias, kernel_size, 
         raise RuntimeError("bias must have %d elements" % Co)
     out = torch.empty((B, Co, OH, OW), dtype=input.dtype, device=input.device)
     lib = _lib.load()
-    ws_bytes = lib.mcx_conv_forward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt)
-    ws = _workspace(ws_bytes, input.device)
+    ws, ws_bytes = _conv_workspace(
+        lib.mcx_conv_forward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt), dt, input.device)
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, IH, IW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
@@ -261,8 +272,8 @@ def _conv_backward(grad_output, sample_map, interp_weights, input, weight, bias,
     grad_weight = torch.empty_like(weight) if needs[1] else None
     grad_bias = torch.empty((Co,), dtype=input.dtype, device=input.device) if needs[2] else None
     lib = _lib.load()
-    ws_bytes = lib.mcx_conv_backward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt)
-    ws = _workspace(ws_bytes, input.device)
+    ws, ws_bytes = _conv_workspace(
+        lib.mcx_conv_backward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt), dt, input.device)
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, IH, IW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
@@ -331,8 +342,8 @@ def _tconv_forward(input, sample_map, interp_weights, weight, bias, output_heigh
         raise RuntimeError("shape mismatch in mapped_transposed_conv_forward")
     out = torch.empty((B, Co, OH, OW), dtype=input.dtype, device=input.device)
     lib = _lib.load()
-    ws_bytes = lib.mcx_tconv_forward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt)
-    ws = _workspace(ws_bytes, input.device)
+    ws, ws_bytes = _conv_workspace(
+        lib.mcx_tconv_forward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt), dt, input.device)
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, OH, OW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
@@ -366,8 +377,8 @@ def _tconv_backward(grad_output, sample_map, interp_weights, input, weight, bias
     if not any(needs):
         return [None, None, None]
     lib = _lib.load()
-    ws_bytes = lib.mcx_tconv_backward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt)
-    ws = _workspace(ws_bytes, input.device)
+    ws, ws_bytes = _conv_workspace(
+        lib.mcx_tconv_backward_workspace(B, Ci, Co, IH, IW, OH, OW, K, P, dt), dt, input.device)
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, OH, OW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)

@@ -12,6 +12,7 @@ from helpers import rel_err
 from oracle import ops as O
 
 from mappedconvolutions_amd import _C, _lib
+from mappedconvolutions_amd.util import synthetic
 
 pytestmark = pytest.mark.gpu
 
@@ -185,6 +186,38 @@ def test_fp64_without_a_workspace(given, device):
     for name, need, got, want in _every_call(lib, workspace):
         assert need > 0, name
         assert rel_err(got, want) < 1e-12, name
+
+
+def test_fp64_where_no_memory_is_left_for_a_workspace(device):
+    """The layers' ops go through without the records' copy of an operand: what the process may
+    hold is limited to the tensors, the results and 16 MB."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.float64)
+    B, ci, co, k, h, w_ = 1, 64, 2, 9, 256, 512
+    torch.cuda.empty_cache()                              # (no blocks of earlier tests to reuse)
+    smap = synthetic.latitude_map(h, w_, 1, dtype=torch.float64).cuda()
+    x, w, b, gy = rnd(B, ci, h, w_), rnd(co, ci, k), rnd(co), rnd(B, co, h, w_)
+    xt, wt, bt = gy, w, rnd(ci)                           # transposed: co channels in, ci out
+    calls = [(lambda: [_C.mapped_conv_forward(x, smap, w, b, k, 1)], gy),
+             (lambda: _C.mapped_conv_backward(gy, smap, x, w, b, k, 1), x),
+             (lambda: [_C.mapped_transposed_conv_forward(xt, smap, wt, bt, h, w_, k, 1)], x),
+             (lambda: _C.mapped_transposed_conv_backward(x, smap, xt, wt, bt, k, 1), xt)]
+    total = torch.cuda.get_device_properties(0).total_memory
+    for call, like in calls:
+        torch.cuda.empty_cache()
+        want = call()
+        torch.cuda.empty_cache()
+        room = torch.cuda.memory_reserved() + like.numel() * 8 + (16 << 20)
+        ooms = torch.cuda.memory_stats()["num_ooms"]
+        torch.cuda.set_per_process_memory_fraction(room / total)
+        try:
+            got = call()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.cuda.memory_stats()["num_ooms"] > ooms
+        for a, c in zip(got, want):
+            assert rel_err(a, c) < 1e-12
+        del got, want, a, c
 
 
 @pytest.mark.parametrize("n", [1 << 13, (1 << 13) + 1, 100003])

@@ -124,6 +124,16 @@ def test_no_cpu_fallback():
         _C.resample_from_map(torch.zeros(1, 1, 2, 4)[..., ::2], torch.zeros(2, 2, 2), 1)
 
 
+def test_only_float64_does_without_a_workspace(monkeypatch):
+    def full(nbytes, device):
+        raise torch.OutOfMemoryError("no memory left")
+    monkeypatch.setattr(_C, "_workspace", full)
+    assert _C._conv_workspace(1 << 20, _lib.MCX_F64, "cpu") == (None, 0)
+    for dt in (_lib.MCX_F32, _lib.MCX_BF16):
+        with pytest.raises(torch.OutOfMemoryError):
+            _C._conv_workspace(1 << 20, dt, "cpu")
+
+
 def test_shipped_package_never_touches_the_oracle():
     pkg = os.path.join(ROOT, "mappedconvolutions_amd")
     for dirpath, _, files in os.walk(pkg):
