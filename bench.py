@@ -26,7 +26,10 @@ from mappedconvolutions_amd import _C  # noqa: E402
 from mappedconvolutions_amd.util import synthetic  # noqa: E402
 
 B, CI, CO, H, W, K = 8, 64, 64, 256, 512, 9
+# Dense peaks of the units the timed calls' dominant kernels multiply on: the fp32 matrix
+# instructions, or (the gather-products) six bf16 matrix instructions per fp32 product.
 PEAK_FP32_MFMA_TFLOPS = 157.3
+PEAK_SPLIT_TFLOPS = 2500.0 / 6
 GEMM_FLOP = 2.0 * B * H * W * CO * CI * K  # one of the three products
 
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "conv_fwd_bwd_headline_hbm_traffic.txt")
@@ -37,22 +40,17 @@ def recorded_traffic():
     committed counter summary (FETCH_SIZE / WRITE_SIZE passes of this script, scaled by copy
     dispatches of known size; bench_traffic_summary.py writes it).  Counters
     cannot be read from inside the process, so these are recorded figures: they are dropped when
-    the kernel source has changed since the counter run."""
-    import hashlib
+    a kernel source has changed since the counter run."""
     import re
-    table, fresh = {}, False
+    from bench_traffic_summary import source_lines
+    table = {}
     try:
         text = open(TRAFFIC_PROFILE).read()
     except OSError:
         return {}, False
-    for line in text.splitlines():
-        m = re.match(r"@source sha256=(\w+) file=(\S+)", line)
-        if m:
-            try:
-                with open(os.path.join(ROOT, m.group(2)), "rb") as f:
-                    fresh = hashlib.sha256(f.read()).hexdigest() == m.group(1)
-            except OSError:
-                fresh = False
+    lines = text.splitlines()
+    fresh = set(source_lines()) == {line for line in lines if line.startswith("@source ")}
+    for line in lines:
         m = re.match(r'@traffic label=(\w+) kernel="([^"]+)" read_bytes=(\d+) written_bytes=(\d+)',
                      line)
         if m:
@@ -158,6 +156,7 @@ def main():
     kernel_ms = {k: sum(v) / len(v) for k, v in per_kernel.items()}
     dominant = max(kernel_ms, key=kernel_ms.get)
     achieved = GEMM_FLOP / (kernel_ms[dominant] * 1e-3) / 1e12
+    peak = PEAK_FP32_MFMA_TFLOPS if dominant == "conv_backward_weight" else PEAK_SPLIT_TFLOPS
 
     ms = elapsed / args.steps * 1e3
     # (the recorded counter runs cover the bilinear headline workload without a plan cache)
@@ -174,8 +173,8 @@ def main():
                                + args.interp, "interpolation": args.interp,
                    "map_plan_cache": bool(args.map_plan_cache)},
         "roofline": {"bound": "mfma", "kernel": recorded.get(dominant, (dominant, None))[0],
-                     "achieved": round(achieved, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
-                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4),
+                     "achieved": round(achieved, 3), "peak": round(peak, 1),
+                     "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
                      "traffic": recorded[dominant][1] if fresh and dominant in recorded else None,
                      "traffic_unit": "bytes per launch",
                      "traffic_source": "profiles/conv_fwd_bwd_headline_hbm_traffic.txt"

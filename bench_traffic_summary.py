@@ -9,7 +9,7 @@ FETCH_DIR / WRITE_DIR: output folders of
 and the same with WRITE_SIZE.  The calibration dispatches (plain elementwise copies of the
 input tensor, bytes known) give the bytes one count stands for; every other kernel's average
 count per dispatch is scaled by it.  Lines that start with '@' are the machine-readable part:
-the hash of the kernel source the run was made with, and per timed C-ABI call the kernel that
+the hashes of the kernel sources the run was made with, and per timed C-ABI call the kernel that
 did its work with the bytes it read and wrote per launch.
 """
 import collections
@@ -21,13 +21,19 @@ import re
 import sys
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
-KERNEL_SOURCE = "mappedconvolutions_amd/csrc/mcx_conv_mfma.hip"
+# The headline's kernels and what they include
+KERNEL_SOURCES = ["mappedconvolutions_amd/csrc/" + name for name in
+                  ("mcx_conv_mfma.hip", "mcx_conv_split.h", "mcx_taps.h", "mcx_device.h")]
 COPY_BYTES = 8 * 64 * 256 * 512 * 4  # one calibration dispatch reads and writes the input once
 
 
-def source_hash():
-    with open(os.path.join(ROOT, KERNEL_SOURCE), "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()
+def source_lines():
+    """A line '@source sha256=... file=...' per kernel source."""
+    lines = []
+    for name in KERNEL_SOURCES:
+        with open(os.path.join(ROOT, name), "rb") as f:
+            lines.append("@source sha256=%s file=%s" % (hashlib.sha256(f.read()).hexdigest(), name))
+    return lines
 
 
 def short_name(name):
@@ -94,7 +100,7 @@ def main(argv):
     for k, n, f, w, rb, wb in rows:
         print("%-58s %8d %12.0f %12.0f %10.1f %10.1f" % (k[:58], n, f, w, rb / 1e6, wb / 1e6))
     print()
-    print("@source sha256=%s file=%s" % (source_hash(), KERNEL_SOURCE))
+    print("\n".join(source_lines()))
     best = {}
     for k, n, f, w, rb, wb in rows:
         for lab in label_of(k):

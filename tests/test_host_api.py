@@ -134,6 +134,28 @@ def test_only_float64_does_without_a_workspace(monkeypatch):
             _C._conv_workspace(1 << 20, dt, "cpu")
 
 
+def test_recorded_traffic_goes_stale_with_any_kernel_source(tmp_path, monkeypatch):
+    import bench
+    import bench_traffic_summary as summary
+    lines = summary.source_lines()
+    assert any("mcx_conv_split.h" in line for line in lines)
+    traffic = '@traffic label=conv_forward kernel="k" read_bytes=3 written_bytes=4'
+    profile = tmp_path / "traffic.txt"
+    monkeypatch.setattr(bench, "TRAFFIC_PROFILE", str(profile))
+
+    def fresh(sources):
+        profile.write_text("\n".join(sources + [traffic]))
+        table, ok = bench.recorded_traffic()
+        assert table == {"conv_forward": ("k", 7)}
+        return ok
+
+    assert fresh(lines)
+    for i, line in enumerate(lines):
+        changed = line.replace("sha256=", "sha256=0")
+        assert not fresh(lines[:i] + lines[i + 1:])
+        assert not fresh(lines[:i] + [changed] + lines[i + 1:])
+
+
 def test_shipped_package_never_touches_the_oracle():
     pkg = os.path.join(ROOT, "mappedconvolutions_amd")
     for dirpath, _, files in os.walk(pkg):
