@@ -140,15 +140,20 @@ int mcx_conv_forward(const void *x, const void *map, const void *iw, const void 
 
 /* mcx_conv_forward for callers that cannot allocate device memory or hand over a workspace
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  It
- * has no counterpart in the reference.  Same arguments and results as mcx_conv_forward, but
- * the scratch (repacked weights, the map's pair mask, staging copies) lives in an array of
+ * has no counterpart in the reference.  Same arguments as mcx_conv_forward, but the scratch
+ * (repacked weights, the map's pair mask, staging copies) lives in an array of
  * MCX_STATIC_SCRATCH_BYTES inside the library's code object, one copy per GPU, held until the
- * process ends; the call makes no hipMalloc / hipFree.  Problems whose
- * mcx_conv_forward_workspace() exceeds that size (bf16 storage and single-row sources need a
- * staging copy as large as the input) return MCX_E_STATIC_LIMIT.  All calls on one GPU share
- * the array: calls that overlap on one GPU (different streams or threads) race; calls on one
- * stream are ordered and safe.  The first call on a device looks up the array's address
- * (hipGetSymbolAddress), so make it outside any graph capture. */
+ * process ends; the call makes no hipMalloc / hipFree.
+ * Where mcx_conv_forward_workspace() fits the array, the results are those of mcx_conv_forward
+ * bit for bit.  Where it does not, fp32 and fp64 run on the kernels that need less (fp32: the
+ * fp32 matrix instructions, whose scratch is the packed weights and, for single-row sources, a
+ * copy of the input; fp64: the scalar kernels, without scratch), whose last bits differ.  What
+ * even these cannot hold in the array, and bf16 storage whose copy of the input does not fit,
+ * returns MCX_E_STATIC_LIMIT.
+ * All calls on one GPU, of every data type, share the array: calls that overlap on one GPU
+ * (different streams or threads) race; calls on one stream are ordered and safe.  The first
+ * call on a device looks up the array's address (hipGetSymbolAddress), so make it outside any
+ * graph capture. */
 #define MCX_STATIC_SCRATCH_BYTES ((size_t)8 << 20)
 int mcx_conv_forward_static(const void *x, const void *map, const void *iw, const void *w,
                             const void *bias, void *y, int64_t B, int64_t Ci, int64_t Co,
@@ -157,7 +162,15 @@ int mcx_conv_forward_static(const void *x, const void *map, const void *iw, cons
 
 /* Bytes of device scratch the matching call needs for these sizes (may be 0).
  * The scratch holds repacked weights, partial sums, staging copies of operands and
- * resolved taps; its contents need not survive the call.  It must be 256-byte aligned. */
+ * resolved taps; its contents need not survive the call.  It must be 256-byte aligned.
+ * fp64 calls accept NULL, or less than this size, and then run scalar kernels without scratch.
+ *
+ * Arithmetic of fp32 forward and input gradient (and their transposed counterparts), given the
+ * whole size: the operands split exactly into three bf16 parts each, six of the nine partial
+ * products summed in fp32.  What is left out is at most 2^-24 of a product; operands of every
+ * magnitude keep their 24 bits, and a pixel tile with a result that is not finite is computed
+ * again on the fp32 instructions.  Against 64 bits the error is no larger than theirs; up to
+ * five gathered channels, where it would be, run on them. */
 size_t mcx_conv_forward_workspace(int64_t B, int64_t Ci, int64_t Co, int64_t IH, int64_t IW,
                                   int64_t OH, int64_t OW, int64_t K, int64_t P, int dtype);
 size_t mcx_conv_backward_workspace(int64_t B, int64_t Ci, int64_t Co, int64_t IH, int64_t IW,

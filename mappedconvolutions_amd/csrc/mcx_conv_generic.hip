@@ -1,6 +1,6 @@
 // Shape-agnostic scalar kernels for the three products of a mapped convolution
 // (gather-product, product-scatter, weight gradient) and the bias gradient.  They
-// carry the fp64 instantiation (used by known-answer and gradcheck tests) and any
+// carry fp64 where the records of mcx_conv_records.hip do not pay or have no scratch, and any
 // fp32 shape the matrix-core kernels do not cover.  Each is written in terms of a
 // "plain" operand read at map locations' own index n and a "gathered"/"scattered"
 // operand reached through the map, so convolution and transposed convolution share

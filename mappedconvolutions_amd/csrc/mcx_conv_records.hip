@@ -10,6 +10,8 @@
 // channels, nine taps of a shuffled map (scalar kernels -> these): forward
 // 210 -> 36 us (7 of them the copy), input gradient 1585 -> 375 us (the atomics: 36 M of them
 // as 3.6 M records; 2 x 8 lanes per record of 10 channels 385), weight gradient 579 -> 70 us.
+// Where a map is coherent the scalar kernels can be the faster ones: see "where the map decides"
+// and "where records pay" below.
 #include <algorithm>
 
 #include "mcx_conv.h"

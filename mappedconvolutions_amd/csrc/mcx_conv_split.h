@@ -27,11 +27,12 @@
 //     through LDS; only the weights do, pre-split by the packing launch.
 // Bound: the matrix instructions (384 clocks a unit) and the vector instructions around them
 // (some 60 x 4), which all but take turns, and what three waves per SIMD leave exposed of the
-// loads' latency.  Measured, fp32 instructions -> these: 8 x 64 channels of 256 x 512 -> 64, nine
-// taps: forward 798 -> 597 us, input gradient 768 -> 597 us; 4 x 64 -> 32 channels onto 256 x 512
-// (transposed) 379 -> 269 us; mesh of 40 962 vertices, 4 x 64 -> 128 channels, four points a tap:
-// forward 411 -> 292 us, input gradient (both levels in one pass) 952 -> 509 us.  Distance from
-// the 64-bit result, in 2-norm: 4.3e-7 -> 3.6e-7 (576 terms).
+// loads' latency.  Measured in one run each, fp32 instructions -> these: 8 x 64 channels of
+// 256 x 512 -> 64, nine taps: forward 798 -> 597 us, input gradient 768 -> 597 us (547 to 600 for
+// the product over the cards seen); 4 x 64 -> 32 channels onto 256 x 512 (transposed) 379 -> 269 us;
+// mesh of 40 962 vertices, 4 x 64 -> 128 channels, four points a tap: forward 411 -> 292 us, input
+// gradient (both levels in one pass) 952 -> 509 us.  Distance from the 64-bit result, in 2-norm:
+// 4.3e-7 -> 3.6e-7 (576 terms).
 // Included by mcx_conv_mfma.hip, inside its anonymous namespace.
 
 constexpr float kSplitUnscale = 1.f / (kSplitScale * kSplitScale);

@@ -2,7 +2,7 @@
 inside the library (one per GPU) instead of a caller's workspace.  Called through the C ABI with
 caller-owned inputs and outputs and compared with mcx_conv_forward on the same inputs: the same
 kernels on the same data, so the same bits.  Two calls in a row, the second on a smaller problem
-(whatever the first left in the array must not matter), then fp64 (no scratch at all), a weighted
+(whatever the first left in the array must not matter), then fp64 (records in the array), a weighted
 nearest map, and a problem whose scratch exceeds the array."""
 import pytest
 import torch
