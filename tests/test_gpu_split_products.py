@@ -242,9 +242,10 @@ def _forward_both(x, smap, w, b, k, interp):
 @pytest.mark.parametrize("c", [1, 2, 3, 5, 6, 8, 9, 10, 11, 16, 17, 24, 33, 64, 128])
 @pytest.mark.parametrize("interp,shift", [(0, 0.0), (1, 0.0), (1, 0.3)])
 def test_accuracy_is_not_below_fp32(c, interp, shift, device):
-    """Distance from the 64-bit result in 2-norm: the forward's is no larger than that of the fp32
-    matrix instructions on the same operands, which serve it themselves where the split products'
-    would be (few channels).  (2 % are allowed for: at nine and ten channels the two are equal.)"""
+    """Distance from the 64-bit result in 2-norm, dense operands: the forward's is no larger than
+    that of the fp32 matrix instructions on the same operands, which serve it themselves where the
+    split products' would be (few channels).  (2 % are allowed for: at nine and ten channels the two
+    are equal.)"""
     g = torch.Generator().manual_seed(9)
     h, w_, k, co = 32, 64, 9, 64
     smap = synthetic.latitude_map(h, w_, 1) + shift
