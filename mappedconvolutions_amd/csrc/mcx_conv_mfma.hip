@@ -11,6 +11,8 @@
 // with v_mfma_f32_32x32x2_f32 (each wave: 32 pixels x 64 channels).  Loads for chunk
 // t+1 are issued before the MFMAs of chunk t.  No column buffer ever reaches HBM.
 #include "mcx_conv.h"
+#include "mcx_conv_runs.h"
+#include "mcx_mfma_common.h"
 #include "mcx_taps.h"
 
 namespace mcx {
@@ -29,22 +31,12 @@ inline void profile_end(hipStream_t s) {
 }
 
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
 constexpr int kThreads = 256;
 constexpr int kTilePx = 128;  // output pixels per workgroup
 constexpr int kGC = 16;       // source channels per reduction chunk
 constexpr int kOT = 64;       // output channels per workgroup
 constexpr int kWtLd = kOT + 4;
 constexpr int kTapCache = 12;  // cached (offset, weight) pairs per tile pixel (12 KB of LDS)
-
-// Workgroups are dealt round-robin to the 8 XCDs; give every XCD one contiguous
-// run of tiles so that neighbouring tiles (which share source rows) share an L2.
-__device__ inline int xcd_contiguous_tile(int wg, int total) {
-  const int q = total >> 3, r = total & 7;
-  const int xcd = wg & 7, slot = wg >> 3;
-  return xcd * q + min(xcd, r) + slot;
-}
 
 // Whether a pair beyond the first two of a tap is in use anywhere in the map, from the pair
 // mask: one word (at least 4 then), or `words` words of which any may say so (one per block
@@ -82,8 +74,6 @@ struct SplitJob {
   int planar;      // the source they meet is planar (else channel-last)
 };
 
-// Factor of the weights and of the samples before they are split.
-constexpr float kSplitScale = 16777216.f;  // 2^24
 __host__ __device__ inline int split_channel(int c, int kg, int j, int G, int planar);
 
 // Bits of the (point, corner) pairs with a nonzero weight anywhere among the entries this
@@ -125,16 +115,6 @@ __device__ inline unsigned block_pair_mask(const float *__restrict__ map,
 //   (channels kg*8 .. kg*8+7, kg = lane / 32) of its row or column in 16 bytes.  Weights are
 //   therefore packed as Wb[k][chunk][kg][o][8] bf16: the 64 x 16 slice of a (tap, chunk) is two
 //   runs of 64 x 16 bytes that are copied linearly into LDS.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-
-// acc + w.lo * word.lo + w.hi * word.hi (v_dot2_f32_bf16: products exact, fp32 sum)
-__device__ inline float dot_bf16(unsigned word, unsigned w, float acc) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, word),
-                                         __builtin_bit_cast(bf16x2, w), acc, false);
-}
-
 // w.lo * word.lo + w.hi * word.hi, the head of such a sum.  (Written out because the compiler
 // renders dot_bf16(word, w, 0) as the accumulating two-operand form behind a move of zero:
 // one instruction in three of an interpolation.)
@@ -1081,7 +1061,6 @@ __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel
 // LDS as S[16][128] (same gather as the forward kernel) and every wave issues 32
 // v_mfma_f32_16x16x4_f32 (bf16: 8 v_mfma_f32_16x16x32_bf16).  Each workgroup writes its partial gW to scratch; a
 // second kernel sums the partials in a fixed order (deterministic result).
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Plain channels and 16-channel blocks of gathered channels per workgroup.  With bf16 storage
 // the gather bounds the kernel, not the MFMAs: a workgroup then takes 128 plain channels (two
@@ -1131,9 +1110,10 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     int G, int GH, int GW, int MH, int MW, int K, int weighted, int wrap, int tiles_x,
     int tiles_per_img, int tw_shift, int total_tiles, int ranges, int cgroups,
     float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask, int run_if_leading,
-    const uint4 *__restrict__ tap_table) {
+    const int *__restrict__ runs_state) {
   constexpr int NE = NP * NCORN;  // (offset, weight) pairs per pixel and tap
   static_assert(NA >= 1 && NA <= NE, "NA counts leading pairs");
+  if (runs_state && runs_done(runs_state)) return;  // (see mcx_conv_runs.h)
   // two variants are launched, with NA == 2 (run_if_leading) and NA == NE; the map's mask of
   // pairs in use decides which of them does the work
   if (pair_mask && (((unsigned)*pair_mask < (1u << 2)) != (run_if_leading != 0))) return;
@@ -1388,47 +1368,20 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
       }
     };
 
-    // (two-pair taps of an image under fp32: resolved before the launch into a table in tile
-    // order, resolve_tap_table_kernel<2, 4, false>, and only copied into the tap cache)
-    constexpr bool kTable = sizeof(TD) == 4 && !CL && NA == 2 && NE == 4 && kCacheTaps;
     if (kCacheTaps) {
       // every wave has its A operands in registers: reuse the plain tile's LDS for the
       // resolved taps of this tile (thread (p, half) takes every other tap of pixel p)
       __syncthreads();
-      bool from_table = false;
-      if constexpr (kTable) {
-        if (tap_table) {
-          // (fetched only here: held across the plain tile's copy, the entries spill)
-          from_table = true;
-          const uint4 *te = tap_table + ((int64_t)t_in * K + k_base) * kTilePx + p;
-          constexpr int kTapsPerThread = (kWgKT + 1) / 2;
-          uint4 tap_entry[kTapsPerThread];
+      for (int k = half; k < ktaps; k += 2) {
+        unsigned o[NE];
+        float w_[NE];
+        resolve_tap(k_base + k, o, w_);
 #pragma unroll
-          for (int t = 0; t < kTapsPerThread; t++)
-            tap_entry[t] = te[(int64_t)min(half + 2 * t, ktaps - 1) * kTilePx];
-#pragma unroll
-          for (int t = 0; t < kTapsPerThread; t++) {
-            const int k = half + 2 * t;
-            if (k < ktaps) {
-              *reinterpret_cast<uint2 *>(&TapOff[k][p][0]) =
-                  make_uint2(tap_entry[t].x, tap_entry[t].y);
-              *reinterpret_cast<uint2 *>(&TapWt[k][p][0]) =
-                  make_uint2(tap_entry[t].z, tap_entry[t].w);
-            }
-          }
+        for (int i = 0; i < NA; i++) {
+          TapOff[k][p][i] = o[i];
+          TapWt[k][p][i] = w_[i];
         }
       }
-      if (!from_table)
-        for (int k = half; k < ktaps; k += 2) {
-          unsigned o[NE];
-          float w_[NE];
-          resolve_tap(k_base + k, o, w_);
-#pragma unroll
-          for (int i = 0; i < NA; i++) {
-            TapOff[k][p][i] = o[i];
-            TapWt[k][p][i] = w_[i];
-          }
-        }
       __syncthreads();
     }
 
@@ -1522,8 +1475,10 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
 template <typename TD>
 __global__ __launch_bounds__(256) void reduce_partials_kernel(
     const float *__restrict__ part, TD *__restrict__ out, int A, int A4, int G, int K,
-    const float *__restrict__ part2, TD *__restrict__ out2, int64_t n2, int ranges) {
+    const float *__restrict__ part2, TD *__restrict__ out2, int64_t n2, int ranges,
+    const int *__restrict__ runs_state, int runs_ranges) {
   __shared__ float quarter[4][64];
+  if (runs_state && runs_done(runs_state)) ranges = runs_ranges;
   int64_t n = (int64_t)K * G * A4;
   const int blocks1 = (int)((n + 63) / 64);
   int64_t e = (int64_t)blockIdx.x * 64 + threadIdx.x;
@@ -1592,16 +1547,14 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(
 //     straight into its operand registers: no LDS tile, no barrier at a tile's start.
 // Partial sums leave in the layout of weight_grad_mfma_kernel.
 
-// The taps of a bilinear map resolved once for a weight-gradient kernel, in the order its
+// The taps of a bilinear map resolved once for weight_grad_bf16_ring_kernel, in the order its
 // workgroups read them: table[tile of an image][tap][pixel of the tile][NA words of byte
-// offsets, then NA words of weights].  ESZ: bytes between neighbouring pixels of the gathered
-// operand (16 in a channel block, the element size in a plane); WBF: weights as bf16 in the low
-// half of the word (what weight_grad_bf16_ring_kernel multiplies by), else as fp32.  Every
+// offsets in a channel block, then NA words of weights as bf16 in their low halves].  Every
 // workgroup of a pixel range (channel groups x tap passes) would otherwise resolve the same
 // taps from the map again, about sixty instructions per tap, which is as much as its products
 // need.  Pixels outside the image weigh zero.  One workgroup per tile: its threads walk the
 // taps of their pixel two apart, so the tile's piece of the map stays in cache.
-template <int NA, int ESZ, bool WBF>
+template <int NA>
 __global__ __launch_bounds__(256) void resolve_tap_table_kernel(
     const float *__restrict__ map, unsigned *__restrict__ table, int GH, int GW, int MH, int MW,
     int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask) {
@@ -1617,13 +1570,12 @@ __global__ __launch_bounds__(256) void resolve_tap_table_kernel(
   // (a weight as bf16 in the low half of a word, the high half zero: the form
   // v_dot2_f32_bf16 multiplies a word of two channels by to get the even one)
   auto wbits = [](float w) {
-    return WBF ? __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{w, 0.f}, bf16x2))
-               : __builtin_bit_cast(unsigned, w);
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{w, 0.f}, bf16x2));
   };
   for (int k = threadIdx.x >> 7; k < K; k += 2) {
     const float2 xy = entry[k];
     PairTap<4> t;
-    resolve_pairs<4, ESZ>(xy.x, xy.y, GH, GW, wrap != 0, live ? 1.f : 0.f, t);
+    resolve_pairs<4, 16>(xy.x, xy.y, GH, GW, wrap != 0, live ? 1.f : 0.f, t);
     uint4 *e = out + (int64_t)k * kTilePx * (NA / 2);
     if constexpr (NA == 2) {
       e[0] = make_uint4(t.off[0], t.off[1], wbits(t.wt[0]), wbits(t.wt[1]));
@@ -2316,8 +2268,6 @@ bool mfma_supported(int64_t P) { return P >= 0 && P <= 4; }
 
 namespace {
 
-inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-
 struct ModeArgs {
   int mode, weighted, wrap, np;
 };
@@ -2804,7 +2754,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
 // Per-range partial sums of gW, per-range partial sums of the plain operand, then
 // (single-row gathered operands) their channel-last copy.
 size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64_t MW, int64_t K,
-                              int64_t GH, int64_t GW, size_t elem) {
+                              int64_t P, int64_t GH, int64_t GW, size_t elem) {
   // (the tiling and the number of ranges depend on the storage type and on the kernel)
   size_t ranges =
       (size_t)std::max(weight_grad_ranges<float>(make_tiling(B, MH, MW, 4).total, A, G, K),
@@ -2812,6 +2762,10 @@ size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64
   if (elem == 2)
     ranges = std::max(
         ranges, (size_t)ring_weight_grad_ranges(make_tiling(B, MH, MW, 2).total, A, G, K));
+  else if (runs_apply(B, A, G, GH, GW, MH, MW, K, P)) {
+    const RunPlan p = run_plan(B, A, G, GW, MH, MW, K);
+    ranges = std::max(ranges, (size_t)p.ranges);
+  }
   size_t n = align256(ranges * (size_t)(round_up(A, 4) * G * K) * sizeof(float));
   n += align256(ranges * (size_t)A * sizeof(float));
   n += 256;  // the map's pair mask
@@ -2821,8 +2775,8 @@ size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64
     n += align256((size_t)(B * GH * GW * round_up(G, kGC)) * sizeof(float));
   else if (elem == 2)
     n += align256((size_t)(B * GH * GW * round_up(G, kGC)) * elem);
-  else  // fp32 images: the table of resolved two-pair taps (resolve_tap_table_kernel)
-    n += align256((size_t)make_tiling(B, MH, MW, 4).tiles_per_img * (size_t)K * kTilePx * 16);
+  else if (runs_apply(B, A, G, GH, GW, MH, MW, K, P))  // fp32 images: the runs' tables
+    n += run_table_bytes(run_plan(B, A, G, GW, MH, MW, K));
   // bf16 images: the plain operand as MFMA fragments per pixel tile (to_plain_fragments_kernel)
   // and the table of resolved taps (resolve_tap_table_kernel, four pairs per tap at most)
   if (GH > 1 && elem == 2) {
@@ -2862,9 +2816,14 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
                     A <= 32 * 65535;
   const int ranges = ring ? ring_weight_grad_ranges(t.total, A, G, K)
                           : weight_grad_ranges<TD>(t.total, A, G, K);
+  // fp32 images: the kernel over runs of pixels, and for what it leaves the general one
+  const bool by_runs = sizeof(TD) == 4 && !cl && runs_apply(B, A, G, GH, GW, MH, MW, K, P);
+  RunPlan rp{};
+  if (by_runs) rp = run_plan(B, A, G, GW, MH, MW, K);
+  const int part_ranges = std::max(ranges, rp.ranges);
   float *sum_part = reinterpret_cast<float *>(
-      (char *)scratch + align256((size_t)ranges * (size_t)(round_up(A, 4) * G * K) * 4));
-  int *pair_mask = reinterpret_cast<int *>((char *)sum_part + align256((size_t)ranges * A * 4));
+      (char *)scratch + align256((size_t)part_ranges * (size_t)(round_up(A, 4) * G * K) * 4));
+  int *pair_mask = reinterpret_cast<int *>((char *)sum_part + align256((size_t)part_ranges * A * 4));
   int *const pair_mask_ws = pair_mask;  // (a plan may supply the mask; the copy's room follows this one)
   if (cl) {
     TD *stage = reinterpret_cast<TD *>((char *)pair_mask + 256);
@@ -2880,29 +2839,35 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   // are ever in use (bilinear maps with integral rows, two of four points weighted) and to
   // launch both variants, of which one returns at once.
   const bool two_variants = m.np * (m.mode == kInterpNearest ? 1 : 4) == 4;
-  if (two_variants) {
+  const int *runs_state = nullptr;
+  if constexpr (sizeof(TD) == 4) {
+    if (by_runs) {
+      char *tables = (char *)pair_mask_ws + 256;
+      if (int rc = resolve_runs(rp, tables, map, iw, GH, GW, MH, MW, K,
+                                m.mode == kInterpNearest ? 1 : 4, m.wrap, m.weighted, s))
+        return rc;
+      profile_begin(s);
+      if (int rc = weight_grad_by_runs(rp, tables, plain, gath, part, plain_sum ? sum_part : nullptr,
+                                       A, G, GH, GW, MH, MW, K, s))
+        return rc;
+      profile_end(s);
+      int *state = run_state(rp, tables);
+      runs_state = state;
+      pair_mask = state + 2;
+    }
+  }
+  if (two_variants && !by_runs) {
     if (plan)  // flag word 4 of a plan built for this map (see mfma_scatter_plan_build)
       pair_mask = (int *)const_cast<void *>(plan) + GH * GW * K + 4;
     else if (int rc = launch_pair_mask(map, iw, pair_mask, m, GH, GW, MH * MW * K, s))
       return rc;
-  }
-  // fp32 images under single-point bilinear taps: the taps of the two-pair form resolved once
-  // (the table follows the pair mask in the scratch)
-  const uint4 *tap_table = nullptr;
-  if (sizeof(TD) == 4 && !cl && GH > 1 && m.np == 1 && m.mode != kInterpNearest && two_variants) {
-    unsigned *table = reinterpret_cast<unsigned *>((char *)pair_mask_ws + 256);
-    hipLaunchKernelGGL((resolve_tap_table_kernel<2, 4, false>), dim3((unsigned)t.tiles_per_img),
-                       dim3(256), 0, s, map, table, (int)GH, (int)GW, (int)MH, (int)MW, (int)K,
-                       m.wrap, t.tiles_x, t.tw_shift, pair_mask);
-    MCX_HIP_CHECK_LAUNCH();
-    tap_table = reinterpret_cast<const uint4 *>(table);
   }
 #define MCX_LAUNCH_NA(NCORN, NP, CL, NA, MASK, LEAD)                                             \
   hipLaunchKernelGGL((weight_grad_mfma_kernel<TD, NCORN, NP, CL, NA>), grid, dim3(kThreads), 0,  \
                      s, plain, gath, map, iw, part, (int)A, (int)G, (int)GH, (int)GW, (int)MH,   \
                      (int)MW, (int)K, m.weighted, m.wrap, t.tiles_x, t.tiles_per_img,            \
                      t.tw_shift, (int)t.total, ranges, cgroups,                                  \
-                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, tap_table)
+                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state)
 #define MCX_LAUNCH_CL(NCORN, NP, CL)                                          \
   if constexpr (NCORN * NP == 4) {                                            \
     if (!ring) {                                                              \
@@ -2939,10 +2904,10 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       unsigned *table = reinterpret_cast<unsigned *>(
           (char *)tiles + align256((size_t)t.total * (size_t)round_up(A, 32) * kTilePx * sizeof(TD)));
       const dim3 rgrid((unsigned)t.tiles_per_img);
-      hipLaunchKernelGGL((resolve_tap_table_kernel<2, 16, true>), rgrid, dim3(256), 0, s, map, table, (int)GH,
+      hipLaunchKernelGGL((resolve_tap_table_kernel<2>), rgrid, dim3(256), 0, s, map, table, (int)GH,
                          (int)GW, (int)MH, (int)MW, (int)K, m.wrap, t.tiles_x, t.tw_shift,
                          pair_mask);
-      hipLaunchKernelGGL((resolve_tap_table_kernel<4, 16, true>), rgrid, dim3(256), 0, s, map, table, (int)GH,
+      hipLaunchKernelGGL((resolve_tap_table_kernel<4>), rgrid, dim3(256), 0, s, map, table, (int)GH,
                          (int)GW, (int)MH, (int)MW, (int)K, m.wrap, t.tiles_x, t.tw_shift,
                          pair_mask);
       MCX_HIP_CHECK_LAUNCH();
@@ -2985,7 +2950,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   const int64_t n2 = plain_sum ? A : 0;
   hipLaunchKernelGGL(reduce_partials_kernel<TD>, dim3((unsigned)((n + 63) / 64 + (n2 + 63) / 64)),
                      dim3(64, 4), 0, s, part, gw, (int)A, (int)round_up(A, 4), (int)G, (int)K,
-                     sum_part, plain_sum, n2, ranges);
+                     sum_part, plain_sum, n2, ranges, runs_state, rp.ranges);
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }

@@ -1,0 +1,36 @@
+// Interface of the weight gradient over runs of neighbouring pixels (mcx_conv_runs.hip).
+#pragma once
+
+#include "mcx_device.h"
+
+namespace mcx {
+
+// Words of `state`: [0] this path has done the work, [1] a sum is not finite, [2] pair mask for
+// weight_grad_mfma_kernel (at least 4: corners of the lower row are in use).
+constexpr int kRunStateWords = 64;
+
+__device__ inline bool runs_done(const int *state) { return state[0] != 0 && state[1] == 0; }
+
+// How the work is cut, from the sizes alone.
+struct RunPlan {
+  int st, cblocks, ablocks, passes, groups, tiles_per_img;
+  int64_t total_tiles;
+  int ranges, stat_words;
+  size_t desc_bytes, wts_bytes;
+};
+RunPlan run_plan(int64_t B, int64_t A, int64_t G, int64_t GW, int64_t MH, int64_t MW, int64_t K);
+bool runs_apply(int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t MH, int64_t MW,
+                int64_t K, int64_t P);
+// Bytes of the tables that resolve_runs fills, and their state words.
+size_t run_table_bytes(const RunPlan &p);
+int *run_state(const RunPlan &p, char *tables);
+int resolve_runs(const RunPlan &p, char *tables, const float *map, const float *iw, int64_t GH,
+                 int64_t GW, int64_t MH, int64_t MW, int64_t K, int ncorn, int wrap, int weighted,
+                 hipStream_t stream);
+// Per-range partial sums [ranges][K][G][A padded to 4]; sum_part (may be NULL): the same of the
+// plain operand, [ranges][A].
+int weight_grad_by_runs(const RunPlan &p, char *tables, const float *plain, const float *gath,
+                        float *part, float *sum_part, int64_t A, int64_t G, int64_t GH, int64_t GW,
+                        int64_t MH, int64_t MW, int64_t K, hipStream_t stream);
+
+}  // namespace mcx

@@ -41,8 +41,6 @@
 // gradient (both levels in one pass) 952 -> 509 us.
 // Included by mcx_conv_mfma.hip, inside its anonymous namespace.
 
-constexpr float kSplitUnscale = 1.f / (kSplitScale * kSplitScale);
-
 struct SplitArgs {
   const float *src, *map, *iw;
   const float2 *map2;     // second-level entries of a transposed map, or NULL (channel-last only)
@@ -55,30 +53,6 @@ struct SplitArgs {
   int G, O, Opad, Gpad, SH, SW, OH, OW, K, np, ncorn, weighted, wrap, packed;
   int tiles_x, tiles_per_img, tw_shift, run_if_zero, mask_words;
 };
-
-// x = p[0] + p[1] + p[2] for 8 values: words of two bf16 each
-__device__ inline void split8(const float *x, bf16x8 *p) {
-  unsigned h[4], m[4], l[4];
-  // {-1, 0} and {0, -1} from registers: as immediates the compiler renders both as the inline
-  // constant -1.0, which the instruction takes for one and the same word.
-  unsigned neg_lo = 0x0000bf80u, neg_hi = 0xbf800000u;
-  asm("" : "+s"(neg_lo), "+s"(neg_hi));
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    // (a remainder is the dot product of the pair word with {-1, 0} or {0, -1} plus the value)
-    h[j] = __builtin_bit_cast(unsigned,
-                              __builtin_convertvector(floatx2{x[2 * j], x[2 * j + 1]}, bf16x2));
-    const float r0 = dot_bf16(h[j], neg_lo, x[2 * j]);
-    const float r1 = dot_bf16(h[j], neg_hi, x[2 * j + 1]);
-    m[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r0, r1}, bf16x2));
-    const float q0 = dot_bf16(m[j], neg_lo, r0);
-    const float q1 = dot_bf16(m[j], neg_hi, r1);
-    l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{q0, q1}, bf16x2));
-  }
-  p[0] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-  p[1] = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
-  p[2] = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
-}
 
 // Channel (of G) that element j of half kg of chunk c stands for, or -1 (a weight of zero).
 // Planar sources read the second half of a partial last chunk `rem - 8` channels after the
