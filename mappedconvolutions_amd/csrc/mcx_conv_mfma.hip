@@ -778,37 +778,30 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 // like those of the general kernel (pair_mask / row_mask).
 constexpr int kDgPx = 256;
 
+template <int NA, int OG>
+struct DirectLds {
+  static constexpr int TG = NA <= 2 ? 13 : 4;  // taps resolved into LDS at a time
+  unsigned off[TG][kDgPx][NA];
+  unsigned w[TG][kDgPx][NA];  // bf16 weights as {w, 0}
+  uint4 wt[2][2][kOT * OG];
+};
+
 template <bool PACKED, int NA, int OG>
-__global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel(
-    const bf16_t *__restrict__ src, const float *__restrict__ map, const float *__restrict__ iw,
-    const uint16_t *__restrict__ wb, const bf16_t *__restrict__ bias, bf16_t *__restrict__ y,
-    int O, int Opad, int Gpad, int SH, int SW, int N, int OW, int K, int weighted, int wrap,
-    int tiles_per_img, const int *__restrict__ gate, int run_if_zero,
-    const float *__restrict__ addend, const int *__restrict__ pair_mask, int run_if_leading,
-    const int *__restrict__ row_mask, int mask_words) {
+__device__ inline void gather_product_bf16_direct(
+    DirectLds<NA, OG> &lds, const bf16_t *__restrict__ src, const float *__restrict__ map,
+    const float *__restrict__ iw, const uint16_t *__restrict__ wb,
+    const bf16_t *__restrict__ bias, bf16_t *__restrict__ y, int O, int Opad, int Gpad, int SH,
+    int SW, int N, int K, int weighted, int wrap, const int *__restrict__ gate,
+    const float *__restrict__ addend, int b, int n0) {
   static_assert(NA == 2 || NA == 4, "two or four entries per tap");
   constexpr int NPR = NA / 2;              // entry pairs per tap
-  constexpr int TG = NA <= 2 ? 13 : 4;     // taps resolved into LDS at a time
+  constexpr int TG = DirectLds<NA, OG>::TG;
   constexpr int kDepth = NA <= 2 ? 3 : 2;  // units whose loads are in flight
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) unsigned TapOff[TG][kDgPx][NA];
-  __shared__ __attribute__((aligned(16))) unsigned TapW[TG][kDgPx][NA];  // bf16 weights as {w, 0}
-  __shared__ __attribute__((aligned(16))) uint4 Wt[2][2][kOT * OG];
-  if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
+  auto &TapOff = lds.off;
+  auto &TapW = lds.w;
+  auto &Wt = lds.wt;
   const int tid = threadIdx.x;
-  const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
-  const int b = tile / tiles_per_img;
-  const int n0 = (tile - b * tiles_per_img) * kDgPx;
-  if (pair_mask) {
-    // the two-entry form serves every tile none of whose rows uses a later entry
-    bool leading = !later_pairs_in_use(pair_mask, mask_words);
-    if (!leading && row_mask) {
-      int any = 0;
-      for (int r = n0 / OW; r <= min(n0 + kDgPx - 1, N - 1) / OW; r++) any |= row_mask[r];
-      leading = any == 0;
-    }
-    if (leading != (run_if_leading != 0)) return;
-  }
   const int o0 = blockIdx.y * (kOT * OG);
   const int64_t plane = (int64_t)SH * SW;
   const unsigned bstride = (unsigned)plane * 16u;  // bytes of a block of 8 channels of an image
@@ -1047,6 +1040,44 @@ __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel
       }
   }
 }
+
+// Tiles none of whose rows uses an entry beyond the first two run the two-entry form, the others
+// the four-entry one, in one launch: as a launch of its own the four-entry form of a few border tiles
+// began when the last of the others had ended (4 x 32 -> 64 channels of 64 x 128: 23 + 30 us for
+// the input gradient's two launches).
+template <bool PACKED, int OG>
+__global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel(
+    const bf16_t *__restrict__ src, const float *__restrict__ map, const float *__restrict__ iw,
+    const uint16_t *__restrict__ wb, const bf16_t *__restrict__ bias, bf16_t *__restrict__ y,
+    int O, int Opad, int Gpad, int SH, int SW, int N, int OW, int K, int weighted, int wrap,
+    int tiles_per_img, const int *__restrict__ gate, int run_if_zero,
+    const float *__restrict__ addend, const int *__restrict__ pair_mask,
+    const int *__restrict__ row_mask, int mask_words) {
+  __shared__ __attribute__((aligned(16))) union {
+    DirectLds<2, OG> two;
+    DirectLds<4, OG> four;
+  } lds;
+  if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
+  const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const int b = tile / tiles_per_img;
+  const int n0 = (tile - b * tiles_per_img) * kDgPx;
+  bool leading = false;
+  if (pair_mask) {
+    leading = !later_pairs_in_use(pair_mask, mask_words);
+    if (!leading && row_mask) {
+      int any = 0;
+      for (int r = n0 / OW; r <= min(n0 + kDgPx - 1, N - 1) / OW; r++) any |= row_mask[r];
+      leading = any == 0;
+    }
+  }
+  if (leading)
+    gather_product_bf16_direct<PACKED, 2, OG>(lds.two, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
+                                              SW, N, K, weighted, wrap, gate, addend, b, n0);
+  else
+    gather_product_bf16_direct<PACKED, 4, OG>(lds.four, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
+                                              SW, N, K, weighted, wrap, gate, addend, b, n0);
+}
+
 
 #include "mcx_conv_split.h"
 
@@ -1555,10 +1586,9 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(
 // need.  Pixels outside the image weigh zero.  One workgroup per tile: its threads walk the
 // taps of their pixel two apart, so the tile's piece of the map stays in cache.
 template <int NA>
-__global__ __launch_bounds__(256) void resolve_tap_table_kernel(
-    const float *__restrict__ map, unsigned *__restrict__ table, int GH, int GW, int MH, int MW,
-    int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask) {
-  if (pair_mask && (((unsigned)*pair_mask < (1u << 2)) != (NA == 2))) return;
+__device__ inline void resolve_tap_table(const float *__restrict__ map,
+                                         unsigned *__restrict__ table, int GH, int GW, int MH,
+                                         int MW, int K, int wrap, int tiles_x, int tw_shift) {
   const int tile = blockIdx.x, p = threadIdx.x & (kTilePx - 1);
   const int tile_y = tile / tiles_x, tile_x = tile - tile_y * tiles_x;
   const int gi = tile_y * (kTilePx >> tw_shift) + (p >> tw_shift);
@@ -1585,6 +1615,14 @@ __global__ __launch_bounds__(256) void resolve_tap_table_kernel(
     }
   }
 }
+__global__ __launch_bounds__(256) void resolve_tap_table_kernel(
+    const float *__restrict__ map, unsigned *__restrict__ table, int GH, int GW, int MH, int MW,
+    int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask) {
+  if ((unsigned)*pair_mask < (1u << 2))
+    resolve_tap_table<2>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
+  else
+    resolve_tap_table<4>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
+}
 
 constexpr int kRgKT = 5;      // taps per pass
 constexpr int kRgG = 32;      // gathered channels per workgroup
@@ -1604,21 +1642,26 @@ inline int ring_weight_grad_ranges(int64_t total_tiles, int64_t A, int64_t G, in
 }
 
 template <int NA>
-__global__ __launch_bounds__(kThreads, 2) void weight_grad_bf16_ring_kernel(
-    const bf16_t *__restrict__ plain, const bf16_t *__restrict__ gath,
+struct RingLds {
+  static constexpr int kTapBufs = NA == 2 ? 2 : 1;
+  uint16_t samples[2][kRgG][kRgLd];
+  unsigned off[kTapBufs][kRgKT][kTilePx][NA];
+  float wt[kTapBufs][kRgKT][kTilePx][NA];
+};
+
+template <int NA>
+__device__ inline void weight_grad_bf16_ring(
+    RingLds<NA> &lds, const bf16_t *__restrict__ plain, const bf16_t *__restrict__ gath,
     const unsigned *__restrict__ table, float *__restrict__ part, int A, int G, int Gpad, int GH,
     int GW, int K, int tiles_per_img, int total_tiles, int ranges, int cgroups, int passes,
-    float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask) {
-  // NA == 2 runs while no tap of the map uses a pair beyond its first two, NA == 4 otherwise
-  if (pair_mask && (((unsigned)*pair_mask < (1u << 2)) != (NA == 2))) return;
+    float *__restrict__ plain_sum_part) {
   static_assert(NA == 2 || NA == 4, "two or four pairs per tap");
   constexpr bool kCross = NA == 2;               // gathers in flight across tile boundaries
   constexpr int kDepth = kCross ? kRgDepth : 1;  // units in flight
-  constexpr int kTapBufs = kCross ? 2 : 1;
   constexpr int MB = kRgA / 64, NB = kRgG / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t SB[2][kRgG][kRgLd];
-  __shared__ __attribute__((aligned(16))) unsigned TapOff[kTapBufs][kRgKT][kTilePx][NA];
-  __shared__ __attribute__((aligned(16))) float TapWt[kTapBufs][kRgKT][kTilePx][NA];
+  auto &SB = lds.samples;
+  auto &TapOff = lds.off;
+  auto &TapWt = lds.wt;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1905,6 +1948,25 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_bf16_ring_kernel(
     }
   }
 }
+
+// (one launch for both forms: the map's pair mask decides)
+__global__ __launch_bounds__(kThreads, 2) void weight_grad_bf16_ring_kernel(
+    const bf16_t *__restrict__ plain, const bf16_t *__restrict__ gath,
+    const unsigned *__restrict__ table, float *__restrict__ part, int A, int G, int Gpad, int GH,
+    int GW, int K, int tiles_per_img, int total_tiles, int ranges, int cgroups, int passes,
+    float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask) {
+  __shared__ __attribute__((aligned(16))) union {
+    RingLds<2> two;
+    RingLds<4> four;
+  } lds;
+  if ((unsigned)*pair_mask < (1u << 2))
+    weight_grad_bf16_ring<2>(lds.two, plain, gath, table, part, A, G, Gpad, GH, GW, K,
+                             tiles_per_img, total_tiles, ranges, cgroups, passes, plain_sum_part);
+  else
+    weight_grad_bf16_ring<4>(lds.four, plain, gath, table, part, A, G, Gpad, GH, GW, K,
+                             tiles_per_img, total_tiles, ranges, cgroups, passes, plain_sum_part);
+}
+
 
 // ---------------------------------------------------------------------------------
 // product_scatter: dst[b,d] += splat(sum_s W[s,d,k] * src[b,s,n], map[n,k])
@@ -2448,37 +2510,29 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
       const int64_t tiles_per_img = (OH * OW + kDgPx - 1) / kDgPx;
       if (tiles_per_img * B > 0x7fffffffLL) return MCX_E_SHAPE;
       const dim3 dgrid((unsigned)(tiles_per_img * B), (unsigned)(Opad / (wide ? 2 * kOT : kOT)));
-#define MCX_LAUNCH_DIRECT(FORM, NA, OG, MASK, LEAD)                                              \
-  hipLaunchKernelGGL((gather_product_bf16_direct_kernel<FORM, NA, OG>), dgrid, dim3(kThreads),   \
-                     0, s, reinterpret_cast<const bf16_t *>(src), map, iw,                       \
+#define MCX_LAUNCH_DIRECT(FORM, OG)                                                              \
+  hipLaunchKernelGGL((gather_product_bf16_direct_kernel<FORM, OG>), dgrid, dim3(kThreads), 0, s, \
+                     reinterpret_cast<const bf16_t *>(src), map, iw,                             \
                      reinterpret_cast<const uint16_t *>(wp),                                     \
                      reinterpret_cast<const bf16_t *>(bias), reinterpret_cast<bf16_t *>(y),      \
                      (int)O, Opad, Gpad, (int)SH, (int)SW, (int)(OH * OW), (int)OW, (int)K,      \
-                     m0.weighted, m0.wrap, (int)tiles_per_img, gate, run_if_zero, addend, MASK,  \
-                     LEAD, row_mask, mask_words)
-#define MCX_LAUNCH_DIRECT_NA(FORM, OG)                                  \
-  if (pair_mask) {                                                      \
-    MCX_LAUNCH_DIRECT(FORM, 2, OG, pair_mask, 1);                       \
-    MCX_LAUNCH_DIRECT(FORM, 4, OG, pair_mask, 0);                       \
-  } else {                                                              \
-    MCX_LAUNCH_DIRECT(FORM, 4, OG, (const int *)nullptr, 0);            \
-  }
+                     m0.weighted, m0.wrap, (int)tiles_per_img, gate, run_if_zero, addend,        \
+                     pair_mask, row_mask, mask_words)
       profile_begin(s);
       if (from_map) {
         if (wide) {
-          MCX_LAUNCH_DIRECT_NA(false, 2)
+          MCX_LAUNCH_DIRECT(false, 2);
         } else {
-          MCX_LAUNCH_DIRECT_NA(false, 1)
+          MCX_LAUNCH_DIRECT(false, 1);
         }
       } else {
         if (wide) {
-          MCX_LAUNCH_DIRECT_NA(true, 2)
+          MCX_LAUNCH_DIRECT(true, 2);
         } else {
-          MCX_LAUNCH_DIRECT_NA(true, 1)
+          MCX_LAUNCH_DIRECT(true, 1);
         }
       }
       profile_end(s);
-#undef MCX_LAUNCH_DIRECT_NA
 #undef MCX_LAUNCH_DIRECT
       MCX_HIP_CHECK_LAUNCH();
       return 0;
@@ -2887,6 +2941,8 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   } else {                                 \
     MCX_LAUNCH_CL(NCORN, NP, false);       \
   }
+  bf16_t *ring_tiles = nullptr;
+  unsigned *ring_table = nullptr;
   if constexpr (sizeof(TD) == 2) {
     if (ring) {
       TD *stage = reinterpret_cast<TD *>((char *)pair_mask_ws + 256);
@@ -2900,16 +2956,13 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
                          dim3(256), 0, s, reinterpret_cast<const bf16_t *>(plain), tiles, (int)A,
                          (int)MH, (int)MW, t.tiles_x, t.tiles_per_img, t.tw_shift);
       MCX_HIP_CHECK_LAUNCH();
+      ring_tiles = tiles;
       // the taps, resolved once for all workgroups (two or four pairs: the mask decides)
-      unsigned *table = reinterpret_cast<unsigned *>(
+      ring_table = reinterpret_cast<unsigned *>(
           (char *)tiles + align256((size_t)t.total * (size_t)round_up(A, 32) * kTilePx * sizeof(TD)));
-      const dim3 rgrid((unsigned)t.tiles_per_img);
-      hipLaunchKernelGGL((resolve_tap_table_kernel<2>), rgrid, dim3(256), 0, s, map, table, (int)GH,
-                         (int)GW, (int)MH, (int)MW, (int)K, m.wrap, t.tiles_x, t.tw_shift,
-                         pair_mask);
-      hipLaunchKernelGGL((resolve_tap_table_kernel<4>), rgrid, dim3(256), 0, s, map, table, (int)GH,
-                         (int)GW, (int)MH, (int)MW, (int)K, m.wrap, t.tiles_x, t.tw_shift,
-                         pair_mask);
+      hipLaunchKernelGGL(resolve_tap_table_kernel, dim3((unsigned)t.tiles_per_img), dim3(256), 0, s,
+                         map, ring_table, (int)GH, (int)GW, (int)MH, (int)MW, (int)K, m.wrap,
+                         t.tiles_x, t.tw_shift, pair_mask);
       MCX_HIP_CHECK_LAUNCH();
     }
   }
@@ -2917,26 +2970,13 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   if constexpr (sizeof(TD) == 2) {
     if (ring) {
       const int rg_groups = (int)((G + kRgG - 1) / kRgG), rg_passes = (int)((K + kRgKT - 1) / kRgKT);
-#define MCX_LAUNCH_RING(NA)                                                                       \
-  hipLaunchKernelGGL(weight_grad_bf16_ring_kernel<NA>,                                            \
-                     dim3((unsigned)(ranges * rg_groups * rg_passes),                             \
-                          (unsigned)((A + kRgA - 1) / kRgA)),                                     \
-                     dim3(kThreads), 0, s,                                                        \
-                     reinterpret_cast<const TD *>(                                                \
-                         (char *)pair_mask_ws + 256 +                                             \
-                         align256((size_t)(B * GH * GW * Gpad) * sizeof(TD))),                    \
-                     reinterpret_cast<const TD *>((char *)pair_mask_ws + 256),                    \
-                     reinterpret_cast<const unsigned *>(                                          \
-                         (char *)pair_mask_ws + 256 +                                             \
-                         align256((size_t)(B * GH * GW * Gpad) * sizeof(TD)) +                    \
-                         align256((size_t)t.total * (size_t)round_up(A, 32) * kTilePx *           \
-                                  sizeof(TD))),                                                   \
-                     part, (int)A, (int)G, (int)Gpad, (int)GH, (int)GW, (int)K, t.tiles_per_img,  \
-                     (int)t.total, ranges, rg_groups, rg_passes,                                  \
-                     plain_sum ? sum_part : (float *)nullptr, pair_mask)
-      MCX_LAUNCH_RING(2);
-      MCX_LAUNCH_RING(4);
-#undef MCX_LAUNCH_RING
+      hipLaunchKernelGGL(
+          weight_grad_bf16_ring_kernel,
+          dim3((unsigned)(ranges * rg_groups * rg_passes), (unsigned)((A + kRgA - 1) / kRgA)),
+          dim3(kThreads), 0, s, reinterpret_cast<const TD *>(ring_tiles),
+          reinterpret_cast<const TD *>((char *)pair_mask_ws + 256), ring_table, part, (int)A, (int)G,
+          (int)Gpad, (int)GH, (int)GW, (int)K, t.tiles_per_img, (int)t.total, ranges, rg_groups,
+          rg_passes, plain_sum ? sum_part : (float *)nullptr, pair_mask);
       MCX_HIP_CHECK_LAUNCH();
     }
   }
