@@ -454,6 +454,81 @@ __global__ __launch_bounds__(kThreads) void reduce_records_kernel(const double *
   }
 }
 
+// ---- scattering before the product ----
+// With few source channels (S) and more destination ones (D) it is S values per corner that are
+// added, into a plane per (tap, source channel), and the product that follows reads every plane
+// once:  T[k][s][p] = sum over the corners on p of weight * src[s],  dst[d][p] = sum W[s][d][k] T[k][s][p].
+// The two corners of a row are neighbouring lanes and neighbouring doubles: one request of 64 bytes
+// for both (a record of ten channels takes one and a half for either), and under a coherent map a
+// wave's 32 pixels are as many neighbours.
+// A double of a plane that nothing was added to keeps its first value, -0: its product is left
+// out, so that an infinite W does not make NaN where no corner lies.  (What -0 adds is nothing.)
+// Bound: the requests of the additions, and clearing the planes.  1 -> 10 channels, nine taps, one
+// image of 200x500, shuffled: 375 -> 120 us for the whole
+// product (16 channels 388 -> 123); see planes_scatter_applies.
+constexpr unsigned long long kUntouched = 0x8000000000000000ull;
+
+__global__ __launch_bounds__(kThreads) void begin_planes_kernel(double2 *__restrict__ t,
+                                                                int64_t count) {
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < count; i += stride)
+    t[i] = make_double2(-0.0, -0.0);
+}
+
+// NC == 4: two lanes a map location, one for either column of corners.
+template <int NC>
+__global__ __launch_bounds__(kThreads) void scatter_planes_kernel(
+    const double *__restrict__ src, const double *__restrict__ map, const double *__restrict__ iw,
+    double *__restrict__ planes, int S, int DH, int DW, int N, int K, int pm, int wrap) {
+  constexpr int kCols = NC == 4 ? 2 : 1;
+  const int n = blockIdx.x * (kThreads / kCols) + threadIdx.x / kCols;
+  const int col = threadIdx.x % kCols, k = blockIdx.y, b = blockIdx.z;
+  if (n >= N) return;
+  const int64_t DN = (int64_t)DH * DW;
+  double *t = planes + ((int64_t)b * K + k) * S * DN;
+  const double *v = src + (int64_t)b * S * N + n;
+  for (int p = 0; p < pm; p++) {
+    int off[NC];
+    double wt[NC];
+    resolve_records<NC>(map, iw, ((int64_t)n * K + k) * pm + p, DH, DW, wrap != 0, -1, off, wt, 1);
+#pragma unroll
+    for (int r = 0; r < (NC == 4 ? 2 : 1); r++) {
+      const int o0 = off[(2 * r) % NC], o1 = off[(2 * r + 1) % NC];
+      const double a0 = wt[(2 * r) % NC], a1 = wt[(2 * r + 1) % NC];
+      const int o = col ? o1 : o0;
+      const double a = col ? a1 : a0;
+      if (o < 0) continue;
+      for (int c = 0; c < S; c++) atomic_add(t + c * DN + o, a * v[(int64_t)c * N]);
+    }
+  }
+}
+
+constexpr int kPlaneD = 16;  // destination channels per workgroup
+__global__ __launch_bounds__(kThreads) void product_planes_kernel(
+    const double *__restrict__ planes, const double *__restrict__ w,
+    const double *__restrict__ bias, double *__restrict__ dst, int S, int D, int64_t DN, int K) {
+  const int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int d0 = blockIdx.y * kPlaneD, b = blockIdx.z;
+  const double *t = planes + (int64_t)b * K * S * DN + min(p, DN - 1);
+  double acc[kPlaneD];
+#pragma unroll
+  for (int d = 0; d < kPlaneD; d++) acc[d] = bias && d0 + d < D ? bias[d0 + d] : 0.0;
+  for (int k = 0; k < K; k++)
+    for (int c = 0; c < S; c++) {
+      const double v = t[((int64_t)k * S + c) * DN];
+      const bool touched = __builtin_bit_cast(unsigned long long, v) != kUntouched;
+#pragma unroll
+      for (int d = 0; d < kPlaneD; d++) {
+        const double a = w[((int64_t)c * D + min(d0 + d, D - 1)) * K + k];
+        acc[d] = touched ? mcx_fma(a, v, acc[d]) : acc[d];
+      }
+    }
+  if (p >= DN) return;
+#pragma unroll
+  for (int d = 0; d < kPlaneD; d++)
+    if (d0 + d < D) dst[((int64_t)b * D + d0 + d) * DN + p] = acc[d];
+}
+
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Tiles, ranges and channel blocks of the weight gradient: about 2048 workgroups, eight per CU.
@@ -566,6 +641,17 @@ bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int
   return B * N >= 2048 || A * G * K * B * N >= ((int64_t)1 << 23);
 }
 
+// Scattering before the product, where the source channels are few beside the destination's (us for
+// the scalar kernel or records, as the rules above have it, against this; nine taps, one image of
+// 200x500): 1 -> 16 channels latitude map 158 / 63, shuffled 388 / 123; 1 -> 10 108 / 61, 375 / 121;
+// 1 -> 4 48 / 57, 187 / 117; 2 -> 16 157 / 107, 389 / 226; 2 -> 5 80 / 100, 205 / 221; 5 -> 16
+// 157 / 231, 390 / 525.  500x1000 1 -> 10 500 / 217, 1721 / 504; up to 64x128 shuffled 1 -> 10 48 / 24,
+// latitude 22 / 22.  The planes are K * S doubles a pixel to clear and to read: not many more than
+// additions, or than a record.
+static bool planes_scatter_applies(int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
+  return D >= 6 * S && K * S <= 64 && (S * DN <= 2 * N || K * S <= D);
+}
+
 #define MCX_LPR(C, CALL)              \
   switch (lanes_per_record(C)) {      \
     case 2: { CALL(2) } break;        \
@@ -612,6 +698,8 @@ int records_gather_product(const double *src, const double *map, const double *i
 }
 
 size_t records_scatter_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
+  if (planes_scatter_applies(S, D, DN, N, K))
+    return align256((size_t)(B * K * S * DN + 1) * sizeof(double));
   return scatter_record_bytes(B, D, DN) + (scatter_asks_map(B, S, N, K) ? 256 : 0);
 }
 
@@ -619,8 +707,29 @@ int records_product_scatter(const double *src, const double *map, const double *
                             const double *w, const double *bias, double *dst, void *ws, int64_t B,
                             int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,
                             int64_t P, int interp, hipStream_t s) {
+  const int64_t DN = DH * DW;
+  if (planes_scatter_applies(S, D, DN, N, K)) {
+    double *planes = (double *)ws;
+    const int64_t pairs = (B * K * S * DN + 1) / 2;
+    const unsigned blocks =
+        (unsigned)std::max<int64_t>(1, std::min<int64_t>((pairs + 1023) / 1024, 8192));
+    hipLaunchKernelGGL(begin_planes_kernel, dim3(blocks), dim3(kThreads), 0, s, (double2 *)ws, pairs);
+    const int pm = (int)(P == 0 ? 1 : P);
+#define MCX_RUN(NC, LOCS)                                                                        \
+  hipLaunchKernelGGL((scatter_planes_kernel<NC>), dim3(div_up(N, LOCS), (unsigned)K, (unsigned)B), \
+                     dim3(kThreads), 0, s, src, map, iw, planes, (int)S, (int)DH, (int)DW, (int)N, \
+                     (int)K, pm, wraps(interp) ? 1 : 0)
+    if (canonical_interp(interp) == kInterpNearest) { MCX_RUN(1, kThreads); }
+    else { MCX_RUN(4, kThreads / 2); }
+#undef MCX_RUN
+    hipLaunchKernelGGL(product_planes_kernel,
+                       dim3(div_up(DN, kThreads), div_up(D, kPlaneD), (unsigned)B), dim3(kThreads), 0,
+                       s, planes, w, bias, dst, (int)S, (int)D, DN, (int)K);
+    MCX_HIP_CHECK_LAUNCH();
+    return 0;
+  }
   double *rec = (double *)ws;
-  const int64_t DN = DH * DW, stride = add_stride(D);
+  const int64_t stride = add_stride(D);
   int *coherent = scatter_asks_map(B, S, N, K)
                       ? (int *)((char *)ws + scatter_record_bytes(B, D, DN))
                       : nullptr;

@@ -30,7 +30,13 @@ LARGER = [(1, 1, 1, 32, 32, 0), (2, 1, 9, 31, 67, 0), (3, 4, 6, 32, 33, 0), (5, 
           (33, 20, 3, 45, 53, 0), (1, 3, 9, 320, 308, 0)]
 
 
-@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES + LARGER)
+# few channels scattered into many: planes that are added to before the product (16 destination
+# channels a workgroup, 128 or 256 locations)
+PLANES = [(6, 1, 9, 4, 32, 0), (7, 1, 1, 5, 7, 0), (13, 2, 9, 9, 15, 0), (16, 1, 5, 16, 16, 3),
+          (17, 1, 9, 31, 67, 0), (20, 3, 10, 8, 17, 0), (33, 4, 3, 29, 45, 6), (40, 1, 64, 3, 43, 0)]
+
+
+@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES + LARGER + PLANES)
 @pytest.mark.parametrize("interp", [0, 1, 2])
 def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
     g = torch.Generator().manual_seed(ci * 100 + co)
@@ -59,6 +65,31 @@ def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
         for i, (a, c) in enumerate(zip(*[v if isinstance(v, (list, tuple)) else [v]
                                          for v in (got, want)])):
             assert rel_err(a, c) < 1e-12, (name, i)
+
+
+@pytest.mark.parametrize("interp", [0, 1, 2])
+def test_infinite_weights_reach_what_is_added_to(interp, device):
+    """A product weight that is infinite makes a destination pixel infinite where a tap lands on it
+    and leaves it alone where none does, also where the sums are taken before the product.
+    (Positive operands: no two infinities of different signs meet.)"""
+    g = torch.Generator().manual_seed(22)
+    B, ci, co, k, h, w_ = 2, 12, 1, 9, 9, 20
+    smap = torch.rand(h, w_, k, 2, generator=g, dtype=torch.float64) * 4 + 2.25
+    smap[..., 0] += torch.arange(k) % 3  # (other pixels under every tap)
+    w = torch.rand(co, ci, k, generator=g, dtype=torch.float64) + 0.1
+    w[0, 5, 4] = float("inf")
+    x, gy, b = (torch.rand(s, generator=g, dtype=torch.float64) + 0.1
+                for s in ((B, ci, h, w_), (B, co, h, w_), (co,)))
+    got = _C.mapped_conv_backward(*[t.cuda() for t in (gy, smap, x, w, b)], k, interp,
+                                  needs=(True, False, False))[0].cpu()
+    assert not torch.isnan(got).any() and (got[:, 5] == 0).any()
+    w[0, 5, 4] = 1.0
+    hit = torch.zeros_like(w)
+    hit[0, 5, 4] = 1.0
+    reached = O.mapped_conv_backward(gy, smap, x, hit, b, k, interp)[0] != 0
+    assert torch.equal(torch.isinf(got), reached)
+    want = O.mapped_conv_backward(gy, smap, x, w, b, k, interp)[0]
+    assert ((got - want).abs()[~reached] <= 1e-12 * want.abs().max()).all()
 
 
 @pytest.mark.parametrize("interp", [0, 1, 2])
