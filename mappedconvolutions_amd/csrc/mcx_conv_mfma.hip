@@ -1175,15 +1175,19 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l15 = lane & 15, lq = lane >> 4;
   int range, cg;
-  if ((ranges & 7) == 0) {  // channel groups of one pixel range share an XCD (and its L2)
+  // the channel groups and plain blocks of one pixel range are neighbours, on one XCD (and its L2)
+  const int combos = cgroups * ((A + kWgA - 1) / kWgA);
+  int combo;
+  if ((ranges & 7) == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    cg = slot % cgroups;
-    range = xcd * (ranges >> 3) + slot / cgroups;
+    combo = slot % combos;
+    range = xcd * (ranges >> 3) + slot / combos;
   } else {
-    cg = blockIdx.x % cgroups;
-    range = blockIdx.x / cgroups;
+    combo = blockIdx.x % combos;
+    range = blockIdx.x / combos;
   }
-  const int a0 = blockIdx.y * kWgA;
+  cg = combo % cgroups;
+  const int a0 = combo / cgroups * kWgA;
   const int k_base = blockIdx.z * kWgKT;
   const int ktaps = min(kWgKT, K - k_base);
   const int tpr = (total_tiles + ranges - 1) / ranges;
@@ -1307,6 +1311,9 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
         }
       }
       plain_sum[MB - 1] += t;
+      // (added here and now: put off to the tile's end, the summands stay in registers)
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++) asm volatile("" : "+v"(plain_sum[mb]));
     }
 
     const int gi = i0 + (p >> tw_shift), gj = j0 + (p & tw_mask);
@@ -1315,6 +1322,15 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     const int Gpad = (G + kGC - 1) / kGC * kGC;
     const TD *gath_b = gath + (int64_t)b * (CL ? Gpad : G) * gplane;
 
+    // A thread's samples of a unit are eight channels of one pixel, or over a channel-last copy four
+    // channels of two: four neighbouring lanes then read the 64 bytes of a record's sixteen
+    // channels together, and a load meets 16 lines instead of 64 (40 962 vertices, 4 x 64 -> 128
+    // channels, seven taps of four points: 753 -> 451 us; of three 541 -> 371; of one 150 -> 162,
+    // which stays as it was).
+    constexpr bool kQuads = CL && !kBf16 && kCacheTaps && NA > 1;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    f32x4 vq[kQuads ? 2 : 1][kQuads ? NA : 1];
+    const int qc = (tid & 3) * 4, qp = tid >> 2;  // (pixels qp and qp + 64)
     unsigned off[NE];
     float wt[NE];
     float v[8][NE];
@@ -1333,7 +1349,9 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
       }
     };
     auto load_tap = [&](int k) {  // k: tap within this pass
-      if (kCacheTaps) {
+      if (kQuads) {
+        (void)k;
+      } else if (kCacheTaps) {
 #pragma unroll
         for (int i = 0; i < NA; i++) {
           off[i] = TapOff[k][p][i];
@@ -1343,7 +1361,17 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
         resolve_tap(k_base + k, off, wt);
       }
     };
-    auto issue = [&](int cb) {
+    auto issue = [&](int cb, int k) {
+      if constexpr (kQuads) {
+        const char *base = reinterpret_cast<const char *>(
+            gath_b + min(g_first + cb * kGC + qc, Gpad - 4));
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int i = 0; i < NA; i++)
+            vq[h][i] = *reinterpret_cast<const f32x4 *>(base + TapOff[k][qp + 64 * h][i]);
+        return;
+      }
       const int g0 = g_first + cb * kGC + half * 8;
       if constexpr (CL) {
         // 8 contiguous channels of the pixel row; a workgroup whose channels lie past the
@@ -1376,7 +1404,22 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
         }
       }
     };
-    auto stage = [&](int buf) {
+    auto stage = [&](int buf, int k) {
+      if constexpr (kQuads) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          f32x4 sq = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            const float w = TapWt[k][qp + 64 * h][i];
+#pragma unroll
+            for (int j = 0; j < 4; j++) sq[j] = __builtin_fmaf(w, vq[h][i][j], sq[j]);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; j++) S[buf][qc + j][qp + 64 * h] = sq[j];
+        }
+        return;
+      }
       float sv[8];
 #pragma unroll
       for (int ch = 0; ch < 8; ch++) {
@@ -1419,7 +1462,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     // Units run channel-block-major with the tap fastest: the rows a 16-channel block
     // touches are reused by all taps while they are still in cache.
     load_tap(0);
-    issue(0);
+    issue(0, 0);
     int buf = 0;
 #pragma unroll
     for (int cb = 0; cb < kWgCB; cb++) {
@@ -1427,14 +1470,14 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
       for (int k = 0; k < kWgKT; k++) {
         if (k < ktaps) {
           buf ^= 1;
-          stage(buf);
+          stage(buf, k);
           __syncthreads();
           if (k + 1 < ktaps) {
             load_tap(k + 1);
-            issue(cb);
+            issue(cb, k + 1);
           } else if (cb + 1 < kWgCB) {
             load_tap(0);
-            issue(cb + 1);
+            issue(cb + 1, 0);
           }
           // The products of a unit issue back to back: at the default priority the other
           // waves of the SIMD slip their vector work in between and the matrix pipe idles.
@@ -2887,7 +2930,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
     MCX_HIP_CHECK_LAUNCH();
     gath = stage;
   }
-  dim3 grid((unsigned)(ranges * cgroups), (unsigned)((A + kWgA - 1) / kWgA),
+  dim3 grid((unsigned)(ranges * cgroups * ((A + kWgA - 1) / kWgA)), 1,
             (unsigned)((K + kWgKT - 1) / kWgKT));
   // Four pairs per tap: it pays to find out (on the device) whether only the first two pairs
   // are ever in use (bilinear maps with integral rows, two of four points weighted) and to

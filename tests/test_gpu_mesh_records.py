@@ -1,0 +1,36 @@
+"""fp32 convolutions over vertices (channel-last records that four lanes read together): one to four
+points a tap, channel counts around the 16 of a chunk and the 64 and 128 of a workgroup, vertex
+counts around a tile's 128, and cells of the transposed map of up to eight contributions and more."""
+import pytest
+import torch
+
+from helpers import rel_err
+from oracle import ops as O
+
+from mappedconvolutions_amd import _C
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("points", [1, 2, 3, 4])
+@pytest.mark.parametrize("ci,co,v", [(3, 5, 127), (16, 64, 128), (20, 65, 129), (33, 130, 300),
+                                     (130, 17, 64)])
+@pytest.mark.parametrize("spread", [1.0, 0.2])
+def test_weighted_mesh_convolution(points, ci, co, v, spread, device):
+    g = torch.Generator().manual_seed(100 * points + ci)
+    B, k = 2, 7
+    idx = torch.randint(max(1, int(v * spread)), (1, v, k, points), generator=g).float()
+    smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    iw = torch.rand(1, v, k, points, generator=g)
+    iw[torch.rand(iw.shape, generator=g) < 0.2] = 0  # (corners that weigh nothing)
+    x, w, b, gy = (torch.randn(s, generator=g)
+                   for s in ((B, ci, 1, v), (co, ci, k), (co,), (B, co, 1, v)))
+    dev = [t.cuda() for t in (x, smap, iw, w, b, gy)]
+    # 32-bit sums of up to some thousand terms: a few 1e-7 of the result's magnitude, 1e-5 allowed
+    # as everywhere in these tests
+    y = _C.weighted_mapped_conv_forward(*dev[:5], k, 0)
+    assert rel_err(y, O.weighted_mapped_conv_forward(x, smap, iw, w, b, k, 0)) < 1e-5
+    got = _C.weighted_mapped_conv_backward(dev[5], *dev[1:3], dev[0], *dev[3:5], k, 0)
+    want = O.weighted_mapped_conv_backward(gy, smap, iw, x, w, b, k, 0)
+    for a, e in zip(got, want):
+        assert rel_err(a, e) < 1e-5
