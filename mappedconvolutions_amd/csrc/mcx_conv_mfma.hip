@@ -3112,69 +3112,148 @@ __global__ void build_transposed_map_kernel(const float *__restrict__ map,
   }
 }
 
-// accum[b, d, p] += wt * sum_s W[s, d, k] * src[b, s, n] for every overflow entry: one wave
-// per (entry, image), a lane per destination channel.  `wp` holds the weights in the
-// gather-product's packed layout (fp32: Wp[k][s][d]; bf16: Wb[k][chunk][kg][d][8]); `src_cl`,
-// when not null, is the channel-last copy [B][MN][Spad] of the source, else src is
-// [B][S][MN].  `accum` is a channel-last fp32 image [B][DN][Dpad] (a wave's 64 atomics fall
-// into two cache lines instead of 64) that the gather's epilogue adds.  A fixed grid walks
-// the list, so an empty list costs one launch of idle workgroups.
-template <typename TD>
+// accum[b, d, p] += wt * sum_s W[s, d, k] * src[b, s, n] for every overflow entry, a lane per
+// destination channel: a wave takes 64, 32 or 16 lanes an entry, U entries after one another in
+// each, whose loads are in flight together (an entry is three dependent loads deep), and IB images
+// with one reading of the entry's weights.  One entry and image at a time -> this: 3 x 40 -> 24
+// channels of 125 x 250 under a gnomonic map 58 -> 30 us; mesh of 40 962 vertices, 4 x 128 -> 64
+// channels 85 -> 57.
+// `wp` holds the weights in the gather-product's packed layout (fp32: Wp[k][s][d]; bf16:
+// Wb[k][chunk][kg][d][8]); `src_cl`, when not null, is the channel-last copy [B][MN][Spad] of the
+// source, else src is [B][S][MN].  `accum` is a channel-last fp32 image [B][DN][Dpad] (a wave's 64
+// atomics fall into two cache lines instead of 64) that the gather's epilogue adds.  A fixed grid
+// walks the list, so an empty list costs one launch of idle workgroups.
+template <typename TD, int U, int IB>
 __global__ __launch_bounds__(64) void overflow_scatter_kernel(
     const TD *__restrict__ src, const TD *__restrict__ src_cl, const void *__restrict__ wp,
     float *__restrict__ accum, const OverflowEntry *__restrict__ ovf,
-    const int *__restrict__ overflow, int ovf_cap, int S, int Spad, int D, int Dpad, int64_t MN,
-    int64_t DN) {
+    const int *__restrict__ overflow, int ovf_cap, int B, int S, int Spad, int D, int Dpad,
+    int64_t MN, int64_t DN) {
   if (overflow[0] != 0) return;  // the scatter kernel does the whole product
   const int count = min(overflow[1], ovf_cap);
-  const int b = blockIdx.y, lane = threadIdx.x;
+  const int b0 = blockIdx.y * IB, lane = threadIdx.x;
   const int chunks = Spad / kGC;
-  for (int e = blockIdx.x; e < count; e += gridDim.x) {
-    const OverflowEntry en = ovf[e];
-    for (int d0 = 0; d0 < D; d0 += 64) {
-      const int d = min(d0 + lane, Dpad - 1);
-      float acc = 0.f;
+  const int lanes = D <= 16 ? 16 : D <= 32 ? 32 : 64, per_wave = 64 / lanes;
+  const int sub = lane / lanes, dl = lane % lanes;
+  const int step = U * per_wave;
+  for (int e0 = blockIdx.x * step; e0 < count; e0 += gridDim.x * step) {
+    OverflowEntry en[U];
+    bool live[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int e = e0 + u * per_wave + sub;
+      live[u] = e < count;
+      en[u] = ovf[min(e, count - 1)];
+    }
+    for (int d0 = 0; d0 < D; d0 += lanes) {
+      const int d = min(d0 + dl, Dpad - 1);
+      float acc[U][IB];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int i = 0; i < IB; i++) acc[u][i] = 0.f;
       for (int s8 = 0; s8 < Spad / 8; s8++) {  // 8 source channels at a time (both are padded)
-        float x[8], wv[8];
+        float x[U][IB][8], wv[U][8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const int sc = s8 * 8 + j;
-          x[j] = src_cl ? to_f32(src_cl[((int64_t)b * MN + en.n) * Spad + sc])
-                        : (sc < S ? to_f32(src[((int64_t)b * S + sc) * MN + en.n]) : 0.f);
-        }
-        if constexpr (sizeof(TD) == 2) {
-          const int64_t wi = ((((int64_t)en.k * chunks + (s8 >> 1)) * 2 + (s8 & 1)) * Dpad + d) << 3;
-          const uint4 q = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(wp) + wi);
-          const unsigned w4[4] = {q.x, q.y, q.z, q.w};
+        for (int u = 0; u < U; u++) {
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            wv[2 * j] = __builtin_bit_cast(float, w4[j] << 16);
-            wv[2 * j + 1] = __builtin_bit_cast(float, w4[j] & 0xffff0000u);
+          for (int i = 0; i < IB; i++) {
+            const int64_t b = min(b0 + i, B - 1);  // (past the last image: not added)
+            if (sizeof(TD) == 4 && src_cl) {
+              const float4 *q = reinterpret_cast<const float4 *>(
+                  src_cl + (b * MN + en[u].n) * Spad + s8 * 8);
+              const float4 q0 = q[0], q1 = q[1];
+              x[u][i][0] = q0.x; x[u][i][1] = q0.y; x[u][i][2] = q0.z; x[u][i][3] = q0.w;
+              x[u][i][4] = q1.x; x[u][i][5] = q1.y; x[u][i][6] = q1.z; x[u][i][7] = q1.w;
+            } else {
+#pragma unroll
+              for (int j = 0; j < 8; j++) {
+                const int sc = s8 * 8 + j;
+                x[u][i][j] = src_cl ? to_f32(src_cl[(b * MN + en[u].n) * Spad + sc])
+                                    : (sc < S ? to_f32(src[(b * S + sc) * MN + en[u].n]) : 0.f);
+              }
+            }
           }
-        } else {
+          if constexpr (sizeof(TD) == 2) {
+            const int64_t wi =
+                ((((int64_t)en[u].k * chunks + (s8 >> 1)) * 2 + (s8 & 1)) * Dpad + d) << 3;
+            const uint4 q = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(wp) + wi);
+            const unsigned w4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-          for (int j = 0; j < 8; j++)
-            wv[j] = reinterpret_cast<const float *>(wp)[((int64_t)en.k * Spad + s8 * 8 + j) * Dpad + d];
+            for (int j = 0; j < 4; j++) {
+              wv[u][2 * j] = __builtin_bit_cast(float, w4[j] << 16);
+              wv[u][2 * j + 1] = __builtin_bit_cast(float, w4[j] & 0xffff0000u);
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+              wv[u][j] = reinterpret_cast<const float *>(
+                  wp)[((int64_t)en[u].k * Spad + s8 * 8 + j) * Dpad + d];
+          }
         }
 #pragma unroll
-        for (int j = 0; j < 8; j++) acc = __builtin_fmaf(x[j], wv[j], acc);
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int i = 0; i < IB; i++)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+              acc[u][i] = __builtin_fmaf(x[u][i][j], wv[u][j], acc[u][i]);
       }
-      if (d0 + lane < D) atomic_add(accum + ((int64_t)b * DN + en.p) * Dpad + d, en.wt * acc);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int i = 0; i < IB; i++)
+          if (live[u] && b0 + i < B && d0 + dl < D)
+            atomic_add(accum + ((int64_t)(b0 + i) * DN + en[u].p) * Dpad + d, en[u].wt * acc[u][i]);
     }
   }
 }
 
-// Two jobs that follow the building of a transposed map, in one launch.  (1) mask[0] >= 4
+// What the scatter form needs before it runs: dst[b,c,:] = bias[c] (or 0), and the weights repacked
+// W[s][d][k] -> Wq[k][dc][s][16]: per (tap, 16-channel block) a contiguous [Spad x 16] slice; s
+// padded to 64, d padded to 16, zeros in the padding.
+template <typename TD>
+struct InitScatter {
+  float *dst;
+  const TD *bias, *w;
+  float *wq;
+  int C, S, K, Spad, dchunks;
+  int64_t plane, total;
+};
+template <typename TD>
+__device__ inline void init_scatter(const InitScatter<TD> &a) {
+  const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = first; i < a.total; i += stride)
+    a.dst[i] = a.bias ? to_f32(a.bias[(i / a.plane) % a.C]) : 0.f;
+  const int64_t packed = (int64_t)a.K * a.dchunks * a.Spad * kScDC;
+  for (int64_t e = first; e < packed; e += stride) {
+    const int dl = (int)(e % kScDC);
+    const int sl = (int)((e / kScDC) % a.Spad);
+    const int dc = (int)((e / ((int64_t)kScDC * a.Spad)) % a.dchunks);
+    const int k = (int)(e / ((int64_t)kScDC * a.Spad * a.dchunks));
+    const int d = dc * kScDC + dl;
+    a.wq[e] = (sl < a.S && d < a.C) ? to_f32(a.w[((int64_t)sl * a.C + d) * a.K + k]) : 0.f;
+  }
+}
+template <typename TD>
+__global__ void init_scatter_kernel(const InitScatter<TD> a) {
+  init_scatter(a);
+}
+
+// Three jobs that follow the building of a transposed map, in one launch.  (1) mask[0] >= 4
 // iff some cell holds more than two entries (bits [0, min(cnt, kTransSlots))), and row_mask
 // says in which rows of the destination; with a second level, mask[1] holds the bits of the
 // second-level slots in use (0: none).  (2) Clear
 // the fp32 image the overflow list is accumulated into, only when the list is in use and
-// not empty.
+// not empty.  (3) Where the list overflowed too, what the scatter form needs.
+template <typename TD>
 __global__ void after_transposed_map_kernel(const int *__restrict__ cnt, int64_t cells,
                                             int *__restrict__ mask, int two_level,
                                             float *__restrict__ img, int64_t total,
                                             const int *__restrict__ overflow,
-                                            int *__restrict__ row_mask, int64_t plane, int row_px) {
+                                            int *__restrict__ row_mask, int64_t plane, int row_px,
+                                            const InitScatter<TD> scatter) {
   __shared__ unsigned block_mask;
   if (threadIdx.x == 0) block_mask = 0;
   __syncthreads();
@@ -3197,36 +3276,14 @@ __global__ void after_transposed_map_kernel(const int *__restrict__ cnt, int64_t
                                                    __HIP_MEMORY_SCOPE_AGENT)))
       atomicOr(mask + 1, (int)m2);
   }
-  if (overflow[0] != 0 || overflow[1] <= 0) return;
+  if (overflow[0] != 0) {
+    init_scatter(scatter);
+    return;
+  }
+  if (overflow[1] <= 0) return;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
        i += (int64_t)gridDim.x * blockDim.x)
     img[i] = 0.f;
-}
-
-// What the scatter form needs before it runs, in one launch (a launch costs about 4 us even
-// when every workgroup leaves at once, as here on maps the gather form handles):
-// dst[b,c,:] = bias[c] (or 0), and the weights repacked W[s][d][k] -> Wq[k][dc][s][16]: per
-// (tap, 16-channel block) a contiguous [Spad x 16] slice; s padded to 64, d padded to 16, zeros
-// in the padding.  Runs only when the gate agrees (see above).
-template <typename TD>
-__global__ void init_scatter_kernel(float *__restrict__ dst, const TD *__restrict__ bias, int C,
-                                    int64_t plane, int64_t total, const TD *__restrict__ w,
-                                    float *__restrict__ wq, int S, int K, int Spad, int dchunks,
-                                    const int *__restrict__ gate, int run_if_zero) {
-  if (gate && ((*gate == 0) != (run_if_zero != 0))) return;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x)
-    dst[i] = bias ? to_f32(bias[(i / plane) % C]) : 0.f;
-  const int64_t packed = (int64_t)K * dchunks * Spad * kScDC;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < packed;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int dl = (int)(e % kScDC);
-    const int sl = (int)((e / kScDC) % Spad);
-    const int dc = (int)((e / ((int64_t)kScDC * Spad)) % dchunks);
-    const int k = (int)(e / ((int64_t)kScDC * Spad * dchunks));
-    const int d = dc * kScDC + dl;
-    wq[e] = (sl < S && d < C) ? to_f32(w[((int64_t)sl * C + d) * K + k]) : 0.f;
-  }
 }
 
 template <typename TD>
@@ -3401,10 +3458,10 @@ int mfma_scatter_plan_build(const float *map, const float *iw, void *plan, int64
   const int64_t cells = DH * DW * K;
   int *flag = cnt + cells;
   if (int rc = build_transposed_map(sc, map, iw, cnt, m, DH, DW, MH, MW, K, s)) return rc;
-  hipLaunchKernelGGL(after_transposed_map_kernel,
+  hipLaunchKernelGGL(after_transposed_map_kernel<float>,
                      dim3((unsigned)std::min<int64_t>((cells + 255) / 256, 4096)), dim3(256), 0, s,
                      cnt, cells, flag + 2, sc.two_level ? 1 : 0, (float *)nullptr, (int64_t)0,
-                     flag, flag + 8, DH * DW, (int)DW);
+                     flag, flag + 8, DH * DW, (int)DW, InitScatter<float>{});
   MCX_HIP_CHECK_LAUNCH();
   if (m.np * (m.mode == kInterpNearest ? 1 : 4) == 4)
     if (int rc = launch_pair_mask(map, iw, flag + 4, m, DH, DW, MH * MW * K, s, true)) return rc;
@@ -3444,6 +3501,11 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
   const int Spad = (int)round_up(S, kScSC), dchunks = (int)((D + kScDC - 1) / kScDC);
   const ModeArgs m = mode_args(interp, P);
   const int *gate = nullptr;
+  const int64_t total_dst = B * D * DH * DW;
+  float *acc = sizeof(TD) == 4 ? (float *)dst : (float *)(base + sc.acc32);
+  const InitScatter<TD> init{acc,    bias,    w,       wq,       (int)D,
+                             (int)S, (int)K,  Spad,    dchunks,  DH * DW,
+                             total_dst};
 
   if (sc.transposed_path) {
     // build the transposed map, then try the atomic-free gather form first
@@ -3480,11 +3542,11 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
     float *img = (float *)(base + sc.acc32);
     const int64_t total_img = B * DH * DW * round_up(D, kOT);
     // flag[2]: at least 4 iff some cell holds more than two entries (a plan has it already)
-    hipLaunchKernelGGL(after_transposed_map_kernel,
+    hipLaunchKernelGGL(after_transposed_map_kernel<TD>,
                        dim3((unsigned)std::min<int64_t>(
                            std::max((total_img + 1023) / 1024, (cells + 255) / 256), 4096)),
                        dim3(256), 0, s, cnt, plan ? (int64_t)0 : cells, flag + 2,
-                       sc.two_level ? 1 : 0, img, total_img, flag, flag + 8, DH * DW, (int)DW);
+                       sc.two_level ? 1 : 0, img, total_img, flag, flag + 8, DH * DW, (int)DW, init);
     MCX_HIP_CHECK_LAUNCH();
     if (cl) {  // the overflow pass reads the channel-last copy before the gather would make it
       dim3 tg((unsigned)((MH * MW + 63) / 64), (unsigned)((Spad16 + 63) / 64), (unsigned)B);
@@ -3492,10 +3554,16 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
                          (int)Spad16, MH * MW);
       MCX_HIP_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL(overflow_scatter_kernel<TD>, dim3(2048, (unsigned)B), dim3(64), 0, s, src,
-                       cl ? (const TD *)stage : (const TD *)nullptr, (const void *)wpt, img, ovf,
-                       flag, (int)sc.ovf_cap, (int)S, (int)Spad16, (int)D, (int)round_up(D, kOT),
-                       MH * MW, DH * DW);
+#define MCX_OVERFLOW(U, IB)                                                                       \
+  hipLaunchKernelGGL((overflow_scatter_kernel<TD, U, IB>), dim3(4096, (unsigned)((B + IB - 1) / IB)), \
+                     dim3(64), 0, s, src, cl ? (const TD *)stage : (const TD *)nullptr,           \
+                     (const void *)wpt, img, ovf, flag, (int)sc.ovf_cap, (int)B, (int)S,          \
+                     (int)Spad16, (int)D, (int)round_up(D, kOT), MH * MW, DH * DW)
+    // (a tap's weights that fit an L1 are best shared by entries: 12 KB 30 us where images of two
+    // entries share them in 42; 32 KB 85 and 57)
+    const bool large = Spad16 * round_up(D, kOT) * (int64_t)sizeof(TD) > 16384;
+    if (B > 1 && large) { MCX_OVERFLOW(2, 4); } else { MCX_OVERFLOW(4, 1); }
+#undef MCX_OVERFLOW
     MCX_HIP_CHECK_LAUNCH();
     if (int rc = launch_gather_product<TD>(src, (const float *)tmap, nullptr, wpt, bias, dst,
                                            stage, B, S, D, MH, MW, DH, DW, K, kTransSlots,
@@ -3513,12 +3581,11 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
   }
 
   // atomic path (runs when there is no transposed map or it overflowed)
-  const int64_t total_dst = B * D * DH * DW;
-  float *acc = sizeof(TD) == 4 ? (float *)dst : (float *)(base + sc.acc32);
   const unsigned fill_blocks = (unsigned)std::min<int64_t>((total_dst + 1023) / 1024, 8192);
-  hipLaunchKernelGGL(init_scatter_kernel<TD>, dim3(fill_blocks), dim3(256), 0, s, acc, bias, (int)D,
-                     DH * DW, total_dst, w, wq, (int)S, (int)K, Spad, dchunks, gate, 0);
-  MCX_HIP_CHECK_LAUNCH();
+  if (!sc.transposed_path) {
+    hipLaunchKernelGGL(init_scatter_kernel<TD>, dim3(fill_blocks), dim3(256), 0, s, init);
+    MCX_HIP_CHECK_LAUNCH();
+  }
   const int tiles_x = (int)((MW + kScPx - 1) / kScPx);
   const int64_t tiles_per_img = (int64_t)tiles_x * MH;
   const int64_t total = tiles_per_img * B;

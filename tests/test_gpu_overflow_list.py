@@ -1,0 +1,34 @@
+"""Input gradients whose transposed map overfills cells: the list of what is left, by entries and by
+images, channel counts around the 16, 32 and 64 lanes of an entry, and lists that overflow as well."""
+import pytest
+import torch
+
+from helpers import rel_err
+from oracle import ops as O
+
+from mappedconvolutions_amd import _C
+
+pytestmark = pytest.mark.gpu
+
+
+# (ci is the gradient's channel count; 128 x 64 weights of a tap: images share their reading)
+@pytest.mark.parametrize("B", [1, 2, 5])
+@pytest.mark.parametrize("ci,co", [(3, 5), (16, 20), (17, 8), (33, 64), (64, 128), (65, 40)])
+@pytest.mark.parametrize("share", [0.1, 0.4, 1.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_many_contributions_to_few_pixels(B, ci, co, share, dtype, device):
+    g = torch.Generator().manual_seed(ci + co)
+    h, w_, k = 12, 20, 3
+    y, x = torch.meshgrid(torch.arange(h).float(), torch.arange(w_).float(), indexing="ij")
+    smap = torch.stack((x, y), -1).unsqueeze(2).repeat(1, 1, k, 1)
+    crowd = torch.rand(h, w_, k, 1, generator=g) < share  # (these meet in six pixels)
+    smap = torch.where(crowd, torch.rand(h, w_, k, 2, generator=g) * torch.tensor([2.0, 1.0]) + 3, smap)
+    smap = smap.contiguous()
+    rnd = lambda *s: torch.randn(s, generator=g).to(dtype).float()
+    xs, wt, b, gy = rnd(B, ci, h, w_), rnd(co, ci, k), rnd(co), rnd(B, co, h, w_)
+    gx = _C.mapped_conv_backward(gy.cuda().to(dtype), smap.cuda(), xs.cuda().to(dtype),
+                                 wt.cuda().to(dtype), b.cuda().to(dtype), k, 1,
+                                 needs=(True, False, False))[0]
+    want = O.mapped_conv_backward(gy, smap, xs, wt, b, k, 1)[0]
+    # (the bars of the other tests: 32-bit sums, and results and samples rounded to bf16)
+    assert rel_err(gx.float(), want) < (1e-5 if dtype == torch.float32 else 2e-2)
