@@ -106,6 +106,83 @@ __device__ inline unsigned block_pair_mask(const float *__restrict__ map,
   return block_mask;
 }
 
+// x[b][g][n] -> xt[b][g/8][n][g%8] (channels past G zero): a thread gathers the 8 channels of
+// one pixel (each of the 8 loads is contiguous across the wave) and writes them as one vector.
+template <typename TD>
+struct ChannelBlocksJob {
+  const TD *x;     // nullptr: no job
+  TD *xt;
+  int G, groups;   // channels, blocks of 8 of them (padded)
+  int64_t plane;
+  int per_plane;   // workgroups a block of channels
+  int64_t count;   // workgroups
+};
+template <typename TD>
+__device__ inline void to_channel_blocks(const ChannelBlocksJob<TD> &a, int block) {
+  const int64_t n = (int64_t)(block % a.per_plane) * 256 + threadIdx.x;
+  const int g8 = block / a.per_plane % a.groups, b = block / a.per_plane / a.groups;
+  if (n >= a.plane) return;
+  struct alignas(8 * sizeof(TD)) Block { TD c[8]; } v;
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const int g = g8 * 8 + c;
+    v.c[c] = g < a.G ? a.x[((int64_t)b * a.G + g) * a.plane + n] : TD{};
+  }
+  reinterpret_cast<Block *>(a.xt)[((int64_t)b * a.groups + g8) * a.plane + n] = v;
+}
+
+// Gather part of a map plan: every (map location, tap) resolved once to four (element index of
+// the sampled image as bits, weight) entries - the four bilinear corners, or up to four
+// nearest points with the rest zero - in the layout the gather-product kernel reads with
+// `packed_map` (the same as a transposed map's cells).
+constexpr int kPlanSlots = 4;  // resolved entries per (location, tap)
+struct GatherPlanJob {
+  const float *map, *iw;  // map nullptr: no job
+  float2 *gmap;
+  int np, weighted, wrap, SH, SW, K, ncorn;
+  int64_t total;   // (location, tap) pairs
+  int count;       // workgroups
+};
+template <int NCORN>
+__device__ inline void build_gather_plan(const float *__restrict__ map,
+                                         const float *__restrict__ iw, float2 *__restrict__ gmap,
+                                         int np, int weighted, int wrap, int SH, int SW, int K,
+                                         int64_t total, int block) {
+  // (a wave takes 64 consecutive locations of one tap: its stores are 512-byte runs)
+  const int64_t t0 = (int64_t)block * 256 + threadIdx.x;
+  const int64_t run = t0 / (64 * (int64_t)K), pixels = total / K;
+  const int r = (int)(t0 - run * 64 * K);
+  const int64_t n = run * 64 + (r & 63);
+  const int k = r >> 6;
+  if (n >= pixels) return;
+  const int64_t e = n * K + k;  // (location, tap)
+  float2 out[kPlanSlots];
+#pragma unroll
+  for (int i = 0; i < kPlanSlots; i++) out[i] = make_float2(0.f, 0.f);
+  for (int sp = 0; sp < np; sp++) {
+    const int64_t q = e * np + sp;
+    PairTap<NCORN> t;
+    resolve_pairs<NCORN, 1>(map[q * 2], map[q * 2 + 1], SH, SW, wrap != 0,
+                            weighted ? iw[q] : 1.f, t);
+#pragma unroll
+    for (int i = 0; i < NCORN; i++)
+      if (sp * NCORN + i < kPlanSlots)
+        out[sp * NCORN + i] = make_float2(__builtin_bit_cast(float, t.off[i]), t.wt[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < kPlanSlots; i++)  // stored [tap][slot][location]
+    gmap[((int64_t)k * kPlanSlots + i) * pixels + n] = out[i];
+}
+
+//   * ChannelBlocksJob and GatherPlanJob: the gathered operand in blocks of eight channels, and the
+//     map's taps resolved, for the product that follows (bf16 images): 4 x 32 -> 64 channels of
+//     64 x 128, forward five launches -> two.
+template <typename TD>
+struct PrepJobs {
+  ChannelBlocksJob<TD> blocks;
+  GatherPlanJob plan;
+};
+
 // Repack W[o][g][k] for the matrix-core kernels, with g padded to 16 and o padded to 64
 // (zeros); `transposed` reads W[g][o][k] instead (weights stored source-channel major).
 //   fp32 storage: Wp[k][g][o] floats, so that a reduction chunk's weights are 16 rows of
@@ -128,9 +205,27 @@ template <typename TD>
 __global__ __launch_bounds__(256) void pack_weights_kernel(
     const TD *__restrict__ w, void *__restrict__ packed_out, int O, int G, int K, int Opad,
     int Gpad, int transposed, int *__restrict__ clear, ZeroJob zero, PairMaskJob pm,
-    SplitJob split) {
+    SplitJob split, PrepJobs<TD> prep) {
   if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // a flag word of the caller
   int blocks = gridDim.x;
+  if (prep.blocks.x) {
+    blocks -= (int)prep.blocks.count;
+    if ((int)blockIdx.x >= blocks) return to_channel_blocks(prep.blocks, (int)blockIdx.x - blocks);
+  }
+  if (prep.plan.map) {
+    const GatherPlanJob &g = prep.plan;
+    blocks -= g.count;
+    if ((int)blockIdx.x >= blocks) {
+      const int block = (int)blockIdx.x - blocks;
+      if (g.ncorn == 1)
+        build_gather_plan<1>(g.map, g.iw, g.gmap, g.np, g.weighted, g.wrap, g.SH, g.SW, g.K, g.total,
+                             block);
+      else
+        build_gather_plan<4>(g.map, g.iw, g.gmap, g.np, g.weighted, g.wrap, g.SH, g.SW, g.K, g.total,
+                             block);
+      return;
+    }
+  }
   if (pm.mask) {
     blocks -= pm.blocks;
     if ((int)blockIdx.x >= blocks) {  // the last blocks: the map's pair mask, nothing else
@@ -217,27 +312,6 @@ __global__ __launch_bounds__(256) void to_channel_last_kernel(const TD *__restri
     const int g = g0 + lx;
     if (n < plane && g < Gpad) xt[((int64_t)b * plane + n) * Gpad + g] = tile[lx][ly + 4 * r];
   }
-}
-
-// x[b][g][n] -> xt[b][g/8][n][g%8] (channels past G zero): a thread gathers the 8 channels of
-// one pixel (each of the 8 loads is contiguous across the wave) and writes them as one vector.
-template <typename TD>
-__global__ __launch_bounds__(256) void to_channel_blocks_kernel(const TD *__restrict__ x,
-                                                                TD *__restrict__ xt, int G,
-                                                                int64_t plane,
-                                                                const int *__restrict__ pair_mask) {
-  // (with a pair mask: the copy is for a kernel that only runs while the mask is below 4)
-  if (pair_mask && (unsigned)*pair_mask >= (1u << 2)) return;
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int g8 = blockIdx.y, b = blockIdx.z;
-  if (n >= plane) return;
-  struct alignas(8 * sizeof(TD)) Block { TD c[8]; } v;
-#pragma unroll
-  for (int c = 0; c < 8; c++) {
-    const int g = g8 * 8 + c;
-    v.c[c] = g < G ? x[((int64_t)b * G + g) * plane + n] : TD{};
-  }
-  reinterpret_cast<Block *>(xt)[((int64_t)b * gridDim.y + g8) * plane + n] = v;
 }
 
 // y[b][a][pixel] -> yt[b][tile][a / 32][mb][s4][lane][8]: the plain operand of a weight gradient
@@ -1660,8 +1734,8 @@ __device__ inline void resolve_tap_table(const float *__restrict__ map,
 }
 __global__ __launch_bounds__(256) void resolve_tap_table_kernel(
     const float *__restrict__ map, unsigned *__restrict__ table, int GH, int GW, int MH, int MW,
-    int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask) {
-  if ((unsigned)*pair_mask < (1u << 2))
+    int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask, int mask_words) {
+  if (!later_pairs_in_use(pair_mask, mask_words))
     resolve_tap_table<2>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
   else
     resolve_tap_table<4>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
@@ -1997,12 +2071,12 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_bf16_ring_kernel(
     const bf16_t *__restrict__ plain, const bf16_t *__restrict__ gath,
     const unsigned *__restrict__ table, float *__restrict__ part, int A, int G, int Gpad, int GH,
     int GW, int K, int tiles_per_img, int total_tiles, int ranges, int cgroups, int passes,
-    float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask) {
+    float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask, int mask_words) {
   __shared__ __attribute__((aligned(16))) union {
     RingLds<2> two;
     RingLds<4> four;
   } lds;
-  if ((unsigned)*pair_mask < (1u << 2))
+  if (!later_pairs_in_use(pair_mask, mask_words))
     weight_grad_bf16_ring<2>(lds.two, plain, gath, table, part, A, G, Gpad, GH, GW, K,
                              tiles_per_img, total_tiles, ranges, cgroups, passes, plain_sum_part);
   else
@@ -2423,14 +2497,17 @@ inline bool use_channel_blocks(int64_t SH, int interp, size_t elem) {
   return elem == 2 && !use_channel_last(SH, interp) && SH > 1;
 }
 template <typename TD>
-int launch_channel_blocks(const TD *src, TD *stage, int64_t B, int64_t G, int64_t plane,
-                          hipStream_t s, const int *pair_mask = nullptr) {
-  const int64_t Gpad = round_up(G, kGC);
-  dim3 tg((unsigned)((plane + 255) / 256), (unsigned)(Gpad / 8), (unsigned)B);
-  hipLaunchKernelGGL(to_channel_blocks_kernel<TD>, tg, dim3(256), 0, s, src, stage, (int)G, plane,
-                     pair_mask);
-  MCX_HIP_CHECK_LAUNCH();
-  return 0;
+ChannelBlocksJob<TD> channel_blocks_job(const TD *src, TD *stage, int64_t B, int64_t G,
+                                        int64_t plane) {
+  const int64_t groups = round_up(G, kGC) / 8, per_plane = (plane + 255) / 256;
+  return ChannelBlocksJob<TD>{src, stage, (int)G, (int)groups, plane, (int)per_plane,
+                              per_plane * groups * B};
+}
+GatherPlanJob gather_plan_job(const float *map, const float *iw, float2 *gmap, const ModeArgs &m,
+                              int64_t SH, int64_t SW, int64_t MN, int64_t K) {
+  return GatherPlanJob{map, iw, gmap, m.np, m.weighted, m.wrap, (int)SH, (int)SW, (int)K,
+                       m.mode == kInterpNearest ? 1 : 4, MN * K,
+                       (int)(((MN + 63) / 64 * 64 * K + 255) / 256)};
 }
 
 // `stage`: room for the channel-last copy (B * SH * SW * Gpad elements) when
@@ -2505,6 +2582,19 @@ int launch_gather_split(SplitArgs a, const PixelTiling &t, bool cl, hipStream_t 
 
 // `split` (fp32 storage; w NULL: not available): where the packing launch put the split weights.
 // `map2`: second-level entries of a packed map, read by the split kernels only.
+// Whether launch_gather_product reads blocks of eight channels: the packing launch makes them then.
+template <typename TD>
+bool gathers_blocks(const TD *stage, int64_t SH, int64_t SW, int interp) {
+  return stage != nullptr && use_channel_blocks(SH, interp, sizeof(TD)) &&
+         SH * SW * 8 * (int64_t)sizeof(TD) <= 0xffffffffLL;
+}
+template <typename TD>
+ChannelBlocksJob<TD> blocks_for(const TD *src, TD *stage, int64_t B, int64_t G, int64_t SH,
+                                int64_t SW, int interp) {
+  return gathers_blocks(stage, SH, SW, interp) ? channel_blocks_job<TD>(src, stage, B, G, SH * SW)
+                                               : ChannelBlocksJob<TD>{};
+}
+
 template <typename TD>
 int launch_gather_product(const TD *src, const float *map, const float *iw, const float *wp,
                           const TD *bias, TD *y, TD *stage, int64_t B, int64_t G, int64_t O,
@@ -2516,14 +2606,10 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
                           int mask_words = 1, SplitJob split = SplitJob{},
                           const float2 *map2 = nullptr, const int *only_if = nullptr) {
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
-  const bool blocked = stage != nullptr && use_channel_blocks(SH, interp, sizeof(TD)) &&
-                       SH * SW * 8 * (int64_t)sizeof(TD) <= 0xffffffffLL;
+  const bool blocked = gathers_blocks(stage, SH, SW, interp);
   const bool cl = blocked || gathers_channel_last(stage != nullptr, SH, SW, G, interp, sizeof(TD));
-  if (cl && staged) {
-    src = stage;  // the caller has made the copy already
-  } else if (blocked) {
-    if (int rc = launch_channel_blocks<TD>(src, stage, B, G, SH * SW, s)) return rc;
-    src = stage;
+  if (blocked || (cl && staged)) {
+    src = stage;  // the copy is there already (blocks come with the packing launch: blocks_for)
   } else if (cl) {
     dim3 tg((unsigned)((SH * SW + 63) / 64), (unsigned)((Gpad + 63) / 64), (unsigned)B);
     hipLaunchKernelGGL(to_channel_last_kernel<TD>, tg, dim3(256), 0, s, src, stage, (int)G, Gpad,
@@ -2662,15 +2748,36 @@ constexpr int64_t kTinyMapEntries = 4096;
 template <typename TD>
 int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K, int transposed,
                         hipStream_t s, int *clear = nullptr, ZeroJob zero = ZeroJob{nullptr, 0},
-                        PairMaskJob pm = PairMaskJob{}, SplitJob split = SplitJob{}) {
+                        PairMaskJob pm = PairMaskJob{}, SplitJob split = SplitJob{},
+                        PrepJobs<TD> prep = PrepJobs<TD>{}) {
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const int64_t packed = (int64_t)K * Gpad * Opad;
+  // (a launch has at most 2^32 threads: beyond a quarter of them, image by image)
+  if (prep.blocks.x && prep.blocks.count > ((int64_t)1 << 22)) {
+    const int64_t image = (int64_t)prep.blocks.per_plane * prep.blocks.groups;
+    const int64_t images = prep.blocks.count / image;
+    if (image > ((int64_t)1 << 22)) return MCX_E_SHAPE;
+    for (int64_t b = 0; b < images; b++) {
+      PrepJobs<TD> one{};
+      one.blocks = prep.blocks;
+      one.blocks.x += b * prep.blocks.G * prep.blocks.plane;
+      one.blocks.xt += b * prep.blocks.groups * 8 * prep.blocks.plane;
+      one.blocks.count = image;
+      hipLaunchKernelGGL(pack_weights_kernel<TD>, dim3((unsigned)image), dim3(256), 0, s, w,
+                         (void *)wp, 0, 0, 0, 0, 0, 0, (int *)nullptr, ZeroJob{nullptr, 0},
+                         PairMaskJob{}, SplitJob{}, one);
+      MCX_HIP_CHECK_LAUNCH();
+    }
+    prep.blocks = ChannelBlocksJob<TD>{};
+  }
   // (bf16 storage: the bf16 MFMA operand layout in the same scratch, half the bytes)
   const int64_t work = std::max({packed, zero.count * 4, split.tiles});
   const dim3 grid((unsigned)std::min<int64_t>((work + 255) / 256, 4096) +
-                  (pm.mask ? (unsigned)pm.blocks : 0u));
+                  (pm.mask ? (unsigned)pm.blocks : 0u) +
+                  (prep.plan.map ? (unsigned)prep.plan.count : 0u) +
+                  (prep.blocks.x ? (unsigned)prep.blocks.count : 0u));
   hipLaunchKernelGGL(pack_weights_kernel<TD>, grid, dim3(256), 0, s, w, (void *)wp, (int)O, (int)G,
-                     (int)K, Opad, Gpad, transposed, clear, zero, pm, split);
+                     (int)K, Opad, Gpad, transposed, clear, zero, pm, split, prep);
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }
@@ -2706,13 +2813,7 @@ int launch_pair_mask(const float *map, const float *iw, int *mask, const ModeArg
 
 // (defined with the map plans below)
 namespace {
-constexpr int kPlanSlots = 4;  // resolved entries per (location, tap) of a plan's gather part
 bool gather_plan_applies(int interp, int64_t P);
-template <int NCORN>
-__global__ void build_gather_plan_kernel(const float *__restrict__ map,
-                                         const float *__restrict__ iw, float2 *__restrict__ gmap,
-                                         int np, int weighted, int wrap, int SH, int SW, int K,
-                                         int64_t total);
 // bf16 images under single-point bilinear taps: a forward call without a plan resolves the
 // taps once into the same form before its product (a tenth of a millisecond where the product
 // kernel would spend four resolving them tile by tile)
@@ -2789,8 +2890,9 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
         room && split_applies(G, O, SH, SW, K, mode_args(kInterpNearest, kPlanSlots), true, cl)
             ? split_job(split_region, !cl, tiles)
             : SplitJob{};
-    if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s, nullptr, ZeroJob{nullptr, 0},
-                                         PairMaskJob{}, split))
+    if (int rc = launch_pack_weights<TD>(
+            w, wp, O, G, K, 0, s, nullptr, ZeroJob{nullptr, 0}, PairMaskJob{}, split,
+            PrepJobs<TD>{blocks_for(src, stage, B, G, SH, SW, kInterpNearest), GatherPlanJob{}}))
       return rc;
     return launch_gather_product<TD>(src, gmap, nullptr, wp, bias, y, stage, B, G, O, SH, SW, OH,
                                      OW, K, kPlanSlots, kInterpNearest, nullptr, 0, s, nullptr,
@@ -2806,18 +2908,21 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
   if (!plan && resolves_per_call(sizeof(TD), SH, interp, P, OH, OW, K)) {
     float2 *gmap = reinterpret_cast<float2 *>(
         (char *)stage + align256((size_t)(B * SH * SW * round_up(G, kGC)) * sizeof(float)));
-    if (int rc = launch_pack_weights<TD>(w, wp, O, G, K, 0, s, pair_mask)) return rc;
-    if (int rc = launch_pair_mask(map, iw, pair_mask, m, SH, SW, OH * OW * K, s, true)) return rc;
-    const int64_t total = OH * OW * K;
-    hipLaunchKernelGGL(build_gather_plan_kernel<4>,
-                       dim3((unsigned)(((OH * OW + 63) / 64 * 64 * K + 255) / 256)), dim3(256), 0,
-                       s, map, iw, gmap, m.np, m.weighted, m.wrap, (int)SH, (int)SW, (int)K,
-                       total);
-    MCX_HIP_CHECK_LAUNCH();
+    // one launch for the weights, the taps, the staged operand and, of a small map, the pair mask
+    const bool on_pack = OH * OW * K <= kSmallMapEntries;
+    const PairMaskJob job =
+        on_pack ? pair_mask_job(map, iw, pair_mask, m, SH, SW, OH * OW * K) : PairMaskJob{};
+    if (int rc = launch_pack_weights<TD>(
+            w, wp, O, G, K, 0, s, on_pack ? nullptr : pair_mask, ZeroJob{nullptr, 0}, job, SplitJob{},
+            PrepJobs<TD>{blocks_for(src, stage, B, G, SH, SW, kInterpNearest),
+                         gather_plan_job(map, iw, gmap, m, SH, SW, OH * OW, K)}))
+      return rc;
+    if (!on_pack)
+      if (int rc = launch_pair_mask(map, iw, pair_mask, m, SH, SW, OH * OW * K, s, true)) return rc;
     return launch_gather_product<TD>(src, reinterpret_cast<const float *>(gmap), nullptr, wp, bias,
                                      y, stage, B, G, O, SH, SW, OH, OW, K, kPlanSlots,
                                      kInterpNearest, nullptr, 0, s, nullptr, false, pair_mask,
-                                     true);
+                                     true, false, nullptr, on_pack ? job.blocks : 1);
   }
   const int *mask = pair_mask;
   // the pair mask of a small map is made by the last block of the packing launch
@@ -2830,7 +2935,7 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
           w, wp, O, G, K, 0, s, mask_on_pack ? nullptr : pair_mask, ZeroJob{nullptr, 0},
           mask_on_pack ? pair_mask_job(map, iw, pair_mask, m, SH, SW, OH * OW * K)
                        : PairMaskJob{},
-          split))
+          split, PrepJobs<TD>{blocks_for(src, stage, B, G, SH, SW, interp), GatherPlanJob{}}))
     return rc;
   if (four_pairs) {
     if (plan)  // flag word 4 of a plan built for this map
@@ -2953,7 +3058,12 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       pair_mask = state + 2;
     }
   }
-  if (two_variants && !by_runs) {
+  // (the pair mask of a small map under the ring kernel is made with the staged operand)
+  PairMaskJob mask_job{};
+  if (ring && !plan && MH * MW * K <= kSmallMapEntries)
+    mask_job = pair_mask_job(map, iw, pair_mask, m, GH, GW, MH * MW * K);
+  const int mask_words = mask_job.mask ? mask_job.blocks : 1;
+  if (two_variants && !by_runs && !mask_job.mask) {
     if (plan)  // flag word 4 of a plan built for this map (see mfma_scatter_plan_build)
       pair_mask = (int *)const_cast<void *>(plan) + GH * GW * K + 4;
     else if (int rc = launch_pair_mask(map, iw, pair_mask, m, GH, GW, MH * MW * K, s))
@@ -2989,7 +3099,11 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   if constexpr (sizeof(TD) == 2) {
     if (ring) {
       TD *stage = reinterpret_cast<TD *>((char *)pair_mask_ws + 256);
-      if (int rc = launch_channel_blocks<TD>(gath, stage, B, G, GH * GW, s)) return rc;
+      PrepJobs<TD> prep{};
+      prep.blocks = channel_blocks_job<TD>(gath, stage, B, G, GH * GW);
+      if (int rc = launch_pack_weights<TD>(nullptr, nullptr, 0, 0, 0, 0, s, nullptr,
+                                           ZeroJob{nullptr, 0}, mask_job, SplitJob{}, prep))
+        return rc;
       // the plain operand tile by tile, after the blocks of the gathered one
       bf16_t *tiles = reinterpret_cast<bf16_t *>(
           (char *)stage + align256((size_t)(B * GH * GW * Gpad) * sizeof(TD)));
@@ -3005,7 +3119,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
           (char *)tiles + align256((size_t)t.total * (size_t)round_up(A, 32) * kTilePx * sizeof(TD)));
       hipLaunchKernelGGL(resolve_tap_table_kernel, dim3((unsigned)t.tiles_per_img), dim3(256), 0, s,
                          map, ring_table, (int)GH, (int)GW, (int)MH, (int)MW, (int)K, m.wrap,
-                         t.tiles_x, t.tw_shift, pair_mask);
+                         t.tiles_x, t.tw_shift, pair_mask, mask_words);
       MCX_HIP_CHECK_LAUNCH();
     }
   }
@@ -3019,7 +3133,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
           dim3(kThreads), 0, s, reinterpret_cast<const TD *>(ring_tiles),
           reinterpret_cast<const TD *>((char *)pair_mask_ws + 256), ring_table, part, (int)A, (int)G,
           (int)Gpad, (int)GH, (int)GW, (int)K, t.tiles_per_img, (int)t.total, ranges, rg_groups,
-          rg_passes, plain_sum ? sum_part : (float *)nullptr, pair_mask);
+          rg_passes, plain_sum ? sum_part : (float *)nullptr, pair_mask, mask_words);
       MCX_HIP_CHECK_LAUNCH();
     }
   }
@@ -3055,7 +3169,6 @@ namespace {
 // cache lines (counters are [tap][pixel] like the slots); the taps of a run of pixels are
 // neighbouring waves, which read the same lines of the map.
 constexpr int kTransSlots = 4;
-constexpr int kTransSlotsConst = kTransSlots;
 
 // A contribution that finds its cell full goes to the overflow list (destination pixel,
 // source pixel, tap, weight), applied afterwards with atomics by overflow_scatter_kernel;
@@ -3296,41 +3409,6 @@ __global__ void convert_planes_kernel(const float *__restrict__ src, TD *__restr
     dst[i] = from_f32<TD>(src[i]);
 }
 
-// Gather part of a map plan: every (map location, tap) resolved once to four (element index of
-// the sampled image as bits, weight) entries - the four bilinear corners, or up to four
-// nearest points with the rest zero - in the layout the gather-product kernel reads with
-// `packed_map` (the same as a transposed map's cells).
-template <int NCORN>
-__global__ void build_gather_plan_kernel(const float *__restrict__ map,
-                                         const float *__restrict__ iw, float2 *__restrict__ gmap,
-                                         int np, int weighted, int wrap, int SH, int SW, int K,
-                                         int64_t total) {
-  // (a wave takes 64 consecutive locations of one tap: its stores are 512-byte runs)
-  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t run = t0 / (64 * (int64_t)K), pixels = total / K;
-  const int r = (int)(t0 - run * 64 * K);
-  const int64_t n = run * 64 + (r & 63);
-  const int k = r >> 6;
-  if (n >= pixels) return;
-  const int64_t e = n * K + k;  // (location, tap)
-  float2 out[kTransSlotsConst];
-#pragma unroll
-  for (int i = 0; i < kTransSlotsConst; i++) out[i] = make_float2(0.f, 0.f);
-  for (int sp = 0; sp < np; sp++) {
-    const int64_t q = e * np + sp;
-    PairTap<NCORN> t;
-    resolve_pairs<NCORN, 1>(map[q * 2], map[q * 2 + 1], SH, SW, wrap != 0,
-                            weighted ? iw[q] : 1.f, t);
-#pragma unroll
-    for (int i = 0; i < NCORN; i++)
-      if (sp * NCORN + i < kTransSlotsConst)
-        out[sp * NCORN + i] = make_float2(__builtin_bit_cast(float, t.off[i]), t.wt[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < kTransSlotsConst; i++)  // stored [tap][slot][location]
-    gmap[((int64_t)k * kTransSlotsConst + i) * pixels + n] = out[i];
-}
-
 // A map has a gather part when a tap is at most four (offset, weight) pairs.
 static_assert(kPlanSlots == kTransSlots, "a plan's gather part has the cells of a transposed map");
 bool gather_plan_applies(int interp, int64_t P) {
@@ -3467,15 +3545,11 @@ int mfma_scatter_plan_build(const float *map, const float *iw, void *plan, int64
     if (int rc = launch_pair_mask(map, iw, flag + 4, m, DH, DW, MH * MW * K, s, true)) return rc;
   if (gather_plan_applies(interp, P) && MH * MW * K * kTransSlots * 2 <= 0x7fffffffLL) {
     float2 *gmap = (float2 *)((char *)plan + mfma_gather_plan_offset(DH, DW, MH, MW, K, P));
-    const int64_t total = MH * MW * K;
-    const dim3 grid((unsigned)(((MH * MW + 63) / 64 * 64 * K + 255) / 256));
-    if (m.mode == kInterpNearest)
-      hipLaunchKernelGGL(build_gather_plan_kernel<1>, grid, dim3(256), 0, s, map, iw, gmap, m.np,
-                         m.weighted, m.wrap, (int)DH, (int)DW, (int)K, total);
-    else
-      hipLaunchKernelGGL(build_gather_plan_kernel<4>, grid, dim3(256), 0, s, map, iw, gmap, m.np,
-                         m.weighted, m.wrap, (int)DH, (int)DW, (int)K, total);
-    MCX_HIP_CHECK_LAUNCH();
+    PrepJobs<float> prep{};
+    prep.plan = gather_plan_job(map, iw, gmap, m, DH, DW, MH * MW, K);
+    if (int rc = launch_pack_weights<float>(nullptr, nullptr, 0, 0, 0, 0, s, nullptr,
+                                            ZeroJob{nullptr, 0}, PairMaskJob{}, SplitJob{}, prep))
+      return rc;
   }
   return 0;
 }
@@ -3531,7 +3605,8 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
             w, wpt, D, S, K, 1, s, nullptr,
             plan ? ZeroJob{nullptr, 0}
                  : ZeroJob{reinterpret_cast<uint4 *>(cnt), (int64_t)((sc.ovf - sc.cnt) / 16)},
-            PairMaskJob{}, split))
+            PairMaskJob{}, split,
+            PrepJobs<TD>{blocks_for(src, stage, B, S, MH, MW, kInterpNearest), GatherPlanJob{}}))
       return rc;
     if (!plan)
       if (int rc = build_transposed_map(sc, map, iw, cnt, m, DH, DW, MH, MW, K, s, true))
