@@ -23,7 +23,8 @@ import sys
 ROOT = os.path.dirname(os.path.abspath(__file__))
 # The headline's kernels and what they include
 KERNEL_SOURCES = ["mappedconvolutions_amd/csrc/" + name for name in
-                  ("mcx_conv_mfma.hip", "mcx_conv_split.h", "mcx_taps.h", "mcx_device.h")]
+                  ("mcx_conv_mfma.hip", "mcx_conv_split.h", "mcx_conv_runs.hip", "mcx_conv_runs.h",
+                   "mcx_mfma_common.h", "mcx_taps.h", "mcx_device.h")]
 COPY_BYTES = 8 * 64 * 256 * 512 * 4  # one calibration dispatch reads and writes the input once
 
 
@@ -64,7 +65,7 @@ def per_kernel(folder, counter):
 
 def label_of(kernel):
     """The timed C-ABI calls whose work this kernel does (none: a helper kernel)."""
-    if kernel.startswith("weight_grad_mfma_kernel<"):
+    if kernel.startswith(("weight_grad_runs_kernel<", "weight_grad_mfma_kernel<")):
         return ["conv_backward_weight"]
     if kernel.startswith("gather_product_split_kernel<"):
         return ["conv_forward", "conv_backward_input"]  # (one kernel: the average of both calls)

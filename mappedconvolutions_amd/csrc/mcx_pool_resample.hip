@@ -1442,9 +1442,8 @@ int build_transposed(const void *map, const void *iw, void *ws, size_t ws_bytes,
   uint32_t *local = (uint32_t *)(base + l.local), *cursor = (uint32_t *)(base + l.cursor);
   uint32_t *bsum = (uint32_t *)(base + l.bsum), *e_src = (uint32_t *)(base + l.e_src);
   T *e_wt = (T *)(base + l.e_wt);
-  int rc = fill<uint32_t>(local, ndst + 1, 0u, s);
-  if (rc) return rc;
-  if ((rc = fill<uint32_t>(cursor, ndst, 0u, s))) return rc;
+  // (counters and cursors lie next to each other: one launch clears both)
+  if (int rc = fill<uint32_t>(local, (int64_t)((l.cursor - l.local) / 4) + ndst, 0u, s)) return rc;
   const int per_code = (int)(max_codes ? pm : pm * K);
   const dim3 sgrid(div_up(nsrc, kThreads)), blk(kThreads);
   MCX_DISPATCH_MODE(interp, hipLaunchKernelGGL((transposed_map_kernel<T, MODE, false>), sgrid, blk,
