@@ -242,49 +242,46 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
   const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)blocks * blockDim.x;
   const int64_t total = (int64_t)K * Gpad * Opad;
-  if constexpr (sizeof(TD) == 2) {
-    uint16_t *wb = reinterpret_cast<uint16_t *>(packed_out);
-    const int chunks = Gpad / kGC;
-    for (int64_t e = first; e < total; e += stride) {
-      const int j = (int)(e & 7);
-      const int o = (int)((e >> 3) % Opad);
-      const int kg = (int)((e / ((int64_t)8 * Opad)) & 1);
-      const int c = (int)((e / ((int64_t)16 * Opad)) % chunks);
-      const int k = (int)(e / ((int64_t)16 * Opad * chunks));
-      const int g = c * kGC + kg * 8 + j;
-      const int64_t wi = transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k;
-      wb[e] = (o < O && g < G) ? from_f32<bf16_t>(to_f32(w[wi])).v : (uint16_t)0;
-    }
-  } else {
-    float *wp = reinterpret_cast<float *>(packed_out);
-    for (int64_t e = first; e < total; e += stride) {
-      const int o = (int)(e % Opad);
-      const int g = (int)((e / Opad) % Gpad);
-      const int k = (int)(e / ((int64_t)Opad * Gpad));
-      const int64_t wi = transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k;
-      wp[e] = (o < O && g < G) ? to_f32(w[wi]) : 0.f;
-    }
-    // the same in three bf16 parts, [k][chunk][part][kg][o][8 channels] (mcx_conv_split.h)
-    if (split.w) {
-      const int chunks = Gpad / kGC;
-      for (int64_t e = first; e < total; e += stride) {
-        const int o = (int)((e >> 3) % Opad);
-        const int64_t u = (e >> 3) / Opad;  // (tap, chunk, half)
-        const int kg = (int)(u & 1), c = (int)((u >> 1) % chunks), k = (int)((u >> 1) / chunks);
-        const int g = split_channel(c, kg, (int)(e & 7), G, split.planar);
-        float x = 0.f;
-        if (o < O && g >= 0)
-          x = to_f32(w[transposed ? ((int64_t)g * O + o) * K + k : ((int64_t)o * G + g) * K + k]) *
-              kSplitScale;
+  // (indices of 32 bits wherever they suffice: a weight is four to six divisions, and those of 64
+  // bits made this launch of 16 -> 32 weights of nine taps 5.5 us, these 4.8)
+  auto weight = [&](int64_t o, int64_t g, int64_t k) {
+    return to_f32(w[transposed ? (g * O + o) * K + k : (o * G + g) * K + k]);
+  };
+  auto pack = [&](auto index) __attribute__((always_inline)) {
+    using I = decltype(index);
+    const I o_pad = (I)Opad, g_pad = (I)Gpad, chunks = (I)(Gpad / kGC);
+    for (I e = (I)first; e < (I)total; e += (I)stride) {
+      if constexpr (sizeof(TD) == 2) {
+        const I j = e & 7, u = (e >> 3) / o_pad, o = (e >> 3) - u * o_pad;
+        const I c = (u >> 1) % chunks, k = (u >> 1) / chunks, g = c * kGC + (u & 1) * 8 + j;
+        reinterpret_cast<uint16_t *>(packed_out)[e] =
+            (o < (I)O && g < (I)G) ? from_f32<bf16_t>(weight(o, g, k)).v : (uint16_t)0;
+      } else {
+        const I q = e / o_pad, o = e - q * o_pad, k = q / g_pad, g = q - k * g_pad;
+        reinterpret_cast<float *>(packed_out)[e] =
+            (o < (I)O && g < (I)G) ? weight(o, g, k) : 0.f;
+        // the same in three bf16 parts, [k][chunk][part][kg][o][8 channels] (mcx_conv_split.h)
+        if (split.w) {
+          const I u = (e >> 3) / o_pad, so = (e >> 3) - u * o_pad;  // (tap, chunk, half), output
+          const int kg = (int)(u & 1), sc = (int)((u >> 1) % chunks);
+          const I sk = (u >> 1) / chunks;
+          const int sg = split_channel(sc, kg, (int)(e & 7), G, split.planar);
+          float x = 0.f;
+          if (so < (I)O && sg >= 0) x = weight(so, sg, sk) * kSplitScale;
 #pragma unroll
-        for (int part = 0; part < 3; part++) {
-          const uint16_t q = from_f32<bf16_t>(x).v;
-          split.w[((((u >> 1) * 3 + part) * 2 + kg) * Opad + o) * 8 + (e & 7)] = q;
-          x -= __builtin_bit_cast(float, (uint32_t)q << 16);
+          for (int part = 0; part < 3; part++) {
+            const uint16_t h = from_f32<bf16_t>(x).v;
+            split.w[((((int64_t)(u >> 1) * 3 + part) * 2 + kg) * Opad + so) * 8 + (e & 7)] = h;
+            x -= __builtin_bit_cast(float, (uint32_t)h << 16);
+          }
         }
       }
     }
-  }
+  };
+  if (total + stride < 0x7fffffffLL)
+    pack(0u);
+  else
+    pack((int64_t)0);
   for (int64_t i = first; i < zero.count; i += stride) zero.ptr[i] = make_uint4(0u, 0u, 0u, 0u);
   for (int64_t i = first; i < split.tiles; i += stride) split.nonfinite[i] = 0;
 }
@@ -2784,8 +2781,8 @@ int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K,
 
 inline PairMaskJob pair_mask_job(const float *map, const float *iw, int *mask, const ModeArgs &m,
                                  int64_t GH, int64_t GW, int64_t samples) {
-  // (a block of 256 threads per 2048 entries, 64 at most: the readers load a word per lane)
-  const int blocks = (int)std::min<int64_t>(64, (samples + 2047) / 2048);
+  // (a block of 256 threads per 1024 entries, 64 at most: the readers load a word per lane)
+  const int blocks = (int)std::min<int64_t>(64, (samples + 1023) / 1024);
   return PairMaskJob{map, iw, mask, blocks, m.np, m.weighted, m.wrap, (int)GH, (int)GW,
                      m.mode == kInterpNearest ? 1 : 4, samples};
 }
