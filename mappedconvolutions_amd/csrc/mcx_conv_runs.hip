@@ -83,12 +83,13 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
   auto of_group = [&](bool x) {
     return (unsigned)(__builtin_amdgcn_ballot_w64(x) >> first) & 0xffu;
   };
-  for (int t = blockIdx.x * 256 + threadIdx.x; t < ((total + 63) & ~63); t += gridDim.x * 256) {
-    const int e = t & 7, q = min(t, total - 1) >> 3;
+  // One pixel of a (group, tap) q; returns whether the group is no run (the same in its eight
+  // lanes).  `write`: into the tables.
+  auto examine = [&](int q, int e, bool exists, bool write) __attribute__((always_inline)) {
     const int g = q / K, k = q - g * K;
     const GroupPlace at_px = group_place(g, MH, gpr);
     const int row = at_px.row, j = at_px.col + e;
-    const bool live = t < total && j < MW;
+    const bool live = exists && j < MW;
     const int64_t s = ((int64_t)row * MW + min(j, MW - 1)) * K + k;
     const float2 xy = reinterpret_cast<const float2 *>(map)[s];
     const float scale = live ? (weighted ? iw[s] * kSplitScale : kSplitScale) : 0.f;
@@ -125,10 +126,10 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
         const int i = ST * e + c;
         fits = fits && (w[c] == 0.f || o[c] == run[r] + i + (i >= at[r] ? jump[r] : 0));
       }
-      if (t < total) wts[(int64_t)(q * 2 + r) * 8 + e] = make_float2(w[0], w[1]);
+      if (exists && write) wts[(int64_t)(q * 2 + r) * 8 + e] = make_float2(w[0], w[1]);
       if (r == 1) lower |= any[1];
     }
-    if (NCORN == 1 && t < total) wts[(int64_t)(q * 2 + 1) * 8 + e] = make_float2(0.f, 0.f);
+    if (NCORN == 1 && exists && write) wts[(int64_t)(q * 2 + 1) * 8 + e] = make_float2(0.f, 0.f);
     // both rows break at the same element, or one of them is not in use
     if (!any[0]) at[0] = at[1], jump[0] = jump[1];
     const bool same = !any[1] || (at[1] == at[0] && jump[1] == jump[0]);
@@ -136,20 +137,32 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
     bool inside = at[0] == kNowhere;
 #pragma unroll
     for (int r = 0; r < 2; r++) inside = inside && run[r] >= 0 && run[r] + 7 * ST + 1 < GH * GW;
-    if (no_run && t < total) {
+    if (no_run && exists && write) {
 #pragma unroll
       for (int r = 0; r < 2; r++)
         offs[(int64_t)(q * 2 + r) * 8 + e] =
             NCORN == 4 ? make_uint2(tap.off[2 * r % NCORN] * 4u, tap.off[(2 * r + 1) % NCORN] * 4u)
                        : make_uint2(tap.off[0] * 4u, tap.off[0] * 4u);
     }
-    if (e == 0 && t < total) {
+    if (e == 0 && exists && write) {
       RunDesc d{run[0] * 4, run[1] * 4, jump[0] * 4, inside ? 0 : at[0] * 4 + kElements};
       if (no_run) d = RunDesc{0, 0, 0, kNowhere * 4 + kCorners};
       desc[q] = d;
-      no_runs += no_run ? 1 : 0;
     }
+    return no_run;
+  };
+  // Maps without runs (a shuffled one) are not worth tables: where more than half of 32 groups spread
+  // over the map, the same for every block, are none, only the lower row's corners are looked for
+  // (500x1000 shuffled, 10 -> 1 channels: with tables 2220 us for the call, 2121 so, 2092 without a look).
+  const int e = threadIdx.x & 7;
+  const int sample = (int)(((uint64_t)((threadIdx.x >> 3) * 2654435769u) * (uint64_t)(total >> 3)) >> 32);
+  const bool tables = __syncthreads_count(examine(sample, e, true, false)) * 2 <= 256;
+  for (int t = blockIdx.x * 256 + threadIdx.x; t < ((total + 63) & ~63); t += gridDim.x * 256) {
+    const bool exists = t < total;
+    const bool no_run = examine(min(t, total - 1) >> 3, e, exists, tables);
+    no_runs += no_run && exists && e == 0 ? 1 : 0;
   }
+  if (!tables) no_runs = threadIdx.x == 0 ? total / 8 / (int)gridDim.x + 1 : 0;
   if (no_runs) atomicAdd(&count[0], no_runs);
   if (lower) count[1] = 1;
   __syncthreads();
