@@ -3312,9 +3312,33 @@ __global__ __launch_bounds__(64) void overflow_scatter_kernel(
 #pragma unroll
       for (int u = 0; u < U; u++)
 #pragma unroll
+        for (int i = 0; i < IB; i++) acc[u][i] = live[u] ? en[u].wt * acc[u][i] : 0.f;
+      // Additions to one address are served one after the other, and the list of an incoherent map
+      // is mostly one corner pixel, which holds every tap outside the image: what a wave has for
+      // one pixel is added up first.  fp32 backward, 10 -> 1 channels, bilinear map of 500 x 1000
+      // in random order: 4521 us without, 4220 with this.
+      bool same = true;
+#pragma unroll
+      for (int u = 0; u < U; u++) same = same && en[u].p == en[0].p;
+      const int p0 = __builtin_amdgcn_readfirstlane(en[0].p);
+      if (__builtin_amdgcn_ballot_w64(!same || en[0].p != p0) == 0) {
+#pragma unroll
+        for (int i = 0; i < IB; i++) {
+          float v = acc[0][i];
+#pragma unroll
+          for (int u = 1; u < U; u++) v += acc[u][i];
+          for (int m = lanes; m < 64; m <<= 1) v += __shfl_xor(v, m);
+          if (sub == 0 && b0 + i < B && d0 + dl < D)
+            atomic_add(accum + ((int64_t)(b0 + i) * DN + p0) * Dpad + d, v);
+        }
+        continue;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
         for (int i = 0; i < IB; i++)
           if (live[u] && b0 + i < B && d0 + dl < D)
-            atomic_add(accum + ((int64_t)(b0 + i) * DN + en[u].p) * Dpad + d, en[u].wt * acc[u][i]);
+            atomic_add(accum + ((int64_t)(b0 + i) * DN + en[u].p) * Dpad + d, acc[u][i]);
     }
   }
 }

@@ -14,15 +14,18 @@ pytestmark = pytest.mark.gpu
 # (ci is the gradient's channel count; 128 x 64 weights of a tap: images share their reading)
 @pytest.mark.parametrize("B", [1, 2, 5])
 @pytest.mark.parametrize("ci,co", [(3, 5), (16, 20), (17, 8), (33, 64), (64, 128), (65, 40)])
+# (one pixel: what a wave holds for it is added up before the atomics)
+@pytest.mark.parametrize("pixels", [1, 6])
 @pytest.mark.parametrize("share", [0.1, 0.4, 1.0])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_many_contributions_to_few_pixels(B, ci, co, share, dtype, device):
+def test_many_contributions_to_few_pixels(B, ci, co, pixels, share, dtype, device):
     g = torch.Generator().manual_seed(ci + co)
     h, w_, k = 12, 20, 3
     y, x = torch.meshgrid(torch.arange(h).float(), torch.arange(w_).float(), indexing="ij")
     smap = torch.stack((x, y), -1).unsqueeze(2).repeat(1, 1, k, 1)
-    crowd = torch.rand(h, w_, k, 1, generator=g) < share  # (these meet in six pixels)
-    smap = torch.where(crowd, torch.rand(h, w_, k, 2, generator=g) * torch.tensor([2.0, 1.0]) + 3, smap)
+    crowd = torch.rand(h, w_, k, 1, generator=g) < share  # (these meet in one pixel or in six)
+    to = torch.rand(h, w_, k, 2, generator=g) * torch.tensor([2.0, 1.0]) * (pixels > 1) + 3
+    smap = torch.where(crowd, to, smap)
     smap = smap.contiguous()
     rnd = lambda *s: torch.randn(s, generator=g).to(dtype).float()
     xs, wt, b, gy = rnd(B, ci, h, w_), rnd(co, ci, k), rnd(co), rnd(B, co, h, w_)
