@@ -1697,10 +1697,12 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(
 // offsets in a channel block, then NA words of weights as bf16 in their low halves].  Every
 // workgroup of a pixel range (channel groups x tap passes) would otherwise resolve the same
 // taps from the map again, about sixty instructions per tap, which is as much as its products
-// need.  Pixels outside the image weigh zero.  One workgroup per tile: its threads walk the
-// taps of their pixel two apart, so the tile's piece of the map stays in cache.
+// need.  Pixels outside the image weigh zero.  iw (may be NULL): a weight per tap.  One workgroup
+// per tile: its threads walk the taps of their pixel two apart, so the tile's piece of the map
+// stays in cache.
 template <int NA>
 __device__ inline void resolve_tap_table(const float *__restrict__ map,
+                                         const float *__restrict__ iw,
                                          unsigned *__restrict__ table, int GH, int GW, int MH,
                                          int MW, int K, int wrap, int tiles_x, int tw_shift) {
   const int tile = blockIdx.x, p = threadIdx.x & (kTilePx - 1);
@@ -1719,7 +1721,8 @@ __device__ inline void resolve_tap_table(const float *__restrict__ map,
   for (int k = threadIdx.x >> 7; k < K; k += 2) {
     const float2 xy = entry[k];
     PairTap<4> t;
-    resolve_pairs<4, 16>(xy.x, xy.y, GH, GW, wrap != 0, live ? 1.f : 0.f, t);
+    const float scale = live ? (iw ? iw[n_g * K + k] : 1.f) : 0.f;
+    resolve_pairs<4, 16>(xy.x, xy.y, GH, GW, wrap != 0, scale, t);
     uint4 *e = out + (int64_t)k * kTilePx * (NA / 2);
     if constexpr (NA == 2) {
       e[0] = make_uint4(t.off[0], t.off[1], wbits(t.wt[0]), wbits(t.wt[1]));
@@ -1730,12 +1733,13 @@ __device__ inline void resolve_tap_table(const float *__restrict__ map,
   }
 }
 __global__ __launch_bounds__(256) void resolve_tap_table_kernel(
-    const float *__restrict__ map, unsigned *__restrict__ table, int GH, int GW, int MH, int MW,
-    int K, int wrap, int tiles_x, int tw_shift, const int *__restrict__ pair_mask, int mask_words) {
+    const float *__restrict__ map, const float *__restrict__ iw, unsigned *__restrict__ table,
+    int GH, int GW, int MH, int MW, int K, int wrap, int tiles_x, int tw_shift,
+    const int *__restrict__ pair_mask, int mask_words) {
   if (!later_pairs_in_use(pair_mask, mask_words))
-    resolve_tap_table<2>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
+    resolve_tap_table<2>(map, iw, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
   else
-    resolve_tap_table<4>(map, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
+    resolve_tap_table<4>(map, iw, table, GH, GW, MH, MW, K, wrap, tiles_x, tw_shift);
 }
 
 constexpr int kRgKT = 5;      // taps per pass
@@ -3004,9 +3008,9 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   const int64_t Gpad = round_up(G, kGC);
   const bool cl = use_channel_last(GH, interp) &&
                   GH * GW * Gpad * (int64_t)sizeof(TD) <= 0xffffffffLL;
-  // bf16 images under unweighted bilinear taps: the ring kernel, in its two-pair form for maps
+  // bf16 images under bilinear taps of one point: the ring kernel, in its two-pair form for maps
   // whose lower corners weigh nothing and its four-pair form for the others (the pair mask
-  // lets one of the two launches run)
+  // says which)
   // (its 16-byte pieces of the plain operand want rows that are a multiple of 8 pixels, and
   // an image of either operand is addressed as a buffer of less than 4 GiB)
   const bool ring = sizeof(TD) == 2 && !cl && GH > 1 && m.np == 1 && m.mode != kInterpNearest &&
@@ -3115,8 +3119,8 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       ring_table = reinterpret_cast<unsigned *>(
           (char *)tiles + align256((size_t)t.total * (size_t)round_up(A, 32) * kTilePx * sizeof(TD)));
       hipLaunchKernelGGL(resolve_tap_table_kernel, dim3((unsigned)t.tiles_per_img), dim3(256), 0, s,
-                         map, ring_table, (int)GH, (int)GW, (int)MH, (int)MW, (int)K, m.wrap,
-                         t.tiles_x, t.tw_shift, pair_mask, mask_words);
+                         map, m.weighted ? iw : nullptr, ring_table, (int)GH, (int)GW, (int)MH,
+                         (int)MW, (int)K, m.wrap, t.tiles_x, t.tw_shift, pair_mask, mask_words);
       MCX_HIP_CHECK_LAUNCH();
     }
   }

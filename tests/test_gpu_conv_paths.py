@@ -317,6 +317,34 @@ def test_bf16_transposed_conv_under_a_map_with_integral_rows(with_plan, interp, 
     assert_close_elementwise(gr[1].float(), g_o[1], 2e-2, "grad_weight")
 
 
+@pytest.mark.parametrize("op", ["conv", "tconv"])
+@pytest.mark.parametrize("interp", [1, 2])
+@pytest.mark.parametrize("row_shift", [0.0, 0.37])
+@pytest.mark.parametrize("with_plan", [False, True])
+def test_bf16_one_weighted_point_per_tap(op, interp, row_shift, with_plan, device):
+    """bf16 storage, one weighted point per tap, image rows a multiple of 8 pixels: the weight
+    gradient's kernel over staged operands takes the interpolation weights into its tap table, in
+    the two-pair form (integral rows) and in the four-pair one."""
+    B, Ci, Co, H, W, K = 2, 20, 36, 12, 136, 9
+    g = torch.Generator().manual_seed(77)
+    bf = lambda t: t.to(torch.bfloat16)
+    x, gy = bf(torch.randn(B, Ci, H, W, generator=g)), bf(torch.randn(B, Co, H, W, generator=g))
+    w = bf(torch.randn(*((Co, Ci) if op == "conv" else (Ci, Co)), K, generator=g) / (Ci * K) ** 0.5)
+    b = bf(torch.randn(Co, generator=g))
+    smap = synthetic.latitude_map(H, W, 1)
+    smap[..., 1] = (smap[..., 1] + row_shift).clamp(0, H - 1)
+    smap = smap.unsqueeze(3).contiguous()
+    iw = 4 * torch.rand(H, W, K, 1, generator=g) - 2
+    name = "weighted_mapped_%s_backward" % ("conv" if op == "conv" else "transposed_conv")
+    g_o = getattr(O, name)(gy.float(), smap, iw, x.float(), w.float(), b.float(), K, interp)
+    xd, sd, iwd, wd_, bd, gyd = dev(x, smap, iw, w, b, gy)
+    plan = _C.conv_map_plan(sd, iwd, H, W, interp, torch.bfloat16) if with_plan else None
+    gr = getattr(_C, name)(gyd, sd, iwd, xd, wd_, bd, K, interp, plan=plan)
+    for a, r, nm in zip(gr, g_o, ("grad_input", "grad_weight", "grad_bias")):
+        assert rel_err(a.float(), r) < 2e-2, nm
+    assert_close_elementwise(gr[1].float(), g_o[1], 2e-2, "grad_weight")
+
+
 @pytest.mark.parametrize("interp", [1, 2])
 @pytest.mark.parametrize("radius", [1, 2])
 def test_bf16_backward_under_a_map_with_fractional_rows(radius, interp, device):
