@@ -116,9 +116,11 @@ struct ChannelBlocksJob {
   int64_t plane;
   int per_plane;   // workgroups a block of channels
   int64_t count;   // workgroups
+  int first;       // of them, those of earlier launches
 };
 template <typename TD>
 __device__ inline void to_channel_blocks(const ChannelBlocksJob<TD> &a, int block) {
+  block += a.first;
   const int64_t n = (int64_t)(block % a.per_plane) * 256 + threadIdx.x;
   const int g8 = block / a.per_plane % a.groups, b = block / a.per_plane / a.groups;
   if (n >= a.plane) return;
@@ -2502,7 +2504,7 @@ ChannelBlocksJob<TD> channel_blocks_job(const TD *src, TD *stage, int64_t B, int
                                         int64_t plane) {
   const int64_t groups = round_up(G, kGC) / 8, per_plane = (plane + 255) / 256;
   return ChannelBlocksJob<TD>{src, stage, (int)G, (int)groups, plane, (int)per_plane,
-                              per_plane * groups * B};
+                              per_plane * groups * B, 0};
 }
 GatherPlanJob gather_plan_job(const float *map, const float *iw, float2 *gmap, const ModeArgs &m,
                               int64_t SH, int64_t SW, int64_t MN, int64_t K) {
@@ -2753,23 +2755,21 @@ int launch_pack_weights(const TD *w, float *wp, int64_t O, int64_t G, int64_t K,
                         PrepJobs<TD> prep = PrepJobs<TD>{}) {
   const int Opad = (int)round_up(O, kOT), Gpad = (int)round_up(G, kGC);
   const int64_t packed = (int64_t)K * Gpad * Opad;
-  // (a launch has at most 2^32 threads: beyond a quarter of them, image by image)
-  if (prep.blocks.x && prep.blocks.count > ((int64_t)1 << 22)) {
-    const int64_t image = (int64_t)prep.blocks.per_plane * prep.blocks.groups;
-    const int64_t images = prep.blocks.count / image;
-    if (image > ((int64_t)1 << 22)) return MCX_E_SHAPE;
-    for (int64_t b = 0; b < images; b++) {
-      PrepJobs<TD> one{};
-      one.blocks = prep.blocks;
-      one.blocks.x += b * prep.blocks.G * prep.blocks.plane;
-      one.blocks.xt += b * prep.blocks.groups * 8 * prep.blocks.plane;
-      one.blocks.count = image;
-      hipLaunchKernelGGL(pack_weights_kernel<TD>, dim3((unsigned)image), dim3(256), 0, s, w,
+  // (a launch has at most 2^32 threads: what is beyond a quarter of them goes into launches of its own)
+  constexpr int64_t kMostBlocks = (int64_t)1 << 22;
+  if (prep.blocks.x) {
+    if (prep.blocks.count > 0x7fffffffLL) return MCX_E_SHAPE;
+    const int64_t end = prep.blocks.count;
+    for (; end - prep.blocks.first > kMostBlocks; prep.blocks.first += (int)kMostBlocks) {
+      PrepJobs<TD> piece{};
+      piece.blocks = prep.blocks;
+      piece.blocks.count = kMostBlocks;
+      hipLaunchKernelGGL(pack_weights_kernel<TD>, dim3((unsigned)kMostBlocks), dim3(256), 0, s, w,
                          (void *)wp, 0, 0, 0, 0, 0, 0, (int *)nullptr, ZeroJob{nullptr, 0},
-                         PairMaskJob{}, SplitJob{}, one);
+                         PairMaskJob{}, SplitJob{}, piece);
       MCX_HIP_CHECK_LAUNCH();
     }
-    prep.blocks = ChannelBlocksJob<TD>{};
+    prep.blocks.count = end - prep.blocks.first;
   }
   // (bf16 storage: the bf16 MFMA operand layout in the same scratch, half the bytes)
   const int64_t work = std::max({packed, zero.count * 4, split.tiles});

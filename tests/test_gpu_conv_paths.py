@@ -345,6 +345,27 @@ def test_bf16_one_weighted_point_per_tap(op, interp, row_shift, with_plan, devic
     assert_close_elementwise(gr[1].float(), g_o[1], 2e-2, "grad_weight")
 
 
+@pytest.mark.parametrize("with_plan", [False, True])
+def test_bf16_staging_in_several_launches(with_plan, device):
+    """bf16 images are staged in blocks of eight channels, at most 2^22 workgroups a launch: 65 535
+    images of 2x8 pixels and 520 channels are 66 blocks each, more than one launch holds.  One tap
+    that names the pixel itself, so that the results are plain matrix products."""
+    B, Ci, Co, H, W = 65535, 520, 8, 2, 8
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda", dtype=torch.bfloat16)
+    x, gy, w, b = rnd(B, Ci, H, W), rnd(B, Co, H, W), rnd(Co, Ci, 1), rnd(Co)
+    ys, xs = torch.meshgrid(torch.arange(H).float(), torch.arange(W).float(), indexing="ij")
+    smap = torch.stack((xs, ys), -1).unsqueeze(2).contiguous().cuda()
+    plan = _C.conv_map_plan(smap, None, H, W, 1, torch.bfloat16) if with_plan else None
+    y = _C.mapped_conv_forward(x, smap, w, b, 1, 1, plan=plan)
+    gw = _C.mapped_conv_backward(gy, smap, x, w, b, 1, 1, plan=plan, needs=(False, True, False))[1]
+    xf = x.transpose(0, 1).reshape(Ci, -1).float()
+    want_y = w[..., 0].float() @ xf + b.float()[:, None]
+    want_gw = gy.transpose(0, 1).reshape(Co, -1).float() @ xf.t()
+    assert rel_err(y.transpose(0, 1).reshape(Co, -1).float(), want_y) < 2e-2
+    assert rel_err(gw[..., 0].float(), want_gw) < 2e-2
+
+
 @pytest.mark.parametrize("interp", [1, 2])
 @pytest.mark.parametrize("radius", [1, 2])
 def test_bf16_backward_under_a_map_with_fractional_rows(radius, interp, device):
