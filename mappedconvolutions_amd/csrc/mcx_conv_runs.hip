@@ -25,9 +25,21 @@
 // per SIMD do not quite cover.  A wave of 32 plain channels (half the LDS reads) needs 250 registers,
 // and at two waves per SIMD everything is waited for: 820 us where this takes 735.
 // Measured in one run each, fp32 instructions -> this: 8 x 64 -> 64 channels of 256 x 512, nine taps:
-// 880 -> 735 us; 3 x 24 -> 40 of 125 x 250, fractional rows, 71 -> 49; transposed 4 x 64 -> 32 from
-// 128 x 256 onto twice that (taps two pixels apart) 105 -> 71.  Distance from the 64-bit result, in
-// 2-norm: 9.7e-7 -> 2.4e-7, 3.2e-7 -> 2.9e-7 and 3.7e-7 -> 2.5e-7.
+// 793 -> 667 us; 3 x 24 -> 40 of 125 x 250, fractional rows, 100 -> 66; transposed 4 x 64 -> 32 from
+// 128 x 256 onto twice that (taps two pixels apart) 105 -> 71.
+// Accuracy: the instruction rounds its sums downwards, so that 24 of them a tile lose up to 24 units
+// of the last place, all one way.  The products of the leading parts, 16 bits each, are summed in an
+// accumulator of their own, which rounds next to nothing; what the other five lose is 2^-8 of that;
+// and the sign of every other tile is turned.  Distance from 64 bits in 2-norm, in units of 1e-7, fp32
+// instructions / one accumulator / this, 16 -> 64 channels, nine taps:
+//   pixels     operands normal       positive             behind a ReLU
+//   128        1.49 / 1.55 / 0.70    0.93 / 1.25 / 0.67   0.61 / 1.11 / 0.52
+//   256        1.53 / 1.60 / 0.72    0.71 / 0.93 / 0.58   0.55 / 0.88 / 0.48
+//   2 048      2.14 / 1.67 / 0.90    0.60 / 0.52 / 0.45   0.51 / 0.53 / 0.46
+//   131 072    3.73 / 2.87 / 2.57    1.14 / 1.14 / 1.13   1.13 / 1.13 / 1.13
+//   1 048 576  7.21 / 3.02 / 2.71    1.15 / 1.13 / 1.13   1.11 / 1.13 / 1.13
+// (2 to 64 pixels 0.3 to 0.7 against 0.3 to 1.5; two of a hundred values not zero 0.33 to 2.6 against
+// 0.32 to 2.7.)
 #include "mcx_conv.h"
 #include "mcx_conv_runs.h"
 #include "mcx_mfma_common.h"
@@ -243,8 +255,8 @@ __device__ inline void weight_grad_runs(const RunArgs &s, RunLds &lds) {
     const bool plain_tile =
         live == kTileGroups && (strip + 1) * kStrip <= gpr && in + kTileGroups <= strip_groups;
     const auto img = plane_buf(s.gath + (int64_t)b * s.G * (plane >> 2), (unsigned)s.G * plane);
-    // The matrix instruction rounds its sums downwards: every other tile is multiplied with its
-    // sign turned and subtracted, so that what the sums lose does not add up.
+    // (every other tile is multiplied with its sign turned and subtracted, so that what the sums
+    // lose does not add up)
     const float sign = (tile & 1) ? -1.f : 1.f;
     int t0 = tid;  // (opaque: nothing of the preparation is kept in registers through the products)
     asm volatile("" : "+v"(t0));
@@ -424,18 +436,20 @@ __device__ inline void weight_grad_runs(const RunArgs &s, RunLds &lds) {
                 __builtin_bit_cast(bf16x8, lds.samples[buf][part][q * 64 + read_at]);
         };
         samples(0);
-        floatx4 p = floatx4{0.f, 0.f, 0.f, 0.f};
-        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+        // (the leading parts' products apart from the others: see the head of the file)
+        floatx4 p = floatx4{0.f, 0.f, 0.f, 0.f}, low = p;
+        constexpr int pa[5] = {2, 0, 1, 1, 0}, pb[5] = {0, 2, 1, 0, 1};
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           if (q < 3) samples(q + 1);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int i = 0; i < 6; i++)  // (smallest first)
-            p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][pa[i]], bq[q & 1][pb[i]], p, 0, 0, 0);
+          for (int i = 0; i < 5; i++)  // (smallest first)
+            low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][pa[i]], bq[q & 1][pb[i]], low, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][0], bq[q & 1][0], p, 0, 0, 0);
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[k][i] = __builtin_fmaf(sign, p[i], acc[k][i]);
+        for (int i = 0; i < 4; i++) acc[k][i] = __builtin_fmaf(sign, p[i] + low[i], acc[k][i]);
       }
     }
     first += kTileGroups;

@@ -122,10 +122,10 @@ def test_operands_of_every_magnitude_count_in_full(p, q, device):
     assert ((got - want).norm() / want.norm()).item() < 1e-6
 
 
-@pytest.mark.parametrize("B,h,w", [(1, 64, 128), (4, 128, 256)])
-def test_what_the_sums_lose_does_not_add_up(B, h, w, device):
+@pytest.mark.parametrize("B,h,w,bar", [(1, 64, 128, 2.2e-7), (4, 128, 256, 3e-7)])
+def test_what_the_sums_lose_does_not_add_up(B, h, w, bar, device):
     """The matrix instruction rounds downwards; over many pixels that would show as an error of one
-    sign, larger than the fp32 instructions' (which were 2.3e-7 and 3.7e-7 off in 2-norm here)."""
+    sign, larger than the fp32 instructions' (which were 2.2e-7 and 3.7e-7 off in 2-norm here)."""
     g = torch.Generator(device="cuda").manual_seed(11)
     rnd = lambda *s: torch.randn(s, generator=g, device="cuda")
     smap = synthetic.latitude_map(h, w, 1).cuda()
@@ -134,5 +134,23 @@ def test_what_the_sums_lose_does_not_add_up(B, h, w, device):
                                              needs=(False, True, False))[1].double()
     want = grad(torch.float64)
     err = grad(torch.float32) - want
-    assert (err.norm() / want.norm()).item() < 3e-7
+    assert (err.norm() / want.norm()).item() < bar
     assert (err.mean().abs() / err.std()).item() < 0.1
+
+
+# (in 2-norm and units of 1e-7, what the fp32 instructions were off here)
+@pytest.mark.parametrize("B,h,w,normal,positive,relu", [
+    (1, 2, 8, 0.65, 0.47, 0.39), (1, 4, 16, 1.46, 1.23, 0.72), (1, 8, 16, 1.49, 0.93, 0.61),
+    (1, 16, 16, 1.53, 0.71, 0.55), (1, 16, 32, 2.11, 0.95, 0.64), (1, 16, 64, 2.09, 0.74, 0.55),
+    (1, 32, 64, 2.14, 0.60, 0.51)])
+def test_short_sums_are_as_near_to_64_bits_as_fp32_sums(B, h, w, normal, positive, relu, device):
+    """One to eight tiles of 128 pixels, operands of either sign, positive ones, and half zeros."""
+    g = torch.Generator(device="cuda").manual_seed(12)
+    smap = synthetic.latitude_map(h, w, 1).cuda()
+    wt, b = torch.zeros(64, 16, 9, device="cuda"), torch.zeros(64, device="cuda")
+    for kind, bar in ((lambda t: t, normal), (torch.abs, positive), (lambda t: t.clamp_min(0), relu)):
+        x, gy = (kind(torch.randn(B, c, h, w, generator=g, device="cuda")) for c in (16, 64))
+        grad = lambda t: _C.mapped_conv_backward(*[a.to(t) for a in (gy, smap, x, wt, b)], 9, 2,
+                                                 needs=(False, True, False))[1].double()
+        want = grad(torch.float64)
+        assert ((grad(torch.float32) - want).norm() / want.norm()).item() < bar * 1e-7
