@@ -29,9 +29,9 @@
 //     1285 (the fp32 kernel alone, in its two-pair form: 715 to 730; one flag for the whole
 //     product: 1300 in every case with a NaN).  2 x 24 -> 40 of 125 x 250, where the fp32 kernel's
 //     workgroups all run at once: 35, 59, 72, 72 (47).
-//   * A lane gathers, interpolates and splits exactly the elements its matrix B operand holds
-//     (lane (l31, lhi): channels lhi * 8 .. + 7 of pixel l31 of the wave), so samples never pass
-//     through LDS; only the weights do, pre-split by the packing launch.
+//   * In the planar kernel a lane gathers, interpolates and splits exactly the elements its matrix
+//     B operand holds (lane (l31, lhi): channels lhi * 8 .. + 7 of pixel l31 of the wave), so only
+//     the weights, pre-split by the packing launch, pass through LDS.
 // Bound: the matrix instructions (384 clocks a unit) and the vector instructions around them
 // (some 60 x 4), which all but take turns, and what three waves per SIMD leave exposed of the
 // loads' latency.  Measured in one run each, fp32 instructions -> these: 8 x 64 channels of
@@ -526,7 +526,12 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
       }
       *reinterpret_cast<f32x4 *>(&Samples[qp + 16 * h][qc]) = q;
     }
-    float sv[8];  // (of this wave's own pixels: no barrier, LDS serves a wave in order)
+    // (of this wave's own pixels: LDS serves a wave in order, and the fences, which cost nothing,
+    // keep the compiler from moving a lane's reads ahead of what other lanes write)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float sv[8];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       const f32x4 q = *reinterpret_cast<const f32x4 *>(&Samples[pe][lhi * 8 + 4 * j]);
