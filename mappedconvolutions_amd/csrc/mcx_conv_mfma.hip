@@ -3049,11 +3049,10 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       if (int rc = resolve_runs(rp, tables, map, iw, GH, GW, MH, MW, K,
                                 m.mode == kInterpNearest ? 1 : 4, m.wrap, m.weighted, s))
         return rc;
-      profile_begin(s);
+      profile_begin(s);  // (until after the general kernel, which may be the one that does the work)
       if (int rc = weight_grad_by_runs(rp, tables, plain, gath, part, plain_sum ? sum_part : nullptr,
                                        A, G, GH, GW, MH, MW, K, s))
         return rc;
-      profile_end(s);
       int *state = run_state(rp, tables);
       runs_state = state;
       pair_mask = state + 2;
@@ -3124,7 +3123,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       MCX_HIP_CHECK_LAUNCH();
     }
   }
-  profile_begin(s);
+  if (!by_runs) profile_begin(s);
   if constexpr (sizeof(TD) == 2) {
     if (ring) {
       const int rg_groups = (int)((G + kRgG - 1) / kRgG), rg_passes = (int)((K + kRgKT - 1) / kRgKT);

@@ -154,3 +154,28 @@ def test_short_sums_are_as_near_to_64_bits_as_fp32_sums(B, h, w, normal, positiv
                                                  needs=(False, True, False))[1].double()
         want = grad(torch.float64)
         assert ((grad(torch.float32) - want).norm() / want.norm()).item() < bar * 1e-7
+
+
+@pytest.mark.parametrize("runs", [True, False])
+def test_the_timed_kernel_is_the_one_that_does_the_work(runs, device):
+    """A weight gradient's timing request covers the kernel over runs or, for maps without, the
+    general one: the larger part of the call, whichever it is."""
+    B, ci, co, h, w = 2, 64, 64, 128, 256
+    smap = (synthetic.latitude_map(h, w, 1) if runs else synthetic.pixel_shuffle_map(h, w)).cuda()
+    x, gy = torch.randn(B, ci, h, w, device="cuda"), torch.randn(B, co, h, w, device="cuda")
+    wt, b = torch.randn(co, ci, 9, device="cuda"), torch.randn(co, device="cuda")
+    call = lambda: _C.mapped_conv_backward(gy, smap, x, wt, b, 9, 1, needs=(False, True, False))
+    call()
+    (start, end), = _C.make_event_pool(1, device)
+    try:
+        _C.profile_pool, _C.profile_events = _C.make_event_pool(1, device), []
+        torch.cuda.synchronize()
+        start.record()
+        call()
+        end.record()
+        torch.cuda.synchronize()
+        (label, first, last), = _C.profile_events
+    finally:
+        _C.profile_pool, _C.profile_events = [], None
+    assert label == "conv_backward_weight"
+    assert first.elapsed_time(last) > 0.3 * start.elapsed_time(end)
