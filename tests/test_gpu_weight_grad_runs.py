@@ -165,11 +165,12 @@ def test_the_timed_kernel_is_the_one_that_does_the_work(runs, device):
     x, gy = torch.randn(B, ci, h, w, device="cuda"), torch.randn(B, co, h, w, device="cuda")
     wt, b = torch.randn(co, ci, 9, device="cuda"), torch.randn(co, device="cuda")
     call = lambda: _C.mapped_conv_backward(gy, smap, x, wt, b, 9, 1, needs=(False, True, False))
-    call()
     (start, end), = _C.make_event_pool(1, device)
+    pool = _C.make_event_pool(1, device)
+    for _ in range(20):  # (the GPU is behind: what the host takes is not measured)
+        call()
     try:
-        _C.profile_pool, _C.profile_events = _C.make_event_pool(1, device), []
-        torch.cuda.synchronize()
+        _C.profile_pool, _C.profile_events = pool, []
         start.record()
         call()
         end.record()
