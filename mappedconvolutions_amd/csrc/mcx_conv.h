@@ -36,10 +36,11 @@ int records_gather_product(const double *src, const double *map, const double *i
                            int64_t O, int64_t SH, int64_t SW, int64_t N, int64_t K, int64_t P,
                            int interp, hipStream_t s);
 size_t records_scatter_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K);
+size_t records_scatter_min_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K);
 int records_product_scatter(const double *src, const double *map, const double *iw,
-                            const double *w, const double *bias, double *dst, void *ws, int64_t B,
-                            int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,
-                            int64_t P, int interp, hipStream_t s);
+                            const double *w, const double *bias, double *dst, void *ws,
+                            size_t ws_bytes, int64_t B, int64_t S, int64_t D, int64_t DH, int64_t DW,
+                            int64_t N, int64_t K, int64_t P, int interp, hipStream_t s);
 size_t records_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t GN, int64_t N, int64_t K);
 int records_weight_grad(const double *plain, const double *gath, const double *map,
                         const double *iw, double *gw, void *ws, int64_t B, int64_t A, int64_t G,

@@ -182,11 +182,11 @@ int product_scatter<double>(bool, const void *src, const void *map, const void *
                             const void *bias, void *dst, void *ws, size_t ws_bytes, int64_t B,
                             int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t MH, int64_t MW,
                             int64_t K, int64_t P, int interp, hipStream_t s, const void *) {
-  const size_t need = product_scatter_ws(MCX_F64, B, S, D, K, P, DH, DW, MH, MW);
-  if (ws && need > 0 && ws_bytes >= need)
+  if (ws && records_scatter_applies(B, S, D, K) &&
+      ws_bytes >= records_scatter_min_bytes(B, S, D, DH * DW, MH * MW, K))
     return records_product_scatter((const double *)src, (const double *)map, (const double *)iw,
-                                   (const double *)w, (const double *)bias, (double *)dst, ws, B,
-                                   S, D, DH, DW, MH * MW, K, P, interp, s);
+                                   (const double *)w, (const double *)bias, (double *)dst, ws,
+                                   ws_bytes, B, S, D, DH, DW, MH * MW, K, P, interp, s);
   int rc = bias ? fill_bias<double>((double *)dst, (const double *)bias, B, D, DH * DW, s)
                 : fill_zero<double>((double *)dst, B * D * DH * DW, s);
   if (rc) return rc;

@@ -642,14 +642,25 @@ bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int
 }
 
 // Scattering before the product, where the source channels are few beside the destination's (us for
-// the scalar kernel or records, as the rules above have it, against this; nine taps, one image of
-// 200x500): 1 -> 16 channels latitude map 158 / 63, shuffled 388 / 123; 1 -> 10 108 / 61, 375 / 121;
-// 1 -> 4 48 / 57, 187 / 117; 2 -> 16 157 / 107, 389 / 226; 2 -> 5 80 / 100, 205 / 221; 5 -> 16
-// 157 / 231, 390 / 525.  500x1000 1 -> 10 500 / 217, 1721 / 504; up to 64x128 shuffled 1 -> 10 48 / 24,
-// latitude 22 / 22.  The planes are K * S doubles a pixel to clear and to read: not many more than
-// additions, or than a record.
-static bool planes_scatter_applies(int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
-  return D >= 6 * S && K * S <= 64 && (S * DN <= 2 * N || K * S <= D);
+// the scalar kernel or records, as the rules above have it, against this; one image, shuffled maps,
+// coherent ones in brackets).  Nine taps of 128x256: 1 -> 6 63 / 44 (64 / 46), 1 -> 10 117 / 45 (88 / 47),
+// 1 -> 64 434 / 51, 2 -> 12 117 / 82 (98 / 85), 2 -> 32 224 / 86, 4 -> 64 435 / 171; of 200x500 1 -> 10
+// 375 / 121 (108 / 61), 1 -> 4 187 / 117 (48 / 57), 2 -> 5 205 / 221, 5 -> 16 390 / 525 (157 / 231).  Other
+// taps at 128x256, 1 -> 10: one 23 / 22, 25 305 / 112, 64 761 / 279; of 500x1000 one 218 / 66, 25
+// 4494 / 1284, 64 11397 / 3261.
+// A pixel of the product reads its planes one after the other, however few pixels there are: a plane
+// is 0.95 us and 107 ps a location, a record 28 ps a location, tap and channel.  Nine taps of 32x32 2 -> 20
+// 22 / 26, of 45x90 24 / 32 for 2 -> 12 and 36 / 32 for 2 -> 32; 25 taps of 16x16 1 -> 10 22 / 30, of 32x64
+// 31 / 36, of 64x128 80 / 48; 64 taps of 64x128 1 -> 6 104 / 114, of 90x180 191 / 178.
+// The planes are K * S doubles a pixel to clear and to read: not many more than additions, or than a
+// record.  (64 taps of one channel take up to ten times a record's scratch; with less than they need
+// records run.)
+static bool planes_scatter_applies(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
+  return D >= 6 * S && K * S <= 64 && (S * DN <= 2 * N || K * S <= D) &&
+         B * N * (28 * add_stride(D) - 107 * S) > 950000 * S;
+}
+static size_t planes_bytes(int64_t B, int64_t S, int64_t DN, int64_t K) {
+  return align256((size_t)(B * K * S * DN + 1) * sizeof(double));
 }
 
 #define MCX_LPR(C, CALL)              \
@@ -697,18 +708,22 @@ int records_gather_product(const double *src, const double *map, const double *i
                                         s, coherent);
 }
 
+// (what the form that runs with enough scratch takes, and what the call can do with)
 size_t records_scatter_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
-  if (planes_scatter_applies(S, D, DN, N, K))
-    return align256((size_t)(B * K * S * DN + 1) * sizeof(double));
+  if (planes_scatter_applies(B, S, D, DN, N, K)) return planes_bytes(B, S, DN, K);
   return scatter_record_bytes(B, D, DN) + (scatter_asks_map(B, S, N, K) ? 256 : 0);
+}
+size_t records_scatter_min_bytes(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
+  const size_t records = scatter_record_bytes(B, D, DN) + (scatter_asks_map(B, S, N, K) ? 256 : 0);
+  return std::min(records, records_scatter_bytes(B, S, D, DN, N, K));
 }
 
 int records_product_scatter(const double *src, const double *map, const double *iw,
-                            const double *w, const double *bias, double *dst, void *ws, int64_t B,
-                            int64_t S, int64_t D, int64_t DH, int64_t DW, int64_t N, int64_t K,
-                            int64_t P, int interp, hipStream_t s) {
+                            const double *w, const double *bias, double *dst, void *ws,
+                            size_t ws_bytes, int64_t B, int64_t S, int64_t D, int64_t DH, int64_t DW,
+                            int64_t N, int64_t K, int64_t P, int interp, hipStream_t s) {
   const int64_t DN = DH * DW;
-  if (planes_scatter_applies(S, D, DN, N, K)) {
+  if (planes_scatter_applies(B, S, D, DN, N, K) && ws_bytes >= planes_bytes(B, S, DN, K)) {
     double *planes = (double *)ws;
     const int64_t pairs = (B * K * S * DN + 1) / 2;
     const unsigned blocks =

@@ -36,7 +36,12 @@ PLANES = [(6, 1, 9, 4, 32, 0), (7, 1, 1, 5, 7, 0), (13, 2, 9, 9, 15, 0), (16, 1,
           (17, 1, 9, 31, 67, 0), (20, 3, 10, 8, 17, 0), (33, 4, 3, 29, 45, 6), (40, 1, 64, 3, 43, 0)]
 
 
-@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES + LARGER + PLANES)
+# the same with locations enough for planes to pay: more for fewer channels
+MANY = [(64, 1, 9, 17, 43, 0), (40, 1, 64, 17, 43, 0), (33, 1, 3, 31, 67, 6), (16, 1, 5, 48, 48, 3),
+        (13, 1, 9, 45, 53, 0), (7, 1, 10, 72, 70, 0), (20, 3, 9, 72, 70, 0)]
+
+
+@pytest.mark.parametrize("ci,co,k,mh,mw,p", SHAPES + LARGER + PLANES + MANY)
 @pytest.mark.parametrize("interp", [0, 1, 2])
 def test_fp64_products(ci, co, k, mh, mw, p, interp, device):
     g = torch.Generator().manual_seed(ci * 100 + co)
@@ -90,6 +95,28 @@ def test_infinite_weights_reach_what_is_added_to(interp, device):
     assert torch.equal(torch.isinf(got), reached)
     want = O.mapped_conv_backward(gy, smap, x, w, b, k, interp)[0]
     assert ((got - want).abs()[~reached] <= 1e-12 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("share", [1.0, 0.8, 0.2, 0.02])
+def test_planes_with_less_scratch(share, device):
+    """Sums taken before the product ask for more scratch than records; with less, records run, and
+    with less than those the scalar kernels."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(24)
+    B, ci, co, k, h, w_ = 2, 16, 1, 25, 48, 60
+    smap, _ = helpers.random_map(g, h, w_, k, 0, h, w_, torch.float64)
+    x, w, b, gy = (torch.randn(s, generator=g, dtype=torch.float64)
+                   for s in ((B, ci, h, w_), (co, ci, k), (co,), (B, co, h, w_)))
+    size = (B, ci, co, h, w_, h, w_, k, 0)
+    need = int(share * lib.mcx_conv_backward_workspace(*size, _lib.MCX_F64))
+    gyd, sd, xd, wd, gx = *(t.cuda() for t in (gy, smap, x, w)), torch.empty(B, ci, h, w_, device="cuda",
+                                                                          dtype=torch.float64)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    rc = lib.mcx_conv_backward(gyd.data_ptr(), sd.data_ptr(), None, xd.data_ptr(), wd.data_ptr(),
+                               gx.data_ptr(), None, None, ws.data_ptr(), need, *size, 1, _lib.MCX_F64,
+                               torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert rel_err(gx, O.mapped_conv_backward(gy, smap, x, w, b, k, 1)[0]) < 1e-12
 
 
 @pytest.mark.parametrize("interp", [0, 1, 2])
