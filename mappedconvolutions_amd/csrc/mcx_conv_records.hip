@@ -498,7 +498,8 @@ __global__ __launch_bounds__(kThreads) void scatter_planes_kernel(
       const int o = col ? o1 : o0;
       const double a = col ? a1 : a0;
       if (o < 0) continue;
-      for (int c = 0; c < S; c++) atomic_add(t + c * DN + o, a * v[(int64_t)c * N]);
+      // (a product of -0 is added as +0: the pixel has been added to)
+      for (int c = 0; c < S; c++) atomic_add(t + c * DN + o, a * v[(int64_t)c * N] + 0.0);
     }
   }
 }

@@ -97,6 +97,25 @@ def test_infinite_weights_reach_what_is_added_to(interp, device):
     assert ((got - want).abs()[~reached] <= 1e-12 * want.abs().max()).all()
 
 
+@pytest.mark.parametrize("interp", [0, 1, 2])
+@pytest.mark.parametrize("weight", [float("inf"), float("nan")])
+def test_minus_zeros_are_added_too(weight, interp, device):
+    """A pixel that only zeros of negative sign were added to is still one that was added to: an infinite
+    weight makes it NaN, as does a weight that is NaN."""
+    g = torch.Generator().manual_seed(23)
+    B, ci, co, k, h, w_ = 2, 64, 1, 9, 21, 20
+    smap = torch.rand(h, w_, k, 2, generator=g, dtype=torch.float64) * 4 + 2.25
+    smap[..., 0] += torch.arange(k) % 3
+    w = torch.rand(co, ci, k, generator=g, dtype=torch.float64) + 0.1
+    w[0, 5, 4] = weight
+    x, b = torch.zeros(B, ci, h, w_, dtype=torch.float64), torch.zeros(co, dtype=torch.float64)
+    gy = torch.full((B, co, h, w_), -0.0, dtype=torch.float64)
+    got = _C.mapped_conv_backward(*[t.cuda() for t in (gy, smap, x, w, b)], k, interp,
+                                  needs=(True, False, False))[0].cpu()
+    want = O.mapped_conv_backward(gy, smap, x, w, b, k, interp)[0]
+    assert torch.isnan(want).any() and torch.equal(torch.isnan(got), torch.isnan(want))
+
+
 @pytest.mark.parametrize("share", [1.0, 0.8, 0.2, 0.02])
 def test_planes_with_less_scratch(share, device):
     """Sums taken before the product ask for more scratch than records; with less, records run, and
