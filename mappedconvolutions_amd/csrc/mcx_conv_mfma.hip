@@ -3226,122 +3226,100 @@ __global__ void build_transposed_map_kernel(const float *__restrict__ map,
 }
 
 // accum[b, d, p] += wt * sum_s W[s, d, k] * src[b, s, n] for every overflow entry, a lane per
-// destination channel: a wave takes 64, 32 or 16 lanes an entry, U entries after one another in
-// each, whose loads are in flight together (an entry is three dependent loads deep), and IB images
-// with one reading of the entry's weights.  One entry and image at a time -> this: 3 x 40 -> 24
-// channels of 125 x 250 under a gnomonic map 58 -> 30 us; mesh of 40 962 vertices, 4 x 128 -> 64
-// channels 85 -> 57.
+// destination channel: a wave takes 64, 32 or 16 lanes an entry of one image, a workgroup four times
+// that of neighbouring entries.
 // `wp` holds the weights in the gather-product's packed layout (fp32: Wp[k][s][d]; bf16:
 // Wb[k][chunk][kg][d][8]); `src_cl`, when not null, is the channel-last copy [B][MN][Spad] of the
 // source, else src is [B][S][MN].  `accum` is a channel-last fp32 image [B][DN][Dpad] (a wave's 64
-// atomics fall into two cache lines instead of 64) that the gather's epilogue adds.  A fixed grid
-// walks the list, so an empty list costs one launch of idle workgroups.
-template <typename TD, int U, int IB>
-__global__ __launch_bounds__(64) void overflow_scatter_kernel(
+// atomics fall into two cache lines instead of 64) that the gather's epilogue adds.
+// A fixed grid walks entries x images, so that an empty list costs one launch of idle workgroups
+// whatever the batch (64 x 3 <- 16 channels of 32 x 64, whole input gradient: 106 us with a grid for
+// every image, 53 so).
+// Bound: an entry is three dependent loads deep, which waves in flight hide better than entries
+// in flight within a wave do: 64 x 64 <- 128 channels of 64 x 128, gnomonic map, whole input gradient
+// with one entry a wave at a time 1660 us, with two 2040, four 2342, two entries of four images 2666
+// (bf16 2283, 2468, 2797, 2754); 3 x 24 <- 40 of 125 x 250 145, 150, 159, 170 (bf16 117, 116, 126, 153);
+// mesh of 40 962 vertices, 4 x 64 <- 128 657, 660, 655, 664 (bf16 757, 766, 789, 789).
+// UNIFORM: an entry to a wave and known to be one, so that its record comes through the scalar cache:
+// the mesh 647 us where the lanes' vector loads take 683.  (Planar sources the other way: every
+// channel is a line of its own, 8 x 64 <- 64 of 256 x 512 1577 us scalar, 1220 vector.)
+template <typename TD, bool UNIFORM>
+__global__ __launch_bounds__(256) void overflow_scatter_kernel(
     const TD *__restrict__ src, const TD *__restrict__ src_cl, const void *__restrict__ wp,
     float *__restrict__ accum, const OverflowEntry *__restrict__ ovf,
     const int *__restrict__ overflow, int ovf_cap, int B, int S, int Spad, int D, int Dpad,
     int64_t MN, int64_t DN) {
   if (overflow[0] != 0) return;  // the scatter kernel does the whole product
   const int count = min(overflow[1], ovf_cap);
-  const int b0 = blockIdx.y * IB, lane = threadIdx.x;
-  const int chunks = Spad / kGC;
-  const int lanes = D <= 16 ? 16 : D <= 32 ? 32 : 64, per_wave = 64 / lanes;
-  const int sub = lane / lanes, dl = lane % lanes;
-  const int step = U * per_wave;
-  for (int e0 = blockIdx.x * step; e0 < count; e0 += gridDim.x * step) {
-    OverflowEntry en[U];
-    bool live[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int e = e0 + u * per_wave + sub;
-      live[u] = e < count;
-      en[u] = ovf[min(e, count - 1)];
-    }
-    for (int d0 = 0; d0 < D; d0 += lanes) {
+  const int lane = threadIdx.x & 63, chunks = Spad / kGC;
+  const int lanes = UNIFORM ? 64 : D <= 16 ? 16 : D <= 32 ? 32 : 64, per_wave = 64 / lanes;
+  const int sub = UNIFORM ? 0 : lane / lanes, dl = lane % lanes;
+  // Additions to one address are served one after the other, and the list of an incoherent map is
+  // mostly one corner pixel, which holds every tap outside the image: what a workgroup has for one
+  // pixel is added up before the atomics (1 x 128 <- 32 channels of 100 x 200, shuffled: 269 us where
+  // a wave adds up its own, 224 so; bf16 189 and 144).
+  __shared__ float part[2][4][64];
+  __shared__ int pixel[2][4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pieces = (count + 4 * per_wave - 1) / (4 * per_wave);
+  const int64_t items = (int64_t)pieces * B;
+  int buf = 0;
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const int b = (int)(it / pieces);
+    const int e = (((int)(it - (int64_t)b * pieces) * 4) + wave) * per_wave + sub;
+    const OverflowEntry en = ovf[min(e, count - 1)];
+    for (int d0 = 0; d0 < D; d0 += lanes, buf ^= 1) {
       const int d = min(d0 + dl, Dpad - 1);
-      float acc[U][IB];
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int i = 0; i < IB; i++) acc[u][i] = 0.f;
+      float sum = 0.f;
       for (int s8 = 0; s8 < Spad / 8; s8++) {  // 8 source channels at a time (both are padded)
-        float x[U][IB][8], wv[U][8];
+        float x[8], wv[8];
+        if (sizeof(TD) == 4 && src_cl) {
+          const float4 *q = reinterpret_cast<const float4 *>(
+              src_cl + ((int64_t)b * MN + en.n) * Spad + s8 * 8);
+          const float4 q0 = q[0], q1 = q[1];
+          x[0] = q0.x; x[1] = q0.y; x[2] = q0.z; x[3] = q0.w;
+          x[4] = q1.x; x[5] = q1.y; x[6] = q1.z; x[7] = q1.w;
+        } else {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-#pragma unroll
-          for (int i = 0; i < IB; i++) {
-            const int64_t b = min(b0 + i, B - 1);  // (past the last image: not added)
-            if (sizeof(TD) == 4 && src_cl) {
-              const float4 *q = reinterpret_cast<const float4 *>(
-                  src_cl + (b * MN + en[u].n) * Spad + s8 * 8);
-              const float4 q0 = q[0], q1 = q[1];
-              x[u][i][0] = q0.x; x[u][i][1] = q0.y; x[u][i][2] = q0.z; x[u][i][3] = q0.w;
-              x[u][i][4] = q1.x; x[u][i][5] = q1.y; x[u][i][6] = q1.z; x[u][i][7] = q1.w;
-            } else {
-#pragma unroll
-              for (int j = 0; j < 8; j++) {
-                const int sc = s8 * 8 + j;
-                x[u][i][j] = src_cl ? to_f32(src_cl[(b * MN + en[u].n) * Spad + sc])
-                                    : (sc < S ? to_f32(src[(b * S + sc) * MN + en[u].n]) : 0.f);
-              }
-            }
-          }
-          if constexpr (sizeof(TD) == 2) {
-            const int64_t wi =
-                ((((int64_t)en[u].k * chunks + (s8 >> 1)) * 2 + (s8 & 1)) * Dpad + d) << 3;
-            const uint4 q = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(wp) + wi);
-            const unsigned w4[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-              wv[u][2 * j] = __builtin_bit_cast(float, w4[j] << 16);
-              wv[u][2 * j + 1] = __builtin_bit_cast(float, w4[j] & 0xffff0000u);
-            }
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-              wv[u][j] = reinterpret_cast<const float *>(
-                  wp)[((int64_t)en[u].k * Spad + s8 * 8 + j) * Dpad + d];
+          for (int j = 0; j < 8; j++) {
+            const int sc = s8 * 8 + j;
+            x[j] = src_cl ? to_f32(src_cl[((int64_t)b * MN + en.n) * Spad + sc])
+                          : (sc < S ? to_f32(src[((int64_t)b * S + sc) * MN + en.n]) : 0.f);
           }
         }
+        if constexpr (sizeof(TD) == 2) {
+          const int64_t wi = ((((int64_t)en.k * chunks + (s8 >> 1)) * 2 + (s8 & 1)) * Dpad + d) << 3;
+          const uint4 q = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(wp) + wi);
+          const unsigned w4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-        for (int u = 0; u < U; u++)
+          for (int j = 0; j < 4; j++) {
+            wv[2 * j] = __builtin_bit_cast(float, w4[j] << 16);
+            wv[2 * j + 1] = __builtin_bit_cast(float, w4[j] & 0xffff0000u);
+          }
+        } else {
 #pragma unroll
-          for (int i = 0; i < IB; i++)
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-              acc[u][i] = __builtin_fmaf(x[u][i][j], wv[u][j], acc[u][i]);
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int i = 0; i < IB; i++) acc[u][i] = live[u] ? en[u].wt * acc[u][i] : 0.f;
-      // Additions to one address are served one after the other, and the list of an incoherent map
-      // is mostly one corner pixel, which holds every tap outside the image: what a wave has for
-      // one pixel is added up first.  fp32 backward, 10 -> 1 channels, bilinear map of 500 x 1000
-      // in random order: 4521 us without, 4220 with this.
-      bool same = true;
-#pragma unroll
-      for (int u = 0; u < U; u++) same = same && en[u].p == en[0].p;
-      const int p0 = __builtin_amdgcn_readfirstlane(en[0].p);
-      if (__builtin_amdgcn_ballot_w64(!same || en[0].p != p0) == 0) {
-#pragma unroll
-        for (int i = 0; i < IB; i++) {
-          float v = acc[0][i];
-#pragma unroll
-          for (int u = 1; u < U; u++) v += acc[u][i];
-          for (int m = lanes; m < 64; m <<= 1) v += __shfl_xor(v, m);
-          if (sub == 0 && b0 + i < B && d0 + dl < D)
-            atomic_add(accum + ((int64_t)(b0 + i) * DN + p0) * Dpad + d, v);
+          for (int j = 0; j < 8; j++)
+            wv[j] = reinterpret_cast<const float *>(wp)[((int64_t)en.k * Spad + s8 * 8 + j) * Dpad + d];
         }
-        continue;
+#pragma unroll
+        for (int j = 0; j < 8; j++) sum = __builtin_fmaf(x[j], wv[j], sum);
       }
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int i = 0; i < IB; i++)
-          if (live[u] && b0 + i < B && d0 + dl < D)
-            atomic_add(accum + ((int64_t)(b0 + i) * DN + en[u].p) * Dpad + d, acc[u][i]);
+      sum = e < count ? en.wt * sum : 0.f;
+      const int p0 = __builtin_amdgcn_readfirstlane(en.p);
+      const bool one = __builtin_amdgcn_ballot_w64(en.p != p0) == 0;
+      if (one)
+        for (int m = lanes; m < 64; m <<= 1) sum += __shfl_xor(sum, m);
+      part[buf][wave][lane] = sum;
+      if (lane == 0) pixel[buf][wave] = one ? p0 : -1 - wave;
+      __syncthreads();
+      bool all = true;
+      for (int q = 1; q < 4; q++) all = all && pixel[buf][q] == pixel[buf][0];
+      if (all) {
+        if (wave != 0) continue;
+        for (int q = 1; q < 4; q++) sum += part[buf][q][lane];
+      }
+      if ((!one || sub == 0) && d0 + dl < D)
+        atomic_add(accum + ((int64_t)b * DN + en.p) * Dpad + d, sum);
     }
   }
 }
@@ -3653,15 +3631,15 @@ int mfma_product_scatter(const TD *src, const float *map, const float *iw, const
                          (int)Spad16, MH * MW);
       MCX_HIP_CHECK_LAUNCH();
     }
-#define MCX_OVERFLOW(U, IB)                                                                       \
-  hipLaunchKernelGGL((overflow_scatter_kernel<TD, U, IB>), dim3(4096, (unsigned)((B + IB - 1) / IB)), \
-                     dim3(64), 0, s, src, cl ? (const TD *)stage : (const TD *)nullptr,           \
-                     (const void *)wpt, img, ovf, flag, (int)sc.ovf_cap, (int)B, (int)S,          \
-                     (int)Spad16, (int)D, (int)round_up(D, kOT), MH * MW, DH * DW)
-    // (a tap's weights that fit an L1 are best shared by entries: 12 KB 30 us where images of two
-    // entries share them in 42; 32 KB 85 and 57)
-    const bool large = Spad16 * round_up(D, kOT) * (int64_t)sizeof(TD) > 16384;
-    if (B > 1 && large) { MCX_OVERFLOW(2, 4); } else { MCX_OVERFLOW(4, 1); }
+    // (64 x 64 <- 128 channels of 64 x 128 1762 us with 2048 workgroups, 1634 with 8192, but an empty
+    // list costs 1.6 us more)
+    const unsigned ovf_blocks = (unsigned)std::min<int64_t>(8192, std::max<int64_t>(2048, B * MH * MW / 64));
+#define MCX_OVERFLOW(UNIFORM)                                                                     \
+  hipLaunchKernelGGL((overflow_scatter_kernel<TD, UNIFORM>), dim3(ovf_blocks), dim3(256), 0, s,   \
+                     src, cl ? (const TD *)stage : (const TD *)nullptr, (const void *)wpt, img,   \
+                     ovf, flag, (int)sc.ovf_cap, (int)B, (int)S, (int)Spad16, (int)D,             \
+                     (int)round_up(D, kOT), MH * MW, DH * DW)
+    if (cl && D > 32) { MCX_OVERFLOW(true); } else { MCX_OVERFLOW(false); }
 #undef MCX_OVERFLOW
     MCX_HIP_CHECK_LAUNCH();
     if (int rc = launch_gather_product<TD>(src, (const float *)tmap, nullptr, wpt, bias, dst,
