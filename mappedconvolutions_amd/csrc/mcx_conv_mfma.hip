@@ -32,7 +32,6 @@ inline void profile_end(hipStream_t s) {
 
 
 constexpr int kThreads = 256;
-constexpr int kTilePx = 128;  // output pixels per workgroup
 constexpr int kGC = 16;       // source channels per reduction chunk
 constexpr int kOT = 64;       // output channels per workgroup
 constexpr int kWtLd = kOT + 4;
@@ -1214,7 +1213,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     int G, int GH, int GW, int MH, int MW, int K, int weighted, int wrap, int tiles_x,
     int tiles_per_img, int tw_shift, int total_tiles, int ranges, int cgroups,
     float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask, int run_if_leading,
-    const int *__restrict__ runs_state) {
+    const int *__restrict__ runs_state, const uint4 *__restrict__ tap_table) {
   constexpr int NE = NP * NCORN;  // (offset, weight) pairs per pixel and tap
   static_assert(NA >= 1 && NA <= NE, "NA counts leading pairs");
   if (runs_state && runs_done(runs_state)) return;  // (see mcx_conv_runs.h)
@@ -1515,20 +1514,47 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
       }
     };
 
+    // (two-pair taps of an fp32 image without runs: resolved into a table in tile order by the launch
+    // that looked for runs, and only copied into the tap cache.  The whole weight gradient of every third
+    // pixel, 3 x 24 -> 40 channels of 125 x 250: resolved by every workgroup 84 us, so 78; of mirrored
+    // rows, 8 x 64 -> 64 of 256 x 512: 826 and 801.)
+    constexpr bool kTable = sizeof(TD) == 4 && !CL && NA == 2 && NE == 4 && kCacheTaps;
     if (kCacheTaps) {
       // every wave has its A operands in registers: reuse the plain tile's LDS for the
       // resolved taps of this tile (thread (p, half) takes every other tap of pixel p)
       __syncthreads();
-      for (int k = half; k < ktaps; k += 2) {
-        unsigned o[NE];
-        float w_[NE];
-        resolve_tap(k_base + k, o, w_);
+      bool from_table = false;
+      if constexpr (kTable) {
+        if (tap_table && runs_table(runs_state)) {
+          // (fetched only here: held across the plain tile's copy, the entries spill)
+          from_table = true;
+          const uint4 *te = tap_table + ((int64_t)t_in * K + k_base) * kTilePx + p;
+          constexpr int kTapsPerThread = (kWgKT + 1) / 2;
+          uint4 entry[kTapsPerThread];
 #pragma unroll
-        for (int i = 0; i < NA; i++) {
-          TapOff[k][p][i] = o[i];
-          TapWt[k][p][i] = w_[i];
+          for (int t = 0; t < kTapsPerThread; t++)
+            entry[t] = te[(int64_t)min(half + 2 * t, ktaps - 1) * kTilePx];
+#pragma unroll
+          for (int t = 0; t < kTapsPerThread; t++) {
+            const int k = half + 2 * t;
+            if (k < ktaps) {
+              *reinterpret_cast<uint2 *>(&TapOff[k][p][0]) = make_uint2(entry[t].x, entry[t].y);
+              *reinterpret_cast<uint2 *>(&TapWt[k][p][0]) = make_uint2(entry[t].z, entry[t].w);
+            }
+          }
         }
       }
+      if (!from_table)
+        for (int k = half; k < ktaps; k += 2) {
+          unsigned o[NE];
+          float w_[NE];
+          resolve_tap(k_base + k, o, w_);
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            TapOff[k][p][i] = o[i];
+            TapWt[k][p][i] = w_[i];
+          }
+        }
       __syncthreads();
     }
 
@@ -2954,6 +2980,10 @@ int mfma_gather_product(const TD *src, const float *map, const float *iw, const 
 }
 
 // ---- weight gradient ---------------------------------------------------------------
+// The two-pair taps of an fp32 image in the order of weight_grad_mfma_kernel's tiles.
+static size_t tap_table_bytes(int64_t MH, int64_t MW, int64_t K) {
+  return align256((size_t)make_tiling(1, MH, MW, 4).tiles_per_img * (size_t)K * kTilePx * 16);
+}
 // Per-range partial sums of gW, per-range partial sums of the plain operand, then
 // (single-row gathered operands) their channel-last copy.
 size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64_t MW, int64_t K,
@@ -2978,8 +3008,8 @@ size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64
     n += align256((size_t)(B * GH * GW * round_up(G, kGC)) * sizeof(float));
   else if (elem == 2)
     n += align256((size_t)(B * GH * GW * round_up(G, kGC)) * elem);
-  else if (runs_apply(B, A, G, GH, GW, MH, MW, K, P))  // fp32 images: the runs' tables
-    n += run_table_bytes(run_plan(B, A, G, GW, MH, MW, K));
+  else if (runs_apply(B, A, G, GH, GW, MH, MW, K, P))  // fp32 images: the runs' tables, the taps' table
+    n += run_table_bytes(run_plan(B, A, G, GW, MH, MW, K)) + tap_table_bytes(MH, MW, K);
   // bf16 images: the plain operand as MFMA fragments per pixel tile (to_plain_fragments_kernel)
   // and the table of resolved taps (resolve_tap_table_kernel, four pairs per tap at most)
   if (GH > 1 && elem == 2) {
@@ -3043,11 +3073,18 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   // launch both variants, of which one returns at once.
   const bool two_variants = m.np * (m.mode == kInterpNearest ? 1 : 4) == 4;
   const int *runs_state = nullptr;
+  const uint4 *tap_table = nullptr;
   if constexpr (sizeof(TD) == 4) {
     if (by_runs) {
       char *tables = (char *)pair_mask_ws + 256;
+      TapTable taps{};
+      if (m.mode != kInterpNearest) {
+        taps = TapTable{reinterpret_cast<uint4 *>(tables + run_table_bytes(rp)), t.tiles_x,
+                        t.tw_shift, t.tiles_per_img};
+        tap_table = taps.table;
+      }
       if (int rc = resolve_runs(rp, tables, map, iw, GH, GW, MH, MW, K,
-                                m.mode == kInterpNearest ? 1 : 4, m.wrap, m.weighted, s))
+                                m.mode == kInterpNearest ? 1 : 4, m.wrap, m.weighted, taps, s))
         return rc;
       profile_begin(s);  // (until after the general kernel, which may be the one that does the work)
       if (int rc = weight_grad_by_runs(rp, tables, plain, gath, part, plain_sum ? sum_part : nullptr,
@@ -3074,7 +3111,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
                      s, plain, gath, map, iw, part, (int)A, (int)G, (int)GH, (int)GW, (int)MH,   \
                      (int)MW, (int)K, m.weighted, m.wrap, t.tiles_x, t.tiles_per_img,            \
                      t.tw_shift, (int)t.total, ranges, cgroups,                                  \
-                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state)
+                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state, tap_table)
 #define MCX_LAUNCH_CL(NCORN, NP, CL)                                          \
   if constexpr (NCORN * NP == 4) {                                            \
     if (!ring) {                                                              \

@@ -6,10 +6,12 @@
 namespace mcx {
 
 // Words of `state`: [0] this path has done the work, [1] a sum is not finite, [2] pair mask for
-// weight_grad_mfma_kernel (at least 4: corners of the lower row are in use).
+// weight_grad_mfma_kernel (at least 4: corners of the lower row are in use), [3] the table of its taps
+// is there.
 constexpr int kRunStateWords = 64;
 
 __device__ inline bool runs_done(const int *state) { return state[0] != 0 && state[1] == 0; }
+__device__ inline bool runs_table(const int *state) { return state[3] != 0; }
 
 // How the work is cut, from the sizes alone.
 struct RunPlan {
@@ -24,9 +26,16 @@ bool runs_apply(int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t
 // Bytes of the tables that resolve_runs fills, and their state words.
 size_t run_table_bytes(const RunPlan &p);
 int *run_state(const RunPlan &p, char *tables);
+// What weight_grad_mfma_kernel reads where this path leaves a map of two-pair taps to it: the taps in
+// the order of its tiles, [tile of an image][tap][pixel of the tile] two byte offsets in a plane and
+// their two weights.  table NULL: taps of one corner.
+struct TapTable {
+  uint4 *table;
+  int tiles_x, tw_shift, tiles;
+};
 int resolve_runs(const RunPlan &p, char *tables, const float *map, const float *iw, int64_t GH,
                  int64_t GW, int64_t MH, int64_t MW, int64_t K, int ncorn, int wrap, int weighted,
-                 hipStream_t stream);
+                 const TapTable &taps, hipStream_t stream);
 // Per-range partial sums [ranges][K][G][A padded to 4]; sum_part (may be NULL): the same of the
 // plain operand, [ranges][A].
 int weight_grad_by_runs(const RunPlan &p, char *tables, const float *plain, const float *gath,

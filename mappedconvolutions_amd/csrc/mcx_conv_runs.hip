@@ -19,7 +19,8 @@
 //   * Maps of which more than one group in eight is no run, and sums that are not finite (an
 //     infinity or NaN among the operands, or values the split does not hold) are left to
 //     weight_grad_mfma_kernel, whose launch follows: state[0] says that this kernel has done the
-//     work, state[1] that a sum was not finite.
+//     work, state[1] that a sum was not finite.  Where resolve_runs_kernel sees at once that the map has
+//     no runs, it resolves the taps for that kernel instead.
 // Bound: vector and matrix instructions, which take turns (90 + 24 a unit: 65 % of the time at the
 // clock that it runs at, 2.0 GHz), and the LDS round trip and barrier of a unit, which three waves
 // per SIMD do not quite cover.  A wave of 32 plain channels (half the LDS reads) needs 250 registers,
@@ -77,12 +78,14 @@ constexpr int kElements = 1, kCorners = 2, kNowhere = 64;
 
 // desc[group][tap]; wts[group][tap][row of corners][pixel][2]: corner weights, scaled for the
 // split; offs (same shape): byte offsets of the corners, where the group is no run.  stats[block]:
-// 2 * groups that are no runs + (a corner of the lower row has a weight).  Eight lanes share a group.
+// 4 * groups that are no runs + 2 * (these tables were not written) + (a corner of the lower row has a
+// weight).  Eight lanes share a group.
 template <int NCORN, int ST>
 __global__ __launch_bounds__(256) void resolve_runs_kernel(
     const float *__restrict__ map, const float *__restrict__ iw, RunDesc *__restrict__ desc,
     float2 *__restrict__ wts, uint2 *__restrict__ offs, int *__restrict__ stats,
-    int *__restrict__ state, int GH, int GW, int MH, int MW, int K, int wrap, int weighted) {
+    int *__restrict__ state, int GH, int GW, int MH, int MW, int K, int wrap, int weighted,
+    const TapTable taps) {
   __shared__ int count[2];
   if (threadIdx.x < 2) count[threadIdx.x] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) state[1] = 0;
@@ -163,22 +166,43 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
     }
     return no_run;
   };
-  // Maps without runs (a shuffled one) are not worth tables: where more than half of 32 groups spread
-  // over the map, the same for every block, are none, only the lower row's corners are looked for
-  // (500x1000 shuffled, 10 -> 1 channels: with tables 2220 us for the call, 2121 so, 2092 without a look).
+  // Maps without runs (a shuffled one) are not worth these tables: more than half of 32 groups spread
+  // over the map, the same for every block, are none (500x1000 shuffled, 10 -> 1 channels: with tables
+  // 2220 us for the call, 2121 so).  The general kernel's taps are resolved instead, which also finds
+  // out whether corners of the lower row are in use; if the samples have shown that they are, nothing
+  // is left to do.
   const int e = threadIdx.x & 7;
   const int sample = (int)(((uint64_t)((threadIdx.x >> 3) * 2654435769u) * (uint64_t)(total >> 3)) >> 32);
   const bool tables = __syncthreads_count(examine(sample, e, true, false)) * 2 <= 256;
-  for (int t = blockIdx.x * 256 + threadIdx.x; t < ((total + 63) & ~63); t += gridDim.x * 256) {
-    const bool exists = t < total;
-    const bool no_run = examine(min(t, total - 1) >> 3, e, exists, tables);
-    no_runs += no_run && exists && e == 0 ? 1 : 0;
+  if (tables) {
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < ((total + 63) & ~63); t += gridDim.x * 256) {
+      const bool exists = t < total;
+      const bool no_run = examine(min(t, total - 1) >> 3, e, exists, true);
+      no_runs += no_run && exists && e == 0 ? 1 : 0;
+    }
+  } else if (NCORN == 4 && !__syncthreads_or(lower)) {
+    const int64_t entries = (int64_t)taps.tiles * K * kTilePx;
+    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < entries; i += gridDim.x * 256) {
+      const int p = (int)(i & (kTilePx - 1)), tk = (int)(i / kTilePx);
+      const int tile = tk / K, k = tk - tile * K;
+      const int tile_y = tile / taps.tiles_x, tile_x = tile - tile_y * taps.tiles_x;
+      const int gi = tile_y * (kTilePx >> taps.tw_shift) + (p >> taps.tw_shift);
+      const int gj = (tile_x << taps.tw_shift) + (p & ((1 << taps.tw_shift) - 1));
+      const int64_t s = ((int64_t)min(gi, MH - 1) * MW + min(gj, MW - 1)) * K + k;
+      const float2 xy = reinterpret_cast<const float2 *>(map)[s];
+      const float scale = gi < MH && gj < MW ? (weighted ? iw[s] : 1.f) : 0.f;
+      PairTap<NCORN> tap;
+      resolve_pairs<NCORN, 4>(xy.x, xy.y, GH, GW, wrap != 0, scale, tap);
+      lower |= tap.wt[2 % NCORN] != 0.f || tap.wt[3 % NCORN] != 0.f;
+      taps.table[i] = make_uint4(tap.off[0], tap.off[1 % NCORN], __builtin_bit_cast(unsigned, tap.wt[0]),
+                                 __builtin_bit_cast(unsigned, tap.wt[1 % NCORN]));
+    }
   }
   if (!tables) no_runs = threadIdx.x == 0 ? total / 8 / (int)gridDim.x + 1 : 0;
   if (no_runs) atomicAdd(&count[0], no_runs);
   if (lower) count[1] = 1;
   __syncthreads();
-  if (threadIdx.x == 0) stats[blockIdx.x] = 2 * count[0] + count[1];
+  if (threadIdx.x == 0) stats[blockIdx.x] = 4 * count[0] + (tables ? 0 : 2) + count[1];
 }
 
 struct RunArgs {
@@ -492,22 +516,34 @@ __device__ inline void weight_grad_runs(const RunArgs &s, RunLds &lds) {
 template <int ST>
 __global__ __launch_bounds__(kRunThreads, 3) void weight_grad_runs_kernel(const RunArgs s) {
   __shared__ __attribute__((aligned(16))) RunLds lds;
-  __shared__ int totals[2];
-  if (threadIdx.x < 2) totals[threadIdx.x] = 0;
-  __syncthreads();
-  int no_runs = 0, lower = 0;
+  __shared__ int totals[kRunThreads / 64][2];
+  int no_runs = 0, bits = 0;
   for (int i = threadIdx.x; i < s.stat_words; i += kRunThreads) {
-    no_runs += s.stats[i] >> 1;
-    lower |= s.stats[i] & 1;
+    no_runs += s.stats[i] >> 2;
+    bits |= s.stats[i];
   }
-  if (no_runs) atomicAdd(&totals[0], no_runs);
-  if (lower) totals[1] = 1;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    no_runs += __shfl_xor(no_runs, m);
+    bits |= __shfl_xor(bits, m);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    totals[threadIdx.x >> 6][0] = no_runs;
+    totals[threadIdx.x >> 6][1] = bits;
+  }
   __syncthreads();
-  const bool runs = (int64_t)totals[0] * 8 <= (int64_t)s.groups * s.K;
-  const bool two_rows = totals[1] != 0;
+  no_runs = bits = 0;
+#pragma unroll
+  for (int w = 0; w < kRunThreads / 64; w++) {
+    no_runs += totals[w][0];
+    bits |= totals[w][1];
+  }
+  const bool runs = (int64_t)no_runs * 8 <= (int64_t)s.groups * s.K;
+  const bool two_rows = (bits & 1) != 0;
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
     s.state[0] = runs ? 1 : 0;
     s.state[2] = two_rows ? 4 : 0;
+    s.state[3] = (bits & 2) != 0 && !two_rows ? 1 : 0;
   }
   if (!runs) return;
   if (two_rows)
@@ -570,12 +606,12 @@ int *run_state(const RunPlan &p, char *tables) { return RunTables(p, tables).sta
 
 int resolve_runs(const RunPlan &p, char *tables, const float *map, const float *iw, int64_t GH,
                  int64_t GW, int64_t MH, int64_t MW, int64_t K, int ncorn, int wrap, int weighted,
-                 hipStream_t stream) {
+                 const TapTable &taps, hipStream_t stream) {
   const RunTables t(p, tables);
 #define MCX_RESOLVE(NCORN, ST)                                                                     \
   hipLaunchKernelGGL((resolve_runs_kernel<NCORN, ST>), dim3((unsigned)p.stat_words), dim3(256), 0, \
                      stream, map, iw, t.desc, t.wts, t.offs, t.stats, t.state, (int)GH, (int)GW,   \
-                     (int)MH, (int)MW, (int)K, wrap, weighted)
+                     (int)MH, (int)MW, (int)K, wrap, weighted, taps)
   if (ncorn == 1) {
     if (p.st == 2) { MCX_RESOLVE(1, 2); } else { MCX_RESOLVE(1, 1); }
   } else {

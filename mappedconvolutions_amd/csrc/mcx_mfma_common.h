@@ -19,6 +19,8 @@ __device__ inline float dot_bf16(unsigned word, unsigned w, float acc) {
                                          __builtin_bit_cast(bf16x2, w), acc, false);
 }
 
+constexpr int kTilePx = 128;  // pixels of a tile
+
 // Factor of the weights and of the samples before they are split.
 constexpr float kSplitScale = 16777216.f;  // 2^24
 constexpr float kSplitUnscale = 1.f / (kSplitScale * kSplitScale);

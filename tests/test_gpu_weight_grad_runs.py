@@ -76,6 +76,22 @@ def test_maps_with_pixels_out_of_place(part, device):
         _check(2, 20, 24, h, w, torch.where(away, anywhere, smap), interp)
 
 
+@pytest.mark.parametrize("interp", [1, 2])
+@pytest.mark.parametrize("h,w", [(2, 130), (3, 33), (4, 32), (5, 33), (9, 72)])
+@pytest.mark.parametrize("k", [1, 9, 10])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_whole_rows_without_runs(interp, h, w, k, weighted, device):
+    """Mirrored rows: no runs, two corners a tap, which the general kernel reads from a table made by
+    the launch that found no runs; tiles of one and of four rows that end ragged."""
+    smap = _grid(h, w, k, 0.25, 0.0)
+    smap[..., 0] = w - 1 - smap[..., 0]
+    weights = None
+    if weighted:
+        weights = torch.rand(h, w, k, 1, generator=torch.Generator().manual_seed(3)) - 0.5
+        smap = smap.unsqueeze(3).contiguous()
+    _check(2, 20, 70, h, w, smap, interp, weights)
+
+
 @pytest.mark.parametrize("interp", [0, 1])
 def test_one_weighted_point_per_tap(interp, device):
     g = torch.Generator().manual_seed(8)
