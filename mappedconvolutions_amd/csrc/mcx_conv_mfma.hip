@@ -3021,6 +3021,17 @@ size_t mfma_weight_grad_bytes(int64_t B, int64_t A, int64_t G, int64_t MH, int64
   return n;
 }
 
+// What weight_grad_mfma_kernel<float> takes, about, in us: a tile is 1.45 a tap and 0.15 for the rest of a
+// CU's time, and where workgroups take several tiles, three of them share it.  (64 -> 64 channels,
+// nine taps, less the launches: 8 of 256 x 512 793, 871 by this; 1 of 200 x 400 77, 79; of 128 x 256
+// 28, 26; of 80 x 160 13, 13; 16 of 32 x 64 26, 26.  One tap of 2 x 128 -> 128 of 128 x 256 26, 29.)
+static double general_weight_grad_us(int64_t tiles, int64_t ranges, int64_t workgroups, int64_t K) {
+  const double one = 1.45 * (double)std::min<int64_t>(K, kWgKT) + 0.15;
+  const int64_t turns = (tiles + ranges - 1) / ranges;
+  if (turns == 1) return one * (double)((workgroups + 255) / 256);
+  return 3 * one * (double)(turns * ((workgroups + 767) / 768));
+}
+
 // scratch: mfma_weight_grad_bytes(...) bytes.  plain_sum (may be NULL): [A], receives the
 // sum of the plain operand over images and pixels (a convolution's bias gradient).
 template <typename TD>
@@ -3050,9 +3061,22 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   const int ranges = ring ? ring_weight_grad_ranges(t.total, A, G, K)
                           : weight_grad_ranges<TD>(t.total, A, G, K);
   // fp32 images: the kernel over runs of pixels, and for what it leaves the general one
-  const bool by_runs = sizeof(TD) == 4 && !cl && runs_apply(B, A, G, GH, GW, MH, MW, K, P);
+  bool by_runs = sizeof(TD) == 4 && !cl && runs_apply(B, A, G, GH, GW, MH, MW, K, P);
   RunPlan rp{};
-  if (by_runs) rp = run_plan(B, A, G, GW, MH, MW, K);
+  if (by_runs) {
+    rp = run_plan(B, A, G, GW, MH, MW, K);
+    // What goes with the general kernel: under taps of one corner it is two launches less, and with a plan,
+    // which says whether the lower row is in use, as well; otherwise it has those of this path and
+    // is the later to begin.  (Nearest taps, general kernel and runs: one of 4 x 32 -> 64 channels of
+    // 64 x 128 20 us, 26; nine 16 -> 32 of 64 x 128 25, 26; 16 x 64 -> 64 of 32 x 64 48, 49; 64 -> 64 of 80 x 160
+    // 33, 34; 4 x 16 -> 32 of 128 x 256 93, 48; two 2 x 128 -> 128 of 128 x 256 69, 81.)
+    const bool one_corner = m.mode == kInterpNearest;
+    const int64_t workgroups = ranges * cgroups * ((A + kWgA - 1) / kWgA) * ((K + kWgKT - 1) / kWgKT);
+    const double general = general_weight_grad_us(t.total, ranges, workgroups, K);
+    set_run_limit(rp, K, one_corner ? 0.9 * (general - 2) : plan ? general - 1 : general + 6);
+    // (of four corners, without a plan, what resolve_runs finds out about the map is wanted all the same)
+    if ((one_corner || plan) && rp.limit < 0) by_runs = false, rp = RunPlan{};
+  }
   const int part_ranges = std::max(ranges, rp.ranges);
   float *sum_part = reinterpret_cast<float *>(
       (char *)scratch + align256((size_t)part_ranges * (size_t)(round_up(A, 4) * G * K) * 4));

@@ -19,10 +19,22 @@ struct RunPlan {
   int64_t total_tiles;
   int ranges, stat_words;
   size_t desc_bytes, wts_bytes;
+  double us;  // of the kernel, about, where all groups are runs under one row of corners
+  // What the groups that are no runs (448 each, 160 under one row of corners) and those fetched element
+  // by element (56 and 10) may come to.  Less than zero: the general kernel is the faster one for every
+  // map.
+  int64_t limit;
 };
 RunPlan run_plan(int64_t B, int64_t A, int64_t G, int64_t GW, int64_t MH, int64_t MW, int64_t K);
 bool runs_apply(int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t MH, int64_t MW,
                 int64_t K, int64_t P);
+// Sets `limit` where the general kernel, and what goes with it, take general_us.  A workgroup waits for
+// its slowest wave, and a wave for corners or elements fetched one by one: each hundredth of the
+// groups that is no run costs a tenth of the time under one row of corners, a quarter under two (8 x 64 -> 64
+// channels of 256 x 512, general kernel in brackets: no such groups 675 us (800), 1.6 % 763 (798), 3.1 % 853
+// (810), 12 % 1260 (871); two rows 865 (974), 1.6 % 1094 (1001), 12 % 2207 (1151)), a group fetched
+// element by element a sixteenth and an eighth of that.
+void set_run_limit(RunPlan &p, int64_t K, double general_us);
 // Bytes of the tables that resolve_runs fills, and their state words.
 size_t run_table_bytes(const RunPlan &p);
 int *run_state(const RunPlan &p, char *tables);

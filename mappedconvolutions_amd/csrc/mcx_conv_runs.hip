@@ -16,8 +16,8 @@
 //     either row of corners and the corner weights of its pixels.  A run that jumps once (the seam
 //     of a wrapping map: one group in 64 of a row of 512) is fetched element by element, a group
 //     that is none corner by corner.
-//   * Maps of which more than one group in eight is no run, and sums that are not finite (an
-//     infinity or NaN among the operands, or values the split does not hold) are left to
+//   * Maps with more groups that are no runs than the gain bears (RunPlan::limit), and sums that are
+//     not finite (an infinity or NaN among the operands, or values the split does not hold) are left to
 //     weight_grad_mfma_kernel, whose launch follows: state[0] says that this kernel has done the
 //     work, state[1] that a sum was not finite.  Where resolve_runs_kernel sees at once that the map has
 //     no runs, it resolves the taps for that kernel instead.
@@ -78,28 +78,29 @@ constexpr int kElements = 1, kCorners = 2, kNowhere = 64;
 
 // desc[group][tap]; wts[group][tap][row of corners][pixel][2]: corner weights, scaled for the
 // split; offs (same shape): byte offsets of the corners, where the group is no run.  stats[block]:
-// 4 * groups that are no runs + 2 * (these tables were not written) + (a corner of the lower row has a
-// weight).  Eight lanes share a group.
+// {4 * groups that are no runs + 2 * (these tables were not written) + (a corner of the lower row has
+// a weight), groups fetched element by element}.  Eight lanes share a group.  wanted: the tables are,
+// should the map have runs.
 template <int NCORN, int ST>
 __global__ __launch_bounds__(256) void resolve_runs_kernel(
     const float *__restrict__ map, const float *__restrict__ iw, RunDesc *__restrict__ desc,
-    float2 *__restrict__ wts, uint2 *__restrict__ offs, int *__restrict__ stats,
+    float2 *__restrict__ wts, uint2 *__restrict__ offs, int2 *__restrict__ stats,
     int *__restrict__ state, int GH, int GW, int MH, int MW, int K, int wrap, int weighted,
-    const TapTable taps) {
-  __shared__ int count[2];
-  if (threadIdx.x < 2) count[threadIdx.x] = 0;
+    int wanted, const TapTable taps) {
+  __shared__ int count[3];
+  if (threadIdx.x < 3) count[threadIdx.x] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) state[1] = 0;
   __syncthreads();
   const int gpr = (MW + 7) >> 3;
   const int total = MH * gpr * K * 8;
   const int lane = threadIdx.x & 63, first = lane & 56;
-  int no_runs = 0;
+  int no_runs = 0, elements = 0;
   bool lower = false;
   auto of_group = [&](bool x) {
     return (unsigned)(__builtin_amdgcn_ballot_w64(x) >> first) & 0xffu;
   };
-  // One pixel of a (group, tap) q; returns whether the group is no run (the same in its eight
-  // lanes).  `write`: into the tables.
+  // One pixel of a (group, tap) q; returns the kind of its group (the same in its
+  // eight lanes).  `write`: into the tables.
   auto examine = [&](int q, int e, bool exists, bool write) __attribute__((always_inline)) {
     const int g = q / K, k = q - g * K;
     const GroupPlace at_px = group_place(g, MH, gpr);
@@ -164,21 +165,22 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
       if (no_run) d = RunDesc{0, 0, 0, kNowhere * 4 + kCorners};
       desc[q] = d;
     }
-    return no_run;
+    return no_run ? kCorners : inside ? 0 : kElements;
   };
-  // Maps without runs (a shuffled one) are not worth these tables: more than half of 32 groups spread
+  // Maps without runs (a shuffled one) are not worth these tables: more than four of 32 groups spread
   // over the map, the same for every block, are none (500x1000 shuffled, 10 -> 1 channels: with tables
   // 2220 us for the call, 2121 so).  The general kernel's taps are resolved instead, which also finds
   // out whether corners of the lower row are in use; if the samples have shown that they are, nothing
   // is left to do.
   const int e = threadIdx.x & 7;
   const int sample = (int)(((uint64_t)((threadIdx.x >> 3) * 2654435769u) * (uint64_t)(total >> 3)) >> 32);
-  const bool tables = __syncthreads_count(examine(sample, e, true, false)) * 2 <= 256;
+  const bool tables = __syncthreads_count(examine(sample, e, true, false) == kCorners) <= 4 * 8 && wanted;
   if (tables) {
     for (int t = blockIdx.x * 256 + threadIdx.x; t < ((total + 63) & ~63); t += gridDim.x * 256) {
       const bool exists = t < total;
-      const bool no_run = examine(min(t, total - 1) >> 3, e, exists, true);
-      no_runs += no_run && exists && e == 0 ? 1 : 0;
+      const int kind = examine(min(t, total - 1) >> 3, e, exists, true);
+      no_runs += exists && e == 0 && kind == kCorners ? 1 : 0;
+      elements += exists && e == 0 && kind == kElements ? 1 : 0;
     }
   } else if (NCORN == 4 && !__syncthreads_or(lower)) {
     const int64_t entries = (int64_t)taps.tiles * K * kTilePx;
@@ -200,9 +202,10 @@ __global__ __launch_bounds__(256) void resolve_runs_kernel(
   }
   if (!tables) no_runs = threadIdx.x == 0 ? total / 8 / (int)gridDim.x + 1 : 0;
   if (no_runs) atomicAdd(&count[0], no_runs);
+  if (elements) atomicAdd(&count[2], elements);
   if (lower) count[1] = 1;
   __syncthreads();
-  if (threadIdx.x == 0) stats[blockIdx.x] = 4 * count[0] + (tables ? 0 : 2) + count[1];
+  if (threadIdx.x == 0) stats[blockIdx.x] = make_int2(4 * count[0] + (tables ? 0 : 2) + count[1], count[2]);
 }
 
 struct RunArgs {
@@ -210,12 +213,13 @@ struct RunArgs {
   const RunDesc *desc;
   const uint2 *offs;
   const float *wts;
-  const int *stats;
+  const int2 *stats;
   int *state;
   float *part, *sum_part;  // sum_part: NULL, or per-range sums of the plain operand
   int A, G, GH, GW, MH, MW, K, stat_words;
   int groups;              // of an image: MH * ceil(MW / 8)
   int tiles_per_img, total_tiles, ranges, cblocks;
+  int64_t limit;           // see RunPlan
 };
 
 constexpr int kTileGroups = 16;  // 128 pixels
@@ -516,30 +520,37 @@ __device__ inline void weight_grad_runs(const RunArgs &s, RunLds &lds) {
 template <int ST>
 __global__ __launch_bounds__(kRunThreads, 3) void weight_grad_runs_kernel(const RunArgs s) {
   __shared__ __attribute__((aligned(16))) RunLds lds;
-  __shared__ int totals[kRunThreads / 64][2];
-  int no_runs = 0, bits = 0;
+  __shared__ int totals[kRunThreads / 64][3];
+  int no_runs = 0, elements = 0, bits = 0;
   for (int i = threadIdx.x; i < s.stat_words; i += kRunThreads) {
-    no_runs += s.stats[i] >> 2;
-    bits |= s.stats[i];
+    const int2 of_block = s.stats[i];
+    no_runs += of_block.x >> 2;
+    bits |= of_block.x;
+    elements += of_block.y;
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
     no_runs += __shfl_xor(no_runs, m);
     bits |= __shfl_xor(bits, m);
+    elements += __shfl_xor(elements, m);
   }
   if ((threadIdx.x & 63) == 0) {
     totals[threadIdx.x >> 6][0] = no_runs;
     totals[threadIdx.x >> 6][1] = bits;
+    totals[threadIdx.x >> 6][2] = elements;
   }
   __syncthreads();
-  no_runs = bits = 0;
+  no_runs = bits = elements = 0;
 #pragma unroll
   for (int w = 0; w < kRunThreads / 64; w++) {
     no_runs += totals[w][0];
     bits |= totals[w][1];
+    elements += totals[w][2];
   }
-  const bool runs = (int64_t)no_runs * 8 <= (int64_t)s.groups * s.K;
   const bool two_rows = (bits & 1) != 0;
+  const bool runs = (int64_t)no_runs * (two_rows ? 448 : 160) +
+                            (int64_t)elements * (two_rows ? 56 : 10) <= s.limit &&
+                    (int64_t)no_runs * 8 <= (int64_t)s.groups * s.K;
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
     s.state[0] = runs ? 1 : 0;
     s.state[2] = two_rows ? 4 : 0;
@@ -556,13 +567,14 @@ struct RunTables {
   RunDesc *desc;
   uint2 *offs;
   float2 *wts;
-  int *stats, *state;
+  int2 *stats;
+  int *state;
   RunTables(const RunPlan &p, char *t) {
     desc = reinterpret_cast<RunDesc *>(t);
     wts = reinterpret_cast<float2 *>(t + p.desc_bytes);
     offs = reinterpret_cast<uint2 *>(t + p.desc_bytes + p.wts_bytes);
-    stats = reinterpret_cast<int *>(t + p.desc_bytes + 2 * p.wts_bytes);
-    state = stats + kRunStatWords;
+    stats = reinterpret_cast<int2 *>(t + p.desc_bytes + 2 * p.wts_bytes);
+    state = reinterpret_cast<int *>(stats + kRunStatWords);
   }
 };
 
@@ -577,13 +589,25 @@ RunPlan run_plan(int64_t B, int64_t A, int64_t G, int64_t GW, int64_t MH, int64_
   p.groups = (int)(MH * ((MW + 7) / 8));
   p.tiles_per_img = (p.groups + kTileGroups - 1) / kTileGroups;
   p.total_tiles = B * p.tiles_per_img;
-  // three workgroups per CU; few tiles: fewer taps per workgroup
-  const int64_t per_tile = (int64_t)p.cblocks * p.ablocks;
-  p.passes = (int)((K + kRunTaps - 1) / kRunTaps);
-  while (p.passes < (K + 2) / 3 && p.total_tiles * per_tile * p.passes < 512)
-    p.passes = (int)std::min<int64_t>(p.passes * 2, (K + 2) / 3);
-  const int64_t want = std::max<int64_t>(1, 768 / (per_tile * p.passes));
-  p.ranges = (int)std::min<int64_t>(want, p.total_tiles);
+  // Three workgroups fit a CU, and a tile takes a workgroup its time however few there are: 1.5 us a
+  // tap and 1.9 for the rest (under taps of one row; a tenth more where they are two pixels apart, and
+  // somewhat more where all three share the taps of one tile).  The taps are cut, to three at least, where
+  // tiles then come out evenly: 16 x 64 -> 64 channels of 32 x 64, nine taps at a time 59 us, three 52;
+  // 4 x 16 -> 32 of 128 x 256 64 and 53; 2 x 128 -> 128 of 45 x 90 in two parts 58 and 54.
+  const int64_t per_tile = (int64_t)p.cblocks * p.ablocks, least = (K + kRunTaps - 1) / kRunTaps;
+  constexpr int64_t kSlots = 768;
+  for (int64_t passes = least; passes <= std::max(least, (K + 2) / 3); passes++) {
+    const int64_t ranges = std::min(std::max<int64_t>(1, kSlots / (per_tile * passes)), p.total_tiles);
+    const int64_t turns = (ranges * per_tile * passes + kSlots - 1) / kSlots;
+    const double us = (double)(turns * ((p.total_tiles + ranges - 1) / ranges)) *
+                      (1.5 * (double)((K + passes - 1) / passes) + 1.9) *
+                      (p.st == 2 ? 1.1 : 1.0) * (1.0 + 0.08 * (double)(passes - least));
+    if (p.passes == 0 || us < p.us) {
+      p.us = us;
+      p.passes = (int)passes;
+      p.ranges = (int)ranges;
+    }
+  }
   const int64_t entries = (int64_t)p.groups * K * 8;
   p.stat_words = (int)std::min<int64_t>(kRunStatWords, (entries + 255) / 256);
   p.desc_bytes = align256((size_t)p.groups * K * sizeof(RunDesc));
@@ -599,7 +623,12 @@ bool runs_apply(int64_t B, int64_t A, int64_t G, int64_t GH, int64_t GW, int64_t
 }
 // desc, weights, corner offsets, statistics and the state words
 size_t run_table_bytes(const RunPlan &p) {
-  return p.desc_bytes + 2 * p.wts_bytes + align256(kRunStatWords * 4) + align256(kRunStateWords * 4);
+  return p.desc_bytes + 2 * p.wts_bytes + align256(kRunStatWords * sizeof(int2)) + align256(kRunStateWords * 4);
+}
+
+void set_run_limit(RunPlan &p, int64_t K, double general_us) {
+  const double gain = general_us / p.us - 1.0;
+  p.limit = gain < 0 ? -1 : (int64_t)(gain * 16 * (double)p.groups * (double)K);
 }
 
 int *run_state(const RunPlan &p, char *tables) { return RunTables(p, tables).state; }
@@ -611,7 +640,7 @@ int resolve_runs(const RunPlan &p, char *tables, const float *map, const float *
 #define MCX_RESOLVE(NCORN, ST)                                                                     \
   hipLaunchKernelGGL((resolve_runs_kernel<NCORN, ST>), dim3((unsigned)p.stat_words), dim3(256), 0, \
                      stream, map, iw, t.desc, t.wts, t.offs, t.stats, t.state, (int)GH, (int)GW,   \
-                     (int)MH, (int)MW, (int)K, wrap, weighted, taps)
+                     (int)MH, (int)MW, (int)K, wrap, weighted, p.limit >= 0 ? 1 : 0, taps)
   if (ncorn == 1) {
     if (p.st == 2) { MCX_RESOLVE(1, 2); } else { MCX_RESOLVE(1, 1); }
   } else {
@@ -633,8 +662,11 @@ int weight_grad_by_runs(const RunPlan &p, char *tables, const float *plain, cons
   a.A = (int)A; a.G = (int)G; a.GH = (int)GH; a.GW = (int)GW; a.MH = (int)MH; a.MW = (int)MW;
   a.K = (int)K; a.stat_words = p.stat_words; a.groups = p.groups;
   a.tiles_per_img = p.tiles_per_img; a.total_tiles = (int)p.total_tiles; a.ranges = p.ranges;
-  a.cblocks = p.cblocks;
-  const dim3 grid((unsigned)(p.ranges * p.cblocks), (unsigned)p.ablocks, (unsigned)p.passes);
+  a.cblocks = p.cblocks; a.limit = p.limit;
+  // (where the work is the general kernel's in any case, one workgroup says so)
+  const dim3 grid = p.limit < 0 ? dim3(1)
+                                : dim3((unsigned)(p.ranges * p.cblocks), (unsigned)p.ablocks,
+                                       (unsigned)p.passes);
   if (p.st == 2)
     hipLaunchKernelGGL(weight_grad_runs_kernel<2>, grid, dim3(kRunThreads), 0, stream, a);
   else
