@@ -504,26 +504,40 @@ __global__ __launch_bounds__(kThreads) void scatter_planes_kernel(
   }
 }
 
-constexpr int kPlaneD = 16;  // destination channels per workgroup
+constexpr int kPlaneD = 16;    // destination channels per workgroup
+constexpr int kPlanes = 64;    // planes of an image, at most
+constexpr int kPlaneRun = 8;   // planes whose loads are in flight
+// The weights sit in LDS and eight planes are read together: a plane of a small image, whose few
+// waves have nothing else to do meanwhile, takes 0.64 us
+// instead of 0.95 (25 taps of 64x128, 1 -> 10 channels: the whole product 51 -> 45 us).
 __global__ __launch_bounds__(kThreads) void product_planes_kernel(
     const double *__restrict__ planes, const double *__restrict__ w,
     const double *__restrict__ bias, double *__restrict__ dst, int S, int D, int64_t DN, int K) {
+  __shared__ double s_w[kPlanes][kPlaneD];
   const int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  const int d0 = blockIdx.y * kPlaneD, b = blockIdx.z;
-  const double *t = planes + (int64_t)b * K * S * DN + min(p, DN - 1);
+  const int d0 = blockIdx.y * kPlaneD, b = blockIdx.z, count = K * S;
+  for (int i = threadIdx.x; i < count * kPlaneD; i += kThreads) {
+    const int q = i / kPlaneD, k = q / S, c = q - k * S, d = min(d0 + i % kPlaneD, D - 1);
+    s_w[q][i % kPlaneD] = w[((int64_t)c * D + d) * K + k];
+  }
+  const double *t = planes + (int64_t)b * count * DN + min(p, DN - 1);
   double acc[kPlaneD];
 #pragma unroll
   for (int d = 0; d < kPlaneD; d++) acc[d] = bias && d0 + d < D ? bias[d0 + d] : 0.0;
-  for (int k = 0; k < K; k++)
-    for (int c = 0; c < S; c++) {
-      const double v = t[((int64_t)k * S + c) * DN];
-      const bool touched = __builtin_bit_cast(unsigned long long, v) != kUntouched;
+  __syncthreads();
+  for (int q0 = 0; q0 < count; q0 += kPlaneRun) {
+    double v[kPlaneRun];
 #pragma unroll
-      for (int d = 0; d < kPlaneD; d++) {
-        const double a = w[((int64_t)c * D + min(d0 + d, D - 1)) * K + k];
-        acc[d] = touched ? mcx_fma(a, v, acc[d]) : acc[d];
-      }
+    for (int j = 0; j < kPlaneRun; j++) v[j] = t[(int64_t)min(q0 + j, count - 1) * DN];
+#pragma unroll
+    for (int j = 0; j < kPlaneRun; j++) {
+      if (q0 + j >= count) break;
+      const bool touched = __builtin_bit_cast(unsigned long long, v[j]) != kUntouched;
+#pragma unroll
+      for (int d = 0; d < kPlaneD; d++)
+        acc[d] = touched ? mcx_fma(s_w[q0 + j][d], v[j], acc[d]) : acc[d];
     }
+  }
   if (p >= DN) return;
 #pragma unroll
   for (int d = 0; d < kPlaneD; d++)
@@ -644,21 +658,23 @@ bool records_weight_grad_applies(int64_t B, int64_t A, int64_t G, int64_t N, int
 
 // Scattering before the product, where the source channels are few beside the destination's (us for
 // the scalar kernel or records, as the rules above have it, against this; one image, shuffled maps,
-// coherent ones in brackets).  Nine taps of 128x256: 1 -> 6 63 / 44 (64 / 46), 1 -> 10 117 / 45 (88 / 47),
-// 1 -> 64 434 / 51, 2 -> 12 117 / 82 (98 / 85), 2 -> 32 224 / 86, 4 -> 64 435 / 171; of 200x500 1 -> 10
+// coherent ones in brackets).  Nine taps of 90x180: 1 -> 6 34 / 28 (35 / 27), 1 -> 10 61 / 28 (46 / 27),
+// 1 -> 64 213 / 30, 2 -> 12 63 / 49 (52 / 46), 2 -> 32 112 / 50, 4 -> 64 217 / 94; of 200x500 1 -> 10
 // 375 / 121 (108 / 61), 1 -> 4 187 / 117 (48 / 57), 2 -> 5 205 / 221, 5 -> 16 390 / 525 (157 / 231).  Other
-// taps at 128x256, 1 -> 10: one 23 / 22, 25 305 / 112, 64 761 / 279; of 500x1000 one 218 / 66, 25
-// 4494 / 1284, 64 11397 / 3261.
-// A pixel of the product reads its planes one after the other, however few pixels there are: a plane
-// is 0.95 us and 107 ps a location, a record 28 ps a location, tap and channel.  Nine taps of 32x32 2 -> 20
-// 22 / 26, of 45x90 24 / 32 for 2 -> 12 and 36 / 32 for 2 -> 32; 25 taps of 16x16 1 -> 10 22 / 30, of 32x64
-// 31 / 36, of 64x128 80 / 48; 64 taps of 64x128 1 -> 6 104 / 114, of 90x180 191 / 178.
+// taps of 90x180, 1 -> 10: 25 151 / 69, 64 378 / 160; of 500x1000 one 218 / 66, 25 4494 / 1284, 64
+// 11397 / 3261.
+// A pixel of the product reads its planes eight at a time, however few pixels there are: a plane
+// is 0.64 us and 100 ps a location, a record 28 ps a location, tap and channel, and 3 us more for all.
+// Nine taps of 10x20 4 -> 64 23 / 36, of 32x64 2 -> 12 23 / 25, of 64x128 38 / 33 (31 / 34); 25 taps of
+// 10x20 1 -> 10 24 / 26, of 32x64 30 / 31, of 45x90 49 / 35 (39 / 34); 64 taps of 45x90 1 -> 6 64 / 77, of
+// 64x128 107 / 105.  (Taps outside the image all meet in one pixel: nine taps of a shuffled 60x90 with
+// such a border 1 -> 10 37 / 20, 2 -> 12 40 / 30.)
 // The planes are K * S doubles a pixel to clear and to read: not many more than additions, or than a
 // record.  (64 taps of one channel take up to ten times a record's scratch; with less than they need
 // records run.)
 static bool planes_scatter_applies(int64_t B, int64_t S, int64_t D, int64_t DN, int64_t N, int64_t K) {
-  return D >= 6 * S && K * S <= 64 && (S * DN <= 2 * N || K * S <= D) &&
-         B * N * (28 * add_stride(D) - 107 * S) > 950000 * S;
+  return D >= 6 * S && K * S <= kPlanes && (S * DN <= 2 * N || K * S <= D) &&
+         K * (B * N * (28 * add_stride(D) - 100 * S) - 640000 * S) > -3000000;
 }
 static size_t planes_bytes(int64_t B, int64_t S, int64_t DN, int64_t K) {
   return align256((size_t)(B * K * S * DN + 1) * sizeof(double));
