@@ -175,14 +175,23 @@ __device__ inline void build_gather_plan(const float *__restrict__ map,
     gmap[((int64_t)k * kPlanSlots + i) * pixels + n] = out[i];
 }
 
-//   * ChannelBlocksJob and GatherPlanJob: the gathered operand in blocks of eight channels, and the
-//     map's taps resolved, for the product that follows (bf16 images): 4 x 32 -> 64 channels of
-//     64 x 128, forward five launches -> two.
+// Jobs of the packing launch (pack_weights_kernel): the gathered operand in blocks of eight channels,
+// and the map's taps resolved, for the product that follows (bf16 images): 4 x 32 -> 64 channels of
+// 64 x 128, forward five launches -> two.
 template <typename TD>
 struct PrepJobs {
   ChannelBlocksJob<TD> blocks;
   GatherPlanJob plan;
 };
+
+// w.lo * word.lo + w.hi * word.hi, the head of such a sum.  (Written out because the compiler
+// renders dot_bf16(word, w, 0) as the accumulating two-operand form behind a move of zero:
+// one instruction in three of an interpolation.)
+__device__ inline float dot_bf16_first(unsigned word, unsigned w) {
+  float r;
+  asm("v_dot2_f32_bf16 %0, %1, %2, 0" : "=v"(r) : "v"(word), "v"(w));
+  return r;
+}
 
 // Repack W[o][g][k] for the matrix-core kernels, with g padded to 16 and o padded to 64
 // (zeros); `transposed` reads W[g][o][k] instead (weights stored source-channel major).
@@ -193,15 +202,6 @@ struct PrepJobs {
 //   (channels kg*8 .. kg*8+7, kg = lane / 32) of its row or column in 16 bytes.  Weights are
 //   therefore packed as Wb[k][chunk][kg][o][8] bf16: the 64 x 16 slice of a (tap, chunk) is two
 //   runs of 64 x 16 bytes that are copied linearly into LDS.
-// w.lo * word.lo + w.hi * word.hi, the head of such a sum.  (Written out because the compiler
-// renders dot_bf16(word, w, 0) as the accumulating two-operand form behind a move of zero:
-// one instruction in three of an interpolation.)
-__device__ inline float dot_bf16_first(unsigned word, unsigned w) {
-  float r;
-  asm("v_dot2_f32_bf16 %0, %1, %2, 0" : "=v"(r) : "v"(word), "v"(w));
-  return r;
-}
-
 template <typename TD>
 __global__ __launch_bounds__(256) void pack_weights_kernel(
     const TD *__restrict__ w, void *__restrict__ packed_out, int O, int G, int K, int Opad,
@@ -389,7 +389,7 @@ struct OperandTiles<bf16_t, OG> {  // bf16: 16-byte groups of 8 channels, [kg][p
 // to_channel_last_kernel): a sample's 8 channels are then one or two 16-byte loads from
 // one cache line instead of 8 loads from 8 lines.  Used for single-row sources (mesh
 // signals), whose maps point anywhere.  With `cl_blocked` the copy is [B][Gpad/8][SH*SW][8]
-// (made by to_channel_blocks_kernel): neighbouring pixels stay neighbours, so image-like
+// (made by to_channel_blocks): neighbouring pixels stay neighbours, so image-like
 // sources keep their coalescing and a sample's 8 channels are still one load; used with bf16
 // storage, where the number of load instructions bounds the kernel.
 // NA: leading (offset, weight) pairs of a tap that are loaded and added.  NA == NP * NCORN is
@@ -843,11 +843,10 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 // Only the weights (linear copies of the pre-packed slices) go through LDS, double buffered,
 // one barrier per unit.  A workgroup is 4 waves = 256 consecutive pixels of an image (in the
 // order of the flattened map, so any image width works) x 64*OG output channels.  The source is
-// the copy in blocks of 8 channels per pixel (to_channel_blocks_kernel).  PACKED: the taps come
+// the copy in blocks of 8 channels per pixel (to_channel_blocks).  PACKED: the taps come
 // from a packed map (a transposed map or a plan's gather part: four (pixel, weight) entries per
 // tap); else from sample_map under single-point bilinear / bispherical interpolation.  NA counts
-// the leading entries of a tap that are read (2 or 4); the launches of both values are gated
-// like those of the general kernel (pair_mask / row_mask).
+// the leading entries of a tap that are read (2 or 4), by the masks of the map (pair_mask / row_mask).
 constexpr int kDgPx = 256;
 
 template <int NA, int OG>
@@ -1694,9 +1693,9 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(
 
 // ---------------------------------------------------------------------------------
 // Weight gradient, bf16 storage, unweighted bilinear taps, gathered operand in blocks of 8
-// channels per pixel ([B][Gpad/8][GH*GW][8], to_channel_blocks_kernel).  NA == 2: maps whose
+// channels per pixel ([B][Gpad/8][GH*GW][8], to_channel_blocks).  NA == 2: maps whose
 // two lower corners weigh nothing anywhere (integral row coordinates); NA == 4: all others (the
-// pair mask of the map lets one of the two launches run).  With bf16 MFMA the products are short
+// pair mask of the map selects the form on the device).  With bf16 MFMA the products are short
 // and the kernel lives or dies by its gather, so this form is built around it:
 //   * a thread gathers two neighbouring pixels x 8 channels of a unit (one tap, 32 gathered
 //     channels): four 16-byte loads instead of 32 two-byte ones (the texture path resolves
@@ -2539,8 +2538,6 @@ GatherPlanJob gather_plan_job(const float *map, const float *iw, float2 *gmap, c
                        (int)(((MN + 63) / 64 * 64 * K + 255) / 256)};
 }
 
-// `stage`: room for the channel-last copy (B * SH * SW * Gpad elements) when
-// use_channel_last(SH, interp), unused otherwise.
 // ---- fp32 on the bf16 matrix instructions (mcx_conv_split.h) ----
 // Room for the flags (a word per tile of the B x OH x OW outputs) and the split weights, at the end
 // of a product's scratch.
@@ -2609,8 +2606,6 @@ int launch_gather_split(SplitArgs a, const PixelTiling &t, bool cl, hipStream_t 
   return 0;
 }
 
-// `split` (fp32 storage; w NULL: not available): where the packing launch put the split weights.
-// `map2`: second-level entries of a packed map, read by the split kernels only.
 // Whether launch_gather_product reads blocks of eight channels: the packing launch makes them then.
 template <typename TD>
 bool gathers_blocks(const TD *stage, int64_t SH, int64_t SW, int interp) {
@@ -2624,6 +2619,10 @@ ChannelBlocksJob<TD> blocks_for(const TD *src, TD *stage, int64_t B, int64_t G, 
                                                : ChannelBlocksJob<TD>{};
 }
 
+// `stage` (may be NULL): room for a copy of the source, B * SH * SW * Gpad elements: channel-last where
+// gathers_channel_last, in blocks of eight channels where gathers_blocks, unused otherwise.
+// `split` (fp32 storage; w NULL: not available): where the packing launch put the split weights.
+// `map2`: second-level entries of a packed map, read by the split kernels only.
 template <typename TD>
 int launch_gather_product(const TD *src, const float *map, const float *iw, const float *wp,
                           const TD *bias, TD *y, TD *stage, int64_t B, int64_t G, int64_t O,

@@ -26,7 +26,7 @@
 // per SIMD do not quite cover.  A wave of 32 plain channels (half the LDS reads) needs 250 registers,
 // and at two waves per SIMD everything is waited for: 820 us where this takes 735.
 // Measured in one run each, fp32 instructions -> this: 8 x 64 -> 64 channels of 256 x 512, nine taps:
-// 793 -> 667 us; 3 x 24 -> 40 of 125 x 250, fractional rows, 100 -> 66; transposed 4 x 64 -> 32 from
+// 793 -> 672 us; 3 x 24 -> 40 of 125 x 250, fractional rows, 100 -> 66; transposed 4 x 64 -> 32 from
 // 128 x 256 onto twice that (taps two pixels apart) 105 -> 71.
 // Accuracy: the instruction rounds its sums downwards, so that 24 of them a tile lose up to 24 units
 // of the last place, all one way.  The products of the leading parts, 16 bits each, are summed in an
