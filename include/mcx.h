@@ -163,7 +163,8 @@ int mcx_conv_forward_static(const void *x, const void *map, const void *iw, cons
 /* Bytes of device scratch the matching call needs for these sizes (may be 0).
  * The scratch holds repacked weights, partial sums, staging copies of operands and
  * resolved taps; its contents need not survive the call.  It must be 256-byte aligned.
- * fp64 calls accept NULL, or less than this size, and then run scalar kernels without scratch.
+ * fp64 calls accept NULL, or less than this size, and then run what fits: in the last resort scalar
+ * kernels without scratch.
  *
  * Arithmetic of fp32 forward and input gradient (and their transposed counterparts), given the
  * whole size: the operands split exactly into three bf16 parts each, six of the nine partial
