@@ -2574,33 +2574,40 @@ int launch_gather_split(SplitArgs a, const PixelTiling &t, bool cl, hipStream_t 
   a.tiles_x = t.tiles_x;
   a.tiles_per_img = t.tiles_per_img;
   a.tw_shift = t.tw_shift;
-  const bool wide = a.Opad % (2 * kOT) == 0;
-  const dim3 grid((unsigned)t.total, (unsigned)(a.Opad / (wide ? 2 * kOT : kOT)));
+  // Blocks of 32 outputs a workgroup computes: a block of zeros costs as many matrix instructions
+  // as one of weights, and its accumulators the registers of a fourth wave.  (Always two or four of
+  // them, against this: 4 x 64 -> 32 channels onto 256 x 512, transposed, forward and backward 450 us, 413;
+  // 3 x 24 -> 40 of 125 x 250, whose input gradient has 24, 257 and 253.  Three blocks keep the two waves
+  // of four.)
+  const int blocks = (a.O + 31) / 32;
+  const int nb = blocks == 1 ? 1 : blocks == 3 ? 3 : a.Opad % (2 * kOT) == 0 ? 4 : 2;
+  const dim3 grid((unsigned)t.total, (unsigned)((blocks + nb - 1) / nb));
 #define MCX_SPLIT(KERNEL, ...) \
   hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(kThreads), 0, s, a)
-#define MCX_SPLIT_OG(KERNEL, ...)        \
-  if (wide) {                            \
-    MCX_SPLIT(KERNEL, __VA_ARGS__, 2);   \
-  } else {                               \
-    MCX_SPLIT(KERNEL, __VA_ARGS__, 1);   \
+#define MCX_SPLIT_NB(KERNEL, ...)                      \
+  switch (nb) {                                        \
+    case 1: MCX_SPLIT(KERNEL, __VA_ARGS__, 1); break;  \
+    case 2: MCX_SPLIT(KERNEL, __VA_ARGS__, 2); break;  \
+    case 3: MCX_SPLIT(KERNEL, __VA_ARGS__, 3); break;  \
+    default: MCX_SPLIT(KERNEL, __VA_ARGS__, 4); break; \
   }
   if (cl) {
     if (a.map2) {
-      MCX_SPLIT_OG(gather_product_split_cl_kernel, 4, true)
+      MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, true)
     } else {
       switch (a.packed ? 4 : a.np) {
-        case 1: MCX_SPLIT_OG(gather_product_split_cl_kernel, 1, false) break;
-        case 2: MCX_SPLIT_OG(gather_product_split_cl_kernel, 2, false) break;
-        case 3: MCX_SPLIT_OG(gather_product_split_cl_kernel, 3, false) break;
-        default: MCX_SPLIT_OG(gather_product_split_cl_kernel, 4, false) break;
+        case 1: MCX_SPLIT_NB(gather_product_split_cl_kernel, 1, false) break;
+        case 2: MCX_SPLIT_NB(gather_product_split_cl_kernel, 2, false) break;
+        case 3: MCX_SPLIT_NB(gather_product_split_cl_kernel, 3, false) break;
+        default: MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, false) break;
       }
     }
   } else if (!a.packed && a.ncorn == 1) {
-    MCX_SPLIT_OG(gather_product_split_kernel, 1)
+    MCX_SPLIT_NB(gather_product_split_kernel, 1)
   } else {
-    MCX_SPLIT_OG(gather_product_split_kernel, 4)
+    MCX_SPLIT_NB(gather_product_split_kernel, 4)
   }
-#undef MCX_SPLIT_OG
+#undef MCX_SPLIT_NB
 #undef MCX_SPLIT
   MCX_HIP_CHECK_LAUNCH();
   return 0;

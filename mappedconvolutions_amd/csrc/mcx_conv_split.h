@@ -70,10 +70,11 @@ __device__ inline int split_upper_half(int c, int G) {
   return rem >= 16 ? 8 : rem > 8 ? rem - 8 : 0;
 }
 
-// The weights of a unit through LDS: [part][kg][output][8 channels], double buffered.
-template <int OG>
+// The weights of a unit through LDS: [part][kg][output][8 channels], double buffered.  NB: blocks of
+// 32 outputs a workgroup computes.
+template <int NB>
 struct SplitWeights {
-  static constexpr int kPieces = 3 * 2 * kOT * OG;                        // of 16 bytes
+  static constexpr int kPieces = 3 * 2 * 32 * NB;                         // of 16 bytes
   static constexpr int kPer = (kPieces + kThreads - 1) / kThreads;        // per thread
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   unsigned off[kPer];
@@ -85,7 +86,7 @@ struct SplitWeights {
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
       const int i = min(t + j * kThreads, kPieces - 1);  // (a last, partial round is not stored)
-      off[j] = (unsigned)((i / (kOT * OG)) * Opad + o0 + i % (kOT * OG)) * 16u;
+      off[j] = (unsigned)((i / (32 * NB)) * Opad + o0 + i % (32 * NB)) * 16u;
     }
   }
   __device__ inline void load(plane_buf_t r, unsigned unit_off, u32x4 *v) const {
@@ -102,27 +103,27 @@ struct SplitWeights {
   }
 };
 
-template <int OG>
+template <int NB>
 __device__ inline void split_products(const uint4 *lds, const bf16x8 *b, int l31, int lhi,
                                       floatx16 *acc) {
-  bf16x8 a[2 * OG][3];
+  bf16x8 a[NB][3];
 #pragma unroll
-  for (int m = 0; m < 2 * OG; m++)
+  for (int m = 0; m < NB; m++)
 #pragma unroll
     for (int part = 0; part < 3; part++)
       a[m][part] =
-          __builtin_bit_cast(bf16x8, lds[(part * 2 + lhi) * (kOT * OG) + 32 * m + l31]);
+          __builtin_bit_cast(bf16x8, lds[(part * 2 + lhi) * (32 * NB) + 32 * m + l31]);
   // (smallest first; the chains of the output blocks are independent)
   constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
   for (int t = 0; t < 6; t++)
 #pragma unroll
-    for (int m = 0; m < 2 * OG; m++)
+    for (int m = 0; m < NB; m++)
       acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m][pa[t]], b[pb[t]], acc[m], 0, 0, 0);
 }
 
 // Bias, addend and stores of a lane's pixel; flags a tile with a result that is not finite.
-template <int OG>
+template <int NB>
 __device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, int tile, int b,
                                       int o0, int ei, int ej, int lhi) {
   const int64_t N = (int64_t)s.OH * s.OW;
@@ -134,7 +135,7 @@ __device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, i
                           ? s.addend + ((int64_t)b * N + n) * s.Opad
                           : nullptr;
 #pragma unroll
-    for (int m = 0; m < 2 * OG; m++)
+    for (int m = 0; m < NB; m++)
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int o = o0 + 32 * m + (i >> 2) * 8 + lhi * 4 + (i & 3);
@@ -155,11 +156,11 @@ __device__ inline void split_epilogue(const SplitArgs &s, const floatx16 *acc, i
 // transposed map) are fetched with one 8-byte load: the texture path takes 16 clocks for a
 // wave's load whatever its width, and 16 single loads a unit would cost it as much as the fp32
 // matrix instructions did.
-template <int NE, int OG>
-__global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gather_product_split_kernel(
+template <int NE, int NB>
+__global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) void gather_product_split_kernel(
     const SplitArgs s) {
   constexpr int kCache = NE == 1 ? 6 : kTapCache;  // cached entries per pixel
-  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<OG>::kPieces];
+  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<NB>::kPieces];
   __shared__ __attribute__((aligned(16))) unsigned TapOff[kCache * kTilePx];
   __shared__ __attribute__((aligned(16))) float TapWt[kCache * kTilePx];
   __shared__ int unpaired;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
       leading = any == 0;
     }
   }
-  const int o0 = blockIdx.y * (kOT * OG);
+  const int o0 = blockIdx.y * (32 * NB);
   const int N = s.OH * s.OW;
   const unsigned plane_bytes = (unsigned)s.SH * (unsigned)s.SW * 4u;
   const int chunks = s.Gpad / kGC;
@@ -196,12 +197,12 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
   const bool live = gi < s.OH && gj < s.OW;
   const int64_t n_g = live ? (int64_t)gi * s.OW + gj : 0;
 
-  floatx16 acc[2 * OG];
+  floatx16 acc[NB];
 #pragma unroll
-  for (int m = 0; m < 2 * OG; m++)
+  for (int m = 0; m < NB; m++)
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[m][i] = 0.f;
-  SplitWeights<OG> wts;
+  SplitWeights<NB> wts;
   wts.init(tid, s.Opad, o0);
   int buf = 0;
 
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
     const int units = chunks * kn;
     float v[kDepth][8][NA];
     float wgt[kDepth][NA];
-    typename SplitWeights<OG>::u32x4 wv[kDepth][SplitWeights<OG>::kPer];
+    typename SplitWeights<NB>::u32x4 wv[kDepth][SplitWeights<NB>::kPer];
     int kl = 0, c = 0;  // the unit whose loads are issued next
     // (issued unconditionally, past the last unit too, where it reads the last chunk again: a
     // load behind a branch would make every wait a full one)
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
         stage(d);
         __syncthreads();
         issue(d);
-        split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+        split_products<NB>(Wt[buf], bq, l31, lhi, acc);
         buf ^= 1;
       }
     }
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
       if (u + d < units) {
         stage(d);
         __syncthreads();
-        split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+        split_products<NB>(Wt[buf], bq, l31, lhi, acc);
         buf ^= 1;
       }
     }
@@ -373,7 +374,7 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
     run(std::integral_constant<int, NE == 4 ? 2 : 1>());
   else
     run(std::integral_constant<int, NE>());
-  split_epilogue<OG>(s, acc, tile, b, o0, tile_y * th + (pe >> s.tw_shift),
+  split_epilogue<NB>(s, acc, tile, b, o0, tile_y * th + (pe >> s.tw_shift),
                      (tile_x << s.tw_shift) + (pe & tw_mask), lhi);
 }
 
@@ -385,10 +386,10 @@ __global__ __launch_bounds__(kThreads, OG == 2 ? 2 : NE == 1 ? 4 : 3) void gathe
 // Tap-major, a tap's entries in registers; NE entries a tap, and with TWO (a
 // transposed map with a second level) four more where any lane of the wave uses one: both levels
 // go through one product.
-template <int NE, bool TWO, int OG>
-__global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_product_split_cl_kernel(const SplitArgs s) {
+template <int NE, bool TWO, int NB>
+__global__ __launch_bounds__(kThreads, TWO || NE * NB > 8 ? 2 : 3) void gather_product_split_cl_kernel(const SplitArgs s) {
   constexpr int NT = TWO ? NE + 4 : NE;
-  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<OG>::kPieces];
+  __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<NB>::kPieces];
   constexpr int kSampleLd = kGC + 4;  // (eight lanes' 16-byte accesses on different banks)
   __shared__ __attribute__((aligned(16))) float Samples[kTilePx][kSampleLd];
   if (s.gate && ((*s.gate == 0) != (s.run_if_zero != 0))) return;
@@ -398,7 +399,7 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
   const int t_in = tile - b * s.tiles_per_img;
   const int tile_y = t_in / s.tiles_x, tile_x = t_in - tile_y * s.tiles_x;
   const int tw_mask = (1 << s.tw_shift) - 1, th = kTilePx >> s.tw_shift;
-  const int o0 = blockIdx.y * (kOT * OG);
+  const int o0 = blockIdx.y * (32 * NB);
   const int N = s.OH * s.OW;
   const int chunks = s.Gpad / kGC;
   const unsigned record = (unsigned)s.Gpad * 4u;
@@ -422,12 +423,12 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
   const auto wbuf = plane_buf(s.w, (unsigned)s.K * chunks * 6u * s.Opad * 16u);
   const unsigned w_unit = 6u * s.Opad * 16u;
 
-  floatx16 acc[2 * OG];
+  floatx16 acc[NB];
 #pragma unroll
-  for (int m = 0; m < 2 * OG; m++)
+  for (int m = 0; m < NB; m++)
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[m][i] = 0.f;
-  SplitWeights<OG> wts;
+  SplitWeights<NB> wts;
   wts.init(tid, s.Opad, o0);
 
   const bool packed = TWO || s.packed;  // (only a transposed map has a second level)
@@ -458,7 +459,7 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
   unsigned off[2][NT];
   float wgt[2][NT];
   f32x4 v[2][NT];
-  typename SplitWeights<OG>::u32x4 wv[SplitWeights<OG>::kPer];
+  typename SplitWeights<NB>::u32x4 wv[SplitWeights<NB>::kPer];
   bool more = false;  // (wave-uniform) an entry beyond the first NE is in use
   auto resolve = [&]() __attribute__((always_inline)) {
     bool any = false;
@@ -551,8 +552,8 @@ __global__ __launch_bounds__(kThreads, TWO || NE * OG > 4 ? 2 : 3) void gather_p
       }
       issue(k, c);
     }
-    split_products<OG>(Wt[buf], bq, l31, lhi, acc);
+    split_products<NB>(Wt[buf], bq, l31, lhi, acc);
     buf ^= 1;
   }
-  split_epilogue<OG>(s, acc, tile, b, o0, ei, ej, lhi);
+  split_epilogue<NB>(s, acc, tile, b, o0, ei, ej, lhi);
 }

@@ -74,6 +74,34 @@ def test_split_products_over_meshes(per_cell, ci, co, device):
     assert rel_err(gx, O.weighted_mapped_conv_backward(gy, smap, iw, x, w, b, k, 0)[0]) < 1e-5
 
 
+@pytest.mark.parametrize("co", [1, 31, 32, 33, 64, 65, 95, 96, 97, 128, 160, 192, 225])
+@pytest.mark.parametrize("mesh", [False, True])
+def test_outputs_in_blocks_of_32(co, mesh, device):
+    """A workgroup computes one to four blocks of 32 outputs.  32-bit sums of 7 * 21 terms: a few 1e-7
+    of the result's magnitude, 1e-5 allowed like everywhere here; a NaN reaches every output of the
+    pixels that sample it and no other pixel."""
+    g = torch.Generator().manual_seed(co)
+    B, ci, k = 2, 21, 7
+    rnd = lambda *s: torch.randn(s, generator=g)
+    if mesh:
+        h, w_ = 1, 150
+        smap = torch.stack((torch.randint(w_, (1, w_, k), generator=g).float(),
+                            torch.zeros(1, w_, k)), -1).contiguous()
+    else:
+        h, w_ = 5, 33
+        smap = _grid(h, w_, k, 0.25, 0.5)
+    interp = 0 if mesh else 1
+    x, w, b = rnd(B, ci, h, w_), rnd(co, ci, k), rnd(co)
+    want = O.mapped_conv_forward(x, smap, w, b, k, interp)
+    y = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp)
+    assert rel_err(y, want) < 1e-5
+    x[1, 4, h // 2, 17] = float("nan")
+    got = _C.mapped_conv_forward(x.cuda(), smap.cuda(), w.cuda(), b.cuda(), k, interp).cpu()
+    ok = torch.isfinite(O.mapped_conv_forward(x, smap, w, b, k, interp))
+    assert torch.equal(torch.isfinite(got), ok) and ok[0].all() and not ok.all()
+    assert ((got - want).abs()[ok] <= 1e-5 * want.abs().max()).all()
+
+
 @pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_inf", "overflow", "large"])
 def test_operands_without_a_split(what, device):
     """An infinity or NaN among the operands and sums beyond fp32 come out as the fp32
