@@ -23,8 +23,8 @@ import sys
 ROOT = os.path.dirname(os.path.abspath(__file__))
 # The headline's kernels and what they include
 KERNEL_SOURCES = ["mappedconvolutions_amd/csrc/" + name for name in
-                  ("mcx_conv_mfma.hip", "mcx_conv_split.h", "mcx_conv_runs.hip", "mcx_conv_runs.h",
-                   "mcx_mfma_common.h", "mcx_taps.h", "mcx_device.h")]
+                  ("mcx_conv_mfma.hip", "mcx_conv_split.hip", "mcx_conv_split.h", "mcx_conv_runs.hip",
+                   "mcx_conv_runs.h", "mcx_mfma_common.h", "mcx_taps.h", "mcx_device.h")]
 COPY_BYTES = 8 * 64 * 256 * 512 * 4  # one calibration dispatch reads and writes the input once
 
 

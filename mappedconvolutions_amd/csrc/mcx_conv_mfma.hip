@@ -12,6 +12,7 @@
 // t+1 are issued before the MFMAs of chunk t.  No column buffer ever reaches HBM.
 #include "mcx_conv.h"
 #include "mcx_conv_runs.h"
+#include "mcx_conv_split.h"
 #include "mcx_mfma_common.h"
 #include "mcx_taps.h"
 
@@ -32,20 +33,8 @@ inline void profile_end(hipStream_t s) {
 
 
 constexpr int kThreads = 256;
-constexpr int kGC = 16;       // source channels per reduction chunk
-constexpr int kOT = 64;       // output channels per workgroup
 constexpr int kWtLd = kOT + 4;
 constexpr int kTapCache = 12;  // cached (offset, weight) pairs per tile pixel (12 KB of LDS)
-
-// Whether a pair beyond the first two of a tap is in use anywhere in the map, from the pair
-// mask: one word (at least 4 then), or `words` words of which any may say so (one per block
-// of the launch that examined the map).  Called by whole waves.
-__device__ inline bool later_pairs_in_use(const int *__restrict__ mask, int words) {
-  if (words <= 1) return (unsigned)*mask >= (1u << 2);
-  const int lane = threadIdx.x & 63;
-  const unsigned v = (unsigned)mask[lane < words ? lane : 0];
-  return __builtin_amdgcn_ballot_w64(v >= (1u << 2)) != 0;
-}
 
 // Small jobs that ride on the weight-packing launch (a launch costs 4 to 8 us even when its
 // kernel does next to nothing, and small problems are made of launches):
@@ -65,15 +54,13 @@ struct PairMaskJob {
 };
 
 //   * SplitJob: the weights in three bf16 parts as well, and the flags that the kernels which
-//     read them set, a word per pixel tile, cleared (mcx_conv_split.h).
+//     read them set, a word per pixel tile, cleared (mcx_conv_split.hip).
 struct SplitJob {
   uint16_t *w;     // nullptr: no job
   int *nonfinite;
   int64_t tiles;
   int planar;      // the source they meet is planar (else channel-last)
 };
-
-__host__ __device__ inline int split_channel(int c, int kg, int j, int G, int planar);
 
 // Bits of the (point, corner) pairs with a nonzero weight anywhere among the entries this
 // block walks (block `block` of `blocks`); valid in every thread on return.
@@ -261,7 +248,7 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
         const I q = e / o_pad, o = e - q * o_pad, k = q / g_pad, g = q - k * g_pad;
         reinterpret_cast<float *>(packed_out)[e] =
             (o < (I)O && g < (I)G) ? weight(o, g, k) : 0.f;
-        // the same in three bf16 parts, [k][chunk][part][kg][o][8 channels] (mcx_conv_split.h)
+        // the same in three bf16 parts, [k][chunk][part][kg][o][8 channels] (mcx_conv_split.hip)
         if (split.w) {
           const I u = (e >> 3) / o_pad, so = (e >> 3) - u * o_pad;  // (tap, chunk, half), output
           const int kg = (int)(u & 1), sc = (int)((u >> 1) % chunks);
@@ -423,7 +410,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
   // (bilinear corners of integral coordinates, unused slots) are neither loaded nor
   // accumulated.
   __shared__ unsigned TapMask[TG][2][2];
-  // nothing of this tile to recompute (see mcx_conv_split.h)
+  // nothing of this tile to recompute (see mcx_conv_split.hip)
   if (only_if && only_if[xcd_contiguous_tile(blockIdx.x, gridDim.x)] == 0) return;
   if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
   if (pair_mask && !row_mask &&
@@ -1150,7 +1137,6 @@ __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel
 }
 
 
-#include "mcx_conv_split.h"
 
 // ---------------------------------------------------------------------------------
 // weight_grad: gW[a,g,k] = sum_{b,n} plain[b,a,n] * sample(gath[b,g], map[n,k])
@@ -2538,7 +2524,7 @@ GatherPlanJob gather_plan_job(const float *map, const float *iw, float2 *gmap, c
                        (int)(((MN + 63) / 64 * 64 * K + 255) / 256)};
 }
 
-// ---- fp32 on the bf16 matrix instructions (mcx_conv_split.h) ----
+// ---- fp32 on the bf16 matrix instructions (mcx_conv_split.hip) ----
 // Room for the flags (a word per tile of the B x OH x OW outputs) and the split weights, at the end
 // of a product's scratch.
 int64_t split_tiles(int64_t B, int64_t OH, int64_t OW) {
@@ -2568,49 +2554,6 @@ bool split_applies(int64_t G, int64_t O, int64_t SH, int64_t SW, int64_t K, cons
   if (SH * SW * (cl ? Gpad : G) * 4 >= (int64_t)kOobOffset) return false;
   if (cl) return m.mode == kInterpNearest && m.np <= 4;
   return packed ? m.np == 4 : m.np == 1;
-}
-
-int launch_gather_split(SplitArgs a, const PixelTiling &t, bool cl, hipStream_t s) {
-  a.tiles_x = t.tiles_x;
-  a.tiles_per_img = t.tiles_per_img;
-  a.tw_shift = t.tw_shift;
-  // Blocks of 32 outputs a workgroup computes: a block of zeros costs as many matrix instructions
-  // as one of weights, and its accumulators the registers of a fourth wave.  (Always two or four of
-  // them, against this: 4 x 64 -> 32 channels onto 256 x 512, transposed, forward and backward 450 us, 413;
-  // 3 x 24 -> 40 of 125 x 250, whose input gradient has 24, 257 and 253.  Three blocks keep the two waves
-  // of four.)
-  const int blocks = (a.O + 31) / 32;
-  const int nb = blocks == 1 ? 1 : blocks == 3 ? 3 : a.Opad % (2 * kOT) == 0 ? 4 : 2;
-  const dim3 grid((unsigned)t.total, (unsigned)((blocks + nb - 1) / nb));
-#define MCX_SPLIT(KERNEL, ...) \
-  hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(kThreads), 0, s, a)
-#define MCX_SPLIT_NB(KERNEL, ...)                      \
-  switch (nb) {                                        \
-    case 1: MCX_SPLIT(KERNEL, __VA_ARGS__, 1); break;  \
-    case 2: MCX_SPLIT(KERNEL, __VA_ARGS__, 2); break;  \
-    case 3: MCX_SPLIT(KERNEL, __VA_ARGS__, 3); break;  \
-    default: MCX_SPLIT(KERNEL, __VA_ARGS__, 4); break; \
-  }
-  if (cl) {
-    if (a.map2) {
-      MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, true)
-    } else {
-      switch (a.packed ? 4 : a.np) {
-        case 1: MCX_SPLIT_NB(gather_product_split_cl_kernel, 1, false) break;
-        case 2: MCX_SPLIT_NB(gather_product_split_cl_kernel, 2, false) break;
-        case 3: MCX_SPLIT_NB(gather_product_split_cl_kernel, 3, false) break;
-        default: MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, false) break;
-      }
-    }
-  } else if (!a.packed && a.ncorn == 1) {
-    MCX_SPLIT_NB(gather_product_split_kernel, 1)
-  } else {
-    MCX_SPLIT_NB(gather_product_split_kernel, 4)
-  }
-#undef MCX_SPLIT_NB
-#undef MCX_SPLIT
-  MCX_HIP_CHECK_LAUNCH();
-  return 0;
 }
 
 // Whether launch_gather_product reads blocks of eight channels: the packing launch makes them then.
@@ -2715,8 +2658,9 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
       a.ncorn = m.mode == kInterpNearest ? 1 : 4;
       a.weighted = m.weighted; a.wrap = m.wrap; a.packed = packed_map ? 1 : 0;
       a.run_if_zero = run_if_zero; a.mask_words = mask_words;
+      a.tiles_x = t.tiles_x; a.tiles_per_img = t.tiles_per_img; a.tw_shift = t.tw_shift;
       profile_begin(s);
-      const int rc = launch_gather_split(a, t, cl, s);
+      const int rc = launch_gather_split(a, t.total, cl, s);
       profile_end(s);
       if (rc) return rc;
       // the fp32 form below recomputes the tiles that have a result that is not finite

@@ -1,7 +1,7 @@
 // Weight gradient of fp32 images over maps whose neighbouring pixels sample neighbouring pixels
 // (every kernel of an equirectangular projection: along a row of the image a tap moves with the
 // pixel), on the bf16 matrix instructions with both operands split into three bf16 parts as in
-// mcx_conv_split.h.
+// mcx_conv_split.hip.
 //   gW[a,g,k] = sum_{b,n} plain[b,a,n] * sample(gath[b,g], map[n,k])
 //   * The sum runs over pixels, so a lane's matrix operand is eight consecutive pixels of one
 //     channel.  Where the eight taps of such a group read a run of neighbouring pixels, a thread

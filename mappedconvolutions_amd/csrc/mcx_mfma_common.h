@@ -1,5 +1,5 @@
 // What the matrix-core kernels share: operand types, the exact split of fp32 values into three
-// bf16 parts (mcx_conv_split.h says what it is for), and the order of workgroups over the chip.
+// bf16 parts (mcx_conv_split.hip says what it is for), and the order of workgroups over the chip.
 #pragma once
 
 #include "mcx_taps.h"
@@ -20,6 +20,8 @@ __device__ inline float dot_bf16(unsigned word, unsigned w, float acc) {
 }
 
 constexpr int kTilePx = 128;  // pixels of a tile
+constexpr int kGC = 16;       // source channels per reduction chunk
+constexpr int kOT = 64;       // outputs are padded to a multiple of this
 
 // Factor of the weights and of the samples before they are split.
 constexpr float kSplitScale = 16777216.f;  // 2^24
@@ -47,6 +49,16 @@ __device__ inline void split8(const float *x, bf16x8 *p) {
   p[0] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
   p[1] = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
   p[2] = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// Whether a pair beyond the first two of a tap is in use anywhere in the map, from the pair
+// mask: one word (at least 4 then), or `words` words of which any may say so (one per block
+// of the launch that examined the map).  Called by whole waves.
+__device__ inline bool later_pairs_in_use(const int *__restrict__ mask, int words) {
+  if (words <= 1) return (unsigned)*mask >= (1u << 2);
+  const int lane = threadIdx.x & 63;
+  const unsigned v = (unsigned)mask[lane < words ? lane : 0];
+  return __builtin_amdgcn_ballot_w64(v >= (1u << 2)) != 0;
 }
 
 // Workgroups are dealt round-robin to the 8 XCDs; give every XCD one contiguous
