@@ -46,8 +46,6 @@ namespace mcx {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTapCache = 12;  // cached (offset, weight) pairs per tile pixel (12 KB of LDS)
-
 // Channels between the two halves of chunk c of a planar source.
 __device__ inline int split_upper_half(int c, int G) {
   const int rem = G - c * 16;
@@ -88,15 +86,16 @@ struct SplitWeights {
 };
 
 template <int NB>
-__device__ inline void split_products(const uint4 *lds, const bf16x8 *b, int l31, int lhi,
-                                      floatx16 *acc) {
-  bf16x8 a[NB][3];
+__device__ inline void read_split_weights(const uint4 *lds, int l31, int lhi, bf16x8 (*a)[3]) {
 #pragma unroll
   for (int m = 0; m < NB; m++)
 #pragma unroll
     for (int part = 0; part < 3; part++)
       a[m][part] =
           __builtin_bit_cast(bf16x8, lds[(part * 2 + lhi) * (32 * NB) + 32 * m + l31]);
+}
+template <int NB>
+__device__ inline void split_products(const bf16x8 (*a)[3], const bf16x8 *b, floatx16 *acc) {
   // (smallest first; the chains of the output blocks are independent)
   constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
@@ -165,18 +164,43 @@ __device__ inline void split_epilogue(const SplitArgs &s, floatx16 *acc, const f
 }
 
 // Planar images.  NE: (offset, weight) entries per tap, 1 or 4; with 4, tiles none of whose taps
-// uses a later entry run with the leading two.  Two entries of a tap that are neighbours in
-// memory for every pixel of the tile (the corners of a row, two contributions of a
-// transposed map) are fetched with one 8-byte load: the texture path takes 16 clocks for a
-// wave's load whatever its width, and 16 single loads a unit would cost it as much as the fp32
-// matrix instructions did.
-template <int NE, int NB>
-__global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) void gather_product_split_kernel(
-    const SplitArgs s) {
-  constexpr int kCache = NE == 1 ? 6 : kTapCache;  // cached entries per pixel
+// uses a later entry run with the leading two.  NB: blocks of 32 outputs.
+//
+// The taps go in groups.  In memory (in_memory): two entries of a tap that are neighbours in memory for
+// every pixel of the tile (the corners of a row, two contributions of a transposed map) are
+// fetched with one 8-byte load; the texture path takes 16 to 25 clocks for a wave's load whatever its
+// width, and 16 single loads a unit would cost it as much as the fp32 matrix instructions did.
+//
+// WINDOW: with four entries a tap that is still 16 loads a unit, and one block of outputs has few
+// matrix instructions to hide even eight.  Where the entries of a group's 128 pixels lie in a small box of
+// the source - those of every kernel over an image do, but next to the poles and at random maps - the
+// box goes into LDS, 16 channels at a time, four channels of a pixel in 16 bytes (a wave copies four of the
+// channels with 16-byte loads, the next chunk's on their way while this one's are multiplied), and an
+// entry is two 16-byte reads of LDS.  A group whose box is too large is tried again in threes of taps, then
+// goes the way through memory.
+constexpr int kMemCache = 12;            // entries a pixel of a group in memory, offsets of 32 bits
+constexpr int kWinCache = 12;            // of a group in a window, offsets of 16 bits
+constexpr int kTapBytes = kMemCache * kTilePx * 8;
+constexpr int kWinPx = 256;              // pixels of a window
+
+// Where pixel i of a window lies: fours of pixels that eight lanes store together are on different banks.
+__device__ inline int window_place(int i) { return i ^ ((i >> 3) & 3); }
+
+// q / d for 0 <= q < 2^31, 0 < d, where the quotient is below 2^16: the estimate is off by one at most.
+__device__ inline int quotient(int q, int d, float inv) {
+  int r = (int)((float)q * inv);
+  r -= r * d > q ? 1 : 0;
+  r += (r + 1) * d <= q ? 1 : 0;
+  return r;
+}
+
+template <int NE, int NB, bool WINDOW>
+__global__ __launch_bounds__(kThreads, NB > 2 ? 2 : !WINDOW && (NE == 1 || NB == 1) ? 4 : 3) void
+gather_product_split_kernel(const SplitArgs s) {
   __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<NB>::kPieces];
-  __shared__ __attribute__((aligned(16))) unsigned TapOff[kCache * kTilePx];
-  __shared__ __attribute__((aligned(16))) float TapWt[kCache * kTilePx];
+  __shared__ __attribute__((aligned(16))) float4 Win[4][kWinPx];  // [channel / 4][pixel]
+  __shared__ __attribute__((aligned(16))) char TapMem[kTapBytes];
+  __shared__ __attribute__((aligned(16))) int box[6][4];  // largest values by wave
   __shared__ __attribute__((aligned(16))) float Bias[32 * NB];
   __shared__ int unpaired;
   if (s.gate && ((*s.gate == 0) != (s.run_if_zero != 0))) return;
@@ -222,7 +246,223 @@ __global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) 
   split_bias<NB>(s, Bias, o0);
   int buf = 0;
 
-  // units of a tap group: chunk-major, the tap fastest (a chunk's source rows stay in cache)
+  // ---- a group in a window: rows of `cols` pixels, a multiple of four, from (row0, col0) on, columns
+  // cyclic, fours of them next to each other in the source ----
+  uint16_t *const win_off = reinterpret_cast<uint16_t *>(TapMem);  // (place in the window)
+  float *const win_wt = reinterpret_cast<float *>(TapMem + kWinCache * kTilePx * 2);
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  auto units_in_window = [&](int k0, int kn, auto na_tag, int row0, int col0, int cols,
+                             int rows) __attribute__((always_inline)) {
+    constexpr int NA = decltype(na_tag)::value;
+    // the four pixels that this lane copies, of this wave's four channels of every chunk
+    const int fours = cols >> 2;
+    const int r = quotient(lane, fours, 1.f / (float)fours);
+    int x4 = col0 + 4 * (lane - r * fours);
+    x4 -= x4 >= s.SW ? s.SW : 0;
+    const unsigned from =
+        lane < rows * fours ? (unsigned)((row0 + r) * s.SW + x4) * 4u : kOobOffset;
+    const unsigned to = (unsigned)(wave * kWinPx + window_place(4 * lane)) * 16u;  // (in Win)
+    f32x4 held[4];
+    // (the last chunk, which may hold few channels, comes first: its products round small sums)
+    auto fetch = [&](int c) __attribute__((always_inline)) {
+      const int cc = max(chunks - 1 - c, 0), last = s.G - 1 - cc * kGC;
+      const int first = cc * kGC + (wave >> 1 ? split_upper_half(cc, s.G) : 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const unsigned so = (unsigned)(first + min((wave & 1) * 4 + i, last)) * plane_bytes;
+        held[i] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       img, (int)from, (int)__builtin_amdgcn_readfirstlane(so), 0));
+      }
+    };
+    auto fill = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        *reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(&Win[0][0]) + (to ^ (j * 16u))) =
+            f32x4{held[0][j], held[1][j], held[2][j], held[3][j]};
+    };
+    f32x4 v[2][NA];
+    float wgt[NA];
+    typename SplitWeights<NB>::u32x4 wv[SplitWeights<NB>::kPer];
+    auto load_weights = [&](int kl, int c) __attribute__((always_inline)) {
+      const int unit = (k0 + kl) * chunks + max(chunks - 1 - c, 0);
+      wts.load(wbuf, __builtin_amdgcn_readfirstlane((unsigned)unit * w_unit), wv);
+    };
+    auto read = [&](int kl) __attribute__((always_inline)) {
+      unsigned at[NA];
+#pragma unroll
+      for (int i = 0; i < NA; i++) at[i] = win_off[(kl * kTilePx + pe) * NA + i] * 16u;
+#pragma unroll
+      for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          v[q][i] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(&Win[q][0]) +
+                                                     at[i] + (unsigned)lhi * (2u * kWinPx * 16u));
+#pragma unroll
+      for (int i = 0; i < NA; i++) wgt[i] = win_wt[(kl * kTilePx + pe) * NA + i];
+    };
+    // One unit: its samples split, the next one's weights and samples on their way, the products.  The
+    // next chunk's pixels (FIRST: after the loads of the weights that the next unit waits for) have two units' time.
+    auto unit = [&](int kl, int c, auto first_tag) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_tag)::value;
+      const bool turn = kl + 1 == kn;
+      const int next = turn ? 0 : kl + 1;  // (past the last unit it is read again)
+      bf16x8 bq[3];
+      float sv[8];
+#pragma unroll
+      for (int ch = 0; ch < 8; ch++) {
+        sv[ch] = wgt[0] * v[ch >> 2][0][ch & 3];
+#pragma unroll
+        for (int i = 1; i < NA; i++) sv[ch] = __builtin_fmaf(wgt[i], v[ch >> 2][i][ch & 3], sv[ch]);
+      }
+      split8(sv, bq);
+      wts.store(Wt[buf], wv);
+      load_weights(next, turn ? c + 1 : c);
+      if constexpr (FIRST) fetch(c + 1);
+      __syncthreads();  // the weights are there, and every wave has read this unit's samples
+      if (turn && c + 1 < chunks) {
+        fill();
+        __syncthreads();
+      }
+      read(next);
+      bf16x8 a[NB][3];
+      read_split_weights<NB>(Wt[buf], l31, lhi, a);
+      split_products<NB>(a, bq, acc);
+      buf ^= 1;
+    };
+    fetch(0);
+    load_weights(0, 0);
+    fill();
+    __syncthreads();
+    read(0);
+    for (int c = 0; c < chunks; c++) {
+      unit(0, c, std::true_type());
+      if (kn > 1) {
+        unit(1, c, std::false_type());
+        for (int kl = 2; kl < kn; kl++) unit(kl, c, std::false_type());
+      }
+    }
+  };
+  // Resolves taps k0 .. k0 + kn - 1 and multiplies them if they fit a window; returns whether they did.
+  const float inv_sw = 1.f / (float)s.SW;
+  auto in_window = [&](int k0, int kn, auto na_tag) __attribute__((always_inline)) {
+    constexpr int NA = decltype(na_tag)::value;
+    constexpr int kMine = NA == 4 ? 2 : 3;  // of three or six taps
+    // (every load is issued before the first is used; past the group's end its last tap is read)
+    constexpr int kRaw = NE == 1 ? 1 : NA;
+    float2 raw[kMine][kRaw];
+    float raw_w[kMine];
+#pragma unroll
+    for (int j = 0; j < kMine; j++) {
+      const int k = k0 + min(half + 2 * j, kn - 1);
+      raw_w[j] = 1.f;
+      if (s.packed) {
+        // pre-resolved entries [tap][slot][pixel]: (pixel index as bits, weight)
+#pragma unroll
+        for (int i = 0; i < kRaw; i++)
+          raw[j][i] = reinterpret_cast<const float2 *>(s.map)[((int64_t)k * 4 + i) * N + n_g];
+      } else {
+        const int64_t e = n_g * s.K + k;
+        raw[j][0] = reinterpret_cast<const float2 *>(s.map)[e];
+        if (s.weighted) raw_w[j] = s.iw[e];
+      }
+    }
+    unsigned cell[kMine][NA];  // row << 16 | column
+    // largest row, column, column with the left half of the image moved to the right of the other
+    // (a seam), and the same of their negatives
+    int most[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) most[i] = -0x7fffffff;
+#pragma unroll
+    for (int j = 0; j < kMine; j++) {
+      const int kl = half + 2 * j;
+      if (kl < kn) {
+        float wt[NA];
+        int y[NA], x[NA];
+        if (s.packed) {
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            const float2 q = raw[j][i < kRaw ? i : 0];
+            wt[i] = live ? q.y * kSplitScale : 0.f;
+            const int e = wt[i] != 0.f ? __builtin_bit_cast(int, q.x) : 0;
+            y[i] = quotient(e, s.SW, inv_sw);
+            x[i] = e - y[i] * s.SW;
+          }
+        } else {
+          CoordTap<NE> t;
+          resolve_coords<NE>(raw[j][0].x, raw[j][0].y, s.SH, s.SW, s.wrap != 0,
+                             live ? raw_w[j] * kSplitScale : 0.f, t);
+#pragma unroll
+          for (int i = 0; i < NA; i++) {
+            wt[i] = (t.ok >> i) & 1u ? t.wt[i] : 0.f;
+            y[i] = t.yy[i];
+            x[i] = t.xx[i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+          const bool use = wt[i] != 0.f;
+          const int turned = x[i] < s.SW / 2 ? x[i] + s.SW : x[i];
+          most[0] = max(most[0], use ? y[i] : -0x7fffffff);
+          most[1] = max(most[1], use ? -y[i] : -0x7fffffff);
+          most[2] = max(most[2], use ? x[i] : -0x7fffffff);
+          most[3] = max(most[3], use ? -x[i] : -0x7fffffff);
+          most[4] = max(most[4], use ? turned : -0x7fffffff);
+          most[5] = max(most[5], use ? -turned : -0x7fffffff);
+          cell[j][i] = use ? (unsigned)y[i] << 16 | (unsigned)x[i] : 0xffffffffu;
+          win_wt[(kl * kTilePx + p) * NA + i] = wt[i];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+      most[i] = wave_max(most[i]);
+      if (lane == 0) box[i][wave] = most[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+      most[i] = __builtin_amdgcn_readfirstlane(
+          max(max(box[i][0], box[i][1]), max(box[i][2], box[i][3])));
+    const bool none = most[0] < 0;  // no entry in use: pixel 0 stands for all
+    const int plain = most[2] + most[3], turned = most[4] + most[5];
+    const int rows = none ? 1 : most[0] + most[1] + 1;
+    const int row0 = none ? 0 : -most[1];
+    int col0 = none ? 0 : plain <= turned ? -most[3] : -most[5];
+    col0 -= col0 >= s.SW ? s.SW : 0;
+    int cols = none ? 1 : min(plain, turned) + 1;
+    // fours of columns, none of which has the seam inside
+    const bool seam = col0 + cols > s.SW;
+    if (seam) {
+      const int back = (col0 - s.SW) & 3;
+      cols += back;
+      col0 -= back;
+    }
+    cols = (cols + 3) & ~3;
+    if (!seam && col0 + cols > s.SW) col0 = s.SW - cols;
+    if (cols > kWinPx || rows > kWinPx || rows * cols > kWinPx || cols > s.SW || col0 < 0) return false;
+#pragma unroll
+    for (int j = 0; j < kMine; j++) {
+      const int kl = half + 2 * j;
+      if (kl < kn) {
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+          int x = (int)(cell[j][i] & 0xffffu) - col0;
+          x += x < 0 ? s.SW : 0;
+          const int at = ((int)(cell[j][i] >> 16) - row0) * cols + x;
+          win_off[(kl * kTilePx + p) * NA + i] =
+              (uint16_t)(cell[j][i] == 0xffffffffu ? 0 : window_place(at));
+        }
+      }
+    }
+    units_in_window(k0, kn, na_tag, row0, col0, cols, rows);
+    return true;
+  };
+
+  // ---- a group in memory ----
+  unsigned *const TapOff = reinterpret_cast<unsigned *>(TapMem);
+  float *const TapWt = reinterpret_cast<float *>(TapMem + kMemCache * kTilePx * 4);
+  // its units: chunk-major, the tap fastest (a chunk's source rows stay in cache)
   auto units_of = [&](int k0, int kn, auto na_tag, auto paired_tag) __attribute__((always_inline)) {
     constexpr int NA = decltype(na_tag)::value;
     constexpr bool PAIRED = decltype(paired_tag)::value;
@@ -295,7 +535,11 @@ __global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) 
         stage(d);
         __syncthreads();
         issue(d);
-        split_products<NB>(Wt[buf], bq, l31, lhi, acc);
+        {
+          bf16x8 a[NB][3];
+          read_split_weights<NB>(Wt[buf], l31, lhi, a);
+          split_products<NB>(a, bq, acc);
+        }
         buf ^= 1;
       }
     }
@@ -304,17 +548,20 @@ __global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) 
       if (u + d < units) {
         stage(d);
         __syncthreads();
-        split_products<NB>(Wt[buf], bq, l31, lhi, acc);
+        {
+          bf16x8 a[NB][3];
+          read_split_weights<NB>(Wt[buf], l31, lhi, a);
+          split_products<NB>(a, bq, acc);
+        }
         buf ^= 1;
       }
     }
   };
-
-  auto run = [&](auto na_tag) __attribute__((always_inline)) {
+  auto in_memory = [&](int from, int count, auto na_tag) __attribute__((always_inline)) {
     constexpr int NA = decltype(na_tag)::value;
-    constexpr int TG = kCache / NA;
-    for (int k0 = 0; k0 < s.K; k0 += TG) {
-      const int kn = min(TG, s.K - k0);
+    constexpr int TG = (NE == 1 ? kMemCache / 2 : kMemCache) / NA;
+    for (int k0 = from; k0 < from + count; k0 += TG) {
+      const int kn = min(TG, from + count - k0);
       __syncthreads();  // the previous group's units are done with the cache
       if (tid == 0) unpaired = NA == 1 ? 1 : 0;
       __syncthreads();
@@ -384,6 +631,30 @@ __global__ __launch_bounds__(kThreads, NB > 2 ? 2 : NE == 1 || NB == 1 ? 4 : 3) 
         }
       }
       units_of(k0, kn, na_tag, std::false_type());
+    }
+  };
+  auto run = [&](auto na_tag) __attribute__((always_inline)) {
+    constexpr int NA = decltype(na_tag)::value;
+    // (two entries a tap of 64 outputs and more: as fast in memory, with the registers of a third wave)
+    if (!WINDOW || (NE == 4 && NA == 2 && NB > 1)) return in_memory(0, s.K, na_tag);
+    constexpr int kMost = kWinCache / NA < 6 ? kWinCache / NA : 6, kFew = 3;
+    // (groups of one size, as far as it goes; a window that holds six taps' pixels holds three of nearly
+    // twice the spread)
+    const int groups = (s.K + kMost - 1) / kMost;
+    int kg = (s.K + groups - 1) / groups;
+    const bool small = s.SH <= 0xffff && s.SW <= 0xffff;
+    for (int k0 = 0; k0 < s.K;) {
+      const int kn = min(kg, s.K - k0);
+      __syncthreads();  // the previous group's units are done with the taps and the window
+      if (!small || !in_window(k0, kn, na_tag)) {
+        if (small && kn > kFew) {
+          kg = kFew;
+          continue;
+        }
+        __syncthreads();
+        in_memory(k0, kn, na_tag);
+      }
+      k0 += kn;
     }
   };
   if (NE == 4 && leading)
@@ -570,7 +841,9 @@ __global__ __launch_bounds__(kThreads, TWO || NE * NB > 8 ? 2 : 3) void gather_p
       }
       issue(k, c);
     }
-    split_products<NB>(Wt[buf], bq, l31, lhi, acc);
+    bf16x8 a[NB][3];
+    read_split_weights<NB>(Wt[buf], l31, lhi, a);
+    split_products<NB>(a, bq, acc);
     buf ^= 1;
   }
   split_epilogue<NB>(s, acc, Bias, tile, b, o0, ei, ej, lhi);
@@ -586,33 +859,55 @@ int launch_gather_split(const SplitArgs &a, int64_t tiles, bool cl, hipStream_t 
   // of four.)
   const int blocks = (a.O + 31) / 32;
   const int nb = blocks == 1 ? 1 : blocks == 3 ? 3 : a.Opad % (2 * kOT) == 0 ? 4 : 2;
-  const dim3 grid((unsigned)tiles, (unsigned)((blocks + nb - 1) / nb));
+  // Two images a workgroup where their accumulators leave two waves a SIMD and the chip is full all
+  // the same.
+  const int64_t by_outputs = (blocks + nb - 1) / nb;
+  // Windows (gather_product_split_kernel) where the grid is three workgroups a CU and more - with fewer,
+  // each waits out a group's taps and then its window, where the form in memory has its loads in flight
+  // - and where two chunks of channels and more share the taps' work; not with four blocks of outputs,
+  // whose matrix instructions hide the loads.  In memory and in windows: 8 x 64 -> 64 channels of 256 x 512, four
+  // corners, 770 us and 669; 3 x 64 -> 64 of 128 x 256 95 and 84; 8 x 32 -> 96 of 128 x 256 156 and 147; 3 x 24 -> 40 of
+  // 125 x 250, a training pass, 246 and 213; 4 x 64 -> 32 onto 256 x 512, transposed, 380 and 355.  Against
+  // them: 4 x 32 -> 32 of 64 x 128 (256 workgroups) 31.3 and 34.4; 8 x 8 -> 3 onto 256 x 512, transposed, 159 and
+  // 188; 4 x 16 -> 20 of 128 x 256 32 and 38; 2 x 40 -> 128 of 128 x 256, 5 x 5, 159 and 176.
+  const bool window = tiles * by_outputs >= 768 && a.G > kGC && nb < 4;
+  const dim3 grid((unsigned)tiles, (unsigned)by_outputs);
 #define MCX_SPLIT(KERNEL, ...) \
   hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(kThreads), 0, s, a)
-#define MCX_SPLIT_NB(KERNEL, ...)                      \
-  switch (nb) {                                        \
-    case 1: MCX_SPLIT(KERNEL, __VA_ARGS__, 1); break;  \
-    case 2: MCX_SPLIT(KERNEL, __VA_ARGS__, 2); break;  \
-    case 3: MCX_SPLIT(KERNEL, __VA_ARGS__, 3); break;  \
-    default: MCX_SPLIT(KERNEL, __VA_ARGS__, 4); break; \
+#define MCX_SPLIT_CL(...)                                                       \
+  switch (nb) {                                                                 \
+    case 1: MCX_SPLIT(gather_product_split_cl_kernel, __VA_ARGS__, 1); break;   \
+    case 2: MCX_SPLIT(gather_product_split_cl_kernel, __VA_ARGS__, 2); break;   \
+    case 3: MCX_SPLIT(gather_product_split_cl_kernel, __VA_ARGS__, 3); break;   \
+    default: MCX_SPLIT(gather_product_split_cl_kernel, __VA_ARGS__, 4); break;  \
+  }
+#define MCX_SPLIT_PLANAR(NE, WINDOW)                                                   \
+  switch (nb) {                                                                        \
+    case 1: MCX_SPLIT(gather_product_split_kernel, NE, 1, WINDOW); break;              \
+    case 2: MCX_SPLIT(gather_product_split_kernel, NE, 2, WINDOW); break;              \
+    case 3: MCX_SPLIT(gather_product_split_kernel, NE, 3, WINDOW); break;              \
+    default: MCX_SPLIT(gather_product_split_kernel, NE, 4, false); break;              \
   }
   if (cl) {
     if (a.map2) {
-      MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, true)
+      MCX_SPLIT_CL(4, true)
     } else {
       switch (a.packed ? 4 : a.np) {
-        case 1: MCX_SPLIT_NB(gather_product_split_cl_kernel, 1, false) break;
-        case 2: MCX_SPLIT_NB(gather_product_split_cl_kernel, 2, false) break;
-        case 3: MCX_SPLIT_NB(gather_product_split_cl_kernel, 3, false) break;
-        default: MCX_SPLIT_NB(gather_product_split_cl_kernel, 4, false) break;
+        case 1: MCX_SPLIT_CL(1, false) break;
+        case 2: MCX_SPLIT_CL(2, false) break;
+        case 3: MCX_SPLIT_CL(3, false) break;
+        default: MCX_SPLIT_CL(4, false) break;
       }
     }
   } else if (!a.packed && a.ncorn == 1) {
-    MCX_SPLIT_NB(gather_product_split_kernel, 1)
+    MCX_SPLIT_PLANAR(1, false)
+  } else if (window) {
+    MCX_SPLIT_PLANAR(4, true)
   } else {
-    MCX_SPLIT_NB(gather_product_split_kernel, 4)
+    MCX_SPLIT_PLANAR(4, false)
   }
-#undef MCX_SPLIT_NB
+#undef MCX_SPLIT_CL
+#undef MCX_SPLIT_PLANAR
 #undef MCX_SPLIT
   MCX_HIP_CHECK_LAUNCH();
   return 0;

@@ -116,6 +116,20 @@ __device__ inline double_pair buf_load_pair(plane_buf_t r, unsigned byte_off, do
                             __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte_off, 0, 0));
 }
 
+// Largest value of the wave (all 64 lanes active), by data-parallel-primitive moves inside the
+// vector unit: shifts within rows of 16 lanes, then the rows' last lanes passed on; lanes a
+// step does not reach keep the identity.  (Shuffles go through LDS, a round trip per step.)
+__device__ inline int wave_max(int v) {
+  constexpr int kId = -0x7fffffff - 1;
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x114, 0xf, 0xe, false));  // row_shr:4
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x118, 0xf, 0xc, false));  // row_shr:8
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // ---- taps -----------------------------------------------------------------
 // A tap is one (x, y) sample location resolved against an H x W plane: up to
 // four in-plane element offsets and their weights.  Offsets are -1 for corners

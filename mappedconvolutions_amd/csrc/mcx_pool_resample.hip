@@ -285,20 +285,6 @@ struct WinShape {
 
 __device__ inline int cyc(int v, int w) { return v < 0 ? v + w : v; }  // v in (-w, w)
 
-// Largest value of the wave (all 64 lanes active), by data-parallel-primitive moves inside the
-// vector unit: shifts within rows of 16 lanes, then the rows' last lanes passed on; lanes a
-// step does not reach keep the identity.  (Shuffles go through LDS, a round trip per step.)
-__device__ inline int wave_max(int v) {
-  constexpr int kId = -0x7fffffff - 1;
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x111, 0xf, 0xf, false));  // row_shr:1
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x112, 0xf, 0xf, false));  // row_shr:2
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x114, 0xf, 0xe, false));  // row_shr:4
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x118, 0xf, 0xc, false));  // row_shr:8
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-  v = max(v, __builtin_amdgcn_update_dpp(kId, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-  return __builtin_amdgcn_readlane(v, 63);
-}
-
 // Returns false (wave-uniform) when the wave's taps do not fit windows; nothing is written then.
 template <typename T, int MODE, int OP>
 __device__ inline bool window_pool(const T *__restrict__ in, const T *__restrict__ map,

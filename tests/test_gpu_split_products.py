@@ -102,6 +102,50 @@ def test_outputs_in_blocks_of_32(co, mesh, device):
     assert ((got - want).abs()[ok] <= 1e-5 * want.abs().max()).all()
 
 
+def _wide_map(kind, h, w_, k, g):
+    """Maps whose tiles' boxes do and do not fit a window, at the seam and at both ends of the rows."""
+    smap = _grid(h, w_, k, 0.3, 0.4)
+    x, y = smap.unbind(-1)
+    if kind == "seam":  # columns that go round the image inside a tile
+        x = (x + w_ - 11.5) % w_
+    elif kind == "spread":  # taps from next to each other to half the image apart, row by row
+        x = x + torch.linspace(0, w_ / 2, h)[:, None, None] * (torch.arange(k) % 3 - 1)
+    elif kind == "steep":  # rows far apart
+        y = y + torch.linspace(-60, 60, w_)[None, :, None]
+    elif kind == "random":
+        x, y = torch.rand(h, w_, k, generator=g) * w_, torch.rand(h, w_, k, generator=g) * h
+    elif kind == "outside":  # tiles of which no tap is inside
+        x = torch.where((torch.arange(h) % 8 < 4)[:, None, None], x, x - 4 * w_)
+    return torch.stack((x, y), -1).contiguous()
+
+
+@pytest.mark.parametrize("kind", ["grid", "seam", "spread", "steep", "random", "outside"])
+@pytest.mark.parametrize("shape,ci,co,k", [((200, 512), 20, 30, 9), ((98, 1001), 33, 70, 5),
+                                           ((402, 250), 17, 9, 4), ((3, 33000), 24, 96, 1),
+                                           ((33000, 3), 18, 20, 3)])
+@pytest.mark.parametrize("interp,weighted", [(1, False), (2, False), (2, True)])
+def test_windows_of_pixels(kind, shape, ci, co, k, interp, weighted, device):
+    """Grids of 768 workgroups and more read their taps from a window of the source where they fit one.
+    32-bit sums of up to 9 * 33 terms against the oracle's 64-bit ones: a few 1e-7 of the largest result."""
+    g = torch.Generator().manual_seed(k)
+    h, w_ = shape
+    smap = _wide_map(kind, h, w_, k, g)
+    rnd = lambda *s: torch.randn(s, generator=g)
+    x, w, b, gy = rnd(1, ci, h, w_), rnd(co, ci, k), rnd(co), rnd(1, co, h, w_)
+    if weighted:
+        smap, iw = smap.unsqueeze(-2).contiguous(), torch.rand(h, w_, k, 1, generator=g)
+        fwd, bwd, maps = _C.weighted_mapped_conv_forward, _C.weighted_mapped_conv_backward, (smap, iw)
+        want, wbwd = O.weighted_mapped_conv_forward, O.weighted_mapped_conv_backward
+    else:
+        fwd, bwd, maps = _C.mapped_conv_forward, _C.mapped_conv_backward, (smap,)
+        want, wbwd = O.mapped_conv_forward, O.mapped_conv_backward
+    cu = lambda *ts: [t.cuda() for t in ts]
+    y = fwd(*cu(x, *maps, w, b), k, interp)
+    assert rel_err(y, want(x, *maps, w, b, k, interp)) < 1e-5
+    gx = bwd(*cu(gy, *maps, x, w, b), k, interp, needs=(True, False, False))[0]
+    assert rel_err(gx, wbwd(gy, *maps, x, w, b, k, interp)[0]) < 1e-5
+
+
 @pytest.mark.parametrize("what", ["x_inf", "x_nan", "w_inf", "overflow", "large"])
 def test_operands_without_a_split(what, device):
     """An infinity or NaN among the operands and sums beyond fp32 come out as the fp32
