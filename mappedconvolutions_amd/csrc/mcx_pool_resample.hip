@@ -1285,13 +1285,13 @@ __device__ inline void transposed_gather_planes(
     if (c < nc) d0[(int64_t)c * ndst] = OP == UN_AVG ? acc[c] / (T)K : acc[c];
 }
 
-// One workgroup: 256 destination pixels x `reps` groups of kTCH planes.
+// One workgroup: 256 destination pixels x `per` planes, kTCH at a time on the register paths.
 template <typename T, int OP>
 __global__ __launch_bounds__(kThreads, OP == UN_AVG ? 4 : OP == UN_MAX ? 3 : 1) void transposed_gather_kernel(
     const T *__restrict__ src, const int64_t *__restrict__ idx, T *__restrict__ dst,
     const uint32_t *__restrict__ local, const uint32_t *__restrict__ bsum,
     const uint32_t *__restrict__ e_src, const T *__restrict__ e_wt, int64_t planes, int nsrc,
-    int ndst, int K, int idx_scale, int groups, int reps, int windows) {
+    int ndst, int K, int idx_scale, int groups, int per, int windows) {
   constexpr int kTCH = planes_per_thread<OP>();
   // (the unpoolings: every XCD takes one contiguous run of the destination, so that the source
   // rows neighbouring destination rows share are read into one L2 only)
@@ -1302,8 +1302,8 @@ __global__ __launch_bounds__(kThreads, OP == UN_AVG ? 4 : OP == UN_MAX ? 3 : 1) 
   const int pc = live ? p : 0;
   const uint32_t start = local[pc] + bsum[pc / kScanBlock];
   const uint32_t end = local[pc + 1] + bsum[(pc + 1) / kScanBlock];
-  const int64_t first_plane = (int64_t)pg * reps * kTCH;
-  const int np = (int)min((int64_t)reps * kTCH, planes - first_plane);
+  const int64_t first_plane = (int64_t)pg * per;
+  const int np = (int)min((int64_t)per, planes - first_plane);
   if constexpr (OP != UN_RESAMPLE) {
     if (windows && window_unpool<T, OP>(src, idx, dst, e_src, e_wt, start, live ? end - start : 0u,
                                         live, p, first_plane, np, nsrc, ndst, K, idx_scale))
@@ -1332,6 +1332,16 @@ int fill(T *p, int64_t n, T v, hipStream_t s) {
   return 0;
 }
 
+// Planes a thread takes where whole ones leave SIMDs idle: halved until the grid is about two waves for
+// each of them, but not below sixteen, a third of what resolving a thread's taps or reading its list
+// costs.  (Average pooling of 64 planes of 249 x 498 to half the size, 500 waves of 64 planes: 73 us, so 28; its
+// gradient 66, 45.  1024 waves and 4096 instead of 2048: 29 and 27, 64 and 45; 128 planes of 128 x 256, forward 30 and
+// 25 against 25, gradient 25 and 24 against 21.)
+inline int fewer_planes(int per, int64_t waves, int64_t planes) {
+  while (per > 16 && waves * div_up(planes, per) < 2048) per /= 2;
+  return per;
+}
+
 template <typename T, int OP>
 int launch_gather(const void *in, const void *map, const void *iw, void *out, int64_t *idx,
                   int64_t B, int64_t C, int64_t IH, int64_t IW, int64_t MH, int64_t MW, int64_t K,
@@ -1349,6 +1359,7 @@ int launch_gather(const void *in, const void *map, const void *iw, void *out, in
     const int64_t waves = (int64_t)div_up(MW, Patch<OP>::kW) * div_up(MH, Patch<OP>::kH) *
                           (kThreads / 64);
     while (cpt < 1024 && cpt * 2 <= C && waves * div_up(C, cpt * 2) >= 8192) cpt *= 2;
+    cpt = fewer_planes(cpt, waves, C);
   }
   // Unweighted resampling: every thread walks a run of planes with a ring of loads in flight.
   // (images and channels are one run of planes, kCH of them per thread: longer runs measured
@@ -1479,7 +1490,9 @@ int gather_transposed(const void *src, const int64_t *idx, void *dst, const void
   while (windows && reps < 4 && (int64_t)reps * 2 * kTCH <= planes &&
          tiles * (kThreads / 64) * ((planes + reps * 2 * kTCH - 1) / (reps * 2 * kTCH)) >= 8192)
     reps *= 2;
-  const int64_t groups = (planes + reps * kTCH - 1) / (reps * kTCH);
+  int per = reps * kTCH;  // planes a workgroup
+  if (OP != UN_RESAMPLE && reps == 1) per = fewer_planes(per, tiles * (kThreads / 64), planes);
+  const int64_t groups = (planes + per - 1) / per;
   const int64_t blocks = groups * tiles;
   if (blocks > 0x7fffffffLL) return kNotApplicable;
   const char *base = (const char *)ws;
@@ -1487,7 +1500,7 @@ int gather_transposed(const void *src, const int64_t *idx, void *dst, const void
                      s, (const T *)src, idx, (T *)dst, (const uint32_t *)(base + l.local),
                      (const uint32_t *)(base + l.bsum), (const uint32_t *)(base + l.e_src),
                      (const T *)(base + l.e_wt), planes, (int)nsrc, (int)ndst, (int)K,
-                     (int)(pm * 2), (int)groups, reps, windows ? 1 : 0);
+                     (int)(pm * 2), (int)groups, per, windows ? 1 : 0);
   MCX_HIP_CHECK_LAUNCH();
   return 0;
 }

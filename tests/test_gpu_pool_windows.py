@@ -205,3 +205,17 @@ def test_weighted_unpoolings_through_windows(interp, device):
                                             K, interp)
     assert _rel(got_avg, want_avg) < 1e-5
     assert _rel(got_max, want_max) < 1e-5
+
+
+@pytest.mark.parametrize("planes", [15, 16, 17, 31, 33, 64, 65, 150, 600])
+@pytest.mark.parametrize("W,fractional", [(128, False), (128, True), (130, False)])
+def test_planes_are_spread_over_idle_simds(planes, W, fractional, device):
+    """Where whole runs of 64 planes would leave SIMDs idle a thread takes 32 or 16 of them: ragged last
+    groups, through windows, lists in registers (fractional rows) and rows that are no whole chunks."""
+    H = 40
+    g = torch.Generator().manual_seed(planes + W)
+    smap = synthetic.latitude_map(H, W, 1)
+    if fractional:
+        smap[..., 1] += 0.25
+    _check(torch.randn(1, planes, H, W, generator=g), smap, 9, 1)
+    _check_unpool(torch.randn(1, planes, H, W, generator=g), smap, H, W, 9, 1)
