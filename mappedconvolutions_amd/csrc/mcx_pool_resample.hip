@@ -736,6 +736,9 @@ __global__ __launch_bounds__(kThreads) void scan_sums_kernel(uint32_t *__restric
 // that order, and neighbouring lanes of the gather then read neighbouring sources
 // at the same step.  Lists longer than kSortMax stay as filled.
 constexpr uint32_t kSortMax = 512;
+// Lists of more entries than these in half of a wave's lanes go through the network, of fewer by insertion
+// in LDS (124 002 lists of 9 on average: with 2, 4 and 8 10, 12 and 20 us; 524 288 of 3: 18, 19 and 25).
+constexpr uint32_t kFewEntries = 2;
 
 // Batcher's odd-even merge sort for N keys (16 or 32) as a list of compare-exchange pairs, made
 // at compile time so that the unrolled network indexes registers statically.
@@ -759,124 +762,71 @@ constexpr SortNetwork make_network(int N) {
 }
 constexpr SortNetwork kNet32 = make_network(32), kNet16 = make_network(16);
 
+// Weights in the order of their bits: a negative one's turned over, the sign of the others set.
+__device__ inline uint32_t ordered_bits(float w) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, w);
+  return b & 0x80000000u ? ~b : b | 0x80000000u;
+}
+__device__ inline float from_ordered_bits(uint32_t b) {
+  return __builtin_bit_cast(float, b & 0x80000000u ? b & 0x7fffffffu : ~b);
+}
+
 // Sorts the list [start, end) of this lane (at most N entries) in registers: read once, run
 // through the network, written back.  Order: by source, ties by weight.
 template <typename T, int N>
 __device__ inline void network_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint32_t end) {
   constexpr const SortNetwork &net = N == 16 ? kNet16 : kNet32;
-  uint32_t code[N];
-  T w[N];
+  if constexpr (sizeof(T) == 4) {  // source and weight as one number of 64 bits
+    unsigned long long key[N];
 #pragma unroll
-  for (int u = 0; u < N; u++) {
-    const bool in = start + u < end;
-    code[u] = in ? e_src[start + u] : 0xffffffffu;  // padding sorts to the end
-    w[u] = in ? e_wt[start + u] : T(0);
-  }
+    for (int u = 0; u < N; u++)  // (padding sorts to the end)
+      key[u] = start + u < end
+                   ? (unsigned long long)e_src[start + u] << 32 | ordered_bits(e_wt[start + u])
+                   : ~0ull;
 #pragma unroll
-  for (int c = 0; c < net.n; c++) {
-    const int ia = net.a[c], ib = net.b[c];
-    const bool swap = code[ia] > code[ib] || (code[ia] == code[ib] && w[ia] > w[ib]);
-    const uint32_t ca = swap ? code[ib] : code[ia], cb = swap ? code[ia] : code[ib];
-    const T wa = swap ? w[ib] : w[ia], wb = swap ? w[ia] : w[ib];
-    code[ia] = ca; code[ib] = cb;
-    w[ia] = wa; w[ib] = wb;
-  }
+    for (int c = 0; c < net.n; c++) {
+      const unsigned long long ka = key[net.a[c]], kb = key[net.b[c]];
+      key[net.a[c]] = ka > kb ? kb : ka;
+      key[net.b[c]] = ka > kb ? ka : kb;
+    }
 #pragma unroll
-  for (int u = 0; u < N; u++) {
-    if (start + u < end) {
-      e_src[start + u] = code[u];
-      e_wt[start + u] = w[u];
+    for (int u = 0; u < N; u++) {
+      if (start + u < end) {
+        e_src[start + u] = (uint32_t)(key[u] >> 32);
+        e_wt[start + u] = from_ordered_bits((uint32_t)key[u]);
+      }
+    }
+  } else {
+    uint32_t code[N];
+    T w[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+      const bool in = start + u < end;
+      code[u] = in ? e_src[start + u] : 0xffffffffu;  // padding sorts to the end
+      w[u] = in ? e_wt[start + u] : T(0);
+    }
+#pragma unroll
+    for (int c = 0; c < net.n; c++) {
+      const int ia = net.a[c], ib = net.b[c];
+      const bool swap = code[ia] > code[ib] || (code[ia] == code[ib] && w[ia] > w[ib]);
+      const uint32_t ca = swap ? code[ib] : code[ia], cb = swap ? code[ia] : code[ib];
+      const T wa = swap ? w[ib] : w[ia], wb = swap ? w[ia] : w[ib];
+      code[ia] = ca; code[ib] = cb;
+      w[ia] = wa; w[ib] = wb;
+    }
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+      if (start + u < end) {
+        e_src[start + u] = code[u];
+        e_wt[start + u] = w[u];
+      }
     }
   }
 }
 
+// The list [start, end) of this lane where it lies.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void sort_entries_kernel(
-    const uint32_t *__restrict__ local, const uint32_t *__restrict__ bsum,
-    uint32_t *__restrict__ e_src, T *__restrict__ e_wt, int ndst) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  const bool live = p < ndst;
-  const uint32_t start = live ? local[p] + bsum[p / kScanBlock] : 0u;
-  const uint32_t end = live ? local[p + 1] + bsum[(p + 1) / kScanBlock] : 0u;
-  // Lists of up to kNetN entries in every lane of the wave (pooling and resampling maps):
-  // read once into registers, sorted by the network, written back.  Same order as the
-  // insertion sort below: by source, ties by weight.
-  // (a wave most of whose lists are very short is quicker with the insertion sort)
-  if (__builtin_amdgcn_ballot_w64(end - start > (uint32_t)kNetN) == 0 &&
-      __builtin_popcountll(__builtin_amdgcn_ballot_w64(end - start > 8u)) >= 32) {
-    if (__builtin_amdgcn_ballot_w64(end - start > 16u) == 0) {
-      // The lists of a wave's 64 pixels are one contiguous run of at most 1024 entries: it
-      // is copied to LDS and back with coalesced accesses, and each lane sorts its piece
-      // there (a lane's own list starts 15 or so words after its neighbour's: separate
-      // cache lines in memory, separate banks in LDS).
-      __shared__ uint32_t run_src[kThreads / 64][64 * 16];
-      __shared__ T run_wt[kThreads / 64][64 * 16];
-      const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-      const uint32_t first = __builtin_amdgcn_readfirstlane(start);  // lane 0 is live here
-      uint32_t last = end;
-      for (int d = 32; d > 0; d >>= 1) last = max(last, (uint32_t)__shfl_xor((int)last, d));
-      const uint32_t total = __builtin_amdgcn_readfirstlane(last) - first;
-      for (uint32_t t = lane; t < total; t += 64) {
-        run_src[wv][t] = e_src[first + t];
-        run_wt[wv][t] = e_wt[first + t];
-      }
-      __builtin_amdgcn_wave_barrier();
-      const uint32_t off = live ? start - first : 0u;
-      network_sort<T, 16>(run_src[wv], run_wt[wv], off, off + (end - start));
-      __builtin_amdgcn_wave_barrier();
-      for (uint32_t t = lane; t < total; t += 64) {
-        e_src[first + t] = run_src[wv][t];
-        e_wt[first + t] = run_wt[wv][t];
-      }
-    } else {
-      network_sort<T, 32>(e_src, e_wt, start, end);
-    }
-    return;
-  }
-  // Lists of 33 to 64 entries somewhere in the wave (5 x 5 pooling maps: about fifty): the
-  // wave sorts its lists one after the other, a lane per entry, by rank - the number of
-  // entries that come before it (by source, then weight, then position) - which is where the
-  // entry goes.  Same order as the insertion sort below, which took 5.4 ms for the 524 288
-  // lists of a 5 x 5 map on 512 x 1024.
-  {
-    const uint32_t len = live ? end - start : 0u;
-    const uint32_t longest = (uint32_t)wave_max((int)min(len, 0x7fffffffu));
-    if (longest > (uint32_t)kNetN && longest <= 64u) {
-      const uint32_t lane = threadIdx.x & 63;
-      for (int q = 0; q < 64; q++) {
-        const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)start, q);
-        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, q);
-        if (n < 2u) continue;  // wave-uniform
-        const bool mine = lane < n;
-        const uint32_t code = e_src[s + (mine ? lane : 0u)];
-        const T w = e_wt[s + (mine ? lane : 0u)];
-        uint32_t rank = 0;
-        for (uint32_t j = 0; j < n; j++) {  // (entry j sits in lane j)
-          const uint32_t cj = (uint32_t)__builtin_amdgcn_readlane((int)code, (int)j);
-          T wj;
-          if constexpr (sizeof(T) == 4) {
-            wj = __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), (int)j));
-          } else {
-            const long long wb = __builtin_bit_cast(long long, w);
-            const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)wb, (int)j);
-            const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(wb >> 32), (int)j);
-            wj = __builtin_bit_cast(T, (long long)(((unsigned long long)hi << 32) | lo));
-          }
-          const bool tie = !(wj < w) && !(w < wj);
-          rank += (cj < code || (cj == code && (wj < w || (tie && j < lane)))) ? 1u : 0u;
-        }
-        // (every lane has read the whole list before the first one writes: the stores depend
-        // on all of the wave's loads)
-        if (mine) {
-          e_src[s + rank] = code;
-          e_wt[s + rank] = w;
-        }
-      }
-      return;
-    }
-  }
-  if (!live) return;
-  if (end - start > kSortMax) return;
+__device__ inline void insertion_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint32_t end) {
   for (uint32_t i = start + 1; i < end; i++) {
     const uint32_t code = e_src[i];
     const T w = e_wt[i];
@@ -893,6 +843,118 @@ __global__ __launch_bounds__(kThreads) void sort_entries_kernel(
     e_src[j] = code;
     e_wt[j] = w;
   }
+}
+
+// The list [start, start + n) of one lane, n at most 64, sorted by the wave, a lane per entry, by
+// rank - the number of entries that come before it (by source, then weight, then position) -
+// which is where the entry goes.
+template <typename T>
+__device__ inline void rank_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint32_t n) {
+  const uint32_t lane = threadIdx.x & 63;
+  const bool mine = lane < n;
+  const uint32_t code = e_src[start + (mine ? lane : 0u)];
+  const T w = e_wt[start + (mine ? lane : 0u)];
+  uint32_t rank = 0;
+  if constexpr (sizeof(T) == 4) {
+    const uint32_t low = ordered_bits(w);
+    const unsigned long long key = (unsigned long long)code << 32 | low;
+    for (uint32_t j = 0; j < n; j++) {  // (entry j sits in lane j)
+      const unsigned long long other =
+          (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)code, (int)j) << 32 |
+          (uint32_t)__builtin_amdgcn_readlane((int)low, (int)j);
+      rank += (other < key || (other == key && j < lane)) ? 1u : 0u;
+    }
+  } else {
+    for (uint32_t j = 0; j < n; j++) {
+      const uint32_t cj = (uint32_t)__builtin_amdgcn_readlane((int)code, (int)j);
+      const long long wb = __builtin_bit_cast(long long, w);
+      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)wb, (int)j);
+      const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(wb >> 32), (int)j);
+      const T wj = __builtin_bit_cast(T, (long long)(((unsigned long long)hi << 32) | lo));
+      const bool tie = !(wj < w) && !(w < wj);
+      rank += (cj < code || (cj == code && (wj < w || (tie && j < lane)))) ? 1u : 0u;
+    }
+  }
+  // (every lane has read the whole list before the first one writes: the stores depend on all
+  // of the wave's loads)
+  if (mine) {
+    e_src[start + rank] = code;
+    e_wt[start + rank] = w;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries_kernel(
+    const uint32_t *__restrict__ local, const uint32_t *__restrict__ bsum,
+    uint32_t *__restrict__ e_src, T *__restrict__ e_wt, int ndst) {
+  const int p = blockIdx.x * kThreads + threadIdx.x;
+  const bool live = p < ndst;
+  const uint32_t start = live ? local[p] + bsum[p / kScanBlock] : 0u;
+  const uint32_t end = live ? local[p + 1] + bsum[(p + 1) / kScanBlock] : 0u;
+  // Lists of up to 64 entries in every lane of the wave (pooling and resampling maps).  Those
+  // of neighbouring pixels are one contiguous run, which is copied to LDS and back with
+  // coalesced accesses, as many lanes' lists at a time as surely fit; there each lane sorts its
+  // list (one that starts 15 or so words after its neighbour's: separate cache lines in memory,
+  // separate banks in LDS) in registers, of up to 16 or kNetN entries, and the wave one after the other the
+  // longer ones (5 x 5 pooling maps: about fifty entries).  Same order as the insertion sort below: by
+  // source, ties by weight.  What a wave waits for in LDS and memory bounds it, so its registers are kept to
+  // those of four waves a SIMD.  (With two waves a SIMD, insertion in memory for short lists, lists of 17 to 32
+  // sorted from memory and all lists of a wave by rank where one is longer: 524 288 lists of up to 16 entries 74 us,
+  // now 33; 320 000 of 9 to 40 429, now 190; 124 002 of up to 13 30, now 10.)
+  const uint32_t len = end - start;
+  const uint32_t longest = (uint32_t)wave_max((int)min(len, 0x7fffffffu));
+  if (longest < 2u) return;
+  if (longest <= 64u) {
+    const bool few = longest <= (uint32_t)kNetN &&
+                     __builtin_popcountll(__builtin_amdgcn_ballot_w64(len > kFewEntries)) < 32;
+    constexpr int kRun = 1024;
+    __shared__ uint32_t run_src[kThreads / 64][kRun];
+    __shared__ T run_wt[kThreads / 64][kRun];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lanes = longest <= 16u ? 64 : longest <= 32u ? 32 : 16;
+    for (int l0 = 0; l0 < 64; l0 += lanes) {
+      const bool mine = live && (unsigned)(lane - l0) < (unsigned)lanes;
+      const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)start, l0);
+      const uint32_t last = (uint32_t)wave_max(mine ? (int)end : 0);
+      const uint32_t total = last > first ? last - first : 0u;  // (no pixels here: 0)
+      for (uint32_t t = lane; t < total; t += 64) {
+        run_src[wv][t] = e_src[first + t];
+        run_wt[wv][t] = e_wt[first + t];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const uint32_t off = mine ? start - first : 0u;
+      if (few) {
+        insertion_sort<T>(run_src[wv], run_wt[wv], off, off + (mine ? len : 0u));
+      } else if (longest <= 16u) {
+        network_sort<T, 16>(run_src[wv], run_wt[wv], off, off + (mine ? len : 0u));
+      } else {
+        network_sort<T, kNetN>(run_src[wv], run_wt[wv], off,
+                               off + (mine && len <= (uint32_t)kNetN ? len : 0u));
+        unsigned long long left = __builtin_amdgcn_ballot_w64(mine && len > (uint32_t)kNetN);
+        for (; left != 0; left &= left - 1) {
+          const int q = __builtin_ctzll(left);
+          rank_sort<T>(run_src[wv], run_wt[wv], (uint32_t)__builtin_amdgcn_readlane((int)off, q),
+                       (uint32_t)__builtin_amdgcn_readlane((int)len, q));
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (uint32_t t = lane; t < total; t += 64) {
+        e_src[first + t] = run_src[wv][t];
+        e_wt[first + t] = run_wt[wv][t];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    return;
+  }
+  if (!live) return;
+  if (end - start > kSortMax) return;
+  insertion_sort<T>(e_src, e_wt, start, end);
 }
 
 // Planes per thread of the transposed gather's register paths.  The unpoolings read their list

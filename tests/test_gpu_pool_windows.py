@@ -219,3 +219,27 @@ def test_planes_are_spread_over_idle_simds(planes, W, fractional, device):
         smap[..., 1] += 0.25
     _check(torch.randn(1, planes, H, W, generator=g), smap, 9, 1)
     _check_unpool(torch.randn(1, planes, H, W, generator=g), smap, H, W, 9, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("long", [1, 2, 3, 8, 16, 17, 31, 32, 33, 48, 64, 65, 130])
+@pytest.mark.parametrize("pattern", ["all", "one", "mixed"])
+def test_lists_are_sorted_by_source(dtype, long, pattern, device):
+    """Lists of every length that a pixel's contributions are sorted in: the sums are those of adding
+    the contributions in the order of their sources, bit for bit."""
+    g = torch.Generator().manual_seed(long)
+    H, W = 3, 150
+    n = torch.full((H * W,), long if pattern == "all" else 1)
+    if pattern == "one":      # a single long list in the wave
+        n[::97] = long
+    elif pattern == "mixed":  # from none to the longest
+        n = torch.randint(0, long + 1, (H * W,), generator=g)
+    dest = torch.repeat_interleave(torch.arange(H * W), n)
+    dest = dest[torch.randperm(len(dest), generator=g)]
+    smap = torch.stack((dest % W, dest // W), -1).to(dtype).view(1, -1, 1, 2)
+    gy = torch.randn(1, 3, 1, len(dest), generator=g, dtype=dtype)
+    out = _C.mapped_avg_unpool(gy.cuda(), smap.cuda(), H, W, 1, 0).cpu().view(3, -1)
+    want = np.zeros((3, H * W), gy.numpy().dtype)
+    for i, d in enumerate(dest.tolist()):
+        want[:, d] += gy.numpy()[0, :, 0, i]
+    assert torch.equal(out, torch.from_numpy(want))
