@@ -410,6 +410,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
   // (bilinear corners of integral coordinates, unused slots) are neither loaded nor
   // accumulated.
   __shared__ unsigned TapMask[TG][2][2];
+  __shared__ __attribute__((aligned(16))) float Bias[kOT * OG];
   // nothing of this tile to recompute (see mcx_conv_split.hip)
   if (only_if && only_if[xcd_contiguous_tile(blockIdx.x, gridDim.x)] == 0) return;
   if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
@@ -441,6 +442,8 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
     if (leading != (run_if_leading != 0)) return;
   }
   const int o0 = blockIdx.y * (kOT * OG);
+  if (tid < kOT * OG)  // (there at the first barrier)
+    Bias[tid] = bias && o0 + tid < O ? to_f32(bias[o0 + tid]) : 0.f;
   const int N = OH * OW;
   const int64_t plane = (int64_t)SH * SW;
   const int64_t plane_bytes = plane * (int64_t)sizeof(TD);
@@ -790,21 +793,33 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
   const int pe = wave * 32 + l31;
   const int ei = tile_y * th + (pe >> tw_shift), ej = (tile_x << tw_shift) + (pe & tw_mask);
   if (ei < OH && ej < OW) {
-    TD *yb = y + (int64_t)b * O * N + (int64_t)ei * OW + ej;
-    // `addend`: a channel-last fp32 image [B][N][Opad] of contributions accumulated elsewhere
-    // (the overflow list of a transposed map, gate[1] entries long), added when there are any
-    const float *ab = (addend && gate && gate[1] > 0)
-                          ? addend + ((int64_t)b * N + (int64_t)ei * OW + ej) * Opad
-                          : nullptr;
+    TD *yb = y + ((int64_t)b * O + o0 + lhi * 4) * N + (int64_t)ei * OW + ej;
+    const int left = O - o0 - lhi * 4;  // outputs from yb's on
+    // (No load after the first store: a wait for it would be one for the stores before it as well:
+    // 8 x 3 -> 64 channels of 256 x 512, nine taps, 267 us with the biases read between them, now 248; bf16, 4 x
+    // 64 -> 64 of 128 x 256, nearest taps, 40 and 35.)
 #pragma unroll
     for (int m = 0; m < 2 * OG; m++)
 #pragma unroll
       for (int i = 0; i < 16; i++) {
-        const int o = o0 + 32 * m + (i >> 2) * 8 + lhi * 4 + (i & 3);
-        if (o < O) {
-          const float start = accumulate ? to_f32(yb[(int64_t)o * N]) : (bias ? to_f32(bias[o]) : 0.f);
-          yb[(int64_t)o * N] = from_f32<TD>(acc[m][i] + start + (ab ? ab[o] : 0.f));
-        }
+        const int o = 32 * m + (i >> 2) * 8 + (i & 3);
+        acc[m][i] += accumulate ? to_f32(yb[(int64_t)min(o, left - 1) * N]) : Bias[o + lhi * 4];
+      }
+    // `addend`: a channel-last fp32 image [B][N][Opad] of contributions accumulated elsewhere
+    // (the overflow list of a transposed map, gate[1] entries long), added when there are any
+    if (addend && gate && gate[1] > 0) {
+      const float *ab = addend + ((int64_t)b * N + (int64_t)ei * OW + ej) * Opad + o0 + lhi * 4;
+#pragma unroll
+      for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[m][i] += ab[32 * m + (i >> 2) * 8 + (i & 3)];
+    }
+#pragma unroll
+    for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int o = 32 * m + (i >> 2) * 8 + (i & 3);
+        if (o < left) yb[(int64_t)o * N] = from_f32<TD>(acc[m][i]);
       }
   }
 }
