@@ -165,13 +165,13 @@ __device__ inline void resolve_records(const double *__restrict__ map,
 }
 
 // The taps [k0, k0 + taps) of a workgroup's locations into its cache, [corner][tap][location].
-template <int NC, int LPR>
+template <int NC, int LPR, int TAPS = RecShape<LPR>::kTaps>
 __device__ inline void fill_tap_cache(const double *__restrict__ map,
                                       const double *__restrict__ iw, int n0, int N, int K, int pm,
                                       int p, int k0, int taps, int h, int w, bool wrap, int none,
                                       int *s_off, double *s_wt) {
   using S = RecShape<LPR>;
-  constexpr int kStep = S::kTaps * S::kLocs;
+  constexpr int kStep = TAPS * S::kLocs;
   for (int e = threadIdx.x; e < taps * S::kLocs; e += kThreads) {
     const int l = e / taps, t = e - l * taps;
     const int slot = t * S::kLocs + l;
@@ -335,29 +335,39 @@ __global__ __launch_bounds__(kThreads) void scatter_records_kernel(
 }
 
 // part[range][k][a][g] = sum over a range of (b, n) of plain[b,a,n] * sample(gath[b,g], map[n,k]).
-// A workgroup takes one tap, AT plain channels and 2 * LPR gathered ones; a tile is kSub runs of
-// kLocs locations, whose record reads are in flight together.
-template <int NC, int LPR, int AT>
+// A workgroup takes AT plain channels, 2 * LPR gathered ones and KT taps.  A tile is one run of kLocs
+// locations; for one tap it is kSub, whose record reads are in flight together.
+// KT is grad_taps<LPR, AT>(), as many as a lane has registers for the sums of, where there are locations
+// enough (grad_shape): the taps of a location are one piece of the map, and one by one each workgroup reads the
+// lines of all of them.
+template <int LPR, int AT>
+constexpr int grad_taps() { return AT == 1 ? RecShape<LPR>::kTaps : AT == 4 ? 3 : 1; }
+template <int NC, int LPR, int AT, int KT>
 __global__ __launch_bounds__(kThreads) void weight_grad_records_kernel(
     const double *__restrict__ plain, const double *__restrict__ rec,
     const double *__restrict__ map, const double *__restrict__ iw, double *__restrict__ part,
     int A, int G, int stride, int GH, int GW, int N, int K, int P, int wrap, int tiles_per_img,
     int64_t total_tiles, int ranges) {
   using S = RecShape<LPR>;
-  constexpr int kSub = LPR == 2 ? 2 : 4;  // (tiles of 128 or 256 locations)
+  constexpr int kSub = KT > 1 ? 1 : LPR == 2 ? 2 : 4;
   constexpr int kTile = kSub * S::kLocs;
-  __shared__ int s_off[NC * kTile];
-  __shared__ double s_wt[NC * kTile];
+  constexpr int kSlots = KT * kTile;  // of the tap cache: [tap][location]
+  __shared__ int s_off[NC * kSlots];
+  __shared__ double s_wt[NC * kSlots];
   __shared__ double s_plain[AT * kTile];
   const int loc = threadIdx.x / LPR, j = threadIdx.x % LPR;
-  const int k = blockIdx.x % K, range = blockIdx.x / K;
+  const int kgroups = (K + KT - 1) / KT;
+  const int k0 = (int)(blockIdx.x % kgroups) * KT, range = blockIdx.x / kgroups;
+  const int taps = min(KT, K - k0);
   const int a0 = blockIdx.y * AT, g0 = blockIdx.z * S::kCh;
   const int64_t GN = (int64_t)GH * GW;
   const int pm = P == 0 ? 1 : P;
   const bool live = g0 + 2 * j < stride;
-  double2 acc[AT];
+  double2 acc[KT][AT];
 #pragma unroll
-  for (int a = 0; a < AT; a++) acc[a] = make_double2(0.0, 0.0);
+  for (int t = 0; t < KT; t++)
+#pragma unroll
+    for (int a = 0; a < AT; a++) acc[t][a] = make_double2(0.0, 0.0);
   const int64_t t0 = total_tiles * range / ranges, t1 = total_tiles * (range + 1) / ranges;
   for (int64_t tile = t0; tile < t1; tile++) {
     const int b = (int)(tile / tiles_per_img);
@@ -370,64 +380,83 @@ __global__ __launch_bounds__(kThreads) void weight_grad_records_kernel(
           const int l = i % kTile, a = a0 + i / kTile;
           s_plain[i] = (a < A && n0 + l < N) ? plain[((int64_t)b * A + a) * N + n0 + l] : 0.0;
         }
-      for (int l = threadIdx.x; l < kTile; l += kThreads) {
-        if (n0 + l < N) {
-          resolve_records<NC>(map, iw, ((int64_t)(n0 + l) * K + k) * pm + p, GH, GW, wrap != 0,
-                              (int)GN, s_off + l, s_wt + l, kTile);
-        } else {
+      if constexpr (KT > 1) {
+        fill_tap_cache<NC, LPR, KT>(map, iw, n0, N, K, pm, p, k0, taps, GH, GW, wrap != 0, (int)GN,
+                                    s_off, s_wt);
+      } else {
+        for (int l = threadIdx.x; l < kTile; l += kThreads) {
+          if (n0 + l < N) {
+            resolve_records<NC>(map, iw, ((int64_t)(n0 + l) * K + k0) * pm + p, GH, GW, wrap != 0,
+                                (int)GN, s_off + l, s_wt + l, kTile);
+          } else {
 #pragma unroll
-          for (int i = 0; i < NC; i++) {
-            s_off[i * kTile + l] = (int)GN;
-            s_wt[i * kTile + l] = 0.0;
+            for (int i = 0; i < NC; i++) {
+              s_off[i * kTile + l] = (int)GN;
+              s_wt[i * kTile + l] = 0.0;
+            }
           }
         }
       }
       __syncthreads();
       if (live) {
-        double2 d[kSub][NC];
+        // units: the taps of a location, or one tap's locations; kRun of them are in flight
+        constexpr int kUnits = KT > 1 ? KT : kSub, kRun = KT > 1 ? (KT % 3 == 0 ? 3 : KT) : kSub;
 #pragma unroll
-        for (int u = 0; u < kSub; u++)
+        for (int u0 = 0; u0 < kUnits; u0 += kRun) {
+          if (KT > 1 && u0 >= taps) break;
+          double2 d[kRun][NC];
 #pragma unroll
-          for (int i = 0; i < NC; i++)
-            d[u][i] = *reinterpret_cast<const double2 *>(
-                src + (int64_t)s_off[i * kTile + u * S::kLocs + loc] * stride);
+          for (int q = 0; q < kRun; q++) {
+            // (past the last tap it is read again and not used)
+            const int u = KT > 1 ? min(u0 + q, taps - 1) : u0 + q;
 #pragma unroll
-        for (int u = 0; u < kSub; u++) {
-          double vx = 0.0, vy = 0.0;
-#pragma unroll
-          for (int i = 0; i < NC; i++) {
-            const double f = s_wt[i * kTile + u * S::kLocs + loc];
-            vx = mcx_fma(f, d[u][i].x, vx);
-            vy = mcx_fma(f, d[u][i].y, vy);
+            for (int i = 0; i < NC; i++)
+              d[q][i] = *reinterpret_cast<const double2 *>(
+                  src + (int64_t)s_off[i * kSlots + u * S::kLocs + loc] * stride);
           }
 #pragma unroll
-          for (int a = 0; a < AT; a++) {
-            const double q = s_plain[a * kTile + u * S::kLocs + loc];
-            acc[a].x = mcx_fma(q, vx, acc[a].x);
-            acc[a].y = mcx_fma(q, vy, acc[a].y);
+          for (int q = 0; q < kRun; q++) {
+            const int u = u0 + q;
+            if (KT > 1 && u >= taps) break;
+            double vx = 0.0, vy = 0.0;
+#pragma unroll
+            for (int i = 0; i < NC; i++) {
+              const double f = s_wt[i * kSlots + u * S::kLocs + loc];
+              vx = mcx_fma(f, d[q][i].x, vx);
+              vy = mcx_fma(f, d[q][i].y, vy);
+            }
+#pragma unroll
+            for (int a = 0; a < AT; a++) {
+              const double g = s_plain[a * kTile + (KT > 1 ? 0 : u * S::kLocs) + loc];
+              double2 &sum = acc[KT > 1 ? u : 0][a];
+              sum.x = mcx_fma(g, vx, sum.x);
+              sum.y = mcx_fma(g, vy, sum.y);
+            }
           }
         }
       }
     }
   }
   // sum over the locations' lanes of each wave, then over the four waves through LDS
-  __shared__ double2 s_red[kThreads / 64][AT][LPR];
+  __shared__ double2 s_red[kThreads / 64][KT * AT][LPR];
 #pragma unroll
-  for (int a = 0; a < AT; a++) {
+  for (int t = 0; t < KT; t++)
 #pragma unroll
-    for (int m = 32; m >= LPR; m >>= 1) {
-      acc[a].x += __shfl_xor(acc[a].x, m);
-      acc[a].y += __shfl_xor(acc[a].y, m);
+    for (int a = 0; a < AT; a++) {
+#pragma unroll
+      for (int m = 32; m >= LPR; m >>= 1) {
+        acc[t][a].x += __shfl_xor(acc[t][a].x, m);
+        acc[t][a].y += __shfl_xor(acc[t][a].y, m);
+      }
+      if ((int)(threadIdx.x & 63) < LPR) s_red[threadIdx.x >> 6][t * AT + a][j] = acc[t][a];
     }
-    if ((int)(threadIdx.x & 63) < LPR) s_red[threadIdx.x >> 6][a][j] = acc[a];
-  }
   __syncthreads();
-  for (int i = threadIdx.x; i < AT * LPR; i += kThreads) {
-    const int a = i / LPR, jj = i % LPR, g = g0 + 2 * jj;
-    double2 v = s_red[0][a][jj];
+  for (int i = threadIdx.x; i < taps * AT * LPR; i += kThreads) {
+    const int ta = i / LPR, jj = i % LPR, g = g0 + 2 * jj, k = k0 + ta / AT, a = ta % AT;
+    double2 v = s_red[0][ta][jj];
     for (int q = 1; q < kThreads / 64; q++) {
-      v.x += s_red[q][a][jj].x;
-      v.y += s_red[q][a][jj].y;
+      v.x += s_red[q][ta][jj].x;
+      v.y += s_red[q][ta][jj].y;
     }
     if (a0 + a < A) {
       double *out = part + (((int64_t)range * K + k) * A + a0 + a) * G + g;
@@ -546,10 +575,11 @@ __global__ __launch_bounds__(kThreads) void product_planes_kernel(
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Tiles, ranges and channel blocks of the weight gradient: about 2048 workgroups, eight per CU.
+// Tiles, ranges and channel blocks of the weight gradient: about 2048 workgroups, eight per CU; of several
+// taps, whose registers leave room for two or three, 1024 or 768.
 struct GradShape {
-  int lpr, at;
-  int64_t tiles_per_img, total, ranges, ablocks, gblocks;
+  int lpr, at, taps;
+  int64_t tiles_per_img, total, ranges, ablocks, gblocks, kgroups;
 };
 GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
   GradShape q;
@@ -557,11 +587,20 @@ GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
   q.at = A == 1 ? 1 : A <= 4 ? 4 : 16;
   q.ablocks = (A + q.at - 1) / q.at;
   q.gblocks = (read_stride(G) + 2 * q.lpr - 1) / (2 * q.lpr);
-  const int64_t tile = (q.lpr == 2 ? 2 : 4) * (kThreads / q.lpr);
+  // Several taps a workgroup from 98304 locations on, with two to four plain channels 65536; with fewer,
+  // workgroups of one tap are more and wait less (us, one tap and several, nine taps of shuffled maps.  10 -> 1
+  // channels: 50 x 80 4.6, 7.6; 2 of 100 x 350 31, 35; 200 x 500 59, 43; 400 x 700 202, 97.  2 of 200 x 300,
+  // 3 -> 1 38, 29.  220 x 300, 6 -> 1 25, 29, but 7 -> 4 31, 21.  2 of 300 x 500, 16 -> 3 216, 99.  Four waves a SIMD
+  // spill: twice as slow.)
+  const int64_t many = q.at == 1 ? (q.lpr == 2 ? RecShape<2>::kTaps : RecShape<8>::kTaps) : q.at == 4 ? 3 : 1;
+  const int64_t taps = B * N >= (q.at == 1 ? 98304 : 65536) ? many : 1;
+  q.taps = (int)taps;
+  const int64_t tile = (taps > 1 ? 1 : q.lpr == 2 ? 2 : 4) * (kThreads / q.lpr);
   q.tiles_per_img = (N + tile - 1) / tile;
   q.total = B * q.tiles_per_img;
-  const int64_t per_range = K * q.ablocks * q.gblocks;
-  q.ranges = std::max<int64_t>(1, std::min(q.total, 2048 / per_range));
+  q.kgroups = (K + taps - 1) / taps;
+  const int64_t per_range = q.kgroups * q.ablocks * q.gblocks;
+  q.ranges = std::max<int64_t>(1, std::min(q.total, (taps == 1 ? 2048 : q.at == 1 ? 1024 : 768) / per_range));
   return q;
 }
 
@@ -803,12 +842,15 @@ int records_weight_grad(const double *plain, const double *gath, const double *m
   if (int rc = make_records(gath, rec, B, G, GH * GW, s)) return rc;
   const GradShape q = grad_shape(B, A, G, N, K);
   const bool one = canonical_interp(interp) == kInterpNearest;
-#define MCX_RUN(NC, LPR, AT)                                                                     \
-  hipLaunchKernelGGL((weight_grad_records_kernel<NC, LPR, AT>),                                  \
-                     dim3((unsigned)(q.ranges * K), (unsigned)q.ablocks, (unsigned)q.gblocks),   \
+#define MCX_RUN_TAPS(NC, LPR, AT, KT)                                                            \
+  hipLaunchKernelGGL((weight_grad_records_kernel<NC, LPR, AT, KT>),                              \
+                     dim3((unsigned)(q.ranges * q.kgroups), (unsigned)q.ablocks, (unsigned)q.gblocks),   \
                      dim3(kThreads), 0, s, plain, rec, map, iw, part, (int)A, (int)G,            \
                      (int)read_stride(G), (int)GH, (int)GW, (int)N, (int)K, (int)P,              \
                      wraps(interp) ? 1 : 0, (int)q.tiles_per_img, q.total, (int)q.ranges);
+#define MCX_RUN(NC, LPR, AT)                                          \
+  if (q.taps == 1) { MCX_RUN_TAPS(NC, LPR, AT, 1) }                   \
+  else { MCX_RUN_TAPS(NC, LPR, AT, (grad_taps<LPR, AT>())) }
 #define MCX_AT(NC, LPR)                             \
   if (q.at == 1) { MCX_RUN(NC, LPR, 1) }            \
   else if (q.at == 4) { MCX_RUN(NC, LPR, 4) }       \
@@ -817,6 +859,7 @@ int records_weight_grad(const double *plain, const double *gath, const double *m
   MCX_LPR(G, MCX_NC)
 #undef MCX_NC
 #undef MCX_AT
+#undef MCX_RUN_TAPS
 #undef MCX_RUN
   MCX_HIP_CHECK_LAUNCH();
   hipLaunchKernelGGL(reduce_records_kernel, dim3(div_up(A * G * K, kThreads / 64)), dim3(kThreads),

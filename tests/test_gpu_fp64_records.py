@@ -308,3 +308,25 @@ def test_bias_gradient_of_one_channel(n, device):
     want = gy.sum().item()
     # n terms of magnitude one in 64 bits: at most n * 2^-53 * sum|gy| apart, far less in practice
     assert abs(gb.item() - want) <= 1e-12 * gy.abs().sum().item()
+
+
+@pytest.mark.parametrize("ci,co,k,p", [(3, 1, 9, 0), (4, 1, 5, 2), (7, 1, 10, 0), (10, 1, 9, 0),
+                                       (17, 1, 11, 0), (1, 1, 4, 0), (2, 2, 4, 0), (8, 4, 9, 0), (9, 3, 1, 3),
+                                       (17, 4, 8, 0), (6, 5, 3, 0)])
+@pytest.mark.parametrize("interp", [0, 1, 2])
+@pytest.mark.parametrize("few", [False, True])
+def test_weight_gradient_of_several_taps_a_workgroup(ci, co, k, p, interp, few, device):
+    """From 98 304 locations (65 536 with two to four outputs) a workgroup takes several taps: below and
+    above, taps that fill no whole group, channels around a pass of lanes.  Sums of 100 000 terms in 64 bits
+    differ by some 1e-14 of the result with their order; 1e-12 is allowed like everywhere here."""
+    g = torch.Generator().manual_seed(ci * 100 + k)
+    B, ih, iw_ = 2, 60, 90
+    mh, mw = (180, 181) if few else (221, 223)
+    smap, wts = helpers.random_map(g, mh, mw, k, p, ih, iw_, torch.float64)
+    x, gy, w, b = (torch.randn(s, generator=g, dtype=torch.float64)
+                   for s in ((B, ci, ih, iw_), (B, co, mh, mw), (co, ci, k), (co,)))
+    maps = [smap] + ([wts] if p else [])
+    name = ("weighted_" if p else "") + "mapped_conv_backward"
+    got = getattr(_C, name)(*[t.cuda() for t in (gy, *maps, x, w, b)], k, interp,
+                            needs=(False, True, False))[1]
+    assert rel_err(got, getattr(O, name)(gy, *maps, x, w, b, k, interp)[1]) < 1e-12
