@@ -7,6 +7,8 @@ include/nn/layers/*.h wrappers do, allocates the outputs with torch, and calls
 the C ABI of libmcx_hip.so on the current HIP stream.  Tensors must live on the
 GPU: there is no CPU implementation behind these names.
 """
+import contextlib
+
 import torch
 
 from . import _lib
@@ -64,8 +66,9 @@ def _on_gpu(ref_name, ref, **tensors):
     if not ref.is_cuda:
         raise RuntimeError(
             "%s must be a GPU tensor: this backend has no CPU implementation" % ref_name)
+    device = ref.get_device()
     for name, t in tensors.items():
-        if t is not None and t.device != ref.device:
+        if t is not None and t.get_device() != device:
             raise RuntimeError("%s must be on the same device as %s" % (name, ref_name))
 
 
@@ -90,8 +93,22 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# (the handle alone: a Stream object takes two microseconds to make, a call of a small layer thirty)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
+
+
+_here = contextlib.nullcontext()
+
+
+def _device(t):
+    """A context in which t's device is the current one: nothing to switch where it is already."""
+    return _here if torch.cuda.current_device() == t.get_device() else torch.cuda.device(t.device)
 
 
 def _workspace(nbytes, device):
@@ -148,7 +165,7 @@ def _conv_forward(input, sample_map, interp_weights, weight, bias, kernel_size, 
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, IH, IW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = _timed("conv_forward", input.device, lambda: lib.mcx_conv_forward_planned(
             _ptr(input), _ptr(sample_map), _ptr(interp_weights), _ptr(weight), _ptr(bias),
             _ptr(out), _ptr(ws), ws_bytes, plan_ptr, plan_bytes, plan_desc, B, Ci, Co, IH, IW, OH,
@@ -222,7 +239,7 @@ def conv_map_plan(sample_map, interp_weights, input_height, input_width, interpo
         return None
     plan = torch.empty((nbytes,), dtype=torch.uint8, device=sample_map.device)
     desc = _lib.PlanDesc()
-    with torch.cuda.device(sample_map.device):
+    with _device(sample_map):
         rc = lib.mcx_conv_plan_build(_ptr(sample_map), _ptr(interp_weights), _ptr(plan), nbytes,
                                      desc, IH, IW, OH, OW, K, P, int(interpolation), dt,
                                      _stream(sample_map))
@@ -277,12 +294,15 @@ def _conv_backward(grad_output, sample_map, interp_weights, input, weight, bias,
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, IH, IW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
-    # Two C-ABI calls (NULL skips a gradient) so that the input gradient and the weight
-    # gradient can be timed alone; the bias gradient rides on the weight gradient's pass
-    # over grad_output.
-    outs = {"conv_backward_input": (grad_input, None, None),
-            "conv_backward_weight": (None, grad_weight, grad_bias)}
-    with torch.cuda.device(input.device):
+    # Where kernels are timed, two C-ABI calls (NULL skips a gradient), so that the input gradient
+    # and the weight gradient can be timed alone; the bias gradient rides on the weight
+    # gradient's pass over grad_output.
+    if profile_events is None:
+        outs = {"conv_backward": (grad_input, grad_weight, grad_bias)}
+    else:
+        outs = {"conv_backward_input": (grad_input, None, None),
+                "conv_backward_weight": (None, grad_weight, grad_bias)}
+    with _device(input):
         for label, (gx, gw, gb) in outs.items():
             if gx is None and gw is None and gb is None:
                 continue
@@ -347,7 +367,7 @@ def _tconv_forward(input, sample_map, interp_weights, weight, bias, output_heigh
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, OH, OW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = lib.mcx_tconv_forward_planned(_ptr(input), _ptr(sample_map), _ptr(interp_weights),
                                            _ptr(weight), _ptr(bias), _ptr(out), _ptr(ws),
                                            ws_bytes, plan_ptr, plan_bytes, plan_desc, B, Ci, Co,
@@ -382,7 +402,7 @@ def _tconv_backward(grad_output, sample_map, interp_weights, input, weight, bias
     if plan is None and map_plan_cache is not None:
         plan = _cached_plan(sample_map, interp_weights, OH, OW, interpolation, input.dtype)
     plan_ptr, plan_bytes, plan_desc = _plan_args(plan)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = lib.mcx_tconv_backward_planned(
             _ptr(grad_output), _ptr(sample_map), _ptr(interp_weights), _ptr(input), _ptr(weight),
             _ptr(grad_input), _ptr(grad_weight), _ptr(grad_bias), _ptr(ws), ws_bytes, plan_ptr,
@@ -448,7 +468,7 @@ def scatter_map_plan(sample_map, interp_weights, dest_height, dest_width, interp
         return None
     plan = torch.empty((nbytes,), dtype=torch.uint8, device=sample_map.device)
     desc = _lib.PlanDesc()
-    with torch.cuda.device(sample_map.device):
+    with _device(sample_map):
         rc = lib.mcx_scatter_plan_build(_ptr(sample_map), _ptr(interp_weights), _ptr(plan), nbytes,
                                         desc, MH, MW, DH, DW, K, P, int(interpolation), dt,
                                         1 if for_max_unpool else 0, _stream(sample_map))
@@ -484,7 +504,7 @@ def _max_pool(input, sample_map, interp_weights, kernel_size, interpolation):
     OH, OW = sample_map.shape[0], sample_map.shape[1]
     out = torch.empty((B, C, OH, OW), dtype=input.dtype, device=input.device)
     idx = torch.empty((B, C, OH, OW), dtype=torch.int64, device=input.device)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = _lib.load().mcx_max_pool(_ptr(input), _ptr(sample_map), _ptr(interp_weights),
                                       _ptr(out), _ptr(idx), B, C, IH, IW, OH, OW, K, P,
                                       int(interpolation), dt, _stream(input))
@@ -511,7 +531,7 @@ def _max_unpool(grad_output, idx_mask, sample_map, interp_weights, input_height,
     plan = _scatter_plan_for("max_unpool", plan, sample_map, interp_weights, IH, IW,
                              interpolation, True)
     if plan is not None:
-        with torch.cuda.device(grad_output.device):
+        with _device(grad_output):
             rc = lib.mcx_max_unpool_planned(_ptr(grad_output), _ptr(idx_mask), *_plan_args(plan),
                                             _ptr(gin), B, C, IH, IW, OH, OW, K, P,
                                             int(interpolation), dt, _stream(grad_output))
@@ -520,7 +540,7 @@ def _max_unpool(grad_output, idx_mask, sample_map, interp_weights, input_height,
     ws_bytes = lib.mcx_unpool_workspace(IH, IW, OH, OW, K, P, int(interpolation), dt) \
         if scatter_as_gather else 0
     ws = _workspace(ws_bytes, grad_output.device)
-    with torch.cuda.device(grad_output.device):
+    with _device(grad_output):
         rc = lib.mcx_max_unpool(_ptr(grad_output), _ptr(idx_mask), _ptr(sample_map),
                                 _ptr(interp_weights), _ptr(gin), _ptr(ws), ws_bytes, B, C, IH, IW,
                                 OH, OW, K, P, int(interpolation), dt, _stream(grad_output))
@@ -536,7 +556,7 @@ def _avg_pool(input, sample_map, interp_weights, kernel_size, interpolation):
     B, C, IH, IW = input.shape
     OH, OW = sample_map.shape[0], sample_map.shape[1]
     out = torch.empty((B, C, OH, OW), dtype=input.dtype, device=input.device)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = _lib.load().mcx_avg_pool(_ptr(input), _ptr(sample_map), _ptr(interp_weights),
                                       _ptr(out), B, C, IH, IW, OH, OW, K, P, int(interpolation),
                                       dt, _stream(input))
@@ -559,7 +579,7 @@ def _avg_unpool(grad_output, sample_map, interp_weights, input_height, input_wid
     plan = _scatter_plan_for("avg_unpool", plan, sample_map, interp_weights, IH, IW,
                              interpolation, True)
     if plan is not None:
-        with torch.cuda.device(grad_output.device):
+        with _device(grad_output):
             rc = lib.mcx_avg_unpool_planned(_ptr(grad_output), *_plan_args(plan), _ptr(gin),
                                             B, C, IH, IW, OH, OW, K, P, int(interpolation), dt,
                                             _stream(grad_output))
@@ -568,7 +588,7 @@ def _avg_unpool(grad_output, sample_map, interp_weights, input_height, input_wid
     ws_bytes = lib.mcx_unpool_workspace(IH, IW, OH, OW, K, P, int(interpolation), dt) \
         if scatter_as_gather else 0
     ws = _workspace(ws_bytes, grad_output.device)
-    with torch.cuda.device(grad_output.device):
+    with _device(grad_output):
         rc = lib.mcx_avg_unpool(_ptr(grad_output), _ptr(sample_map), _ptr(interp_weights),
                                 _ptr(gin), _ptr(ws), ws_bytes, B, C, IH, IW, OH, OW, K, P,
                                 int(interpolation), dt, _stream(grad_output))
@@ -642,7 +662,7 @@ def _resample_to_map(input, sample_map, interp_weights, output_height, output_wi
     plan = _scatter_plan_for("resample", plan, sample_map, interp_weights, OH, OW, interpolation,
                              False)
     if plan is not None:
-        with torch.cuda.device(input.device):
+        with _device(input):
             rc = lib.mcx_resample_to_map_planned(_ptr(input), *_plan_args(plan), _ptr(out),
                                                  B, C, IH, IW, OH, OW, P, int(interpolation), dt,
                                                  _stream(input))
@@ -651,7 +671,7 @@ def _resample_to_map(input, sample_map, interp_weights, output_height, output_wi
     ws_bytes = lib.mcx_resample_to_map_workspace(IH, IW, OH, OW, P, int(interpolation), dt) \
         if scatter_as_gather else 0
     ws = _workspace(ws_bytes, input.device)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = lib.mcx_resample_to_map(_ptr(input), _ptr(sample_map), _ptr(interp_weights),
                                      _ptr(out), _ptr(ws), ws_bytes, B, C, IH, IW, OH, OW, P,
                                      int(interpolation), dt, _stream(input))
@@ -669,7 +689,7 @@ def _resample_from_map(input, sample_map, interp_weights, interpolation):
     B, C, SH, SW = input.shape
     MH, MW = sample_map.shape[0], sample_map.shape[1]
     out = torch.empty((B, C, MH, MW), dtype=input.dtype, device=input.device)
-    with torch.cuda.device(input.device):
+    with _device(input):
         rc = _lib.load().mcx_resample_from_map(_ptr(input), _ptr(sample_map),
                                                _ptr(interp_weights), _ptr(out), B, C, SH, SW, MH,
                                                MW, P, int(interpolation), dt, _stream(input))
@@ -713,7 +733,7 @@ def knn_forward(ref, query, k):
     idx = torch.empty((B, k, Q), dtype=torch.int64, device=ref.device)
     dist = torch.empty((B, k, Q), dtype=ref.dtype, device=ref.device)
     lib = _lib.load()
-    with torch.cuda.device(ref.device):
+    with _device(ref):
         # (the grid search's bins; 0 bytes where it does not apply and every point is walked)
         ws_bytes = lib.mcx_knn_workspace(B, D, R, dt)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=ref.device) if ws_bytes else None
@@ -774,7 +794,7 @@ def cube2rect(cubemap, rect_height, rect_width, interpolation):
     C, dim = cubemap.shape[0], cubemap.shape[1]
     RH, RW = int(rect_height), int(rect_width)
     rect = torch.empty((C, RH, RW), dtype=cubemap.dtype, device=cubemap.device)
-    with torch.cuda.device(cubemap.device):
+    with _device(cubemap):
         rc = _lib.load().mcx_cube2rect(_ptr(cubemap), _ptr(rect), C, dim, RH, RW,
                                        int(interpolation), _DTYPES[cubemap.dtype],
                                        _stream(cubemap))
@@ -792,7 +812,7 @@ def gnomonic_samples(centres, kh, kw, res_lat, res_lon):
         raise RuntimeError("spherical_coords must be a float32 tensor [V, 2]")
     V = centres.shape[0]
     out = torch.empty((1, V, int(kh) * int(kw), 2), dtype=torch.float32, device=centres.device)
-    with torch.cuda.device(centres.device):
+    with _device(centres):
         rc = _lib.load().mcx_gnomonic_samples(_ptr(centres), _ptr(out), V, int(kh), int(kw),
                                               float(res_lat), float(res_lon), _stream(centres))
     _lib.check(rc, "gnomonic_kernel")
