@@ -275,8 +275,13 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
 }
 
 // x[b][g][n] -> xt[b][n][Gpad] (channels past G zero): 64 pixels x 64 channels per
-// workgroup through LDS, coalesced on both sides.
-template <typename TD>
+// workgroup through LDS, coalesced on both sides.  CHUNKED: xt[b][Gpad/16][n][16], a record's sixteen
+// channels of a chunk with the same chunk of the other records (see weight_grad_mfma_kernel).
+template <bool CHUNKED>
+__device__ inline int64_t record_offset(int64_t n, int g, int Gpad, int64_t plane) {
+  return CHUNKED ? ((int64_t)(g / kGC) * plane + n) * kGC + g % kGC : n * Gpad + g;
+}
+template <typename TD, bool CHUNKED = false>
 __global__ __launch_bounds__(256) void to_channel_last_kernel(const TD *__restrict__ x,
                                                               TD *__restrict__ xt, int G, int Gpad,
                                                               int64_t plane) {
@@ -295,7 +300,8 @@ __global__ __launch_bounds__(256) void to_channel_last_kernel(const TD *__restri
   for (int r = 0; r < 16; r++) {
     const int64_t n = n0 + ly + 4 * r;
     const int g = g0 + lx;
-    if (n < plane && g < Gpad) xt[((int64_t)b * plane + n) * Gpad + g] = tile[lx][ly + 4 * r];
+    if (n < plane && g < Gpad)
+      xt[(int64_t)b * plane * Gpad + record_offset<CHUNKED>(n, g, Gpad, plane)] = tile[lx][ly + 4 * r];
   }
 }
 
@@ -1199,6 +1205,14 @@ constexpr int wg_plain_channels() { return sizeof(TD) == 2 ? 128 : 64; }
 template <typename TD>
 constexpr int wg_gathered_blocks() { return sizeof(TD) == 2 ? 1 : 2; }
 constexpr int kWgKT = 9;            // taps per pass (accumulators in registers)
+constexpr int kWgKTMesh = 7;        // and of fp32 mesh signals with no more
+// Layout of the channel-last copy: several points a tap read their records from [chunk of 16][n][16],
+// so that what the channel groups of one XCD read of an image comes near its 4 MB of L2 (see `spread`
+// in the kernel).  One point a tap gains nothing by it, nor do two in bf16 (weight gradients over 40 962
+// vertices, 4 x 64 -> 128 channels, without and with it: one point 222 us, 226, bf16 164, 167; two points 264, 255, bf16
+// 200, 202).
+template <typename TD>
+constexpr bool chunked_records(bool cl, int np) { return cl && np > (sizeof(TD) == 4 ? 1 : 2); }
 constexpr int kLdPx = kTilePx + 4;  // LDS row stride (floats)
 
 // The consumers of a pair mask only ask whether a pair beyond the first two is in use
@@ -1225,13 +1239,13 @@ __global__ void map_pair_mask_kernel(const float *__restrict__ map, const float 
   report_pairs_beyond_two(mask, m);
 }
 
-// CL: `gath` is a channel-last copy [B][GH*GW][Gpad] of the gathered operand (see the
-// gather-product kernel).
+// CL: `gath` is a channel-last copy of the gathered operand, [B][GH*GW][Gpad] or in chunks (see
+// chunked_records).
 // NA: leading (offset, weight) pairs of a tap that are loaded and added.  NA < NP*NCORN is
 // valid when the remaining pairs are zero for every sample of the map (bilinear corners of
 // integral row coordinates, unused points); map_pair_mask_kernel finds that out on the
 // device and `pair_mask` / `run_if_leading` let exactly one of two launched variants run.
-template <typename TD, int NCORN, int NP, bool CL, int NA>
+template <typename TD, int NCORN, int NP, bool CL, int NA, int KT = kWgKT>
 __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad_mfma_kernel(
     const TD *__restrict__ plain, const TD *__restrict__ gath,
     const float *__restrict__ map, const float *__restrict__ iw, float *__restrict__ part, int A,
@@ -1251,11 +1265,12 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // different rows on different banks) and feed v_mfma_f32_16x16x32_bf16, whose lanes take
   // 8 consecutive pixels of their row.
   constexpr bool kBf16 = sizeof(TD) == 2;
+  constexpr bool kChunked = chunked_records<TD>(CL, NP);
   constexpr int kLdPxB = kTilePx + 8;
   constexpr int kWgA = wg_plain_channels<TD>(), kWgCB = wg_gathered_blocks<TD>();
   constexpr int MB = kWgA / 64;  // 16-row blocks of plain channels per wave
   constexpr int kPtFloats = kBf16 ? kWgA * kLdPxB / 2 : kWgA * kLdPx;
-  constexpr int kTapFloats = 2 * kWgKT * kTilePx * NA;
+  constexpr int kTapFloats = 2 * KT * kTilePx * NA;
   constexpr bool kCacheTaps = kTapFloats <= kPtFloats + 1024;
   __shared__ __attribute__((aligned(16))) float PtMem[kCacheTaps && kTapFloats > kPtFloats ? kTapFloats : kPtFloats];
   __shared__ __attribute__((aligned(16))) float SMem[kBf16 ? kGC * kLdPxB : 2 * kGC * kLdPx];
@@ -1267,7 +1282,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // wave read consecutive words)
   unsigned(*TapOff)[kTilePx][NA] = reinterpret_cast<unsigned(*)[kTilePx][NA]>(PtMem);
   float(*TapWt)[kTilePx][NA] =
-      reinterpret_cast<float(*)[kTilePx][NA]>(PtMem + kWgKT * kTilePx * NA);
+      reinterpret_cast<float(*)[kTilePx][NA]>(PtMem + KT * kTilePx * NA);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l15 = lane & 15, lq = lane >> 4;
@@ -1275,7 +1290,19 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // the channel groups and plain blocks of one pixel range are neighbours, on one XCD (and its L2)
   const int combos = cgroups * ((A + kWgA - 1) / kWgA);
   int combo;
-  if ((ranges & 7) == 0) {
+  // Records in chunks: an XCD takes one channel group, and its workgroups walk the images together (tile t
+  // goes to range t % ranges).  40 962 vertices, 4 x 64 -> 128 channels, seven taps of four random points: an
+  // image's records are 10.5 MB and the kernel was bound by L2 misses, 2.5 GB of them at 5.7 TB/s, as many as
+  // the gather reads; now 1.25 GB, and 338 us for 443 (with the taps read side by side, see below, and seven
+  // taps' accumulators, which do not spill).  Whole weight gradients, before and now: one of these images
+  // 167 -> 127, bf16 130 -> 100; two of 20 000 vertices, 128 -> 128 channels, nine taps 366 -> 211, bf16 220 -> 142;
+  // a real mesh kernel of three points, 4 x 64 -> 128 322 -> 287, bf16 256 -> 214.
+  const bool spread = kChunked && (ranges & 7) == 0 && cgroups > 1 && 8 % cgroups == 0;
+  if (spread) {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, ablocks = combos / cgroups;
+    combo = slot % ablocks * cgroups + xcd % cgroups;
+    range = slot / ablocks * (8 / cgroups) + xcd / cgroups;
+  } else if ((ranges & 7) == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     combo = slot % combos;
     range = xcd * (ranges >> 3) + slot / combos;
@@ -1285,10 +1312,11 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   }
   cg = combo % cgroups;
   const int a0 = combo / cgroups * kWgA;
-  const int k_base = blockIdx.z * kWgKT;
-  const int ktaps = min(kWgKT, K - k_base);
+  const int k_base = blockIdx.z * KT;
+  const int ktaps = min(KT, K - k_base);
   const int tpr = (total_tiles + ranges - 1) / ranges;
-  const int t_begin = range * tpr, t_end = min(total_tiles, t_begin + tpr);
+  const int t_begin = spread ? range : range * tpr, t_step = spread ? ranges : 1;
+  const int t_end = spread ? total_tiles : min(total_tiles, t_begin + tpr);
   const int tw_mask = (1 << tw_shift) - 1, th = kTilePx >> tw_shift;
   const int N = MH * MW;
   const int64_t gplane = (int64_t)GH * GW;
@@ -1299,9 +1327,9 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   const bool vec_ok = (MW & (16 / (int)sizeof(TD) - 1)) == 0 &&
                       (reinterpret_cast<uintptr_t>(plain) & 15) == 0;
 
-  floatx4 acc[kWgKT][kWgCB][MB];
+  floatx4 acc[KT][kWgCB][MB];
 #pragma unroll
-  for (int k = 0; k < kWgKT; k++)
+  for (int k = 0; k < KT; k++)
 #pragma unroll
     for (int cb = 0; cb < kWgCB; cb++)
 #pragma unroll
@@ -1314,7 +1342,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
 #pragma unroll
   for (int mb = 0; mb < MB; mb++) plain_sum[mb] = 0.f;
 
-  for (int tile = t_begin; tile < t_end; ++tile) {
+  for (int tile = t_begin; tile < t_end; tile += t_step) {
     const int b = tile / tiles_per_img;
     const int t_in = tile - b * tiles_per_img;
     const int tile_y = t_in / tiles_x, tile_x = t_in - tile_y * tiles_x;
@@ -1431,19 +1459,22 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     unsigned off[NE];
     float wt[NE];
     float v[8][NE];
-    auto resolve_tap = [&](int k, unsigned *o, float *w_) {  // tap k of this thread's pixel
+    auto resolve_at = [&](int64_t n, bool live, int k, unsigned *o, float *w_) {
 #pragma unroll
       for (int sp = 0; sp < NP; sp++) {
-        const int64_t e = (n_g * K + k) * NP + sp;
+        const int64_t e = (n * K + k) * NP + sp;
         PairTap<NCORN> t;
         resolve_pairs<NCORN, sizeof(TD)>(map[e * 2], map[e * 2 + 1], GH, GW, wrap != 0,
                                          live ? (weighted ? iw[e] : 1.f) : 0.f, t);
 #pragma unroll
         for (int i = 0; i < NCORN; i++) {
-          o[sp * NCORN + i] = CL ? t.off[i] * (unsigned)Gpad : t.off[i];
+          o[sp * NCORN + i] = CL ? t.off[i] * (unsigned)(kChunked ? kGC : Gpad) : t.off[i];
           w_[sp * NCORN + i] = t.wt[i];
         }
       }
+    };
+    auto resolve_tap = [&](int k, unsigned *o, float *w_) {  // tap k of this thread's pixel
+      resolve_at(n_g, live, k, o, w_);
     };
     auto load_tap = [&](int k) {  // k: tap within this pass
       if (kQuads) {
@@ -1461,7 +1492,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     auto issue = [&](int cb, int k) {
       if constexpr (kQuads) {
         const char *base = reinterpret_cast<const char *>(
-            gath_b + min(g_first + cb * kGC + qc, Gpad - 4));
+            gath_b + record_offset<kChunked>(0, min(g_first + cb * kGC + qc, Gpad - 4), Gpad, gplane));
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
@@ -1473,7 +1504,8 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
       if constexpr (CL) {
         // 8 contiguous channels of the pixel row; a workgroup whose channels lie past the
         // padded count reads the last valid group (its products are not stored)
-        const char *base = reinterpret_cast<const char *>(gath_b + min(g0, Gpad - 8));
+        const char *base = reinterpret_cast<const char *>(
+            gath_b + record_offset<kChunked>(0, min(g0, Gpad - 8), Gpad, gplane));
 #pragma unroll
         for (int i = 0; i < NA; i++) {
           const char *row = base + off[i];
@@ -1554,7 +1586,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
           // (fetched only here: held across the plain tile's copy, the entries spill)
           from_table = true;
           const uint4 *te = tap_table + ((int64_t)t_in * K + k_base) * kTilePx + p;
-          constexpr int kTapsPerThread = (kWgKT + 1) / 2;
+          constexpr int kTapsPerThread = (KT + 1) / 2;
           uint4 entry[kTapsPerThread];
 #pragma unroll
           for (int t = 0; t < kTapsPerThread; t++)
@@ -1569,7 +1601,25 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
           }
         }
       }
-      if (!from_table)
+      if constexpr (kChunked) {
+        // Consecutive threads take consecutive taps of a pixel, which lie side by side in the map: a
+        // pixel to a thread, the lines of all taps of all pixels (43 KB at seven taps of four points)
+        // are wanted again after the L1 has lost them.  (The mesh above, in fp32: 391 us a pixel to a thread,
+        // 338 so.)
+        for (int i = tid; i < ktaps * kTilePx; i += kThreads) {
+          const int px = i / ktaps, k = i - px * ktaps;
+          const int qi = i0 + (px >> tw_shift), qj = j0 + (px & tw_mask);
+          const bool there = qi < MH && qj < MW;
+          unsigned o[NE];
+          float w_[NE];
+          resolve_at(there ? (int64_t)qi * MW + qj : 0, there, k_base + k, o, w_);
+#pragma unroll
+          for (int e = 0; e < NA; e++) {
+            TapOff[k][px][e] = o[e];
+            TapWt[k][px][e] = w_[e];
+          }
+        }
+      } else if (!from_table)
         for (int k = half; k < ktaps; k += 2) {
           unsigned o[NE];
           float w_[NE];
@@ -1591,7 +1641,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
 #pragma unroll
     for (int cb = 0; cb < kWgCB; cb++) {
 #pragma unroll
-      for (int k = 0; k < kWgKT; k++) {
+      for (int k = 0; k < KT; k++) {
         if (k < ktaps) {
           buf ^= 1;
           stage(buf, k);
@@ -1648,7 +1698,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   const int A4 = (A + 3) & ~3;
   float *pr = part + (int64_t)range * A4 * G * K;
 #pragma unroll
-  for (int k = 0; k < kWgKT; k++) {
+  for (int k = 0; k < KT; k++) {
     if (k < ktaps) {
 #pragma unroll
       for (int cb = 0; cb < kWgCB; cb++) {
@@ -3075,8 +3125,12 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   if (cl) {
     TD *stage = reinterpret_cast<TD *>((char *)pair_mask + 256);
     dim3 tg((unsigned)((GH * GW + 63) / 64), (unsigned)((Gpad + 63) / 64), (unsigned)B);
-    hipLaunchKernelGGL(to_channel_last_kernel<TD>, tg, dim3(256), 0, s, gath, stage, (int)G,
-                       (int)Gpad, GH * GW);
+    if (chunked_records<TD>(cl, m.np))
+      hipLaunchKernelGGL((to_channel_last_kernel<TD, true>), tg, dim3(256), 0, s, gath, stage, (int)G,
+                         (int)Gpad, GH * GW);
+    else
+      hipLaunchKernelGGL(to_channel_last_kernel<TD>, tg, dim3(256), 0, s, gath, stage, (int)G,
+                         (int)Gpad, GH * GW);
     MCX_HIP_CHECK_LAUNCH();
     gath = stage;
   }
@@ -3120,12 +3174,24 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
     else if (int rc = launch_pair_mask(map, iw, pair_mask, m, GH, GW, MH * MW * K, s))
       return rc;
   }
-#define MCX_LAUNCH_NA(NCORN, NP, CL, NA, MASK, LEAD)                                             \
-  hipLaunchKernelGGL((weight_grad_mfma_kernel<TD, NCORN, NP, CL, NA>), grid, dim3(kThreads), 0,  \
-                     s, plain, gath, map, iw, part, (int)A, (int)G, (int)GH, (int)GW, (int)MH,   \
+#define MCX_LAUNCH_KT(NCORN, NP, CL, NA, KT, MASK, LEAD)                                         \
+  hipLaunchKernelGGL((weight_grad_mfma_kernel<TD, NCORN, NP, CL, NA, KT>), grid, dim3(kThreads), \
+                     0, s, plain, gath, map, iw, part, (int)A, (int)G, (int)GH, (int)GW, (int)MH,   \
                      (int)MW, (int)K, m.weighted, m.wrap, t.tiles_x, t.tiles_per_img,            \
                      t.tw_shift, (int)t.total, ranges, cgroups,                                  \
                      plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state, tap_table)
+// (seven taps, those of a mesh vertex and its neighbours, leave the registers that nine spill: a pass of
+// nine for the kernel of seven taps of four points 402 us, of seven 391)
+#define MCX_LAUNCH_NA(NCORN, NP, CL, NA, MASK, LEAD)                           \
+  if constexpr (CL && sizeof(TD) == 4 && NA > 1) {                            \
+    if (K <= kWgKTMesh) {                                                     \
+      MCX_LAUNCH_KT(NCORN, NP, CL, NA, kWgKTMesh, MASK, LEAD);                \
+    } else {                                                                  \
+      MCX_LAUNCH_KT(NCORN, NP, CL, NA, kWgKT, MASK, LEAD);                    \
+    }                                                                         \
+  } else {                                                                    \
+    MCX_LAUNCH_KT(NCORN, NP, CL, NA, kWgKT, MASK, LEAD);                      \
+  }
 #define MCX_LAUNCH_CL(NCORN, NP, CL)                                          \
   if constexpr (NCORN * NP == 4) {                                            \
     if (!ring) {                                                              \
@@ -3192,6 +3258,7 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
   profile_end(s);
 #undef MCX_LAUNCH
 #undef MCX_LAUNCH_NA
+#undef MCX_LAUNCH_KT
 #undef MCX_LAUNCH_CL
   MCX_HIP_CHECK_LAUNCH();
   const int64_t n = round_up(A, 4) * G * K;

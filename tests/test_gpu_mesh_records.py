@@ -34,3 +34,29 @@ def test_weighted_mesh_convolution(points, ci, co, v, spread, device):
     want = O.weighted_mapped_conv_backward(gy, smap, iw, x, w, b, k, 0)
     for a, e in zip(got, want):
         assert rel_err(a, e) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("points,k", [(1, 7), (2, 7), (3, 8), (4, 1), (4, 7), (4, 9), (4, 10)])
+@pytest.mark.parametrize("ci,co,v", [(32, 40, 1030), (33, 129, 1100), (64, 64, 2100), (100, 8, 520),
+                                     (256, 64, 1025)])
+def test_weight_gradient_over_chunks_of_records(dtype, points, k, ci, co, v, device):
+    """Channel groups that share out the XCDs (two, four and eight of them) and others, ranges of tiles that
+    are a multiple of eight and not, and taps around the seven and nine of a pass."""
+    g = torch.Generator().manual_seed(1000 * points + ci + k)
+    B = 2
+    idx = torch.randint(v, (1, v, k, points), generator=g).float()
+    smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    iw = torch.rand(1, v, k, points, generator=g)
+    x, gy = (torch.randn(s, generator=g).to(dtype) for s in ((B, ci, 1, v), (B, co, 1, v)))
+    w, b = torch.zeros(co, ci, k, dtype=dtype), torch.zeros(co, dtype=dtype)
+    got = _C.weighted_mapped_conv_backward(gy.cuda(), smap.cuda(), iw.cuda(), x.cuda(), w.cuda(),
+                                           b.cuda(), k, 0, needs=(False, True, True))
+    # in 64 bits, tap by tap: [B, ci, v] samples against [B, co, v]
+    cols = torch.stack([(x.double()[:, :, 0, idx[0, :, t].long()] * iw[0, :, t].double()).sum(-1)
+                        for t in range(k)])
+    gw = torch.einsum("bon,kbcn->ock", gy.double()[:, :, 0], cols)
+    # fp32: some thousand terms, a few 1e-7; bf16: samples rounded to 2^-9 each and the result once
+    tol = 1e-5 if dtype == torch.float32 else 8e-3
+    assert rel_err(got[1], gw) < tol
+    assert rel_err(got[2], gy.double().sum((0, 2, 3))) < tol
