@@ -838,7 +838,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 // tile once per 32 pixels.  Here
 //   * a lane gathers and interpolates exactly the elements its MFMA B operand holds
 //     (v_mfma_f32_32x32x16_bf16: lane (l31, lhi) holds channels lhi*8 .. lhi*8+7 of pixel column
-//     l31), so samples never touch LDS, and a wave multiplies two 32-pixel blocks by all 64*OG
+//     l31), so samples never touch LDS, and a wave multiplies one or two 32-pixel blocks by all 64*OG
 //     output channels per weight fetch: half the LDS bytes per product;
 //   * a tap is NA (pixel, weight) entries; a 32-bit word of an entry (two channels of its
 //     pixel) is multiplied by {w, 0} for the even and by {0, w} for the odd channel with
@@ -849,7 +849,7 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 //     arithmetic in the loop), the loads of kDepth units are in flight, and the LDS reads of a
 //     unit are issued a step ahead of their use.
 // Only the weights (linear copies of the pre-packed slices) go through LDS, double buffered,
-// one barrier per unit.  A workgroup is 4 waves = 256 consecutive pixels of an image (in the
+// one barrier per unit.  A workgroup is 4 waves = 256 or 128 consecutive pixels of an image (in the
 // order of the flattened map, so any image width works) x 64*OG output channels.  The source is
 // the copy in blocks of 8 channels per pixel (to_channel_blocks).  PACKED: the taps come
 // from a packed map (a transposed map or a plan's gather part: four (pixel, weight) entries per
@@ -857,25 +857,33 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 // the leading entries of a tap that are read (2 or 4), by the masks of the map (pair_mask / row_mask).
 constexpr int kDgPx = 256;
 
-template <int NA, int OG>
+// Q: pixels a lane, of which a workgroup has 128 * Q.  Two of them share a fetch of the weights, one leaves
+// registers for four waves a SIMD and fills the chip with half the pixels; over 64 outputs, whose
+// weights are few, one is the better form (forward and input gradient, us, of two pixels and of one:
+// 4 x 32 -> 64 channels of 64 x 128 16 + 31, 11 + 18; 16 x 32 -> 64 22 + 41, 22 + 37; 8 x 64 -> 64 of 256 x 512, four
+// corners, 312 + 302, 284 + 278; 5 x 5 508 + 519, 476 + 485; 128 -> 64 349, 355).  Over 128 it is where two make no
+// more than one workgroup a CU (kSmallDirectGrid): 8 x 128 -> 128 of 64 x 128, four corners, which are 256, 62 + 65, 52 +
+// 51; 4 of 128 x 256, which are 512, 69 + 65, 73 + 71.
+constexpr int64_t kSmallDirectGrid = 256;
+template <int NA, int OG, int Q>
 struct DirectLds {
-  static constexpr int TG = NA <= 2 ? 13 : 4;  // taps resolved into LDS at a time
-  unsigned off[TG][kDgPx][NA];
-  unsigned w[TG][kDgPx][NA];  // bf16 weights as {w, 0}
+  static constexpr int TG = NA <= 2 ? 13 : Q == 1 ? 9 : 4;  // taps resolved into LDS at a time
+  unsigned off[TG][128 * Q][NA];
+  unsigned w[TG][128 * Q][NA];  // bf16 weights as {w, 0}
   uint4 wt[2][2][kOT * OG];
   float bias[kOT * OG];
 };
 
-template <bool PACKED, int NA, int OG>
+template <bool PACKED, int NA, int OG, int Q>
 __device__ inline void gather_product_bf16_direct(
-    DirectLds<NA, OG> &lds, const bf16_t *__restrict__ src, const float *__restrict__ map,
+    DirectLds<NA, OG, Q> &lds, const bf16_t *__restrict__ src, const float *__restrict__ map,
     const float *__restrict__ iw, const uint16_t *__restrict__ wb,
     const bf16_t *__restrict__ bias, bf16_t *__restrict__ y, int O, int Opad, int Gpad, int SH,
     int SW, int N, int K, int weighted, int wrap, const int *__restrict__ gate,
     const float *__restrict__ addend, int b, int n0) {
   static_assert(NA == 2 || NA == 4, "two or four entries per tap");
   constexpr int NPR = NA / 2;              // entry pairs per tap
-  constexpr int TG = DirectLds<NA, OG>::TG;
+  constexpr int TG = DirectLds<NA, OG, Q>::TG;
   constexpr int kDepth = NA <= 2 ? 3 : 2;  // units whose loads are in flight
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   auto &TapOff = lds.off;
@@ -888,7 +896,9 @@ __device__ inline void gather_product_bf16_direct(
   const int chunks = Gpad / kGC;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, lhi = lane >> 5;
-  const int px[2] = {wave * 64 + l31, wave * 64 + 32 + l31};  // this lane's pixels of the tile
+  int px[Q];  // this lane's pixels of the tile
+#pragma unroll
+  for (int q = 0; q < Q; q++) px[q] = (wave * Q + q) * 32 + l31;
   // the image's staged copy as a buffer: the lane's offset selects pixel and (through lhi) the
   // upper or lower block of a chunk, the scalar offset the chunk
   const auto img = __builtin_amdgcn_make_buffer_rsrc(
@@ -903,76 +913,109 @@ __device__ inline void gather_product_bf16_direct(
   const int wt = min(tid, 2 * kPerKg - 1);
   const unsigned w_lane = ((unsigned)(wt / kPerKg) * Opad + o0 + wt % kPerKg) * 16u;
 
-  floatx16 acc[2 * OG][2];
+  floatx16 acc[2 * OG][Q];
 #pragma unroll
   for (int m = 0; m < 2 * OG; m++)
 #pragma unroll
-    for (int q = 0; q < 2; q++)
+    for (int q = 0; q < Q; q++)
 #pragma unroll
       for (int i = 0; i < 16; i++) acc[m][q][i] = 0.f;
 
   if (tid < kOT * OG) lds.bias[tid] = bias && o0 + tid < O ? to_f32(bias[o0 + tid]) : 0.f;
+  auto read_tap = [&](int64_t ng, int k, float2 *raw, float &raw_w) __attribute__((always_inline)) {
+    raw_w = 1.f;
+    if constexpr (PACKED) {
+      // pre-resolved entries [tap][slot][pixel]: (pixel index of the source as bits, weight)
+#pragma unroll
+      for (int r = 0; r < NA; r++)
+        raw[r] = reinterpret_cast<const float2 *>(map)[((int64_t)k * 4 + r) * N + ng];
+    } else {
+      const int64_t e = ng * K + k;
+      raw[0] = make_float2(map[e * 2], map[e * 2 + 1]);
+      if (weighted) raw_w = iw[e];
+    }
+  };
+  auto put_tap = [&](int kl, int p, bool live, const float2 *raw, float raw_w)
+      __attribute__((always_inline)) {
+    unsigned off[4];
+    float wgt[4];
+    if constexpr (PACKED) {
+#pragma unroll
+      for (int r = 0; r < NA; r++) {
+        off[r] = __builtin_bit_cast(unsigned, raw[r].x) * 16u;
+        wgt[r] = live ? raw[r].y : 0.f;
+      }
+    } else {
+      PairTap<4> t;
+      resolve_pairs<4, 16>(raw[0].x, raw[0].y, SH, SW, wrap != 0, live ? raw_w : 0.f, t);
+#pragma unroll
+      for (int r = 0; r < NA; r++) {
+        off[r] = t.off[r];
+        wgt[r] = t.wt[r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < NA; r++) TapOff[kl][p][r] = off[r];
+    // entry r weighs w[r] (rounded to bf16, the precision of the samples themselves), kept
+    // as the word {w, 0} that weighs the even channel of a sample word; a lane-side shift
+    // makes the {0, w} of the odd one
+#pragma unroll
+    for (int r = 0; r < NA; r++)
+      TapW[kl][p][r] = __builtin_bit_cast(
+          unsigned, __builtin_convertvector(floatx2{wgt[r], 0.f}, bf16x2));
+  };
   int buf = 0;
   for (int k0 = 0; k0 < K; k0 += TG) {
     const int kn = min(TG, K - k0);
     __syncthreads();  // the previous group's units are done with the tap cache
-    {                 // thread tid resolves the group's taps of pixel tid
+    if constexpr (Q == 2) {  // thread tid resolves the group's taps of pixel tid
       const int n = n0 + tid;
       const bool live = n < N;
       const int64_t ng = live ? n : 0;
       for (int kl = 0; kl < kn; kl++) {
-        unsigned off[4];
-        float wgt[4];
-        if constexpr (PACKED) {
-          // pre-resolved entries [tap][slot][pixel]: (pixel index of the source as bits, weight)
+        float2 raw[PACKED ? NA : 1];
+        float raw_w;
+        read_tap(ng, k0 + kl, raw, raw_w);
+        put_tap(kl, tid, live, raw, raw_w);
+      }
+    } else {  // a thread resolves every other tap of a pixel
+      const int p = tid & 127, part = tid >> 7;
+      const int n = n0 + p;
+      const bool live = n < N;
+      const int64_t ng = live ? n : 0;
+      // kBatch of them are read at a time: one after the other each waits out a load's way to memory.  (Not with
+      // two pixels a lane: 16 x 128 -> 128 channels of 512 x 1024, 5 x 5, 30.2 ms a training pass, 30.8 in batches.)
+      constexpr int kBatch = 5;
+      for (int kl0 = part; kl0 < kn; kl0 += 2 * kBatch) {
+        float2 raw[kBatch][PACKED ? NA : 1];
+        float raw_w[kBatch];
 #pragma unroll
-          for (int r = 0; r < NA; r++) {
-            const float2 q =
-                reinterpret_cast<const float2 *>(map)[((int64_t)(k0 + kl) * 4 + r) * N + ng];
-            off[r] = __builtin_bit_cast(unsigned, q.x) * 16u;
-            wgt[r] = live ? q.y : 0.f;
-          }
-        } else {
-          const int64_t e = ng * K + k0 + kl;
-          PairTap<4> t;
-          resolve_pairs<4, 16>(map[e * 2], map[e * 2 + 1], SH, SW, wrap != 0,
-                               live ? (weighted ? iw[e] : 1.f) : 0.f, t);
+        for (int t = 0; t < kBatch; t++)
+          read_tap(ng, k0 + min(kl0 + 2 * t, kn - 1), raw[t], raw_w[t]);
 #pragma unroll
-          for (int r = 0; r < NA; r++) {
-            off[r] = t.off[r];
-            wgt[r] = t.wt[r];
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < NA; r++) TapOff[kl][tid][r] = off[r];
-        // entry r weighs w[r] (rounded to bf16, the precision of the samples themselves), kept
-        // as the word {w, 0} that weighs the even channel of a sample word; a lane-side shift
-        // makes the {0, w} of the odd one
-#pragma unroll
-        for (int r = 0; r < NA; r++)
-          TapW[kl][tid][r] = __builtin_bit_cast(
-              unsigned, __builtin_convertvector(floatx2{wgt[r], 0.f}, bf16x2));
+        for (int t = 0; t < kBatch; t++)
+          if (kl0 + 2 * t < kn) put_tap(kl0 + 2 * t, p, live, raw[t], raw_w[t]);
       }
     }
     __syncthreads();
 
     // units: chunk-major, the tap fastest (a chunk's source rows stay in cache for all taps)
     const int units = chunks * kn;
-    u32x4 ring[kDepth][2][NA];
+    u32x4 ring[kDepth][Q][NA];
     u32x4 wring[kDepth];
     int ki = 0, ci = 0, ks = 0;
     // `offn`: the offsets of the unit whose loads are issued next; `wnext`: the packed weights
     // of the unit that is interpolated next (both read from LDS a step ahead)
-    unsigned offn[2][NA], wnext[2][NA];
+    unsigned offn[Q][NA], wnext[Q][NA];
     auto fetch_offsets = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int q = 0; q < 2; q++)
+      for (int q = 0; q < Q; q++)
 #pragma unroll
         for (int r = 0; r < NA; r++) offn[q][r] = TapOff[ki][px[q]][r] + lane_block;
     };
     auto fetch_weights = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int q = 0; q < 2; q++)
+      for (int q = 0; q < Q; q++)
 #pragma unroll
         for (int r = 0; r < NA; r++) wnext[q][r] = TapW[ks][px[q]][r];
     };
@@ -983,7 +1026,7 @@ __device__ inline void gather_product_bf16_direct(
       const int w_off = __builtin_amdgcn_readfirstlane(
           (int)((unsigned)((k0 + ki) * chunks + cc) * 2u * (unsigned)Opad * 16u));
 #pragma unroll
-      for (int q = 0; q < 2; q++)
+      for (int q = 0; q < Q; q++)
 #pragma unroll
         for (int r = 0; r < NA; r++)
           ring[d][q][r] = __builtin_bit_cast(
@@ -995,10 +1038,10 @@ __device__ inline void gather_product_bf16_direct(
         ++ci;
       }
     };
-    bf16x8 bq[2];
+    bf16x8 bq[Q];
     auto stage_slot = [&](int d, int bb) __attribute__((always_inline)) {
 #pragma unroll
-      for (int q = 0; q < 2; q++) {
+      for (int q = 0; q < Q; q++) {
         float sv[8];
 #pragma unroll
         for (int r = 0; r < NPR; r++) {
@@ -1041,7 +1084,7 @@ __device__ inline void gather_product_bf16_direct(
 #pragma unroll
       for (int m = 0; m < 2 * OG; m++)
 #pragma unroll
-        for (int q = 0; q < 2; q++)
+        for (int q = 0; q < Q; q++)
           acc[m][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq[m], bq[q], acc[m][q], 0, 0, 0);
     };
     // (loads are issued unconditionally, past the last unit too, where they read the last
@@ -1097,7 +1140,7 @@ __device__ inline void gather_product_bf16_direct(
       const int o = 32 * m + 8 * g + lhi * 4;
       const f32x4 at = *reinterpret_cast<const f32x4 *>(&lds.bias[o]);
 #pragma unroll
-      for (int q = 0; q < 2; q++) {
+      for (int q = 0; q < Q; q++) {
         f32x4 more = at;
         if (add && n0 + px[q] < N)
           more += *reinterpret_cast<const f32x4 *>(
@@ -1109,7 +1152,7 @@ __device__ inline void gather_product_bf16_direct(
   const bool pack2 = (N & 1) == 0 && (reinterpret_cast<uintptr_t>(y) & 3) == 0;
   const bool odd = (l31 & 1) != 0, whole = o0 + kOT * OG <= O;  // (every output of the workgroup)
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
+  for (int q = 0; q < Q; q++) {
     const int n = n0 + px[q];
     if (n >= N) continue;
     bf16_t *yb = y + ((int64_t)b * O + o0 + lhi * 4) * N + n;
@@ -1149,7 +1192,7 @@ __device__ inline void gather_product_bf16_direct(
 // the four-entry one, in one launch: as a launch of its own the four-entry form of a few border tiles
 // began when the last of the others had ended (4 x 32 -> 64 channels of 64 x 128: 23 + 30 us for
 // the input gradient's two launches).
-template <bool PACKED, int OG>
+template <bool PACKED, int OG, int Q>
 __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel(
     const bf16_t *__restrict__ src, const float *__restrict__ map, const float *__restrict__ iw,
     const uint16_t *__restrict__ wb, const bf16_t *__restrict__ bias, bf16_t *__restrict__ y,
@@ -1158,27 +1201,27 @@ __global__ __launch_bounds__(kThreads, 2) void gather_product_bf16_direct_kernel
     const float *__restrict__ addend, const int *__restrict__ pair_mask,
     const int *__restrict__ row_mask, int mask_words) {
   __shared__ __attribute__((aligned(16))) union {
-    DirectLds<2, OG> two;
-    DirectLds<4, OG> four;
+    DirectLds<2, OG, Q> two;
+    DirectLds<4, OG, Q> four;
   } lds;
   if (gate && ((*gate == 0) != (run_if_zero != 0))) return;  // device-side path selection
   const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
   const int b = tile / tiles_per_img;
-  const int n0 = (tile - b * tiles_per_img) * kDgPx;
+  const int n0 = (tile - b * tiles_per_img) * (128 * Q);
   bool leading = false;
   if (pair_mask) {
     leading = !later_pairs_in_use(pair_mask, mask_words);
     if (!leading && row_mask) {
       int any = 0;
-      for (int r = n0 / OW; r <= min(n0 + kDgPx - 1, N - 1) / OW; r++) any |= row_mask[r];
+      for (int r = n0 / OW; r <= min(n0 + 128 * Q - 1, N - 1) / OW; r++) any |= row_mask[r];
       leading = any == 0;
     }
   }
   if (leading)
-    gather_product_bf16_direct<PACKED, 2, OG>(lds.two, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
+    gather_product_bf16_direct<PACKED, 2, OG, Q>(lds.two, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
                                               SW, N, K, weighted, wrap, gate, addend, b, n0);
   else
-    gather_product_bf16_direct<PACKED, 4, OG>(lds.four, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
+    gather_product_bf16_direct<PACKED, 4, OG, Q>(lds.four, src, map, iw, wb, bias, y, O, Opad, Gpad, SH,
                                               SW, N, K, weighted, wrap, gate, addend, b, n0);
 }
 
@@ -2704,12 +2747,21 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
     if ((from_map || from_packed) && !accumulate && OH * OW <= 0x7fffffffLL - kDgPx &&
         (int64_t)(Gpad / 8) * SH * SW * 16 < 0xffffff00LL &&
         K * (int64_t)(Gpad / kGC) * 2 * Opad * 16 < 0xffffff00LL) {
-      const int64_t tiles_per_img = (OH * OW + kDgPx - 1) / kDgPx;
+      const int64_t oblocks = Opad / (wide ? 2 * kOT : kOT);
+      const bool half = !wide || (OH * OW + kDgPx - 1) / kDgPx * B * oblocks <= kSmallDirectGrid;
+      const int tile_px = half ? kDgPx / 2 : kDgPx;
+      const int64_t tiles_per_img = (OH * OW + tile_px - 1) / tile_px;
       if (tiles_per_img * B > 0x7fffffffLL) return MCX_E_SHAPE;
-      const dim3 dgrid((unsigned)(tiles_per_img * B), (unsigned)(Opad / (wide ? 2 * kOT : kOT)));
-#define MCX_LAUNCH_DIRECT(FORM, OG)                                                              \
-  hipLaunchKernelGGL((gather_product_bf16_direct_kernel<FORM, OG>), dgrid, dim3(kThreads), 0, s, \
-                     reinterpret_cast<const bf16_t *>(src), map, iw,                             \
+      const dim3 dgrid((unsigned)(tiles_per_img * B), (unsigned)oblocks);
+#define MCX_LAUNCH_DIRECT(FORM, OG)              \
+  if (OG == 1 || half) {                         \
+    MCX_LAUNCH_DIRECT_PX(FORM, OG, 1);           \
+  } else {                                       \
+    MCX_LAUNCH_DIRECT_PX(FORM, 2, 2);            \
+  }
+#define MCX_LAUNCH_DIRECT_PX(FORM, OG, Q)                                                        \
+  hipLaunchKernelGGL((gather_product_bf16_direct_kernel<FORM, OG, Q>), dgrid, dim3(kThreads), 0, \
+                     s, reinterpret_cast<const bf16_t *>(src), map, iw,                             \
                      reinterpret_cast<const uint16_t *>(wp),                                     \
                      reinterpret_cast<const bf16_t *>(bias), reinterpret_cast<bf16_t *>(y),      \
                      (int)O, Opad, Gpad, (int)SH, (int)SW, (int)(OH * OW), (int)OW, (int)K,      \
@@ -2731,6 +2783,7 @@ int launch_gather_product(const TD *src, const float *map, const float *iw, cons
       }
       profile_end(s);
 #undef MCX_LAUNCH_DIRECT
+#undef MCX_LAUNCH_DIRECT_PX
       MCX_HIP_CHECK_LAUNCH();
       return 0;
     }

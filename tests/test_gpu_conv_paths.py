@@ -415,6 +415,30 @@ def test_weight_gradient_with_staged_operands_over_ragged_channel_groups(row_shi
     assert_close_elementwise(gr[1].float(), g_o[1], tol, "grad_weight")
 
 
+@pytest.mark.parametrize("row_shift", [0.0, 0.37])
+@pytest.mark.parametrize("taps", [1, 9, 10, 14, 25])
+@pytest.mark.parametrize("shape", [(2, 16, 64, 2, 63), (1, 20, 65, 2, 64), (3, 64, 40, 3, 43),
+                                   (1, 33, 128, 5, 51), (2, 128, 24, 7, 37)])
+def test_bf16_direct_products_over_tiles_of_128_pixels(shape, taps, row_shift, device):
+    """Pixel counts around one and two tiles of 128, odd and even; outputs of one and two groups of 64 on
+    either side (forward and input gradient); taps that fill a resolved group (13 of two entries, nine of
+    four) and its batches of five a thread and that do not."""
+    B, Ci, Co, H, W = shape
+    g = torch.Generator().manual_seed(taps + Ci)
+    bf = lambda t: t.to(torch.bfloat16)
+    x, gy = bf(torch.randn(B, Ci, H, W, generator=g)), bf(torch.randn(B, Co, H, W, generator=g))
+    w = bf(torch.randn(Co, Ci, taps, generator=g) / (Ci * taps) ** 0.5)
+    b = bf(torch.randn(Co, generator=g))
+    smap = synthetic.latitude_map(H, W, 2)[:, :, :taps].contiguous()
+    smap[..., 1] = (smap[..., 1] + row_shift).clamp(0, H - 1)
+    y_o = O.mapped_conv_forward(x.float(), smap, w.float(), b.float(), taps, 1)
+    gx_o = O.mapped_conv_backward(gy.float(), smap, x.float(), w.float(), b.float(), taps, 1)[0]
+    xd, sd, wd_, bd, gyd = dev(x, smap, w, b, gy)
+    # samples and interpolation weights rounded to 2^-9 each, the result once: as in the tests around
+    assert rel_err(_C.mapped_conv_forward(xd, sd, wd_, bd, taps, 1).float(), y_o) < 2e-2
+    assert rel_err(_C.mapped_conv_backward(gyd, sd, xd, wd_, bd, taps, 1)[0].float(), gx_o) < 2e-2
+
+
 @pytest.mark.parametrize("row_shift", [0.0, 0.5])
 @pytest.mark.parametrize("shape", [(1, 3, 5, 6, 16), (2, 1, 2, 3, 8), (1, 9, 17, 5, 264)])
 def test_bf16_backward_with_very_few_channels(shape, row_shift, device):
