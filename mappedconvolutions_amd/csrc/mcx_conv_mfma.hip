@@ -277,9 +277,8 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(
 // x[b][g][n] -> xt[b][n][Gpad] (channels past G zero): 64 pixels x 64 channels per
 // workgroup through LDS, coalesced on both sides.  CHUNKED: xt[b][Gpad/16][n][16], a record's sixteen
 // channels of a chunk with the same chunk of the other records (see weight_grad_mfma_kernel).
-template <bool CHUNKED>
-__device__ inline int64_t record_offset(int64_t n, int g, int Gpad, int64_t plane) {
-  return CHUNKED ? ((int64_t)(g / kGC) * plane + n) * kGC + g % kGC : n * Gpad + g;
+__device__ inline int64_t record_offset(int64_t n, int g, int Gpad, int64_t plane, bool chunked) {
+  return chunked ? ((int64_t)(g / kGC) * plane + n) * kGC + g % kGC : n * Gpad + g;
 }
 template <typename TD, bool CHUNKED = false>
 __global__ __launch_bounds__(256) void to_channel_last_kernel(const TD *__restrict__ x,
@@ -301,7 +300,7 @@ __global__ __launch_bounds__(256) void to_channel_last_kernel(const TD *__restri
     const int64_t n = n0 + ly + 4 * r;
     const int g = g0 + lx;
     if (n < plane && g < Gpad)
-      xt[(int64_t)b * plane * Gpad + record_offset<CHUNKED>(n, g, Gpad, plane)] = tile[lx][ly + 4 * r];
+      xt[(int64_t)b * plane * Gpad + record_offset(n, g, Gpad, plane, CHUNKED)] = tile[lx][ly + 4 * r];
   }
 }
 
@@ -1255,7 +1254,23 @@ constexpr int kWgKTMesh = 7;        // and of fp32 mesh signals with no more
 // vertices, 4 x 64 -> 128 channels, without and with it: one point 222 us, 226, bf16 164, 167; two points 264, 255, bf16
 // 200, 202).
 template <typename TD>
-constexpr bool chunked_records(bool cl, int np) { return cl && np > (sizeof(TD) == 4 ? 1 : 2); }
+constexpr bool chunks_pay(bool cl, int np) { return cl && np > (sizeof(TD) == 4 ? 1 : 2); }
+// Whether every XCD can take one channel group.
+__host__ __device__ inline bool groups_by_xcd(int ranges, int cgroups) {
+  return (ranges & 7) == 0 && cgroups > 1 && 8 % cgroups == 0;
+}
+// Where they cannot, an XCD meets all chunks of a record.  In fp32 they are as good as whole records then (4 x 96
+// -> 128 channels, 40 962 vertices, seven taps of four random points 667 us, whole 686; 160 -> 32 778 and 863; 512 -> 128
+// of 20 000 1742 and 2122); in bf16 a line of a whole record holds the chunks of four groups, and where there are more of them and an image's
+// records are more than half an L2 they are the better form (four of 40 962 vertices, 160 -> 128 833 us, whole 695; 256 -> 32
+// 1189 and 890; 10 242 vertices, 160 -> 32, 3.3 MB, 178 and 164; 96 -> 32, 2 MB, 109 and 110; 2562 vertices,
+// 256 -> 32, 1.3 MB, 74 and 81; kernels of real meshes, three points, 40 962 vertices, 160 -> 128 504 and 520).
+template <typename TD>
+bool chunked_records(bool cl, int np, int ranges, int cgroups, int64_t image_bytes) {
+  return chunks_pay<TD>(cl, np) &&
+         (sizeof(TD) == 4 || cgroups <= 4 || groups_by_xcd(ranges, cgroups) ||
+          image_bytes <= (int64_t)1 << 21);
+}
 constexpr int kLdPx = kTilePx + 4;  // LDS row stride (floats)
 
 // The consumers of a pair mask only ask whether a pair beyond the first two is in use
@@ -1295,7 +1310,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     int G, int GH, int GW, int MH, int MW, int K, int weighted, int wrap, int tiles_x,
     int tiles_per_img, int tw_shift, int total_tiles, int ranges, int cgroups,
     float *__restrict__ plain_sum_part, const int *__restrict__ pair_mask, int run_if_leading,
-    const int *__restrict__ runs_state, const uint4 *__restrict__ tap_table) {
+    const int *__restrict__ runs_state, const uint4 *__restrict__ tap_table, int in_chunks) {
   constexpr int NE = NP * NCORN;  // (offset, weight) pairs per pixel and tap
   static_assert(NA >= 1 && NA <= NE, "NA counts leading pairs");
   if (runs_state && runs_done(runs_state)) return;  // (see mcx_conv_runs.h)
@@ -1308,7 +1323,8 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // different rows on different banks) and feed v_mfma_f32_16x16x32_bf16, whose lanes take
   // 8 consecutive pixels of their row.
   constexpr bool kBf16 = sizeof(TD) == 2;
-  constexpr bool kChunked = chunked_records<TD>(CL, NP);
+  constexpr bool kSideBySide = chunks_pay<TD>(CL, NP);  // (taps are resolved side by side)
+  const bool chunked = kSideBySide && (!kBf16 || in_chunks != 0);
   constexpr int kLdPxB = kTilePx + 8;
   constexpr int kWgA = wg_plain_channels<TD>(), kWgCB = wg_gathered_blocks<TD>();
   constexpr int MB = kWgA / 64;  // 16-row blocks of plain channels per wave
@@ -1336,11 +1352,11 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // Records in chunks: an XCD takes one channel group, and its workgroups walk the images together (tile t
   // goes to range t % ranges).  40 962 vertices, 4 x 64 -> 128 channels, seven taps of four random points: an
   // image's records are 10.5 MB and the kernel was bound by L2 misses, 2.5 GB of them at 5.7 TB/s, as many as
-  // the gather reads; now 1.25 GB, and 338 us for 443 (with the taps read side by side, see below, and seven
-  // taps' accumulators, which do not spill).  Whole weight gradients, before and now: one of these images
+  // the gather reads; now 1.25 GB, and 338 us for 443 (with the taps read side by side, see below, and the accumulators
+  // of seven taps, with which 14 registers spill and not 36).  Whole weight gradients, before and now: one of these images
   // 167 -> 127, bf16 130 -> 100; two of 20 000 vertices, 128 -> 128 channels, nine taps 366 -> 211, bf16 220 -> 142;
   // a real mesh kernel of three points, 4 x 64 -> 128 322 -> 287, bf16 256 -> 214.
-  const bool spread = kChunked && (ranges & 7) == 0 && cgroups > 1 && 8 % cgroups == 0;
+  const bool spread = chunked && groups_by_xcd(ranges, cgroups);
   if (spread) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, ablocks = combos / cgroups;
     combo = slot % ablocks * cgroups + xcd % cgroups;
@@ -1513,7 +1529,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
                                          live ? (weighted ? iw[e] : 1.f) : 0.f, t);
 #pragma unroll
         for (int i = 0; i < NCORN; i++) {
-          o[sp * NCORN + i] = CL ? t.off[i] * (unsigned)(kChunked ? kGC : Gpad) : t.off[i];
+          o[sp * NCORN + i] = CL ? t.off[i] * (unsigned)(chunked ? kGC : Gpad) : t.off[i];
           w_[sp * NCORN + i] = t.wt[i];
         }
       }
@@ -1534,7 +1550,8 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
     auto issue = [&](int cb, int k) {
       if constexpr (kQuads) {
         const char *base = reinterpret_cast<const char *>(
-            gath_b + record_offset<kChunked>(0, min(g_first + cb * kGC + qc, Gpad - 4), Gpad, gplane));
+            gath_b +
+            record_offset(0, min(g_first + cb * kGC + qc, Gpad - 4), Gpad, gplane, chunked));
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
@@ -1547,7 +1564,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
         // 8 contiguous channels of the pixel row; a workgroup whose channels lie past the
         // padded count reads the last valid group (its products are not stored)
         const char *base = reinterpret_cast<const char *>(
-            gath_b + record_offset<kChunked>(0, min(g0, Gpad - 8), Gpad, gplane));
+            gath_b + record_offset(0, min(g0, Gpad - 8), Gpad, gplane, chunked));
 #pragma unroll
         for (int i = 0; i < NA; i++) {
           const char *row = base + off[i];
@@ -1643,7 +1660,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
           }
         }
       }
-      if constexpr (kChunked) {
+      if constexpr (kSideBySide) {
         // Consecutive threads take consecutive taps of a pixel, which lie side by side in the map: a
         // pixel to a thread, the lines of all taps of all pixels (43 KB at seven taps of four points)
         // are wanted again after the L1 has lost them.  (The mesh above, in fp32: 391 us a pixel to a thread,
@@ -3174,10 +3191,12 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
       (char *)scratch + align256((size_t)part_ranges * (size_t)(round_up(A, 4) * G * K) * 4));
   int *pair_mask = reinterpret_cast<int *>((char *)sum_part + align256((size_t)part_ranges * A * 4));
   int *const pair_mask_ws = pair_mask;  // (a plan may supply the mask; the copy's room follows this one)
+  const bool in_chunks =
+      chunked_records<TD>(cl, m.np, ranges, cgroups, GH * GW * Gpad * (int64_t)sizeof(TD));
   if (cl) {
     TD *stage = reinterpret_cast<TD *>((char *)pair_mask + 256);
     dim3 tg((unsigned)((GH * GW + 63) / 64), (unsigned)((Gpad + 63) / 64), (unsigned)B);
-    if (chunked_records<TD>(cl, m.np))
+    if (in_chunks)
       hipLaunchKernelGGL((to_channel_last_kernel<TD, true>), tg, dim3(256), 0, s, gath, stage, (int)G,
                          (int)Gpad, GH * GW);
     else
@@ -3231,9 +3250,10 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
                      0, s, plain, gath, map, iw, part, (int)A, (int)G, (int)GH, (int)GW, (int)MH,   \
                      (int)MW, (int)K, m.weighted, m.wrap, t.tiles_x, t.tiles_per_img,            \
                      t.tw_shift, (int)t.total, ranges, cgroups,                                  \
-                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state, tap_table)
-// (seven taps, those of a mesh vertex and its neighbours, leave the registers that nine spill: a pass of
-// nine for the kernel of seven taps of four points 402 us, of seven 391)
+                     plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state, tap_table, \
+                     in_chunks ? 1 : 0)
+// (a pass of seven taps, those of a mesh vertex and its neighbours, spills 14 registers at four points where one
+// of nine spills 40: a pass of nine for the kernel of seven taps 402 us, of seven 391)
 #define MCX_LAUNCH_NA(NCORN, NP, CL, NA, MASK, LEAD)                           \
   if constexpr (CL && sizeof(TD) == 4 && NA > 1) {                            \
     if (K <= kWgKTMesh) {                                                     \

@@ -60,3 +60,27 @@ def test_weight_gradient_over_chunks_of_records(dtype, points, k, ci, co, v, dev
     tol = 1e-5 if dtype == torch.float32 else 8e-3
     assert rel_err(got[1], gw) < tol
     assert rel_err(got[2], gy.double().sum((0, 2, 3))) < tol
+
+
+@pytest.mark.parametrize("points,k,ci,co,v", [
+    (4, 7, 96, 40, 10922), (4, 7, 96, 40, 10923),  # 2 MB of records, in chunks and whole
+    (3, 9, 70, 130, 22000),                        # five groups of channels, two of plain ones
+    (4, 1, 160, 8, 6600), (3, 10, 250, 20, 4200),  # ten and sixteen groups
+])
+def test_bf16_weight_gradient_over_whole_records(points, k, ci, co, v, device):
+    """bf16 records of more than 2 MB an image stay whole where the groups of channels are more than four
+    and do not share out the XCDs.  Samples are rounded to 2^-9 each and the result once: as above."""
+    g = torch.Generator().manual_seed(ci + k)
+    B = 2
+    idx = torch.randint(v, (1, v, k, points), generator=g).float()
+    smap = torch.stack((idx, torch.zeros_like(idx)), -1).contiguous()
+    iw = torch.rand(1, v, k, points, generator=g)
+    x, gy = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((B, ci, 1, v), (B, co, 1, v)))
+    w, b = torch.zeros(co, ci, k, dtype=torch.bfloat16), torch.zeros(co, dtype=torch.bfloat16)
+    got = _C.weighted_mapped_conv_backward(gy.cuda(), smap.cuda(), iw.cuda(), x.cuda(), w.cuda(),
+                                           b.cuda(), k, 0, needs=(False, True, False))[1]
+    gw = torch.zeros(co, ci, k, dtype=torch.float64)
+    for t in range(k):
+        col = (x.double()[:, :, 0, idx[0, :, t].long()] * iw[0, :, t].double()).sum(-1)
+        gw[:, :, t] = torch.bmm(gy.double()[:, :, 0], col.transpose(1, 2).contiguous()).sum(0)
+    assert rel_err(got, gw) < 8e-3
