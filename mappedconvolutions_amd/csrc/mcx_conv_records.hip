@@ -587,13 +587,18 @@ GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
   q.at = A == 1 ? 1 : A <= 4 ? 4 : 16;
   q.ablocks = (A + q.at - 1) / q.at;
   q.gblocks = (read_stride(G) + 2 * q.lpr - 1) / (2 * q.lpr);
-  // Several taps a workgroup from 98304 locations on, with two to four plain channels 65536; with fewer,
-  // workgroups of one tap are more and wait less (us, one tap and several, nine taps of shuffled maps.  10 -> 1
-  // channels: 50 x 80 4.6, 7.6; 2 of 100 x 350 31, 35; 200 x 500 59, 43; 400 x 700 202, 97.  2 of 200 x 300,
-  // 3 -> 1 38, 29.  220 x 300, 6 -> 1 25, 29, but 7 -> 4 31, 21.  2 of 300 x 500, 16 -> 3 216, 99.  Four waves a SIMD
-  // spill: twice as slow.)
+  // Several taps a workgroup where eight taps and more fill eight ninths of the workgroups' and there are locations
+  // enough: with fewer of either, workgroups of one tap are more and have the loads of four locations in flight
+  // (whole weight gradients, us, one tap and several.  Coherent maps, nine taps: 10 -> 1 channels, 100 000 locations 41,
+  // 56; 150 000 62, 69; 200 000 85, 88; 250 000 105, 103; 2 -> 1 100 000 27, 30; 130 000 33, 31; 4 -> 2 50 000 23, 24; 66 000
+  // 27, 26; 10 -> 4 66 000 37, 37; ten taps 100 000 46, 55; 25 taps 66 000 64, 73; 150 000 145, 145.  Shuffled maps gain
+  // earlier: 10 -> 1 100 000 71, 70; 130 000 95, 84; 4 -> 2 66 000 33, 30.  Taps, shuffled, 300 000 locations: 10 -> 1,
+  // groups of nine, one 55, 69; four 114, 114; five 137, 130, coherent 72, 86; ten 261, 292; eleven 281, 302; 18 451, 378;
+  // 2 -> 1, groups of five, five 61, 62; six 76, 89; seven 88, 90; nine 112, 92.  Four waves a SIMD spill: twice as slow.)
   const int64_t many = q.at == 1 ? (q.lpr == 2 ? RecShape<2>::kTaps : RecShape<8>::kTaps) : q.at == 4 ? 3 : 1;
-  const int64_t taps = B * N >= (q.at == 1 ? 98304 : 65536) ? many : 1;
+  const int64_t enough = q.at == 1 ? (q.lpr == 2 ? 1 << 17 : 3 << 16) : K > 9 ? 1 << 17 : 1 << 16;
+  const bool filled = K >= 8 && K * 9 >= (K + many - 1) / many * many * 8;
+  const int64_t taps = filled && B * N >= enough ? many : 1;
   q.taps = (int)taps;
   const int64_t tile = (taps > 1 ? 1 : q.lpr == 2 ? 2 : 4) * (kThreads / q.lpr);
   q.tiles_per_img = (N + tile - 1) / tile;

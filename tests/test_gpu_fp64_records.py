@@ -330,3 +330,23 @@ def test_weight_gradient_of_several_taps_a_workgroup(ci, co, k, p, interp, few, 
     got = getattr(_C, name)(*[t.cuda() for t in (gy, *maps, x, w, b)], k, interp,
                             needs=(False, True, False))[1]
     assert rel_err(got, getattr(O, name)(gy, *maps, x, w, b, k, interp)[1]) < 1e-12
+
+
+@pytest.mark.parametrize("ci,co,k,locations", [
+    # one output: 196 608 locations, groups of nine taps; up to four channels 131 072, groups of five
+    (10, 1, 9, 196607), (10, 1, 9, 196608), (6, 1, 8, 196608), (10, 1, 7, 196608), (16, 1, 17, 196608),
+    (10, 1, 10, 196608), (3, 1, 5, 131072), (3, 1, 9, 131071), (3, 1, 9, 131072), (4, 1, 14, 131074),
+    # two to four: 65 536 locations, with more than nine taps 131 072, groups of three
+    (4, 2, 8, 65535), (4, 2, 8, 65536), (4, 2, 7, 65536), (10, 4, 9, 65539),
+    (5, 3, 17, 131071), (5, 3, 17, 131072), (5, 3, 25, 131073)])
+def test_weight_gradient_around_the_rule_for_several_taps(ci, co, k, locations, device):
+    """Locations and taps on either side of where a workgroup takes several taps.  Sums of 200 000
+    terms of both signs in 64 bits: up to some 1e-14 of the result with their order, 1e-12 allowed."""
+    g = torch.Generator().manual_seed(ci + 31 * k)
+    ih, iw_ = 20, 33
+    smap, _ = helpers.random_map(g, 1, locations, k, 0, ih, iw_, torch.float64)
+    x, gy, w, b = (torch.randn(s, generator=g, dtype=torch.float64)
+                   for s in ((1, ci, ih, iw_), (1, co, 1, locations), (co, ci, k), (co,)))
+    got = _C.mapped_conv_backward(*[t.cuda() for t in (gy, smap, x, w, b)], k, 1,
+                                  needs=(False, True, False))[1]
+    assert rel_err(got, O.mapped_conv_backward(gy, smap, x, w, b, k, 1)[1]) < 1e-12
