@@ -1396,11 +1396,16 @@ int fill(T *p, int64_t n, T v, hipStream_t s) {
 
 // Planes a thread takes where whole ones leave SIMDs idle: halved until the grid is about two waves for
 // each of them, but not below sixteen, a third of what resolving a thread's taps or reading its list
-// costs.  (Average pooling of 64 planes of 249 x 498 to half the size, 500 waves of 64 planes: 73 us, so 28; its
+// costs, and as long as `resident` waves, those that the chip holds at once, are not exceeded.  (Average pooling of 64
+// planes of 249 x 498 to half the size, 500 waves of 64 planes: 73 us, so 28; its
 // gradient 66, 45.  1024 waves and 4096 instead of 2048: 29 and 27, 64 and 45; 128 planes of 128 x 256, forward 30 and
-// 25 against 25, gradient 25 and 24 against 21.)
-inline int fewer_planes(int per, int64_t waves, int64_t planes) {
-  while (per > 16 && waves * div_up(planes, per) < 2048) per /= 2;
+// 25 against 25, gradient 25 and 24 against 21.  Max unpooling, three waves a SIMD: 64 planes of 249 x 498, 1940 waves,
+// in two rounds of 3880 351 us, in one 299; of 180 x 360, 1012, in 2024 314, in 4048 413; of 200 x 400, 1252, in 2504 400 for
+// 509.  Maps of random taps, whose planes come from the caches, lose where more planes are read side by side: gradient of
+// average pooling, 64 planes of 249 x 498, 1940 waves 2083 us, 3880 2615; forward, 256 planes of 64 x 128 78 and 97.)
+inline int fewer_planes(int per, int64_t waves, int64_t planes, int64_t resident = 4096) {
+  while (per > 16 && waves * div_up(planes, per) < 2048 && waves * div_up(planes, per / 2) <= resident)
+    per /= 2;
   return per;
 }
 
@@ -1553,7 +1558,8 @@ int gather_transposed(const void *src, const int64_t *idx, void *dst, const void
          tiles * (kThreads / 64) * ((planes + reps * 2 * kTCH - 1) / (reps * 2 * kTCH)) >= 8192)
     reps *= 2;
   int per = reps * kTCH;  // planes a workgroup
-  if (OP != UN_RESAMPLE && reps == 1) per = fewer_planes(per, tiles * (kThreads / 64), planes);
+  if (OP != UN_RESAMPLE && reps == 1)
+    per = fewer_planes(per, tiles * (kThreads / 64), planes, OP == UN_MAX ? 3072 : 4096);
   const int64_t groups = (planes + per - 1) / per;
   const int64_t blocks = groups * tiles;
   if (blocks > 0x7fffffffLL) return kNotApplicable;
