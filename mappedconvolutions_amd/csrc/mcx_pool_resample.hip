@@ -737,8 +737,11 @@ __global__ __launch_bounds__(kThreads) void scan_sums_kernel(uint32_t *__restric
 // at the same step.  Lists longer than kSortMax stay as filled.
 constexpr uint32_t kSortMax = 512;
 // Lists of more entries than these in half of a wave's lanes go through the network, of fewer by insertion
-// in LDS (124 002 lists of 9 on average: with 2, 4 and 8 10, 12 and 20 us; 524 288 of 3: 18, 19 and 25).
-constexpr uint32_t kFewEntries = 2;
+// in LDS (124 002 lists of 9 on average: with 2, 4 and 8 10, 12 and 20 us; 524 288 of 3: 18, 19 and 25).  The network
+// of fp64 weights compares them beside the sources, at some three times the instructions (three planes onto 512 x 1024
+// from 256 x 1536, lists of three, with 2 and 8 176 and 145 us).
+template <typename T>
+constexpr uint32_t few_entries() { return sizeof(T) == 4 ? 2 : 8; }
 
 // Batcher's odd-even merge sort for N keys (16 or 32) as a list of compare-exchange pairs, made
 // at compile time so that the unrolled network indexes registers statically.
@@ -906,7 +909,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
   if (longest < 2u) return;
   if (longest <= 64u) {
     const bool few = longest <= (uint32_t)kNetN &&
-                     __builtin_popcountll(__builtin_amdgcn_ballot_w64(len > kFewEntries)) < 32;
+                     __builtin_popcountll(__builtin_amdgcn_ballot_w64(len > few_entries<T>())) < 32;
     constexpr int kRun = 1024;
     __shared__ uint32_t run_src[kThreads / 64][kRun];
     __shared__ T run_wt[kThreads / 64][kRun];
@@ -930,8 +933,10 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
       } else if (longest <= 16u) {
         network_sort<T, 16>(run_src[wv], run_wt[wv], off, off + (mine ? len : 0u));
       } else {
-        network_sort<T, kNetN>(run_src[wv], run_wt[wv], off,
-                               off + (mine && len <= (uint32_t)kNetN ? len : 0u));
+        // (not where every list is a longer one: the network takes the same time over none)
+        if (__builtin_amdgcn_ballot_w64(mine && len - 2u <= (uint32_t)kNetN - 2u) != 0)
+          network_sort<T, kNetN>(run_src[wv], run_wt[wv], off,
+                                 off + (mine && len <= (uint32_t)kNetN ? len : 0u));
         unsigned long long left = __builtin_amdgcn_ballot_w64(mine && len > (uint32_t)kNetN);
         for (; left != 0; left &= left - 1) {
           const int q = __builtin_ctzll(left);
