@@ -766,9 +766,14 @@ constexpr SortNetwork make_network(int N) {
 constexpr SortNetwork kNet32 = make_network(32), kNet16 = make_network(16);
 
 // Weights in the order of their bits: a negative one's turned over, the sign of the others set.
+// (A NaN has its place among them: entries compared as numbers lost one beside it.)
 __device__ inline uint32_t ordered_bits(float w) {
   const uint32_t b = __builtin_bit_cast(uint32_t, w);
   return b & 0x80000000u ? ~b : b | 0x80000000u;
+}
+__device__ inline unsigned long long ordered_bits(double w) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, w);
+  return b >> 63 ? ~b : b | 1ull << 63;
 }
 __device__ inline float from_ordered_bits(uint32_t b) {
   return __builtin_bit_cast(float, b & 0x80000000u ? b & 0x7fffffffu : ~b);
@@ -858,8 +863,8 @@ __device__ inline void rank_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint3
   const uint32_t code = e_src[start + (mine ? lane : 0u)];
   const T w = e_wt[start + (mine ? lane : 0u)];
   uint32_t rank = 0;
+  const auto low = ordered_bits(w);
   if constexpr (sizeof(T) == 4) {
-    const uint32_t low = ordered_bits(w);
     const unsigned long long key = (unsigned long long)code << 32 | low;
     for (uint32_t j = 0; j < n; j++) {  // (entry j sits in lane j)
       const unsigned long long other =
@@ -870,12 +875,10 @@ __device__ inline void rank_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint3
   } else {
     for (uint32_t j = 0; j < n; j++) {
       const uint32_t cj = (uint32_t)__builtin_amdgcn_readlane((int)code, (int)j);
-      const long long wb = __builtin_bit_cast(long long, w);
-      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)wb, (int)j);
-      const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(wb >> 32), (int)j);
-      const T wj = __builtin_bit_cast(T, (long long)(((unsigned long long)hi << 32) | lo));
-      const bool tie = !(wj < w) && !(w < wj);
-      rank += (cj < code || (cj == code && (wj < w || (tie && j < lane)))) ? 1u : 0u;
+      const unsigned long long other =
+          (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(low >> 32), (int)j) << 32 |
+          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)low, (int)j);
+      rank += (cj < code || (cj == code && (other < low || (other == low && j < lane)))) ? 1u : 0u;
     }
   }
   // (every lane has read the whole list before the first one writes: the stores depend on all

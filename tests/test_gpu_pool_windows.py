@@ -243,3 +243,23 @@ def test_lists_are_sorted_by_source(dtype, long, pattern, device):
     for i, d in enumerate(dest.tolist()):
         want[:, d] += gy.numpy()[0, :, 0, i]
     assert torch.equal(out, torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("k", [3, 20, 40, 64, 70])
+def test_a_nan_among_the_weights_of_one_source_is_not_lost(dtype, k, device):
+    """A pixel that one source reaches through all taps, one of which weighs NaN: ties of the source are
+    sorted by weight, and the NaN and every number beside it stay in the list."""
+    g = torch.Generator().manual_seed(k)
+    W = 6
+    smap = torch.zeros(1, W, k, 1, 2, dtype=dtype)
+    smap[..., 0] = torch.arange(W)[:, None, None]
+    iw = torch.rand(1, W, k, 1, generator=g, dtype=dtype) + 1
+    iw[0, 2, k // 2] = float("nan")
+    gy = torch.ones(1, 1, 1, W, dtype=dtype)
+    out = _C.weighted_mapped_avg_unpool(gy.cuda(), smap.cuda(), iw.cuda(), 1, W, k, 0).cpu().view(-1)
+    want = iw.sum((2, 3)).view(-1) / k
+    assert torch.isnan(out[2])
+    ok = torch.arange(W) != 2
+    # sums of up to 70 positive terms: at most 70 roundings of 2^-24 (2^-53)
+    assert ((out - want).abs()[ok] <= want[ok] * (5e-6 if dtype == torch.float32 else 1e-14)).all()
