@@ -730,8 +730,7 @@ __global__ __launch_bounds__(kThreads) void scan_sums_kernel(uint32_t *__restric
   }
 }
 
-// Orders the entries of every destination pixel by source location (insertion sort,
-// one thread per pixel; lists are short).  The fill kernel places entries in the
+// Orders the entries of every destination pixel by source location.  The fill kernel places entries in the
 // order its atomics happen to retire: sorted lists make the result independent of
 // that order, and neighbouring lanes of the gather then read neighbouring sources
 // at the same step.  Lists longer than kSortMax stay as filled.
@@ -771,12 +770,15 @@ __device__ inline uint32_t ordered_bits(float w) {
   const uint32_t b = __builtin_bit_cast(uint32_t, w);
   return b & 0x80000000u ? ~b : b | 0x80000000u;
 }
+__device__ inline float from_ordered_bits(uint32_t b) {
+  return __builtin_bit_cast(float, b & 0x80000000u ? b & 0x7fffffffu : ~b);
+}
 __device__ inline unsigned long long ordered_bits(double w) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, w);
   return b >> 63 ? ~b : b | 1ull << 63;
 }
-__device__ inline float from_ordered_bits(uint32_t b) {
-  return __builtin_bit_cast(float, b & 0x80000000u ? b & 0x7fffffffu : ~b);
+__device__ inline double from_ordered_bits(unsigned long long b) {
+  return __builtin_bit_cast(double, b >> 63 ? b & ~(1ull << 63) : ~b);
 }
 
 // Sorts the list [start, end) of this lane (at most N entries) in registers: read once, run
@@ -889,6 +891,51 @@ __device__ inline void rank_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint3
   }
 }
 
+// The list [start, start + n) of one lane, n at most kSortMax, sorted by the wave as rank_sort does, through LDS
+// (`code` and `low`: room for n entries and three more).
+template <typename T, typename Bits>
+__device__ inline void long_rank_sort(uint32_t *e_src, T *e_wt, uint32_t start, uint32_t n,
+                                      uint32_t *code, Bits *low) {
+  const uint32_t lane = threadIdx.x & 63, padded = (n + 3u) & ~3u;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // (the list before this one was read there)
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  for (uint32_t t = lane; t < padded; t += 64) {
+    code[t] = t < n ? e_src[start + t] : 0xffffffffu;  // (comes before no entry)
+    low[t] = t < n ? ordered_bits(e_wt[start + t]) : ~(Bits)0;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  for (uint32_t t0 = 0; t0 < n; t0 += 128) {  // two entries a lane
+    const uint32_t t[2] = {t0 + lane, t0 + 64 + lane};
+    uint32_t c[2], rank[2] = {0u, 0u};
+    Bits w[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) c[q] = code[min(t[q], n - 1)], w[q] = low[min(t[q], n - 1)];
+    for (uint32_t j0 = 0; j0 < padded; j0 += 4) {
+      uint32_t oc[4];
+      Bits ow[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) oc[u] = code[j0 + u], ow[u] = low[j0 + u];
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          rank[q] += (oc[u] < c[q] ||
+                      (oc[u] == c[q] && (ow[u] < w[q] || (ow[u] == w[q] && j0 + u < t[q]))))
+                         ? 1u
+                         : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      if (t[q] < n) {
+        e_src[start + rank[q]] = c[q];
+        e_wt[start + rank[q]] = from_ordered_bits(w[q]);
+      }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries_kernel(
     const uint32_t *__restrict__ local, const uint32_t *__restrict__ bsum,
@@ -902,7 +949,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
   // coalesced accesses, as many lanes' lists at a time as surely fit; there each lane sorts its
   // list (one that starts 15 or so words after its neighbour's: separate cache lines in memory,
   // separate banks in LDS) in registers, of up to 16 or kNetN entries, and the wave one after the other the
-  // longer ones (5 x 5 pooling maps: about fifty entries).  Same order as the insertion sort below: by
+  // longer ones (5 x 5 pooling maps: about fifty entries).  Order: by
   // source, ties by weight.  What a wave waits for in LDS and memory bounds it, so its registers are kept to
   // those of four waves a SIMD.  (With two waves a SIMD, insertion in memory for short lists, lists of 17 to 32
   // sorted from memory and all lists of a wave by rank where one is longer: 524 288 lists of up to 16 entries 74 us,
@@ -910,13 +957,14 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
   const uint32_t len = end - start;
   const uint32_t longest = (uint32_t)wave_max((int)min(len, 0x7fffffffu));
   if (longest < 2u) return;
+  constexpr int kRun = 1024;
+  __shared__ __attribute__((aligned(16))) uint32_t run_src[kThreads / 64][kRun];
+  __shared__ __attribute__((aligned(16))) T run_wt[kThreads / 64][kRun];
+  const int wv = threadIdx.x >> 6;
   if (longest <= 64u) {
     const bool few = longest <= (uint32_t)kNetN &&
                      __builtin_popcountll(__builtin_amdgcn_ballot_w64(len > few_entries<T>())) < 32;
-    constexpr int kRun = 1024;
-    __shared__ uint32_t run_src[kThreads / 64][kRun];
-    __shared__ T run_wt[kThreads / 64][kRun];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63;
     const int lanes = longest <= 16u ? 64 : longest <= 32u ? 32 : 16;
     for (int l0 = 0; l0 < 64; l0 += lanes) {
       const bool mine = live && (unsigned)(lane - l0) < (unsigned)lanes;
@@ -960,9 +1008,21 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
     }
     return;
   }
-  if (!live) return;
-  if (end - start > kSortMax) return;
-  insertion_sort<T>(e_src, e_wt, start, end);
+  // Longer lists (5 x 5 taps between pixels: about a hundred entries), and the others of their waves: one list at a
+  // time by the whole wave.  (A lane to a list, by insertion in memory, each step waits for memory, the longer the more
+  // waves share the caches: gradient of average pooling, three planes
+  // of 512 x 1024, 25 taps, 23.9 ms at two waves a SIMD, 29.8 at four, so 3.2; fp64 20.5 and 4.6; of 16 x 32 1.9 and 0.7.)
+  unsigned long long left = __builtin_amdgcn_ballot_w64(len >= 2u && len <= kSortMax);
+  for (; left != 0; left &= left - 1) {
+    const int q = __builtin_ctzll(left);
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)start, q);
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, q);
+    if (n <= 64u)
+      rank_sort<T>(e_src, e_wt, s0, n);
+    else
+      long_rank_sort<T>(e_src, e_wt, s0, n, run_src[wv],
+                        reinterpret_cast<decltype(ordered_bits(T(0))) *>(run_wt[wv]));
+  }
 }
 
 // Planes per thread of the transposed gather's register paths.  The unpoolings read their list

@@ -263,3 +263,11 @@ def test_a_nan_among_the_weights_of_one_source_is_not_lost(dtype, k, device):
     ok = torch.arange(W) != 2
     # sums of up to 70 positive terms: at most 70 roundings of 2^-24 (2^-53)
     assert ((out - want).abs()[ok] <= want[ok] * (5e-6 if dtype == torch.float32 else 1e-14)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("long,pattern", [(67, "all"), (127, "one"), (128, "mixed"), (129, "one"), (193, "mixed"),
+                                          (257, "one"), (511, "one"), (512, "one"), (512, "mixed")])
+def test_long_lists_are_sorted_by_source(dtype, long, pattern, device):
+    """Lists that a wave sorts one at a time, of one to eight entries a lane."""
+    test_lists_are_sorted_by_source(dtype, long, pattern, device)
