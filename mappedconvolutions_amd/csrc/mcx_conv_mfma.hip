@@ -814,10 +814,16 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
     // (the overflow list of a transposed map, gate[1] entries long), added when there are any
     if (addend && gate && gate[1] > 0) {
       const float *ab = addend + ((int64_t)b * N + (int64_t)ei * OW + ej) * Opad + o0 + lhi * 4;
+      // (only those of outputs that there are, here and in the other products: all read, the input gradient of 4 x 8 ->
+      // 5 channels of 64 x 129 took 57 us, so 55; bf16, 2 x 6 -> 12 of 256 x 512 under a projection's kernel 126 and 115)
 #pragma unroll
       for (int m = 0; m < 2 * OG; m++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[m][i] += ab[32 * m + (i >> 2) * 8 + (i & 3)];
+        for (int g = 0; g < 4; g++)
+          if (o0 + 32 * m + 8 * g < O) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[m][4 * g + i] += ab[32 * m + 8 * g + i];
+          }
     }
 #pragma unroll
     for (int m = 0; m < 2 * OG; m++)
@@ -1141,7 +1147,7 @@ __device__ inline void gather_product_bf16_direct(
 #pragma unroll
       for (int q = 0; q < Q; q++) {
         f32x4 more = at;
-        if (add && n0 + px[q] < N)
+        if (add && o0 + 32 * m + 8 * g < O && n0 + px[q] < N)
           more += *reinterpret_cast<const f32x4 *>(
               addend + ((int64_t)b * N + n0 + px[q]) * Opad + o0 + o);
 #pragma unroll

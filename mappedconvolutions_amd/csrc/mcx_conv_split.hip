@@ -139,6 +139,7 @@ __device__ inline void split_epilogue(const SplitArgs &s, floatx16 *acc, const f
       for (int m = 0; m < NB; m++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
+          if (o0 + 32 * m + 8 * g >= s.O) continue;  // (no such outputs)
           const f32x4 add = *reinterpret_cast<const f32x4 *>(ab + 32 * m + 8 * g);
 #pragma unroll
           for (int i = 0; i < 4; i++) acc[m][4 * g + i] += add[i];
