@@ -871,7 +871,10 @@ int launch_gather_split(const SplitArgs &a, int64_t tiles, bool cl, hipStream_t 
   // 125 x 250, a training pass, 246 and 213; 4 x 64 -> 32 onto 256 x 512, transposed, 380 and 355.  Against
   // them: 4 x 32 -> 32 of 64 x 128 (256 workgroups) 31.3 and 34.4; 8 x 8 -> 3 onto 256 x 512, transposed, 159 and
   // 188; 4 x 16 -> 20 of 128 x 256 32 and 38; 2 x 40 -> 128 of 128 x 256, 5 x 5, 159 and 176.
-  const bool window = tiles * by_outputs >= 768 && a.G > kGC && nb < 4;
+  // One tap and one block of outputs have nothing else that would share the window (one tap, in windows and in memory:
+  // 2 x 64 -> 3 of 256 x 512 39 and 28; 4 x 128 -> 1 97 and 66; 4 x 32 -> 32 57 and 40, of a random map, whose groups do not
+  // fit and are the fewer at a time for it, 489 and 577).
+  const bool window = tiles * by_outputs >= 768 && a.G > kGC && nb < 4 && (a.K > 1 || nb > 1);
   const dim3 grid((unsigned)tiles, (unsigned)by_outputs);
 #define MCX_SPLIT(KERNEL, ...) \
   hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(kThreads), 0, s, a)
