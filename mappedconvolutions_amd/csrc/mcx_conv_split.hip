@@ -195,7 +195,7 @@ __device__ inline int quotient(int q, int d, float inv) {
   return r;
 }
 
-template <int NE, int NB, bool WINDOW>
+template <int NE, int NB, bool WINDOW>  // (windows for four entries only)
 __global__ __launch_bounds__(kThreads, NB > 2 ? 2 : !WINDOW && (NE == 1 || NB == 1) ? 4 : 3) void
 gather_product_split_kernel(const SplitArgs s) {
   __shared__ __attribute__((aligned(16))) uint4 Wt[2][SplitWeights<NB>::kPieces];
@@ -204,6 +204,7 @@ gather_product_split_kernel(const SplitArgs s) {
   __shared__ __attribute__((aligned(16))) int box[6][4];  // largest values by wave
   __shared__ __attribute__((aligned(16))) float Bias[32 * NB];
   __shared__ int unpaired;
+  static_assert(!WINDOW || NE == 4, "four entries");
   if (s.gate && ((*s.gate == 0) != (s.run_if_zero != 0))) return;
   const int tid = threadIdx.x;
   const int tile = xcd_contiguous_tile(blockIdx.x, gridDim.x);
@@ -350,8 +351,7 @@ gather_product_split_kernel(const SplitArgs s) {
     constexpr int NA = decltype(na_tag)::value;
     constexpr int kMine = NA == 4 ? 2 : 3;  // of three or six taps
     // (every load is issued before the first is used; past the group's end its last tap is read)
-    constexpr int kRaw = NE == 1 ? 1 : NA;
-    float2 raw[kMine][kRaw];
+    float2 raw[kMine][NA];
     float raw_w[kMine];
 #pragma unroll
     for (int j = 0; j < kMine; j++) {
@@ -360,7 +360,7 @@ gather_product_split_kernel(const SplitArgs s) {
       if (s.packed) {
         // pre-resolved entries [tap][slot][pixel]: (pixel index as bits, weight)
 #pragma unroll
-        for (int i = 0; i < kRaw; i++)
+        for (int i = 0; i < NA; i++)
           raw[j][i] = reinterpret_cast<const float2 *>(s.map)[((int64_t)k * 4 + i) * N + n_g];
       } else {
         const int64_t e = n_g * s.K + k;
@@ -383,16 +383,16 @@ gather_product_split_kernel(const SplitArgs s) {
         if (s.packed) {
 #pragma unroll
           for (int i = 0; i < NA; i++) {
-            const float2 q = raw[j][i < kRaw ? i : 0];
+            const float2 q = raw[j][i];
             wt[i] = live ? q.y * kSplitScale : 0.f;
             const int e = wt[i] != 0.f ? __builtin_bit_cast(int, q.x) : 0;
             y[i] = quotient(e, s.SW, inv_sw);
             x[i] = e - y[i] * s.SW;
           }
         } else {
-          CoordTap<NE> t;
-          resolve_coords<NE>(raw[j][0].x, raw[j][0].y, s.SH, s.SW, s.wrap != 0,
-                             live ? raw_w[j] * kSplitScale : 0.f, t);
+          CoordTap<4> t;
+          resolve_coords<4>(raw[j][0].x, raw[j][0].y, s.SH, s.SW, s.wrap != 0,
+                            live ? raw_w[j] * kSplitScale : 0.f, t);
 #pragma unroll
           for (int i = 0; i < NA; i++) {
             wt[i] = (t.ok >> i) & 1u ? t.wt[i] : 0.f;
@@ -637,25 +637,28 @@ gather_product_split_kernel(const SplitArgs s) {
   auto run = [&](auto na_tag) __attribute__((always_inline)) {
     constexpr int NA = decltype(na_tag)::value;
     // (two entries a tap of 64 outputs and more: as fast in memory, with the registers of a third wave)
-    if (!WINDOW || (NE == 4 && NA == 2 && NB > 1)) return in_memory(0, s.K, na_tag);
-    constexpr int kMost = kWinCache / NA < 6 ? kWinCache / NA : 6, kFew = 3;
-    // (groups of one size, as far as it goes; a window that holds six taps' pixels holds three of nearly
-    // twice the spread)
-    const int groups = (s.K + kMost - 1) / kMost;
-    int kg = (s.K + groups - 1) / groups;
-    const bool small = s.SH <= 0xffff && s.SW <= 0xffff;
-    for (int k0 = 0; k0 < s.K;) {
-      const int kn = min(kg, s.K - k0);
-      __syncthreads();  // the previous group's units are done with the taps and the window
-      if (!small || !in_window(k0, kn, na_tag)) {
-        if (small && kn > kFew) {
-          kg = kFew;
-          continue;
+    if constexpr (!WINDOW || (NA == 2 && NB > 1)) {
+      in_memory(0, s.K, na_tag);
+    } else {
+      constexpr int kMost = kWinCache / NA < 6 ? kWinCache / NA : 6, kFew = 3;
+      // (groups of one size, as far as it goes; a window that holds six taps' pixels holds three of nearly
+      // twice the spread)
+      const int groups = (s.K + kMost - 1) / kMost;
+      int kg = (s.K + groups - 1) / groups;
+      const bool small = s.SH <= 0xffff && s.SW <= 0xffff;
+      for (int k0 = 0; k0 < s.K;) {
+        const int kn = min(kg, s.K - k0);
+        __syncthreads();  // the previous group's units are done with the taps and the window
+        if (!small || !in_window(k0, kn, na_tag)) {
+          if (small && kn > kFew) {
+            kg = kFew;
+            continue;
+          }
+          __syncthreads();
+          in_memory(k0, kn, na_tag);
         }
-        __syncthreads();
-        in_memory(k0, kn, na_tag);
+        k0 += kn;
       }
-      k0 += kn;
     }
   };
   if (NE == 4 && leading)
@@ -860,8 +863,6 @@ int launch_gather_split(const SplitArgs &a, int64_t tiles, bool cl, hipStream_t 
   // of four.)
   const int blocks = (a.O + 31) / 32;
   const int nb = blocks == 1 ? 1 : blocks == 3 ? 3 : a.Opad % (2 * kOT) == 0 ? 4 : 2;
-  // Two images a workgroup where their accumulators leave two waves a SIMD and the chip is full all
-  // the same.
   const int64_t by_outputs = (blocks + nb - 1) / nb;
   // Windows (gather_product_split_kernel) where the grid is three workgroups a CU and more - with fewer,
   // each waits out a group's taps and then its window, where the form in memory has its loads in flight
