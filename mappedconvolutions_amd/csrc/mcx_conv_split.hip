@@ -345,7 +345,8 @@ gather_product_split_kernel(const SplitArgs s) {
       }
     }
   };
-  // Resolves taps k0 .. k0 + kn - 1 and multiplies them if they fit a window; returns whether they did.
+  // Resolves taps k0 .. k0 + kn - 1 and multiplies them if they fit a window; returns 1 then, else at
+  // least 2: one more than the windows that their box would fill.
   const float inv_sw = 1.f / (float)s.SW;
   auto in_window = [&](int k0, int kn, auto na_tag) __attribute__((always_inline)) {
     constexpr int NA = decltype(na_tag)::value;
@@ -441,7 +442,8 @@ gather_product_split_kernel(const SplitArgs s) {
     }
     cols = (cols + 3) & ~3;
     if (!seam && col0 + cols > s.SW) col0 = s.SW - cols;
-    if (cols > kWinPx || rows > kWinPx || rows * cols > kWinPx || cols > s.SW || col0 < 0) return false;
+    if (cols > kWinPx || rows > kWinPx || rows * cols > kWinPx || cols > s.SW || col0 < 0)
+      return max(2, 1 + (int)(min((unsigned)rows, 0xffffu) * min((unsigned)cols, 0xffffu) / kWinPx));
 #pragma unroll
     for (int j = 0; j < kMine; j++) {
       const int kl = half + 2 * j;
@@ -457,7 +459,7 @@ gather_product_split_kernel(const SplitArgs s) {
       }
     }
     units_in_window(k0, kn, na_tag, row0, col0, cols, rows);
-    return true;
+    return 1;
   };
 
   // ---- a group in memory ----
@@ -649,12 +651,19 @@ gather_product_split_kernel(const SplitArgs s) {
       for (int k0 = 0; k0 < s.K;) {
         const int kn = min(kg, s.K - k0);
         __syncthreads();  // the previous group's units are done with the taps and the window
-        if (!small || !in_window(k0, kn, na_tag)) {
-          if (small && kn > kFew) {
+        const int size = small ? in_window(k0, kn, na_tag) : 2;
+        if (size > 1) {
+          if (small && kn > kFew && size < 3) {
             kg = kFew;
             continue;
           }
           __syncthreads();
+          if constexpr (NA == 2) {
+            // (the others hardly fit, and six taps at a time are better off in memory than three: the map of every
+            // other pixel, samples of 8 x 32 channels of 256 x 512 -> 24 of 128 x 256, 102 us, so 83)
+            in_memory(k0, s.K - k0, na_tag);
+            return;
+          }
           in_memory(k0, kn, na_tag);
         }
         k0 += kn;

@@ -327,3 +327,21 @@ def test_accuracy_is_not_below_fp32(c, interp, shift, device):
     far = lambda y: ((y - want).norm() / want.norm()).item()
     assert torch.equal(split, fp32) == (c <= 5)
     assert far(split) <= 1.02 * far(fp32), (far(split), far(fp32))
+
+
+@pytest.mark.parametrize("f,shift", [(2, 0.0), (3, 0.0), (2, 0.4)])
+@pytest.mark.parametrize("ci,co,k", [(20, 18, 9), (9, 33, 9), (16, 17, 1), (32, 40, 1), (20, 30, 25)])
+def test_taps_whose_boxes_are_larger_than_windows(f, shift, ci, co, k, device):
+    """Maps of every second and third pixel, whose tiles' boxes are two windows and more: the rest of the
+    taps reads memory; and one tap, of one block of outputs, always does.  32-bit sums of up to 25 * 40 terms."""
+    g = torch.Generator().manual_seed(ci + k)
+    h, w_ = 150, 330
+    smap = synthetic.latitude_map(f * h, f * w_, 2)[::f, ::f, :k].contiguous()
+    smap[..., 1] = (smap[..., 1] + shift).clamp(0, f * h - 1)
+    rnd = lambda *s: torch.randn(s, generator=g)
+    x, w, b, gy = rnd(2, co, f * h, f * w_), rnd(ci, co, k), rnd(ci), rnd(2, ci, h, w_)
+    cu = lambda *ts: [t.cuda() for t in ts]
+    y = _C.mapped_conv_forward(*cu(x, smap, w, b), k, 1)
+    assert rel_err(y, O.mapped_conv_forward(x, smap, w, b, k, 1)) < 1e-5
+    gx = _C.mapped_conv_backward(*cu(gy, smap, x, w, b), k, 1, needs=(True, False, False))[0]
+    assert rel_err(gx, O.mapped_conv_backward(gy, smap, x, w, b, k, 1)[0]) < 1e-5
