@@ -1471,10 +1471,19 @@ int fill(T *p, int64_t n, T v, hipStream_t s) {
 // in two rounds of 3880 351 us, in one 299; of 180 x 360, 1012, in 2024 314, in 4048 413; of 200 x 400, 1252, in 2504 400 for
 // 509.  Maps of random taps, whose planes come from the caches, lose where more planes are read side by side: gradient of
 // average pooling, 64 planes of 249 x 498, 1940 waves 2083 us, 3880 2615; forward, 256 planes of 64 x 128 78 and 97.)
-inline int fewer_planes(int per, int64_t waves, int64_t planes, int64_t resident = 4096) {
-  while (per > 16 && waves * div_up(planes, per) < 2048 && waves * div_up(planes, per / 2) <= resident)
+// The waves then share the planes out evenly: of 17 planes a wave of sixteen takes as long as one of all, and beside it
+// stands one for the last.  (fp64, 17 planes of 137 x 275, all planes a wave, 16 and 1, nine and eight: average pooling 60,
+// 69, 50 us; max 93, 97, 79; gradients 78, 85, 77 and 128, 150, 119.  fp32, 20 planes of 200 x 400, gradients 78, 79, 75 and 115, 122,
+// 107.)  `light` (poolings from windows in fp32): nearly all is set-up, so that less than 32 planes a wave are worth no
+// more than three waves for each SIMD, and short waves hardly add to it (26 planes of 180 x 360, 1440 waves, all planes a
+// wave 24.6 us, 16 and ten 20.6, of 208 x 416, 1664 waves, 22 planes 19.5, 20.7; 20 planes of 200 x 400, all planes a wave 19, ten
+// each 21, 16 and four 18).
+inline int fewer_planes(int per, int64_t waves, int64_t planes, int64_t resident, bool light) {
+  const int whole = per;
+  while (per > 16 && waves * div_up(planes, per) < 2048 &&
+         waves * div_up(planes, per / 2) <= (light && per <= 32 ? 3072 : resident))
     per /= 2;
-  return per;
+  return per < whole && !light ? (int)div_up(planes, div_up(planes, per)) : per;
 }
 
 template <typename T, int OP>
@@ -1484,6 +1493,10 @@ int launch_gather(const void *in, const void *map, const void *iw, void *out, in
   const int64_t N = MH * MW;
   // (the same test as in direct_gather: unweighted pooling with at most 9 taps)
   const bool tap_registers = OP != OP_RESAMPLE && P == 0;
+  // (the LDS-window path copies 16-byte chunks of source rows)
+  const bool pool_windows = tap_registers && K <= 9 && N * 8 < (int64_t)kOobOffset &&
+                            IW % (16 / (int)sizeof(T)) == 0 &&
+                            (reinterpret_cast<uintptr_t>(in) & 15) == 0;
   int cpt = tap_registers ? kPoolCH : kCH;
   if (tap_registers && B * C <= 0x7fffffffLL) {
     // Images and channels are one run of planes to these kernels, and resolving a thread's
@@ -1494,7 +1507,7 @@ int launch_gather(const void *in, const void *map, const void *iw, void *out, in
     const int64_t waves = (int64_t)div_up(MW, Patch<OP>::kW) * div_up(MH, Patch<OP>::kH) *
                           (kThreads / 64);
     while (cpt < 1024 && cpt * 2 <= C && waves * div_up(C, cpt * 2) >= 8192) cpt *= 2;
-    cpt = fewer_planes(cpt, waves, C);
+    cpt = fewer_planes(cpt, waves, C, 4096, sizeof(T) == 4 && pool_windows);
   }
   // Unweighted resampling: every thread walks a run of planes with a ring of loads in flight.
   // (images and channels are one run of planes, kCH of them per thread: longer runs measured
@@ -1510,12 +1523,7 @@ int launch_gather(const void *in, const void *map, const void *iw, void *out, in
   }
   if ((C + cpt - 1) / cpt > 65535) return MCX_E_SHAPE;
   dim3 grid(div_up(MW, Patch<OP>::kW) * div_up(MH, Patch<OP>::kH), div_up(C, cpt), (unsigned)B);
-  // (the LDS-window path copies 16-byte chunks of source rows)
-  const int windows = plane_ring || (tap_registers && K <= 9 && N * 8 < (int64_t)kOobOffset &&
-                                     IW % (16 / (int)sizeof(T)) == 0 &&
-                                     (reinterpret_cast<uintptr_t>(in) & 15) == 0)
-                          ? 1
-                          : 0;
+  const int windows = plane_ring || pool_windows ? 1 : 0;
   MCX_DISPATCH_MODE(interp, hipLaunchKernelGGL((gather_kernel<T, MODE, OP>), grid, dim3(kThreads),
                                                0, s, (const T *)in, (const T *)map,
                                                (const T *)iw, (T *)out, idx, (int)C, (int)IH,
@@ -1626,8 +1634,16 @@ int gather_transposed(const void *src, const int64_t *idx, void *dst, const void
          tiles * (kThreads / 64) * ((planes + reps * 2 * kTCH - 1) / (reps * 2 * kTCH)) >= 8192)
     reps *= 2;
   int per = reps * kTCH;  // planes a workgroup
-  if (OP != UN_RESAMPLE && reps == 1)
-    per = fewer_planes(per, tiles * (kThreads / 64), planes, OP == UN_MAX ? 3072 : 4096);
+  if (OP != UN_RESAMPLE && reps == 1) {
+    const int64_t waves = tiles * (kThreads / 64);
+    // (fp64, gradient of average pooling, 17 planes of 249 x 498, 1940 waves 128 us, 3880 136; 52 planes 170, 173)
+    per = fewer_planes(per, waves, planes, OP == UN_MAX || sizeof(T) == 8 ? 3072 : 4096, false);
+    // (Three waves of max unpooling fit a SIMD.  In three parts it is faster than in two, and nowhere slower than undivided: fp64, 17
+    // planes of 180 x 360 137 us in one and in three, 144 in two; of 137 x 275 128, 109, 119; 128 of 180 x 360, of 64 each, 538, in
+    // three 445; fp32 247, 221, in four 205, but fractional rows, 64 planes, 486, in two 314, in four 413.)
+    if (OP == UN_MAX && div_up(planes, per) == 2 && waves * 3 <= 3072)
+      per = div_up(planes, 3);
+  }
   const int64_t groups = (planes + per - 1) / per;
   const int64_t blocks = groups * tiles;
   if (blocks > 0x7fffffffLL) return kNotApplicable;

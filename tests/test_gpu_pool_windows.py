@@ -222,6 +222,18 @@ def test_planes_are_spread_over_idle_simds(planes, W, fractional, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("planes", [17, 20, 33, 47, 67])
+@pytest.mark.parametrize("H,W", [(40, 129), (136, 272), (180, 361)])
+def test_planes_are_shared_out_evenly(H, W, planes, dtype, device):
+    """Plane counts that are no multiple of a thread's, on grids of one wave for ten SIMDs to one for each:
+    two, three and more parts of nine planes and more."""
+    g = torch.Generator().manual_seed(planes + W)
+    smap = synthetic.latitude_map(H, W, 1).to(dtype)
+    _check(torch.randn(1, planes, H, W, generator=g, dtype=dtype), smap, 9, 1)
+    _check_unpool(torch.randn(1, planes, H, W, generator=g, dtype=dtype), smap, H, W, 9, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("long", [1, 2, 3, 8, 16, 17, 31, 32, 33, 48, 64, 65, 130])
 @pytest.mark.parametrize("pattern", ["all", "one", "mixed"])
 def test_lists_are_sorted_by_source(dtype, long, pattern, device):
