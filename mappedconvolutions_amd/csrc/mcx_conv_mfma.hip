@@ -881,8 +881,9 @@ __global__ __launch_bounds__(kThreads, OG == 1 ? 4 : 3) void gather_product_mfma
 // the leading entries of a tap that are read (2 or 4), by the masks of the map (pair_mask / row_mask).
 constexpr int kDgPx = 256;
 
-// Q: pixels a lane, of which a workgroup has 128 * Q.  Two of them share a fetch of the weights, one leaves
-// registers for four waves a SIMD and fills the chip with half the pixels; over 64 outputs, whose
+// Q: pixels a lane, of which a workgroup has 128 * Q.  Two of them share a fetch of the weights, one
+// fills the chip with half the pixels and over 64 outputs (127 registers, 41 KB of LDS) leaves room for three waves a
+// SIMD where two (and 128 outputs, 246 and 248 registers) leave it for two; over 64 outputs, whose
 // weights are few, one is the better form (forward and input gradient, us, of two pixels and of one:
 // 4 x 32 -> 64 channels of 64 x 128 16 + 31, 11 + 18; 16 x 32 -> 64 22 + 41, 22 + 37; 8 x 64 -> 64 of 256 x 512, four
 // corners, 312 + 302, 284 + 278; 5 x 5 508 + 519, 476 + 485; 128 -> 64 349, 355).  Over 128 it is where two make no
@@ -1166,50 +1167,88 @@ __device__ inline void gather_product_bf16_direct(
 #pragma unroll
       for (int q = 0; q < Q; q++) {
         f32x4 more = at;
-        // (with two pixels a lane most outputs are there, and the test costs 2 % of 8 x 128 -> 128 of 256 x 512)
-        if (add && (Q == 2 || o0 + 32 * m + 8 * g < O) && n0 + px[q] < N)
+        if (Q == 1 && add && o0 + 32 * m + 8 * g < O && n0 + px[q] < N)
           more += *reinterpret_cast<const f32x4 *>(
               addend + ((int64_t)b * N + n0 + px[q]) * Opad + o0 + o);
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[m][q][4 * g + i] += more[i];
       }
     }
+  if (Q == 2 && add) {
+    // (With two pixels a lane most outputs are there: a test for it costs 2 % of 8 x 128 -> 128 of 256 x 512.  The sums
+    // of 32 outputs are read at a time: all of them spill.)
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      if (n0 + px[q] < N) {
+        const float *ab = addend + ((int64_t)b * N + n0 + px[q]) * Opad + o0 + lhi * 4;
+#pragma unroll
+        for (int m = 0; m < 2 * OG; m++) {
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const f32x4 more = *reinterpret_cast<const f32x4 *>(ab + 32 * m + 8 * g);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[m][q][4 * g + i] += more[i];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+  }
   const bool pack2 = (N & 1) == 0 && (reinterpret_cast<uintptr_t>(y) & 3) == 0;
-  const bool odd = (l31 & 1) != 0, whole = o0 + kOT * OG <= O;  // (every output of the workgroup)
+  const bool odd = (l31 & 1) != 0;
+  const int left = O - o0 - lhi * 4;  // outputs from the lane's first on
+  // outputs oa (at `at`) and the next one of a pixel; `all`: both are there
+  auto put = [&](char *at, int64_t row, int oa, float va, float vb, bool all) __attribute__((always_inline)) {
+    if (pack2) {
+      const float send = odd ? va : vb;
+      const float recv = __builtin_bit_cast(
+          float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, send), 0xB1, 0xf, 0xf,
+                                          true));  // quad_perm [1, 0, 3, 2]
+      const unsigned two = __builtin_bit_cast(
+          unsigned, __builtin_convertvector(floatx2{odd ? recv : va, odd ? vb : recv}, bf16x2));
+      if (all || (odd ? oa + 1 : oa) < left) *reinterpret_cast<unsigned *>(at) = two;
+    } else {
+      if (all || oa < left) *reinterpret_cast<bf16_t *>(at) = from_f32<bf16_t>(va);
+      if (all || oa + 1 < left) *reinterpret_cast<bf16_t *>(at + row) = from_f32<bf16_t>(vb);
+    }
+  };
 #pragma unroll
   for (int q = 0; q < Q; q++) {
     const int n = n0 + px[q];
     if (n >= N) continue;
     bf16_t *yb = y + ((int64_t)b * O + o0 + lhi * 4) * N + n;
-    auto store = [&](auto whole_tag) __attribute__((always_inline)) {
-      constexpr bool WHOLE = decltype(whole_tag)::value;
+    if constexpr (Q == 2) {
+      // One address, stepped from output to output: as multiples of the plane they are 64 scalar pairs, and with the
+      // sums above 72 vector registers and 500 scalar ones spilled, none now (us, then and now: 8 x 126 -> 7 channels of 446 x
+      // 892, input gradient 784, 625; 8 x 128 -> 128 of 256 x 512, nine taps, 551 + 582, 512 + 543; 8 x 16 -> 128, one tap, 135,
+      // 102; 4 x 128 -> 128 of 512 x 1024, 5 x 5, 2421 + 2551, 2370 + 2494).  One pixel's fit, and stepped its loop before
+      // comes out the slower one (8 x 64 -> 64 of 256 x 512, four corners, 330, stepped 352).
+      const int64_t row = (int64_t)N * 2;
+      char *at = reinterpret_cast<char *>(yb);
+      if (pack2 && odd) at += row - 2;
 #pragma unroll
       for (int m = 0; m < 2 * OG; m++)
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-          const int oa = 32 * m + (t >> 1) * 8 + (t & 1) * 2, ob = oa + 1;  // (from yb's on)
-          const int left = O - o0 - lhi * 4;
-          const float va = acc[m][q][2 * t], vb = acc[m][q][2 * t + 1];
-          if (pack2) {
-            const float send = odd ? va : vb;
-            const float recv = __builtin_bit_cast(
-                float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, send), 0xB1, 0xf, 0xf,
-                                                true));  // quad_perm [1, 0, 3, 2]
-            const unsigned two = __builtin_bit_cast(
-                unsigned,
-                __builtin_convertvector(floatx2{odd ? recv : va, odd ? vb : recv}, bf16x2));
-            if (WHOLE || (odd ? ob : oa) < left)
-              *reinterpret_cast<unsigned *>(yb + (int64_t)oa * N + (odd ? N - 1 : 0)) = two;
-          } else {
-            if (WHOLE || oa < left) yb[(int64_t)oa * N] = from_f32<bf16_t>(va);
-            if (WHOLE || ob < left) yb[(int64_t)ob * N] = from_f32<bf16_t>(vb);
-          }
+          put(at, row, 32 * m + (t >> 1) * 8 + (t & 1) * 2, acc[m][q][2 * t], acc[m][q][2 * t + 1], false);
+          at += row * (t & 1 ? 6 : 2);
+          asm volatile("" : "+v"(at));  // (no multiple of the plane to the compiler)
         }
-    };
-    if (whole)
-      store(std::true_type());
-    else
-      store(std::false_type());
+    } else {
+      auto store = [&](auto all_tag) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < 2 * OG; m++)
+#pragma unroll
+          for (int t = 0; t < 8; t++) {
+            const int oa = 32 * m + (t >> 1) * 8 + (t & 1) * 2;
+            put(reinterpret_cast<char *>(yb + (int64_t)oa * N + (pack2 && odd ? N - 1 : 0)), (int64_t)N * 2, oa,
+                acc[m][q][2 * t], acc[m][q][2 * t + 1], decltype(all_tag)::value);
+          }
+      };
+      if (o0 + kOT * OG <= O)
+        store(std::true_type());
+      else
+        store(std::false_type());
+    }
   }
 }
 

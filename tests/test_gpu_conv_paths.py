@@ -439,6 +439,38 @@ def test_bf16_direct_products_over_tiles_of_128_pixels(shape, taps, row_shift, d
     assert rel_err(_C.mapped_conv_backward(gyd, sd, xd, wd_, bd, taps, 1)[0].float(), gx_o) < 2e-2
 
 
+@pytest.mark.parametrize("overflow", [False, True])
+@pytest.mark.parametrize("row_shift", [0.0, 0.37])
+@pytest.mark.parametrize("taps", [1, 5, 14])
+@pytest.mark.parametrize("shape", [(5, 24, 100, 109, 123), (3, 200, 20, 109, 124), (5, 72, 128, 109, 123),
+                                   (9, 128, 65, 80, 93)])
+def test_bf16_direct_products_over_tiles_of_256_pixels(shape, taps, row_shift, overflow, device):
+    """More than 256 workgroups of 256 pixels and 128 outputs (forward, input gradient or both): odd
+    and even pixel counts with ragged last tiles, outputs that fill a workgroup and that do not,
+    taps within and beyond a resolved group (13 of two entries, four of four), and a map that has 60 pixels
+    read one place, which leaves an overflow list.  Against the fp32 kernels over the same values."""
+    B, Ci, Co, H, W = shape
+    g = torch.Generator().manual_seed(taps + Ci)
+    bf = lambda t: t.to(torch.bfloat16)
+    x, gy = bf(torch.randn(B, Ci, H, W, generator=g)), bf(torch.randn(B, Co, H, W, generator=g))
+    w = bf(torch.randn(Co, Ci, taps, generator=g) / (Ci * taps) ** 0.5)
+    b = bf(torch.randn(Co, generator=g))
+    smap = synthetic.latitude_map(H, W, 2)[:, :, :taps].contiguous()
+    smap[..., 1] = (smap[..., 1] + row_shift).clamp(0, H - 1)
+    if overflow:
+        smap[H // 2, 10:70, 0] = torch.tensor([20.5, 30.25])
+    xd, sd, wd_, bd, gyd = dev(x, smap, w, b, gy)
+    y_f = _C.mapped_conv_forward(xd.float(), sd, wd_.float(), bd.float(), taps, 1)
+    gx_f = _C.mapped_conv_backward(gyd.float(), sd, xd.float(), wd_.float(), bd.float(), taps, 1)[0]
+    # samples and interpolation weights rounded to 2^-9 each, the result once: as in the tests around
+    y = _C.mapped_conv_forward(xd, sd, wd_, bd, taps, 1).float()
+    assert rel_err(y, y_f) < 2e-2
+    assert_close_elementwise(y, y_f, TOL[torch.bfloat16])
+    gx = _C.mapped_conv_backward(gyd, sd, xd, wd_, bd, taps, 1)[0].float()
+    assert rel_err(gx, gx_f) < 2e-2
+    assert_close_elementwise(gx, gx_f, TOL[torch.bfloat16])
+
+
 @pytest.mark.parametrize("row_shift", [0.0, 0.5])
 @pytest.mark.parametrize("shape", [(1, 3, 5, 6, 16), (2, 1, 2, 3, 8), (1, 9, 17, 5, 264)])
 def test_bf16_backward_with_very_few_channels(shape, row_shift, device):
