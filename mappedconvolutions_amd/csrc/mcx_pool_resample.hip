@@ -962,7 +962,9 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) void sort_entries
   __shared__ __attribute__((aligned(16))) T run_wt[kThreads / 64][kRun];
   const int wv = threadIdx.x >> 6;
   if (longest <= 64u) {
-    const bool few = longest <= (uint32_t)kNetN &&
+    // (a single longer one would be inserted by its lane alone, in some n * n / 2 steps through LDS: 5 x 5 nearest taps at every second
+    // pixel of 86 x 172, lists of up to 32 at the poles, gradient of 82 fp64 planes 102 us, with the network 75)
+    const bool few = longest <= 16u &&
                      __builtin_popcountll(__builtin_amdgcn_ballot_w64(len > few_entries<T>())) < 32;
     const int lane = threadIdx.x & 63;
     const int lanes = longest <= 16u ? 64 : longest <= 32u ? 32 : 16;
