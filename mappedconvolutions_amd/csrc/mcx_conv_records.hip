@@ -337,11 +337,13 @@ __global__ __launch_bounds__(kThreads) void scatter_records_kernel(
 // part[range][k][a][g] = sum over a range of (b, n) of plain[b,a,n] * sample(gath[b,g], map[n,k]).
 // A workgroup takes AT plain channels, 2 * LPR gathered ones and KT taps.  A tile is one run of kLocs
 // locations; for one tap it is kSub, whose record reads are in flight together.
-// KT is grad_taps<LPR, AT>(), as many as a lane has registers for the sums of, where there are locations
-// enough (grad_shape): the taps of a location are one piece of the map, and one by one each workgroup reads the
-// lines of all of them.
-template <int LPR, int AT>
-constexpr int grad_taps() { return AT == 1 ? RecShape<LPR>::kTaps : AT == 4 ? 3 : 1; }
+// KT is 1, or kGradTaps over up to four plain channels where there are taps and locations enough (grad_shape): the
+// taps of a location are one piece of the map, and one by one each workgroup reads the lines of all of them;
+// neighbouring taps often meet each other's records too.  Three, not as many as a lane has registers for the sums of:
+// with nine, two waves a SIMD instead of four, coherent maps were slower than tap by tap (whole weight gradient, 10 -> 1 channels,
+// nine taps, us, tap by tap, three and nine: 100 000 locations, shuffled pixels 70, 47, 60, coherent 43, 42, 58; 300 000 240, 117,
+// 132 and 131, 95, 125).
+constexpr int kGradTaps = 3;
 template <int NC, int LPR, int AT, int KT>
 __global__ __launch_bounds__(kThreads) void weight_grad_records_kernel(
     const double *__restrict__ plain, const double *__restrict__ rec,
@@ -399,39 +401,34 @@ __global__ __launch_bounds__(kThreads) void weight_grad_records_kernel(
       }
       __syncthreads();
       if (live) {
-        // units: the taps of a location, or one tap's locations; kRun of them are in flight
-        constexpr int kUnits = KT > 1 ? KT : kSub, kRun = KT > 1 ? (KT % 3 == 0 ? 3 : KT) : kSub;
+        // units, whose records are in flight together: the taps of a location, or one tap's locations
+        constexpr int kUnits = KT > 1 ? KT : kSub;
+        double2 d[kUnits][NC];
 #pragma unroll
-        for (int u0 = 0; u0 < kUnits; u0 += kRun) {
-          if (KT > 1 && u0 >= taps) break;
-          double2 d[kRun][NC];
+        for (int u = 0; u < kUnits; u++) {
+          // (past the last tap it is read again and not used)
+          const int v = KT > 1 ? min(u, taps - 1) : u;
 #pragma unroll
-          for (int q = 0; q < kRun; q++) {
-            // (past the last tap it is read again and not used)
-            const int u = KT > 1 ? min(u0 + q, taps - 1) : u0 + q;
+          for (int i = 0; i < NC; i++)
+            d[u][i] = *reinterpret_cast<const double2 *>(
+                src + (int64_t)s_off[i * kSlots + v * S::kLocs + loc] * stride);
+        }
 #pragma unroll
-            for (int i = 0; i < NC; i++)
-              d[q][i] = *reinterpret_cast<const double2 *>(
-                  src + (int64_t)s_off[i * kSlots + u * S::kLocs + loc] * stride);
+        for (int u = 0; u < kUnits; u++) {
+          if (KT > 1 && u >= taps) break;
+          double vx = 0.0, vy = 0.0;
+#pragma unroll
+          for (int i = 0; i < NC; i++) {
+            const double f = s_wt[i * kSlots + u * S::kLocs + loc];
+            vx = mcx_fma(f, d[u][i].x, vx);
+            vy = mcx_fma(f, d[u][i].y, vy);
           }
 #pragma unroll
-          for (int q = 0; q < kRun; q++) {
-            const int u = u0 + q;
-            if (KT > 1 && u >= taps) break;
-            double vx = 0.0, vy = 0.0;
-#pragma unroll
-            for (int i = 0; i < NC; i++) {
-              const double f = s_wt[i * kSlots + u * S::kLocs + loc];
-              vx = mcx_fma(f, d[q][i].x, vx);
-              vy = mcx_fma(f, d[q][i].y, vy);
-            }
-#pragma unroll
-            for (int a = 0; a < AT; a++) {
-              const double g = s_plain[a * kTile + (KT > 1 ? 0 : u * S::kLocs) + loc];
-              double2 &sum = acc[KT > 1 ? u : 0][a];
-              sum.x = mcx_fma(g, vx, sum.x);
-              sum.y = mcx_fma(g, vy, sum.y);
-            }
+          for (int a = 0; a < AT; a++) {
+            const double g = s_plain[a * kTile + (KT > 1 ? 0 : u * S::kLocs) + loc];
+            double2 &sum = acc[KT > 1 ? u : 0][a];
+            sum.x = mcx_fma(g, vx, sum.x);
+            sum.y = mcx_fma(g, vy, sum.y);
           }
         }
       }
@@ -576,7 +573,7 @@ __global__ __launch_bounds__(kThreads) void product_planes_kernel(
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Tiles, ranges and channel blocks of the weight gradient: about 2048 workgroups, eight per CU; of several
-// taps, whose registers leave room for two or three, 1024 or 768.
+// taps, whose registers leave room for four or three, 1024 or 768.
 struct GradShape {
   int lpr, at, taps;
   int64_t tiles_per_img, total, ranges, ablocks, gblocks, kgroups;
@@ -587,18 +584,19 @@ GradShape grad_shape(int64_t B, int64_t A, int64_t G, int64_t N, int64_t K) {
   q.at = A == 1 ? 1 : A <= 4 ? 4 : 16;
   q.ablocks = (A + q.at - 1) / q.at;
   q.gblocks = (read_stride(G) + 2 * q.lpr - 1) / (2 * q.lpr);
-  // Several taps a workgroup where eight taps and more fill eight ninths of the workgroups' and there are locations
-  // enough: with fewer of either, workgroups of one tap are more and have the loads of four locations in flight
-  // (whole weight gradients, us, one tap and several.  Coherent maps, nine taps: 10 -> 1 channels, 100 000 locations 41,
-  // 56; 150 000 62, 69; 200 000 85, 88; 250 000 105, 103; 2 -> 1 100 000 27, 30; 130 000 33, 31; 4 -> 2 50 000 23, 24; 66 000
-  // 27, 26; 10 -> 4 66 000 37, 37; ten taps 100 000 46, 55; 25 taps 66 000 64, 73; 150 000 145, 145.  Shuffled maps gain
-  // earlier: 10 -> 1 100 000 71, 70; 130 000 95, 84; 4 -> 2 66 000 33, 30.  Taps, shuffled, 300 000 locations: 10 -> 1,
-  // groups of nine, one 55, 69; four 114, 114; five 137, 130, coherent 72, 86; ten 261, 292; eleven 281, 302; 18 451, 378;
-  // 2 -> 1, groups of five, five 61, 62; six 76, 89; seven 88, 90; nine 112, 92.  Four waves a SIMD spill: twice as slow.)
-  const int64_t many = q.at == 1 ? (q.lpr == 2 ? RecShape<2>::kTaps : RecShape<8>::kTaps) : q.at == 4 ? 3 : 1;
-  const int64_t enough = q.at == 1 ? (q.lpr == 2 ? 1 << 17 : 3 << 16) : K > 9 ? 1 << 17 : 1 << 16;
-  const bool filled = K >= 8 && K * 9 >= (K + many - 1) / many * many * 8;
-  const int64_t taps = filled && B * N >= enough ? many : 1;
+  // Several taps a workgroup where there are taps and locations enough and the taps fill eight ninths of the
+  // workgroups': with fewer, workgroups of one tap are more and have the loads of four locations in flight (whole weight gradients,
+  // us, one tap and three, shuffled and coherent maps.  10 -> 1 channels, 67 000 locations, six taps 35, 31 and 28, 28; seven 40,
+  // 35 and 30, 33; eight 47, 36 and 33, 33; nine 47, 37 and 33, 33; ten 47, 41 and 35, 36; 25 98, 67 and 61, 60; 49 500, nine 35, 30 and
+  // 27, 28; 100 000, four 41, 38 and 29, 34; five 41, 38 and 31, 34; six 51, 38 and 36, 35.  From 196 608 locations on five taps are
+  // enough: 300 000, four 115, 86 and 68, 73; five 140, 87 and 77, 72; ten 263, 144 and 133, 115.  2 -> 1, 67 000, six 21, 21 and 18,
+  // 18; nine 27, 22 and 23, 19.  Two to four plain channels, whose sums take the registers of a wave, nine coherent taps:
+  // 4 -> 2 50 000 23, 24; 66 000 27, 26; 10 -> 4 66 000 37, 37; ten taps 100 000 46, 55; 25 66 000 64, 73; 150 000 145, 145.)
+  const bool filled = K * 9 >= (K + kGradTaps - 1) / kGradTaps * kGradTaps * 8;
+  const bool several = q.at == 1   ? (filled && K >= 6 && B * N >= 1 << 16) || (K >= 5 && B * N >= 3 << 16)
+                       : q.at == 4 ? filled && K >= 8 && B * N >= (K > 9 ? 1 << 17 : 1 << 16)
+                                   : false;
+  const int64_t taps = several ? kGradTaps : 1;
   q.taps = (int)taps;
   const int64_t tile = (taps > 1 ? 1 : q.lpr == 2 ? 2 : 4) * (kThreads / q.lpr);
   q.tiles_per_img = (N + tile - 1) / tile;
@@ -855,7 +853,7 @@ int records_weight_grad(const double *plain, const double *gath, const double *m
                      wraps(interp) ? 1 : 0, (int)q.tiles_per_img, q.total, (int)q.ranges);
 #define MCX_RUN(NC, LPR, AT)                                          \
   if (q.taps == 1) { MCX_RUN_TAPS(NC, LPR, AT, 1) }                   \
-  else { MCX_RUN_TAPS(NC, LPR, AT, (grad_taps<LPR, AT>())) }
+  else { MCX_RUN_TAPS(NC, LPR, AT, (AT <= 4 ? kGradTaps : 1)) }
 #define MCX_AT(NC, LPR)                             \
   if (q.at == 1) { MCX_RUN(NC, LPR, 1) }            \
   else if (q.at == 4) { MCX_RUN(NC, LPR, 4) }       \

@@ -333,9 +333,12 @@ def test_weight_gradient_of_several_taps_a_workgroup(ci, co, k, p, interp, few, 
 
 
 @pytest.mark.parametrize("ci,co,k,locations", [
-    # one output: 196 608 locations, groups of nine taps; up to four channels 131 072, groups of five
+    # one output
     (10, 1, 9, 196607), (10, 1, 9, 196608), (6, 1, 8, 196608), (10, 1, 7, 196608), (16, 1, 17, 196608),
     (10, 1, 10, 196608), (3, 1, 5, 131072), (3, 1, 9, 131071), (3, 1, 9, 131072), (4, 1, 14, 131074),
+    # groups of three taps, filled and not, on either side of 65 536 and 196 608
+    (10, 1, 6, 65535), (10, 1, 6, 65536), (3, 1, 8, 65537), (2, 1, 7, 65539), (2, 1, 5, 196611), (12, 1, 10, 196608),
+    (16, 1, 4, 196609), (1, 1, 25, 65536),
     # two to four: 65 536 locations, with more than nine taps 131 072, groups of three
     (4, 2, 8, 65535), (4, 2, 8, 65536), (4, 2, 7, 65536), (10, 4, 9, 65539),
     (5, 3, 17, 131071), (5, 3, 17, 131072), (5, 3, 25, 131073)])
