@@ -116,7 +116,7 @@ __device__ inline void split_bias(const SplitArgs &s, float *lds, int o0) {
 // Bias, addend and stores of a lane's pixel; flags a tile with a result that is not finite.  (No
 // load after the first store: a wait for it would be one for the stores before it as well, 500 clocks an
 // output, a quarter of the kernel's time at nine taps of 64 channels.)
-template <int NB>
+template <int NB, int AT_ONCE>
 __device__ inline void split_epilogue(const SplitArgs &s, floatx16 *acc, const float *bias, int tile,
                                       int b, int o0, int ei, int ej, int lhi) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -135,15 +135,32 @@ __device__ inline void split_epilogue(const SplitArgs &s, floatx16 *acc, const f
       }
     if (s.addend && s.gate && s.gate[1] > 0) {
       const float *ab = s.addend + ((int64_t)b * N + n) * s.Opad + o0 + lhi * 4;
+      auto add4 = [&](int m, int g, f32x4 v) __attribute__((always_inline)) {
 #pragma unroll
-      for (int m = 0; m < NB; m++)
+        for (int i = 0; i < 4; i++) acc[m][4 * g + i] += v[i];
+      };
+      // (Those of outputs that there are.  Of AT_ONCE blocks they are read before the first is used: 4 x 64 -> 128 channels over
+      // 40 962 vertices, input gradient 649 us with the test before each use, so 645; of more blocks, they spill.)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          if (o0 + 32 * m + 8 * g >= s.O) continue;  // (no such outputs)
-          const f32x4 add = *reinterpret_cast<const f32x4 *>(ab + 32 * m + 8 * g);
+      for (int m0 = 0; m0 < NB; m0 += AT_ONCE) {
+        f32x4 more[AT_ONCE][4];
 #pragma unroll
-          for (int i = 0; i < 4; i++) acc[m][4 * g + i] += add[i];
+        for (int m = m0; m < m0 + AT_ONCE && m < NB; m++)
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            if (o0 + 32 * m + 8 * g < s.O) {
+              more[m - m0][g] = *reinterpret_cast<const f32x4 *>(ab + 32 * m + 8 * g);
+              if constexpr (AT_ONCE == 1) add4(m, g, more[0][g]);
+            }
+        if constexpr (AT_ONCE > 1) {
+#pragma unroll
+          for (int m = m0; m < m0 + AT_ONCE && m < NB; m++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+              if (o0 + 32 * m + 8 * g < s.O) add4(m, g, more[m - m0][g]);
+          if (NB > AT_ONCE) __builtin_amdgcn_sched_barrier(0);
         }
+      }
     }
     if (o0 + 32 * NB <= s.O) {
 #pragma unroll
@@ -463,13 +480,14 @@ gather_product_split_kernel(const SplitArgs s) {
   };
 
   // ---- a group in memory ----
-  // (Arrays of their own where there is no window to share the memory with: the compiler then moves reads of one past
-  // writes of the other.  Input gradient of 3 x 139 -> 61 channels of 44 x 88, four entries, 78 us in one, 73; 1 x 40 -> 100
-  // of 60 x 120, 5 x 5, 210 and 195.)
-  __shared__ __attribute__((aligned(16))) unsigned OwnOff[WINDOW ? 1 : kMemCache * kTilePx];
-  __shared__ __attribute__((aligned(16))) float OwnWt[WINDOW ? 1 : kMemCache * kTilePx];
-  unsigned *const TapOff = WINDOW ? reinterpret_cast<unsigned *>(TapMem) : OwnOff;
-  float *const TapWt = WINDOW ? reinterpret_cast<float *>(TapMem + kMemCache * kTilePx * 4) : OwnWt;
+  // (Arrays of their own where four entries have no window to share the memory with: the compiler then moves reads of one
+  // past writes of the other.  Input gradient of 3 x 139 -> 61 channels of 44 x 88 78 us in one, 73; 1 x 40 -> 100 of 60 x 120,
+  // 5 x 5, 210 and 195.)
+  constexpr bool kOwn = !WINDOW && NE == 4;
+  __shared__ __attribute__((aligned(16))) unsigned OwnOff[kOwn ? kMemCache * kTilePx : 1];
+  __shared__ __attribute__((aligned(16))) float OwnWt[kOwn ? kMemCache * kTilePx : 1];
+  unsigned *const TapOff = kOwn ? OwnOff : reinterpret_cast<unsigned *>(TapMem);
+  float *const TapWt = kOwn ? OwnWt : reinterpret_cast<float *>(TapMem + kMemCache * kTilePx * 4);
   // its units: chunk-major, the tap fastest (a chunk's source rows stay in cache)
   auto units_of = [&](int k0, int kn, auto na_tag, auto paired_tag) __attribute__((always_inline)) {
     constexpr int NA = decltype(na_tag)::value;
@@ -679,7 +697,7 @@ gather_product_split_kernel(const SplitArgs s) {
     run(std::integral_constant<int, NE == 4 ? 2 : 1>());
   else
     run(std::integral_constant<int, NE>());
-  split_epilogue<NB>(s, acc, Bias, tile, b, o0, tile_y * th + (pe >> s.tw_shift),
+  split_epilogue<NB, (NE == 4 && NB > 1 ? 2 : 1)>(s, acc, Bias, tile, b, o0, tile_y * th + (pe >> s.tw_shift),
                      (tile_x << s.tw_shift) + (pe & tw_mask), lhi);
 }
 
@@ -864,7 +882,7 @@ __global__ __launch_bounds__(kThreads, TWO || NE * NB > 8 ? 2 : 3) void gather_p
     split_products<NB>(a, bq, acc);
     buf ^= 1;
   }
-  split_epilogue<NB>(s, acc, Bias, tile, b, o0, ei, ej, lhi);
+  split_epilogue<NB, (NE == 4 && NB > 1 ? 2 : 1)>(s, acc, Bias, tile, b, o0, ei, ej, lhi);
 }
 
 }  // namespace
