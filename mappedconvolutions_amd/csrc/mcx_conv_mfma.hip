@@ -1154,8 +1154,8 @@ __device__ inline void gather_product_bf16_direct(
   // even lane stores two pixels of the even channel in one 32-bit word and the odd lane two
   // pixels of the odd channel (half the store instructions of 2-byte stores).
   // (No load after the first store: a wait for it would be one for the stores before it as well.  With the
-  // biases read between them 16 x 128 -> 128 channels of 512 x 1024, 5 x 5, took 17.7 ms for the two products,
-  // now 17.0; 4 x 32 -> 64 of 64 x 128, 3 x 3, 52 us, now 45.)
+  // biases read between them 16 x 128 -> 128 channels of 512 x 1024, 5 x 5, took 17.7 ms for the two products, then
+  // 17.0; 4 x 32 -> 64 of 64 x 128, 3 x 3, 52 us, now 45.)
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   const bool add = addend && gate && gate[1] > 0;
 #pragma unroll
@@ -1418,7 +1418,7 @@ __global__ __launch_bounds__(kThreads, NP * NCORN <= 4 ? 3 : 2) void weight_grad
   // goes to range t % ranges).  40 962 vertices, 4 x 64 -> 128 channels, seven taps of four random points: an
   // image's records are 10.5 MB and the kernel was bound by L2 misses, 2.5 GB of them at 5.7 TB/s, as many as
   // the gather reads; now 1.25 GB, and 338 us for 443 (with the taps read side by side, see below, and the accumulators
-  // of seven taps, with which 14 registers spill and not 36).  Whole weight gradients, before and now: one of these images
+  // of seven taps, with which 16 registers spill and not 32).  Whole weight gradients, before and now: one of these images
   // 167 -> 127, bf16 130 -> 100; two of 20 000 vertices, 128 -> 128 channels, nine taps 366 -> 211, bf16 220 -> 142;
   // a real mesh kernel of three points, 4 x 64 -> 128 322 -> 287, bf16 256 -> 214.
   const bool spread = chunked && groups_by_xcd(ranges, cgroups);
@@ -3317,8 +3317,8 @@ int mfma_weight_grad(const TD *plain, const TD *gath, const float *map, const fl
                      t.tw_shift, (int)t.total, ranges, cgroups,                                  \
                      plain_sum ? sum_part : (float *)nullptr, MASK, LEAD, runs_state, tap_table, \
                      in_chunks ? 1 : 0)
-// (a pass of seven taps, those of a mesh vertex and its neighbours, spills 14 registers at four points where one
-// of nine spills 40: a pass of nine for the kernel of seven taps 402 us, of seven 391)
+// (a pass of seven taps, those of a mesh vertex and its neighbours, spills 16 registers at four points where one
+// of nine spills 32: a pass of nine for the kernel of seven taps 402 us, of seven 391)
 #define MCX_LAUNCH_NA(NCORN, NP, CL, NA, MASK, LEAD)                           \
   if constexpr (CL && sizeof(TD) == 4 && NA > 1) {                            \
     if (K <= kWgKTMesh) {                                                     \

@@ -139,6 +139,7 @@ def test_recorded_traffic_goes_stale_with_any_kernel_source(tmp_path, monkeypatc
     import bench_traffic_summary as summary
     lines = summary.source_lines()
     assert any("mcx_conv_split.h" in line for line in lines)
+    assert any(line.endswith("mcx_conv_split.hip") for line in lines)
     traffic = '@traffic label=conv_forward kernel="k" read_bytes=3 written_bytes=4'
     profile = tmp_path / "traffic.txt"
     monkeypatch.setattr(bench, "TRAFFIC_PROFILE", str(profile))
